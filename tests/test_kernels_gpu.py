@@ -1140,6 +1140,25 @@ def test_log_mel_against_the_oracle(pkg, oracle, gpu, n, n_mel):
     assert oracle.nmse(got, want) <= 1e-8
 
 
+@pytest.mark.parametrize("n", [160 * 22 - 200, 160 * 23 - 200, 160 * 24 - 200, 160 * 47 + 1, 160 * 24 * 769])
+def test_log_mel_rounds_and_filter_ranges(pkg, oracle, gpu, n):
+    # frame counts around whole rounds of 24 and beyond one round per workgroup; a bank that is no set of triangles: dense bands,
+    # one of a single bin at either end, one without a nonzero weight (log10(1e-10) in every frame)
+    f = np.abs(rnd((6, 201))) * 0.02
+    f[1, 1:] = 0; f[2, :200] = 0; f[3] = 0; f[4, 70:130] = 0
+    s = mel_test_signal(n, n)
+    got = run_log_mel(pkg, gpu, s, f)
+    if n > 1 << 20:                                         # keep the oracle to a second: the head, up to where the cut begins to show
+        short = mel_test_signal(n, n)[:64000]
+        want, got = oracle.log_mel_spectrogram(short, f)[:, :390], got[:, :390]
+        assert want.max() <= got.max() + 1e-4               # (a louder tail raises the floor; compare above both)
+        floor = max(want.min(), got.min()) + 1e-3
+        want, got = np.maximum(want, floor), np.maximum(got, floor)
+    else:
+        want = oracle.log_mel_spectrogram(s, f)
+    assert np.max(np.abs(got - want)) <= 1e-4
+
+
 def test_log_mel_golden_vectors(pkg, gpu):
     from test_golden import mel_cases
     for _, samples, filters, want in mel_cases():
