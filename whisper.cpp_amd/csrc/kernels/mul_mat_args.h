@@ -3,6 +3,8 @@
 
 #include "common.h"
 
+typedef uint32_t __attribute__((aligned(2))) u32a2;
+struct __attribute__((packed, aligned(2))) u128a2 { uint32_t x, y, z, w; };
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef int      v4i_t __attribute__((ext_vector_type(4)));
 
@@ -24,3 +26,24 @@ struct mm_args {
     int64_t ne12, ne13, r2, r3;      // batch dims of src1/dst and broadcast ratios of src0
     epi_args e;
 };
+
+// one product of a grouped launch
+#define MM_GROUP_MAX 64
+struct mm_group_entry { const char * w; char * d; const float * bias; const char * residual; int64_t d_nb1; int flags; float scale; };
+struct mm_group { mm_group_entry e[MM_GROUP_MAX]; };
+
+#ifdef __HIPCC__
+// four bits -> bit 4 of four bytes
+__device__ __forceinline__ uint32_t spread4_to_bit4(uint32_t nib) {
+    return ((nib * 0x00204081u) & 0x01010101u) << 4;
+}
+// epilogue of one value
+__device__ __forceinline__ float apply_epilogue(float v, const epi_args & e, int64_t m, int64_t n, int64_t res_off) {
+    if (e.flags & MI355X_EPI_BIAS)     v += e.bias[m];
+    if (e.flags & MI355X_EPI_BIAS_COL) v += e.bias[n];
+    if (e.flags & MI355X_EPI_GELU)     v  = gelu_f32(v, e.gelu);
+    if (e.flags & MI355X_EPI_SCALE)    v *= e.scale;
+    if (e.flags & MI355X_EPI_RESIDUAL) v += *(const float *)(e.residual + res_off);
+    return v;
+}
+#endif
