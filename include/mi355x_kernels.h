@@ -149,7 +149,8 @@ MI355X_API int    mi355x_mul_mat_noalloc(const mi355x_tensor * src0, const mi355
 
 /* Several MUL_MATs over the same src1 in one launch (a layer's Q, K and V projections; the cross-attention K and V of all
  * decoder layers): the same arithmetic as `count` calls of mi355x_mul_mat, item by item, but one grid that fills the
- * device where a single 1280-row product covers half of it.  No counterpart in the reference, whose graphs issue these
+ * device where a single 1280-row product covers half of it (which may be a grid of larger tiles than the single product's,
+ * with the f32 sums of a result in another order).  No counterpart in the reference, whose graphs issue these
  * products one node at a time.  Only the shape this exists for: every src0 a dense 2-d F16 matrix of the same size (e.g.
  * the f16 images of quantized weights, with MI355X_MM_ACT_Q8_0 in `flags`), K a multiple of 256, more than 8 columns,
  * count <= 64 — or, for at most 8 columns, every src0 a Q5_0 / Q8_0 matrix of one type and size that takes the

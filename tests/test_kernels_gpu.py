@@ -314,6 +314,48 @@ def test_mul_mat_gelu_epilogue_from_the_lds_table_slice(pkg, oracle, gpu):
     assert oracle.nmse(got[:64], oracle.gelu(plain[:64])) <= 1e-7
 
 
+# (K, M, N): one unit of K; fewer units than wavefronts; odd rows and columns on every tile size; the K split in 8; more rows
+# than one launch of 16-row tiles is chosen for; sizes on both sides of the change to 128-wide tiles
+@pytest.mark.parametrize("k,m,n", [(64, 70, 5), (64, 300, 130), (64, 1500, 700), (128, 33, 17), (192, 1, 3), (1280, 1281, 8), (2048, 515, 16), (1280, 4113, 4),
+                                   (512, 2049, 33), (384, 1000, 487), (448, 513, 900), (256, 1030, 1024), (768, 5001, 27)])
+def test_mul_mat_split_k(pkg, oracle, gpu, k, m, n):
+    # f16 weights, f32 activations rounded to f16: against float64 over the rounded operands, with every part of the epilogue;
+    # a second call over the f16 rows that the first left in the workspace gives the same bits
+    lib = pkg.kernels()
+    w, x, bias, res = rnd((m, k), 0.05), rnd((n, k)), rnd((m,), 0.5), rnd((n, m))
+    w16, x16 = w.astype(np.float16), x.astype(np.float16)
+    base = x16.astype(np.float64) @ w16.astype(np.float64).T
+    d_w, d_x, d_b, d_r = gpu.up(w16.view(np.int16)), gpu.up(x), gpu.up(bias), gpu.up(res)
+    tw, tx = pkg.tensor(d_w, pkg.F16), pkg.tensor(d_x, pkg.F32)
+    need = lib.mi355x_mul_mat_workspace_size(tw, tx)
+    ws = torch.full((need,), 255, dtype=torch.uint8, device=gpu.dev)
+    for flags, out, want in ((0, torch.float32, base), (pkg.EPI_BIAS | pkg.EPI_SCALE | pkg.EPI_RESIDUAL, torch.float32, (base + bias) * 0.5 + res),
+                             (pkg.EPI_BIAS | pkg.EPI_OUT_F16, torch.float16, base + bias)):
+        got = []
+        for ready in (0, pkg.MM_WS_READY):
+            d_y = torch.full((n + 1, m), 7.0, dtype=out, device=gpu.dev)
+            epi = pkg.Epilogue(flags | ready, 0.5, d_b.data_ptr(), d_r.data_ptr(), None)
+            pkg.check(lib.mi355x_mul_mat(tw, tx, pkg.tensor(d_y[:n], pkg.F16 if out == torch.float16 else pkg.F32), C.byref(epi), ws.data_ptr(), need, gpu.stream))
+            assert torch.all(d_y[n] == 7.0)
+            got.append(gpu.down(d_y[:n].float()))
+        assert np.array_equal(got[0], got[1])
+        assert oracle.nmse(got[0], want) <= (1e-12 if out == torch.float32 else 1e-6)
+
+
+# rows that are not 16-byte aligned, any K (the transposed V of a window of 1500, 37 or 1501 positions), one or two columns
+@pytest.mark.parametrize("k,m,n,batch", [(1500, 64, 300, 3), (37, 64, 37, 2), (1501, 64, 5, 2), (1500, 64, 1, 4), (64, 1500, 2, 2), (512, 1000, 1, 1), (1280, 5003, 2, 1), (2048, 48, 1, 1), (3, 5, 40, 1)])
+def test_mul_mat_f16_keeps_f32_activations(pkg, oracle, gpu, k, m, n, batch):
+    lib = pkg.kernels()
+    w16, x = rnd((batch, m, k), 0.5).astype(np.float16), np.abs(rnd((batch, n, k), 1.0 / k))
+    want = np.einsum("bnk,bmk->bnm", x.astype(np.float64), w16.astype(np.float64))
+    d_w, d_x = gpu.up(w16.view(np.int16)), gpu.up(x)
+    d_y = torch.full((batch, n, m), 7.0, dtype=torch.float32, device=gpu.dev)
+    tw, tx = pkg.tensor(d_w, pkg.F16), pkg.tensor(d_x, pkg.F32)
+    assert lib.mi355x_mul_mat_workspace_size(tw, tx) == 0
+    pkg.check(lib.mi355x_mul_mat(tw, tx, pkg.tensor(d_y, pkg.F32), None, None, 0, gpu.stream))
+    assert oracle.nmse(gpu.down(d_y), want) <= 1e-12
+
+
 @pytest.mark.parametrize("k,m,n", [(256, 320, 150), (256, 5120, 1500), (128, 2080, 2950)])
 def test_mul_mat_epilogue_emits_the_next_products_activation_image(pkg, oracle, gpu, k, m, n):
     # MI355X_EPI_EMIT_F16: besides dst (here with bias and GELU, the FFN's first matrix), its rows rounded to Q8_0 as f16(q * d).

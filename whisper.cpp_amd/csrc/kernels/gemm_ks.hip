@@ -1,0 +1,452 @@
+// MUL_MAT over f16 weights for problems too small to fill the device with 128-wide tiles, for a handful of columns, and for
+// operands whose rows are not 16-byte aligned: k_gemm_ks.
+//
+// What bounds such a product is not the matrix cores but the time until the first operands are there and how much of the
+// device asks for them: a decoder's 1280 x 1280 product over 5 columns is 20 tiles of 64 x 64 with 20 dependent K steps each,
+// 10.3 us where its 3.3 MB of weights need 1.  Here tiles are small and the K range of a tile is dealt to the KW wavefronts of
+// a workgroup (units of 64 values, round robin: the wavefronts together read consecutive 128-byte lines).  No operand is used
+// by two wavefronts, so each streams its own and the K loop has no barrier; the partial tiles meet once, in LDS, where the
+// epilogue reads them.  k_gemm_ks streams through LDS, k_gemm_kd (any alignment, any K) straight into registers.
+//
+// The weights are the A operand of v_mfma_f32_16x16x32_f16, the activations (src1) the B operand: lane l holds row / column
+// l % 16 and k = 8 (l / 16) .. + 7 of a 32-deep step, and the result's registers are 4 consecutive m of one dst row.
+// Rows past M and columns past N are read from the last valid one and not stored; a K that is no multiple of 64 ends in one
+// unit whose loads are guarded value by value.
+#include "gemm_ks.h"
+
+#include <atomic>
+
+#define KS_UNIT 64
+
+template <int N>
+__device__ __forceinline__ void ks_wait_vmcnt() {             // s_waitcnt vmcnt(N) only; what is read from LDS stays behind it
+    static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+typedef float ks_f4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef half_t ks_h8 __attribute__((ext_vector_type(8), aligned(2)));
+typedef half_t ks_h4 __attribute__((ext_vector_type(4), aligned(2)));
+
+template <int MT, int NT, int KW> constexpr size_t ks_red_bytes() { return (size_t) KW * 16 * NT * (16 * MT + 4) * sizeof(float); }
+
+// The partial tiles of the KW wavefronts meet in `red` ([KW][16 NT][LD] floats, free when every wavefront is past its loop) and
+// leave through the epilogue.  EMIT: MI355X_EPI_EMIT_F16 (a block of 32 m is 8 consecutive lanes).
+template <int MT, int NT, int KW, bool EMIT>
+__device__ __forceinline__ void ks_finish(float4_t (&acc)[MT][NT], float * red, const mm_args & a, char * db, const epi_args & epi, int64_t batch_off,
+                                          int64_t d_nb1, int64_t m0, int64_t n0) {
+    static_assert(!EMIT || MT % 2 == 0, "whole Q8_0 blocks per tile");
+    constexpr int LD = 16 * MT + 4;                     // (+ 4: the 16 rows n of a result register start 4 banks apart)
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r16 = lane & 15, q = lane >> 4;
+    // result register e of a 16x16 tile: column (n) lane % 16, row (m) 4 (lane / 16) + e
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) *(float4_t *)(red + (wave * 16 * NT + 16 * j + r16) * LD + 16 * i + 4 * q) = acc[i][j];
+    __syncthreads();
+    constexpr int PIECES = 16 * NT * 4 * MT;            // (n, four consecutive m)
+#pragma unroll
+    for (int p0 = 0; p0 < PIECES; p0 += 64 * KW) {
+        const int p = p0 + tid;
+        if (PIECES % (64 * KW) != 0 && p >= PIECES) break;
+        const int nl = p / (4 * MT), ml = p % (4 * MT) * 4;
+        float4_t v = *(const float4_t *)(red + nl * LD + ml);
+#pragma unroll
+        for (int w = 1; w < KW; ++w) v += *(const float4_t *)(red + (w * 16 * NT + nl) * LD + ml);
+        const int64_t n = n0 + nl, m = m0 + ml;
+        const bool row = n < a.N, whole = m + 3 < a.M;
+        if (!EMIT && (!row || m >= a.M)) continue;
+        const int64_t nc = row ? n : a.N - 1;
+        if (whole) {
+            if (epi.flags & MI355X_EPI_BIAS) v += *(const ks_f4 *)(epi.bias + m);
+            if (epi.flags & MI355X_EPI_BIAS_COL) v += epi.bias[nc];
+            if (epi.flags & MI355X_EPI_GELU) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = gelu_f32(v[e], epi.gelu);
+            }
+            if (epi.flags & MI355X_EPI_SCALE) v *= epi.scale;
+            if (epi.flags & MI355X_EPI_RESIDUAL) v += *(const ks_f4 *)(epi.residual + batch_off + nc * d_nb1 + m * 4);
+            if (row) {
+                if (epi.flags & MI355X_EPI_OUT_F16) *(ks_h4 *)(db + n * d_nb1 + m * 2) = (ks_h4){ (half_t) v[0], (half_t) v[1], (half_t) v[2], (half_t) v[3] };
+                else if (!EMIT || !(epi.flags & MI355X_EPI_IMAGE_ONLY)) *(ks_f4 *)(db + n * d_nb1 + m * 4) = v;
+            }
+        } else if (row && m < a.M) {
+            for (int e = 0; e < 4 && m + e < a.M; ++e) {
+                const float y = apply_epilogue(v[e], epi, m + e, n, batch_off + n * d_nb1 + (m + e) * 4);
+                if (epi.flags & MI355X_EPI_OUT_F16) *(half_t *)(db + n * d_nb1 + (m + e) * 2) = (half_t) y;
+                else                                *(float  *)(db + n * d_nb1 + (m + e) * 4) = y;
+            }
+        }
+        if (EMIT) {                                     // M is a multiple of 32: a block of 8 lanes is inside dst or outside
+            float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+            amax = lanes_max<8>(amax);
+            const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
+            const float dq = h2f(f2h_bits(div127(amax)));
+            if (row && whole)
+                *(half4_t *)(epi.image + n * a.M + m) = (half4_t){ (half_t)((rintf(v[0] * id) + 0.0f) * dq), (half_t)((rintf(v[1] * id) + 0.0f) * dq),
+                                                                   (half_t)((rintf(v[2] * id) + 0.0f) * dq), (half_t)((rintf(v[3] * id) + 0.0f) * dq) };
+        }
+    }
+}
+
+// The same with the operands streamed through LDS: rows at 16-byte alignment, K a multiple of 64.  A fragment load straight
+// from global memory takes 16 rows in every 16 lanes, 16 cache lines where 16 consecutive lanes could share two, and the
+// L1 cache looks up one line a clock: 16 B per clock and CU.  global_load_lds reads 8 whole 128-byte row pieces instead, and
+// the fragments come out of LDS.  Every wavefront streams its own units through its own D buffers, so the loop has no
+// barrier in it.
+// LDS layout of f16 rows: row pairs form 256-byte lines, the 16-byte chunk c of row r sits in slot (r & 1) * 8 + (c ^ (line & 7))
+// of line r / 2 (the 16 rows of a fragment read then cover all banks once); f32 rows are one line each, chunk c in slot c ^ (r & 15).
+// XR: rows of src1 that are loaded (8 with at most 8 columns: the other columns of the result are not stored).
+template <int MT, int NT, int KW, int D, int XR, int XM, bool EMIT>
+__device__ __forceinline__ void gemm_ks_tile(const mm_args & a, const char * wb, const char * xb, char * db, const epi_args & epi, int64_t batch_off,
+                                             int64_t d_nb1, int64_t m0, int64_t n0, half_t * x16) {
+    constexpr int XE = XM == KS_X_F16 ? 2 : 4;
+    constexpr int WL = 2 * MT, XL = XR * XE / 16;       // 1 KB loads per unit
+    constexpr int UNIT_BYTES = (WL + XL) * 1024;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r16 = lane & 15, q = lane >> 4;
+    char * mine = smem + wave * (D * UNIT_BYTES);
+
+    // load i covers lines 4 i .. + 3; this lane: line 4 i + lane / 16, slot lane % 16
+    const char * wp[WL]; const char * xp[XL];
+    auto row_of = [&](int i, int & chunk) __attribute__((always_inline)) { const int line = 4 * i + q; chunk = (lane & 7) ^ (line & 7); return 2 * line + ((lane >> 3) & 1); };
+#pragma unroll
+    for (int i = 0; i < WL; ++i) { int c; const int64_t m = m0 + row_of(i, c); wp[i] = wb + (m < a.M ? m : a.M - 1) * a.w_nb1 + c * 16; }
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+        int c; int64_t n;
+        if constexpr (XM == KS_X_F16) n = n0 + row_of(i, c);
+        else { const int r = 4 * i + q; c = r16 ^ (r & 15); n = n0 + r; }
+        xp[i] = xb + (n < a.N ? n : a.N - 1) * a.x_nb1 + c * 16;
+    }
+    auto load = [&](int64_t u, int buf) __attribute__((always_inline)) {
+        char * to = mine + buf * UNIT_BYTES;
+#pragma unroll
+        for (int i = 0; i < WL; ++i)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(wp[i] + u * (KS_UNIT * 2)), (__attribute__((address_space(3))) void *)(to + i * 1024), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < XL; ++i)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(xp[i] + u * (KS_UNIT * XE)), (__attribute__((address_space(3))) void *)(to + (WL + i) * 1024), 16, 0, 0);
+    };
+    float4_t acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = (float4_t){ 0.f, 0.f, 0.f, 0.f };
+    // fragment addresses inside a unit: f16 rows 16 i + r16 (line 8 i + r16 / 2), chunk 4 s + q
+    const int frow = (r16 >> 1) * 256 + (r16 & 1) * 128, fsw = (r16 >> 1) & 7;
+    auto mma = [&](int64_t u, int buf) __attribute__((always_inline)) {
+        const char * ws = mine + buf * UNIT_BYTES, * xs = ws + WL * 1024;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int fo = frow + ((4 * s + q) ^ fsw) * 16;
+            half8_t wv[MT];
+#pragma unroll
+            for (int i = 0; i < MT; ++i) wv[i] = *(const half8_t *)(ws + i * 2048 + fo);
+            if constexpr (XM == KS_X_F16) {
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    const half8_t xv = *(const half8_t *)(xs + j * 2048 + fo);
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[i], xv, acc[i][j], 0, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    const int r = XR == 8 ? r16 & 7 : r16;
+                    const float4_t lo = *(const float4_t *)(xs + (16 * j + r) * 256 + ((8 * s + 2 * q) ^ r) * 16);
+                    const float4_t hi = *(const float4_t *)(xs + (16 * j + r) * 256 + ((8 * s + 2 * q + 1) ^ r) * 16);
+                    if constexpr (XM == KS_X_CVT) {
+                        const half8_t xv = { (half_t) lo.x, (half_t) lo.y, (half_t) lo.z, (half_t) lo.w, (half_t) hi.x, (half_t) hi.y, (half_t) hi.z, (half_t) hi.w };
+                        if (x16) {
+                            const int64_t n = n0 + 16 * j + r16;
+                            if (r16 < XR && n < a.N) *(half8_t *)(x16 + n * a.K + u * KS_UNIT + 32 * s + 8 * q) = xv;
+                        }
+#pragma unroll
+                        for (int i = 0; i < MT; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[i], xv, acc[i][j], 0, 0, 0);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+#pragma unroll
+                            for (int i = 0; i < MT; ++i)
+                                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32((float) wv[i][e], e < 4 ? lo[e & 3] : hi[e & 3], acc[i][j], 0, 0, 0);
+                    }
+                }
+            }
+        }
+    };
+    const int units = (int)(a.K / KS_UNIT), n_mine = units > wave ? (units - wave + KW - 1) / KW : 0;
+#pragma unroll
+    for (int t = 0; t < D - 1; ++t) if (t < n_mine) load(wave + t * KW, t);
+    int t = 0, buf = 0;
+    for (; t + D - 1 < n_mine; ++t) {
+        load(wave + (int64_t)(t + D - 1) * KW, buf == 0 ? D - 1 : buf - 1);
+        ks_wait_vmcnt<(D - 1) * (WL + XL)>();           // unit t is in LDS
+        mma(wave + (int64_t) t * KW, buf);
+        buf = buf + 1 == D ? 0 : buf + 1;
+    }
+    ks_wait_vmcnt<0>();
+    for (; t < n_mine; ++t) { mma(wave + (int64_t) t * KW, buf); buf = buf + 1 == D ? 0 : buf + 1; }
+    __syncthreads();                                    // (the partial tiles take the buffers' place)
+    ks_finish<MT, NT, KW, EMIT>(acc, (float *) smem, a, db, epi, batch_off, d_nb1, m0, n0);
+}
+
+template <int MT, int NT, int KW, int XM>
+__device__ __forceinline__ void gemm_kd_tile(const mm_args & a, const char * wb, const char * xb, char * db, const epi_args & epi, int64_t batch_off,
+                                             int64_t d_nb1, int64_t m0, int64_t n0) {
+    constexpr int XE = XM == KS_X_F16 ? 2 : 4;          // bytes per src1 element
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    float * red = (float *) smem;                       // [KW][16 NT][LD]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r16 = lane & 15, q = lane >> 4;
+
+    const char * wp[MT]; const char * xp[NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) { const int64_t m = m0 + 16 * i + r16; wp[i] = wb + (m < a.M ? m : a.M - 1) * a.w_nb1 + q * 16; }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) { const int64_t n = n0 + 16 * j + r16; xp[j] = xb + (n < a.N ? n : a.N - 1) * a.x_nb1 + q * 8 * XE; }
+
+    struct frags { ks_h8 w[2][MT]; ks_h8 x[2][XM == KS_X_F16 ? NT : 1]; ks_f4 xf[2][XM == KS_X_F16 ? 1 : NT][2]; };
+    float4_t acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = (float4_t){ 0.f, 0.f, 0.f, 0.f };
+
+    auto load = [&](frags & f, int64_t u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int64_t k = u * KS_UNIT + 32 * s;
+#pragma unroll
+            for (int i = 0; i < MT; ++i) f.w[s][i] = *(const ks_h8 *)(wp[i] + k * 2);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                if constexpr (XM == KS_X_F16) f.x[s][j] = *(const ks_h8 *)(xp[j] + k * 2);
+                else { f.xf[s][j][0] = *(const ks_f4 *)(xp[j] + k * 4); f.xf[s][j][1] = *(const ks_f4 *)(xp[j] + k * 4 + 16); }
+            }
+        }
+    };
+    auto load_tail = [&](frags & f, int64_t u) __attribute__((always_inline)) {       // values past K are zero
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int64_t k = u * KS_UNIT + 32 * s;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const bool in = k + 8 * q + e < a.K;
+                const int64_t at = in ? k + e : -(int64_t) 8 * q;                     // (k = 0 of the row, which exists)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) { const half_t v = *(const half_t *)(wp[i] + at * 2); f.w[s][i][e] = in ? v : (half_t) 0.f; }
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    if constexpr (XM == KS_X_F16) { const half_t v = *(const half_t *)(xp[j] + at * 2); f.x[s][j][e] = in ? v : (half_t) 0.f; }
+                    else { const float v = *(const float *)(xp[j] + at * 4); f.xf[s][j][e / 4][e % 4] = in ? v : 0.f; }
+                }
+            }
+        }
+    };
+    auto mma = [&](const frags & f, int64_t u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if constexpr (XM == KS_X_F32) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+#pragma unroll
+                    for (int i = 0; i < MT; ++i)
+#pragma unroll
+                        for (int j = 0; j < NT; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32((float) f.w[s][i][e], f.xf[s][j][e / 4][e % 4], acc[i][j], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.w[s][i], f.x[s][j], acc[i][j], 0, 0, 0);
+            }
+        }
+    };
+
+    // Two units in flight.  Every load is unconditional (past the end it re-reads the last unit): with a load behind a
+    // branch the compiler cannot count what is outstanding and waits for everything.
+    const int64_t full = a.K / KS_UNIT;
+    int64_t u = wave;
+    if (u < full) {
+        frags f0, f1;
+        load(f0, u);
+        while (true) {
+            load(f1, u + KW < full ? u + KW : full - 1);
+            mma(f0, u); u += KW; if (u >= full) break;
+            load(f0, u + KW < full ? u + KW : full - 1);
+            mma(f1, u); u += KW; if (u >= full) break;
+        }
+    }
+    if (a.K % KS_UNIT != 0 && wave == (int)(full % KW)) {
+        frags f;
+        load_tail(f, full);
+        mma(f, full);
+    }
+
+    ks_finish<MT, NT, KW, false>(acc, red, a, db, epi, batch_off, d_nb1, m0, n0);
+}
+
+// grids: m tiles x n tiles x batch
+#define KS_SLICES const int64_t b2 = blockIdx.z % a.ne12, b3 = blockIdx.z / a.ne12; \
+    const char * wb = a.w + (b2 / a.r2) * a.w_nb2 + (b3 / a.r3) * a.w_nb3, * xb = a.x + b2 * a.x_nb2 + b3 * a.x_nb3; \
+    const int64_t d_off = b2 * a.d_nb2 + b3 * a.d_nb3, m0 = (int64_t) blockIdx.x * 16 * MT, n0 = (int64_t) blockIdx.y * 16 * NT;
+
+template <int MT, int NT, int KW, int D, int XR, int XM, bool EMIT>
+__global__ void __launch_bounds__(64 * KW) k_gemm_ks(mm_args a, half_t * x16, int64_t x16_slice) {
+    KS_SLICES
+    gemm_ks_tile<MT, NT, KW, D, XR, XM, EMIT>(a, wb, xb, a.d + d_off, a.e, d_off, a.d_nb1, m0, n0, x16 && blockIdx.x == 0 ? x16 + blockIdx.z * x16_slice : nullptr);
+}
+// several products over the same activations: blockIdx.z picks the weights, the destination and the epilogue
+struct ks_group { mm_group_entry e[KS_GROUP_MAX]; };
+template <int MT, int NT, int KW, int D, int XR>
+__global__ void __launch_bounds__(64 * KW) k_gemm_ks_group(mm_args a, ks_group grp) {
+    const mm_group_entry & ge = grp.e[blockIdx.z];
+    epi_args e;
+    e.flags = ge.flags; e.scale = ge.scale; e.bias = ge.bias; e.residual = ge.residual; e.gelu = a.e.gelu; e.image = nullptr;
+    gemm_ks_tile<MT, NT, KW, D, XR, KS_X_F16, false>(a, ge.w, a.x, ge.d, e, 0, ge.d_nb1, (int64_t) blockIdx.x * 16 * MT, (int64_t) blockIdx.y * 16 * NT, nullptr);
+}
+template <int MT, int NT, int KW, int XM>
+__global__ void __launch_bounds__(64 * KW) k_gemm_kd(mm_args a) {
+    KS_SLICES
+    gemm_kd_tile<MT, NT, KW, XM>(a, wb, xb, a.d + d_off, a.e, d_off, a.d_nb1, m0, n0);
+}
+
+template <int MT, int NT>
+static int ks_grid(const mm_args & a, dim3 & grid) {
+    const int64_t tm = (a.M + 16 * MT - 1) / (16 * MT), tn = (a.N + 16 * NT - 1) / (16 * NT), nb = a.ne12 * a.ne13;
+    if (tm > 0x7fffffff || tn > 65535 || nb > 65535) return MI355X_ERR_UNSUPPORTED;
+    grid = dim3((unsigned) tm, (unsigned) tn, (unsigned) nb);
+    return MI355X_OK;
+}
+// more than the default 64 KB of LDS have to be asked for, once per kernel and device
+static int ks_configure(const void * fn, size_t lds, std::atomic<bool> * configured) {
+    if (lds <= 64 * 1024) return MI355X_OK;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return MI355X_ERR_HIP;
+    if (configured[dev].load(std::memory_order_acquire)) return MI355X_OK;
+    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds) != hipSuccess) return MI355X_ERR_HIP;
+    configured[dev].store(true, std::memory_order_release);
+    return MI355X_OK;
+}
+
+template <int MT, int NT, int KW, int D, int XR, int XM, bool EMIT>
+static int launch_ks_t(const mm_args & a, half_t * x16, int64_t slice, hipStream_t st) {
+    constexpr size_t ring = (size_t) KW * D * (2 * MT + XR * (XM == KS_X_F16 ? 2 : 4) / 16) * 1024, red = ks_red_bytes<MT, NT, KW>(), lds = ring > red ? ring : red;
+    static std::atomic<bool> configured[64];
+    static_assert(lds <= 160 * 1024, "LDS of a CU");
+    dim3 grid;
+    if (int rc = ks_grid<MT, NT>(a, grid)) return rc;
+    if (int rc = ks_configure((const void *) k_gemm_ks<MT, NT, KW, D, XR, XM, EMIT>, lds, configured)) return rc;
+    k_gemm_ks<MT, NT, KW, D, XR, XM, EMIT><<<grid, 64 * KW, lds, st>>>(a, x16, slice);
+    return launch_status();
+}
+template <int MT, int NT, int KW, int XM>
+static int launch_kd_t(const mm_args & a, hipStream_t st) {
+    constexpr size_t lds = ks_red_bytes<MT, NT, KW>();
+    static std::atomic<bool> configured[64];
+    dim3 grid;
+    if (int rc = ks_grid<MT, NT>(a, grid)) return rc;
+    if (int rc = ks_configure((const void *) k_gemm_kd<MT, NT, KW, XM>, lds, configured)) return rc;
+    k_gemm_kd<MT, NT, KW, XM><<<grid, 64 * KW, lds, st>>>(a);
+    return launch_status();
+}
+template <int XM, bool EMIT>
+static int launch_ks_x(const mm_args & a, const ks_shape & s, half_t * x16, int64_t slice, hipStream_t st) {
+    const bool few = a.N <= 8;
+#define KS_CASE(MT, NT, KW, D) if (s.mt == MT && s.nt == NT && s.kw == KW && s.d == D) { if constexpr (!EMIT || MT % 2 == 0) { \
+        if constexpr (NT == 1) if (few) return launch_ks_t<MT, NT, KW, D, 8, XM, EMIT>(a, x16, slice, st); \
+        return launch_ks_t<MT, NT, KW, D, 16 * NT, XM, EMIT>(a, x16, slice, st); } }
+    KS_CASE(1, 1, 1, 1) KS_CASE(1, 1, 4, 2) KS_CASE(1, 1, 8, 2) KS_CASE(2, 1, 4, 2)
+    if constexpr (XM != KS_X_F32) { KS_CASE(2, 2, 1, 1) KS_CASE(4, 4, 1, 1) }
+    if constexpr (XM == KS_X_F16) { KS_CASE(2, 2, 4, 2) KS_CASE(4, 4, 4, 2) }
+#undef KS_CASE
+    return MI355X_ERR_UNSUPPORTED;
+}
+
+// Tile and split by size (MI355X, weights from HBM, us per launch; "128-wide" is what the tiled kernels of mul_mat.hip take):
+//   up to 16 columns: 16 x 16 tiles, 4 wavefronts on their K range (1280 x 1280, 5 columns: 4.6; 64 x 64 tiles 10.3), 8 from
+//     K = 2048 (1280 x 5120: 9.6, with 4 11.4, tiled 26.3), 32 rows to a tile from 4096 rows on (51866 x 1280: 26.5; 28.0; 40.4);
+//   one round of 64 x 64 tiles, at least half of one (M = 512, K = 2048, N = 1500: 12.9; 128-wide 14.3; M = 1280, K = 1280,
+//     N = 700: 10.2; 11.3), else 32 x 32 (1280 x 5120, 227 columns: 17.8; 34.9; 384 x 384, 487 columns: 3.9; 7.3), and 16 x 16 where
+//     that is under half a round as well (768 x 768, 27 columns: 3.7; 4.4; 6.8);
+//   more than a round of 64 x 64 tiles: the 128-wide tiles, which move half the bytes per product (M = 768, N = 1500: 8.9;
+//     10.7 here), except with up to 32 columns, where they are mostly padding (51865 x 768, 27 columns: 21.7; 23.9).
+// K = 64 (attention scores) is one unit: no split, one wavefront to a tile, and what counts is the store of the result.
+static bool ks_tiles(int64_t M, int64_t N, int64_t K, int64_t nb, bool emit, ks_shape & s) {
+    const int64_t t44 = (M + 63) / 64 * ((N + 63) / 64) * nb, t22 = (M + 31) / 32 * ((N + 31) / 32) * nb;
+    s.kw = 4; s.d = 2;
+    if (K == KS_UNIT) {
+        s.kw = 1; s.d = 1;
+        s.mt = s.nt = N <= 16 || t22 < 512 ? 1 : t44 < 512 ? 2 : 4;
+        return !emit;
+    }
+    if (N <= 16) {
+        s.nt = 1; s.mt = emit || M > 4096 ? 2 : 1;
+        if (s.mt == 1 && K >= 2048) s.kw = 8;
+        return true;
+    }
+    if (t44 > 256) { s.mt = s.nt = 2; return N <= 32; }
+    s.mt = s.nt = t44 > 128 ? 4 : t22 > 128 ? 2 : 1;
+    if (emit && s.mt == 1) s.mt = 2;
+    return true;
+}
+bool ks_pick(int64_t M, int64_t N, int64_t K, int64_t nb, bool emit, ks_shape & s) {
+    return K > 0 && K % KS_UNIT == 0 && ks_tiles(M, N, K, nb, emit, s);
+}
+// A group goes the way of its single products, on tiles chosen for all of them together; the K split, and with it the order
+// of the sums, is the same for every tile size.  A group that fills the device with 128-wide tiles goes there.
+bool ks_pick_group(int64_t M, int64_t N, int64_t K, int count, ks_shape & s) {
+    ks_shape one;
+    if (count > KS_GROUP_MAX || !ks_pick(M, N, K, 1, false, one) || !ks_pick(M, N, K, count, false, s)) return false;
+    return s.kw == one.kw;
+}
+bool ks_converts(const ks_shape & s) { return s.nt == 1 || s.kw == 1; }
+
+int launch_gemm_ks(const mm_args & a, const ks_shape & s, int xm, half_t * x16, int64_t x16_slice, hipStream_t st) {
+    const bool emit = a.e.flags & MI355X_EPI_EMIT_F16;
+    switch (xm) {
+        case KS_X_F16: return emit ? launch_ks_x<KS_X_F16, true>(a, s, x16, x16_slice, st) : launch_ks_x<KS_X_F16, false>(a, s, x16, x16_slice, st);
+        case KS_X_CVT: return emit ? MI355X_ERR_UNSUPPORTED : launch_ks_x<KS_X_CVT, false>(a, s, x16, x16_slice, st);
+        default:       return emit ? MI355X_ERR_UNSUPPORTED : launch_ks_x<KS_X_F32, false>(a, s, x16, x16_slice, st);
+    }
+}
+
+template <int MT, int NT, int KW, int D, int XR>
+static int launch_ks_group_t(const mm_args & a, const ks_group & grp, int count, hipStream_t st) {
+    constexpr size_t ring = (size_t) KW * D * (2 * MT + XR / 8) * 1024, red = ks_red_bytes<MT, NT, KW>(), lds = ring > red ? ring : red;
+    static std::atomic<bool> configured[64];
+    dim3 grid;
+    if (int rc = ks_grid<MT, NT>(a, grid)) return rc;
+    grid.z = (unsigned) count;
+    if (int rc = ks_configure((const void *) k_gemm_ks_group<MT, NT, KW, D, XR>, lds, configured)) return rc;
+    k_gemm_ks_group<MT, NT, KW, D, XR><<<grid, 64 * KW, lds, st>>>(a, grp);
+    return launch_status();
+}
+int launch_gemm_ks_group(const mm_args & a, const mm_group & all, int count, const ks_shape & s, hipStream_t st) {
+    ks_group grp;
+    for (int i = 0; i < count; ++i) grp.e[i] = all.e[i];
+#define KS_CASE(MT, NT, KW, D) if (s.mt == MT && s.nt == NT && s.kw == KW && s.d == D) { \
+        if constexpr (NT == 1) if (a.N <= 8) return launch_ks_group_t<MT, NT, KW, D, 8>(a, grp, count, st); \
+        return launch_ks_group_t<MT, NT, KW, D, 16 * NT>(a, grp, count, st); }
+    KS_CASE(1, 1, 4, 2) KS_CASE(1, 1, 8, 2) KS_CASE(2, 1, 4, 2) KS_CASE(2, 2, 4, 2) KS_CASE(4, 4, 4, 2)
+#undef KS_CASE
+    return MI355X_ERR_UNSUPPORTED;
+}
+
+// The direct kernel, by size: a few columns on 16 x 16 tiles with as many wavefronts as the K range has units, up to 8; more
+// on 64 x 32 (64 rows are all there are of the transposed V of a head: src1 is then read once).
+int launch_gemm_kd(const mm_args & a, int xm, hipStream_t st) {
+    const bool few = a.N <= 16;
+    const int kw = a.K <= KS_UNIT ? 1 : a.K < 8 * KS_UNIT ? 4 : 8;
+    if (xm == KS_X_F16) {
+        if (!few) return launch_kd_t<4, 2, 4, KS_X_F16>(a, st);
+        return kw == 1 ? launch_kd_t<1, 1, 1, KS_X_F16>(a, st) : kw == 4 ? launch_kd_t<1, 1, 4, KS_X_F16>(a, st) : launch_kd_t<1, 1, 8, KS_X_F16>(a, st);
+    }
+    if (!few) return launch_kd_t<4, 2, 4, KS_X_F32>(a, st);
+    return kw == 1 ? launch_kd_t<1, 1, 1, KS_X_F32>(a, st) : kw == 4 ? launch_kd_t<1, 1, 4, KS_X_F32>(a, st) : launch_kd_t<1, 1, 8, KS_X_F32>(a, st);
+}

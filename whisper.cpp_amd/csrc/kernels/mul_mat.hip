@@ -3,7 +3,7 @@
 //
 // This file: the tiled MFMA GEMM (many columns; f16 operands, f32 accumulation, whatever the weights' type: one pass brings
 // blocks to f16), k_mul_mat_generic for what no other kernel takes, and the dispatch.  The quantized few-column products are
-// in gemv.hip.
+// in gemv.hip, the split-K products over f16 weights in gemm_ks.hip.
 #include "common.h"
 
 #include <algorithm>
@@ -18,6 +18,7 @@
 // ------------------------------------------------------------------------------------------------------
 
 #include "mul_mat_args.h"
+#include "gemm_ks.h"
 #include "gemv.h"
 
 // The same for the 16 registers of one 32x32 accumulator patch (column m, rows n[0..15]) and the stores.  All loads of
@@ -997,13 +998,16 @@ static int launch_gemm_f16_group(const mm_args & a, const mm_group & grp, int co
     return launch_status();
 }
 
-// tile shape: the largest whose grid still covers the 256 CUs about twice
+// tile shape: small problems go to k_gemm_ks; else the largest whose grid still covers the 256 CUs about twice
 static int launch_gemm_f16_auto(const mm_args & a, hipStream_t st) {
     const int64_t nb = a.ne12 * a.ne13;
+    ks_shape ks;
+    if (ks_pick(a.M, a.N, a.K, nb, (a.e.flags & MI355X_EPI_EMIT_F16) != 0, ks)) return launch_gemm_ks(a, ks, KS_X_F16, nullptr, 0, st);
     auto blocks = [&](int bn, int bm) { return ((a.N + bn - 1) / bn) * ((a.M + bm - 1) / bm) * nb; };
     if (blocks(128, 128) >= 384) return launch_gemm_f16<2, 2>(a, st);
-    if (blocks(128, 64)  >= 192 || a.N > 64) return launch_gemm_f16<2, 1>(a, st);
-    return launch_gemm_f16<1, 1>(a, st);
+    if (blocks(128, 64)  >= 192 || a.N > 64 || a.K % GB_K == 0) return launch_gemm_f16<2, 1>(a, st);
+    if (a.e.flags & MI355X_EPI_EMIT_F16) return MI355X_ERR_UNSUPPORTED;
+    return launch_gemm_f16_k<1, 1, 2, true, false>(a, st);       // (few tiles of a K that k_gemm_ks does not take)
 }
 
 // ------------------------------------------------------------------------------------------------------
@@ -1024,7 +1028,6 @@ __device__ __forceinline__ float w_elem(int type, const uint8_t * row, int64_t k
             const uint8_t * b = row + (k / QK) * 34;
             return (float)((const int8_t *) b)[2 + k % QK] * h2f(*(const uint16_t *) b);
         }
-        case MI355X_TYPE_F16: return (float)((const half_t *) row)[k];
         default:              return ((const float *) row)[k];
     }
 }
@@ -1085,7 +1088,7 @@ int mm_path(const mi355x_tensor * src0, const mi355x_tensor * src1) {
         return MM_GEMV;
     }
     bool fast = N > MI355X_GEMV_MAX_COLS || !quant;
-    if (N <= 2) fast = false;                         // a 64-wide tile for one or two columns is mostly padding
+    if (N <= 2) fast = false;                         // (one or two columns keep src1 at its precision)
     fast = fast && aligned16(src1) && K % 8 == 0;
     if (quant)                 fast = fast && w_al2;
     else if (t0 == MI355X_TYPE_F16) fast = fast && aligned16(src0);
@@ -1173,6 +1176,8 @@ extern "C" int mi355x_mul_mat_group(const mi355x_mul_mat_item * items, int count
         a.x = (const char *) workspace; a.x_nb1 = a.K * 2;
     }
     if (flags & MI355X_MM_PREPARE_ONLY) return launch_status();
+    ks_shape ks;
+    if (ks_pick_group(a.M, a.N, a.K, count, ks)) return launch_gemm_ks_group(a, grp, count, ks, st);
     const int64_t blocks22 = ((a.N + 127) / 128) * ((a.M + 127) / 128) * count;
     return blocks22 >= 300 ? launch_gemm_f16_group<2, 2>(a, grp, count, st) : launch_gemm_f16_group<2, 1>(a, grp, count, st);
 }
@@ -1270,6 +1275,10 @@ extern "C" int mi355x_mul_mat(const mi355x_tensor * src0, const mi355x_tensor * 
                 dim3 qgrid((unsigned)((a.K / 4 * a.N + 255) / 256), (unsigned) nbatch);
                 const bool q8 = (quant || (flags & MI355X_MM_ACT_Q8_0)) && !(flags & MI355X_MM_EXACT_ACT);
                 if (q8 && a.K % QK != 0) return MI355X_ERR_INVALID;
+                // a handful of columns: the product rounds src1 to f16 itself and leaves the f16 rows in the workspace on the way
+                ks_shape ks;
+                if (!q8 && !wbytes && !(flags & (MI355X_MM_PREPARE_ONLY | MI355X_EPI_EMIT_F16)) && ks_pick(a.M, a.N, a.K, nbatch, false, ks) && ks_converts(ks))
+                    return launch_gemm_ks(a, ks, KS_X_CVT, (half_t *) workspace, slice / 2, st);
                 if (q8) k_x_to_f16<true ><<<qgrid, 256, 0, st>>>(a.x, (half_t *) workspace, a.K, a.N, a.x_nb1, a.x_nb2, a.ne12, a.x_nb3, slice / 2);
                 else    k_x_to_f16<false><<<qgrid, 256, 0, st>>>(a.x, (half_t *) workspace, a.K, a.N, a.x_nb1, a.x_nb2, a.ne12, a.x_nb3, slice / 2);
             }
@@ -1290,6 +1299,13 @@ extern "C" int mi355x_mul_mat(const mi355x_tensor * src0, const mi355x_tensor * 
         return launch_gemm_f16_auto(g, st);
     }
 
+    // f16 weights that the tiled kernels do not take: one or two columns, or rows that are not 16-byte aligned (the product of
+    // the attention probabilities with the transposed V, whose rows have the length of the window).  src1 keeps its precision.
+    if (t0 == MI355X_TYPE_F16) {
+        ks_shape ks;
+        if (t1 == MI355X_TYPE_F32 && a.N <= 2 && aligned16(src0) && aligned16(src1) && ks_pick(a.M, a.N, a.K, nbatch, false, ks)) return launch_gemm_ks(a, ks, KS_X_F32, nullptr, 0, st);
+        return launch_gemm_kd(a, t1 == MI355X_TYPE_F32 ? KS_X_F32 : KS_X_F16, st);
+    }
     if (a.M > 0x7fffffff || (a.N + 7) / 8 > 65535) return MI355X_ERR_UNSUPPORTED;
     dim3 grid((unsigned) a.M, (unsigned)((a.N + 7) / 8), (unsigned) nbatch);
     k_mul_mat_generic<<<grid, WAVE, 0, st>>>(a, t0, t1);
