@@ -21,6 +21,12 @@ def rnd(shape, scale=1.0, offset=0.0):
     return (RNG.normal(size=shape) * scale + offset).astype(np.float32)
 
 
+@pytest.fixture
+def own_numbers(monkeypatch):
+    # numbers of the test's own: what it draws does not move the draws of the tests behind it
+    monkeypatch.setitem(globals(), "RNG", np.random.default_rng(8))
+
+
 @pytest.fixture(scope="module")
 def gpu(pkg):
     if not torch.cuda.is_available():
@@ -318,7 +324,7 @@ def test_mul_mat_gelu_epilogue_from_the_lds_table_slice(pkg, oracle, gpu):
 # than one launch of 16-row tiles is chosen for; sizes on both sides of the change to 128-wide tiles
 @pytest.mark.parametrize("k,m,n", [(64, 70, 5), (64, 300, 130), (64, 1500, 700), (128, 33, 17), (192, 1, 3), (1280, 1281, 8), (2048, 515, 16), (1280, 4113, 4),
                                    (512, 2049, 33), (384, 1000, 487), (448, 513, 900), (256, 1030, 1024), (768, 5001, 27)])
-def test_mul_mat_split_k(pkg, oracle, gpu, k, m, n):
+def test_mul_mat_split_k(pkg, oracle, gpu, own_numbers, k, m, n):
     # f16 weights, f32 activations rounded to f16: against float64 over the rounded operands, with every part of the epilogue;
     # a second call over the f16 rows that the first left in the workspace gives the same bits
     lib = pkg.kernels()
@@ -344,7 +350,7 @@ def test_mul_mat_split_k(pkg, oracle, gpu, k, m, n):
 
 # rows that are not 16-byte aligned, any K (the transposed V of a window of 1500, 37 or 1501 positions), one or two columns
 @pytest.mark.parametrize("k,m,n,batch", [(1500, 64, 300, 3), (37, 64, 37, 2), (1501, 64, 5, 2), (1500, 64, 1, 4), (64, 1500, 2, 2), (512, 1000, 1, 1), (1280, 5003, 2, 1), (2048, 48, 1, 1), (3, 5, 40, 1)])
-def test_mul_mat_f16_keeps_f32_activations(pkg, oracle, gpu, k, m, n, batch):
+def test_mul_mat_f16_keeps_f32_activations(pkg, oracle, gpu, own_numbers, k, m, n, batch):
     lib = pkg.kernels()
     w16, x = rnd((batch, m, k), 0.5).astype(np.float16), np.abs(rnd((batch, n, k), 1.0 / k))
     want = np.einsum("bnk,bmk->bnm", x.astype(np.float64), w16.astype(np.float64))
@@ -791,6 +797,31 @@ def test_flash_attn_packed_f16_chain(pkg, oracle, gpu, case):
     assert np.array_equal(again.view(np.uint32), got.view(np.uint32))          # the same bits on every run
 
 
+@pytest.mark.parametrize("H,N,KV,masked", [(3, 9, 1, False), (2, 32, 64, True), (2, 33, 65, True), (1, 31, 129, False),            # 32 queries to the workgroup
+                                          (128, 64, 79, False), (129, 64, 80, True), (129, 65, 127, True), (257, 17, 193, False)])   # from 257 workgroups of those on: 64
+def test_flash_attn_packed_tile_sizes(pkg, oracle, gpu, own_numbers, H, N, KV, masked):
+    # both tile sizes of the many-query kernel of the packed form at their edges, ragged ends and odd mask strides; the image
+    # beside dst is its rows' Q8_0 rounding
+    q, kb, vb = _attention_inputs(oracle, H, N, KV)
+    mask = None
+    if masked:
+        m = np.zeros((-(-N // 64) * 64, KV), dtype=np.float32)
+        for r in range(N):
+            m[r, 1 + (r * 7) % KV:] = -np.inf
+        mask = oracle.f32_to_f16_bits(m)
+    got, _ = run_fa(pkg, gpu, q, kb, vb, mask, 0.125, pkg.FA_F16_PK)
+    assert oracle.nmse(got, oracle.flash_attn_ext(q, kb, vb, None if mask is None else mask[:N], 0.125)) <= 1e-5
+    d_q, d_k, d_v, d_m = gpu.up(q), gpu.up(kb), gpu.up(vb), None if mask is None else gpu.up(mask)
+    d_o = torch.empty((N, H, 64), dtype=torch.float32, device=gpu.dev)
+    d_h = torch.zeros((N, H * 64), dtype=torch.float16, device=gpu.dev)
+    pkg.check(pkg.kernels().mi355x_flash_attn_ext(pkg.tensor(d_q, pkg.F32), pkg.tensor(d_k, pkg.F16), pkg.tensor(d_v, pkg.F16), None if mask is None else pkg.tensor(d_m, pkg.F16),
+                                                  pkg.tensor(d_o, pkg.F32), 0.125, pkg.FA_F16_PK | pkg.FA_EMIT_F16, d_h.data_ptr(), d_h.numel() * 2, gpu.stream))
+    y = gpu.down(d_o).reshape(N, H * 64)
+    assert np.array_equal(y.view(np.uint32), got.reshape(N, H * 64).view(np.uint32))
+    image = oracle.dequantize(oracle.Q8_0, oracle.quantize(oracle.Q8_0, y, act=True), H * 64).reshape(N, H * 64)
+    assert np.array_equal(gpu.down(d_h, np.uint16), oracle.f32_to_f16_bits(image))
+
+
 def test_flash_attn_few_queries_take_the_f32_mask(pkg, oracle, gpu):
     # the few-query kernel reads the f32 tensor a graph would cast to f16 and rounds each value as the cast does: the same bits
     # as with the f16 copy, also for values that are not representable in f16; with more than 8 queries it says no
@@ -1183,7 +1214,7 @@ def test_log_mel_against_the_oracle(pkg, oracle, gpu, n, n_mel):
 
 
 @pytest.mark.parametrize("n", [160 * 22 - 200, 160 * 23 - 200, 160 * 24 - 200, 160 * 47 + 1, 160 * 24 * 769])
-def test_log_mel_rounds_and_filter_ranges(pkg, oracle, gpu, n):
+def test_log_mel_rounds_and_filter_ranges(pkg, oracle, gpu, own_numbers, n):
     # frame counts around whole rounds of 24 and beyond one round per workgroup; a bank that is no set of triangles: dense bands,
     # one of a single bin at either end, one without a nonzero weight (log10(1e-10) in every frame)
     f = np.abs(rnd((6, 201))) * 0.02

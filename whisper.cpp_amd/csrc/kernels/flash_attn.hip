@@ -17,7 +17,8 @@
 //       k_fattn_seq_row    N <= 8: one block per (query, head): one wavefront (lane = d) runs the chain while the
 //                                  other three score, scan and stage the next 192 keys.
 //   MI355X_FA_F16_PK             the same sequence with the step of the reference's builds that have f16 vector units: the
-//                                factor rounded to f16, one fused f16 multiply-add per element (k_fattn_pk_tile for N > 8,
+//                                factor rounded to f16, one fused f16 multiply-add per element (k_fattn_pk_tile for N > 8, whose
+//                                maximum moves every 16 keys instead of every key;
 //                                k_fattn_pk_row for N <= 8).
 //   MI355X_FA_F32          f32 accumulators: closer to exact arithmetic, not to the reference (whose f16 accumulator
 //                          loses about 1e-4 NMSE per attention, which whole-model logits then show as several 1e-3).
@@ -25,11 +26,13 @@
 //       k_fattn_vec        N <= 8: one wavefront per (query, head), keys split across lanes
 #include "common.h"
 #include <atomic>
+#include <type_traits>
 
 #define FA_D 64
 #define LOG2E_F 1.44269504088896340736f
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 struct fa_args {
     const char * q; const char * k; const char * v; const char * mask; char * d;
@@ -225,93 +228,26 @@ __device__ __forceinline__ half2_t seq_scale2(half2_t acc, float ms) {
 // rounding (2^-12 of an increment that is itself a small part of the sum) and by one rounding instead of two.  On gfx950
 // that is v_pk_fma_f16, two elements per instruction.
 //
-// One key for a lane that owns 4 queries x 4 d: acc[2 q + j] holds d pair j of query q, v the key's two d pairs, f[q] the
-// factors of two consecutive keys for query q as two f16; SEL picks the first or the second of them for both elements.
-template <int SEL>
-__device__ __forceinline__ void pk_mad8(half2_t (&acc)[8], const uint32_t v0, const uint32_t v1, const u32x4 f) {
-    if (SEL == 0) {
-        asm("v_pk_fma_f16 %0, %8, %10, %0 op_sel_hi:[1,0,1]\n\t"
-            "v_pk_fma_f16 %2, %8, %11, %2 op_sel_hi:[1,0,1]\n\t"
-            "v_pk_fma_f16 %4, %8, %12, %4 op_sel_hi:[1,0,1]\n\t"
-            "v_pk_fma_f16 %6, %8, %13, %6 op_sel_hi:[1,0,1]\n\t"
-            "v_pk_fma_f16 %1, %9, %10, %1 op_sel_hi:[1,0,1]\n\t"
-            "v_pk_fma_f16 %3, %9, %11, %3 op_sel_hi:[1,0,1]\n\t"
-            "v_pk_fma_f16 %5, %9, %12, %5 op_sel_hi:[1,0,1]\n\t"
-            "v_pk_fma_f16 %7, %9, %13, %7 op_sel_hi:[1,0,1]"
-            : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4]), "+v"(acc[5]), "+v"(acc[6]), "+v"(acc[7])
-            : "v"(v0), "v"(v1), "v"(f.x), "v"(f.y), "v"(f.z), "v"(f.w));
-    } else {
-        asm("v_pk_fma_f16 %0, %8, %10, %0 op_sel:[0,1,0] op_sel_hi:[1,1,1]\n\t"
-            "v_pk_fma_f16 %2, %8, %11, %2 op_sel:[0,1,0] op_sel_hi:[1,1,1]\n\t"
-            "v_pk_fma_f16 %4, %8, %12, %4 op_sel:[0,1,0] op_sel_hi:[1,1,1]\n\t"
-            "v_pk_fma_f16 %6, %8, %13, %6 op_sel:[0,1,0] op_sel_hi:[1,1,1]\n\t"
-            "v_pk_fma_f16 %1, %9, %10, %1 op_sel:[0,1,0] op_sel_hi:[1,1,1]\n\t"
-            "v_pk_fma_f16 %3, %9, %11, %3 op_sel:[0,1,0] op_sel_hi:[1,1,1]\n\t"
-            "v_pk_fma_f16 %5, %9, %12, %5 op_sel:[0,1,0] op_sel_hi:[1,1,1]\n\t"
-            "v_pk_fma_f16 %7, %9, %13, %7 op_sel:[0,1,0] op_sel_hi:[1,1,1]"
-            : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4]), "+v"(acc[5]), "+v"(acc[6]), "+v"(acc[7])
-            : "v"(v0), "v"(v1), "v"(f.x), "v"(f.y), "v"(f.z), "v"(f.w));
-    }
+// One key for two of a lane's queries and P pairs of d: x[j] / y[j] hold d pair j of the first / second query, v the key's d pairs,
+// fx / fy the factors of two consecutive keys for the queries as two f16; SEL picks the first or the second of them.
+// (asm with tied operands: the accumulators stay in the registers they are in, whatever branches surround the step)
+#define PK_FMA(acc, v, f, sel) "v_pk_fma_f16 %" #acc ", %" #v ", %" #f ", %" #acc " " sel "\n\t"
+#define PK_LO "op_sel_hi:[1,0,1]"
+#define PK_HI "op_sel:[0,1,0] op_sel_hi:[1,1,1]"
+template <int P, int SEL>
+__device__ __forceinline__ void pk_key(uint32_t (&x)[P], uint32_t (&y)[P], const uint32_t (&v)[P], uint32_t fx, uint32_t fy) {
+    static_assert(P == 2 || P == 4, "4 or 8 d to a lane");
+#define PK_KEY2(sel) asm(PK_FMA(0, 4, 6, sel) PK_FMA(2, 4, 7, sel) PK_FMA(1, 5, 6, sel) PK_FMA(3, 5, 7, sel) \
+                         : "+v"(x[0]), "+v"(x[1]), "+v"(y[0]), "+v"(y[1]) : "v"(v[0]), "v"(v[1]), "v"(fx), "v"(fy))
+#define PK_KEY4(sel) asm(PK_FMA(0, 8, 12, sel) PK_FMA(4, 8, 13, sel) PK_FMA(1, 9, 12, sel) PK_FMA(5, 9, 13, sel) \
+                         PK_FMA(2, 10, 12, sel) PK_FMA(6, 10, 13, sel) PK_FMA(3, 11, 12, sel) PK_FMA(7, 11, 13, sel) \
+                         : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]) \
+                         : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(fx), "v"(fy))
+    if constexpr (P == 2) { if constexpr (SEL == 0) PK_KEY2(PK_LO); else PK_KEY2(PK_HI); }
+    else                  { if constexpr (SEL == 0) PK_KEY4(PK_LO); else PK_KEY4(PK_HI); }
 }
-// acc = f16(acc * ms): m[q] holds -ms of query q in the half SEL picks (the sign is taken off by the instruction)
-template <int SEL>
-__device__ __forceinline__ void pk_scale8(half2_t (&acc)[8], const u32x4 m) {
-    if (SEL == 0) {
-        asm("v_pk_mul_f16 %0, %0, %8 op_sel_hi:[1,0] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %2, %2, %9 op_sel_hi:[1,0] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %4, %4, %10 op_sel_hi:[1,0] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %6, %6, %11 op_sel_hi:[1,0] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %1, %1, %8 op_sel_hi:[1,0] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %3, %3, %9 op_sel_hi:[1,0] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %5, %5, %10 op_sel_hi:[1,0] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %7, %7, %11 op_sel_hi:[1,0] neg_lo:[0,1] neg_hi:[0,1]"
-            : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4]), "+v"(acc[5]), "+v"(acc[6]), "+v"(acc[7])
-            : "v"(m.x), "v"(m.y), "v"(m.z), "v"(m.w));
-    } else {
-        asm("v_pk_mul_f16 %0, %0, %8 op_sel:[0,1] op_sel_hi:[1,1] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %2, %2, %9 op_sel:[0,1] op_sel_hi:[1,1] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %4, %4, %10 op_sel:[0,1] op_sel_hi:[1,1] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %6, %6, %11 op_sel:[0,1] op_sel_hi:[1,1] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %1, %1, %8 op_sel:[0,1] op_sel_hi:[1,1] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %3, %3, %9 op_sel:[0,1] op_sel_hi:[1,1] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %5, %5, %10 op_sel:[0,1] op_sel_hi:[1,1] neg_lo:[0,1] neg_hi:[0,1]\n\t"
-            "v_pk_mul_f16 %7, %7, %11 op_sel:[0,1] op_sel_hi:[1,1] neg_lo:[0,1] neg_hi:[0,1]"
-            : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4]), "+v"(acc[5]), "+v"(acc[6]), "+v"(acc[7])
-            : "v"(m.x), "v"(m.y), "v"(m.z), "v"(m.w));
-    }
-}
-// A key at which some query of the wavefront has a new maximum.  The factor tile marks such a (query, key) by its sign:
-// -ms in place of vs (then vs is exactly 1).  Rescales the accumulators — the queries that stay as they are multiply by 1,
-// which leaves the value — and puts 1 in place of -ms in the factor registers, so that the multiply-add that follows is the
-// same instruction sequence with or without a rescale.  Everything happens in the registers it finds (tied asm operands):
-// written as C++ selects, the compiler gives the changed factors or accumulators new registers and copies them back on the
-// path without a rescale, eight or four v_mov per key on the path that matters.
-template <int SEL>
-__device__ __forceinline__ void pk_rescale(half2_t (&acc)[8], u32x4 & f) {
-    const uint32_t keep = SEL ? 0x0000ffffu : 0xffff0000u, one = SEL ? 0x3c000000u : 0x00003c00u, neg_one = 0xbc00bc00u;
-    u32x4 msn;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        uint32_t fq = f[q], m, t;
-        if (SEL == 0)
-            asm("v_and_b32 %1, 0x8000, %0\n\t"
-                "v_cmp_ne_u32 vcc, 0, %1\n\t"
-                "v_and_or_b32 %2, %0, %3, %5\n\t"
-                "s_nop 0\n\t"
-                "v_cndmask_b32 %1, %4, %0, vcc\n\t"           // -ms, or -1
-                "v_cndmask_b32 %0, %0, %2, vcc"                 // 1 in place of -ms
-                : "+v"(fq), "=&v"(m), "=&v"(t) : "v"(keep), "v"(neg_one), "v"(one) : "vcc");
-        else
-            asm("v_cmp_gt_i32 vcc, 0, %0\n\t"
-                "v_and_or_b32 %2, %0, %3, %5\n\t"
-                "s_nop 0\n\t"
-                "v_cndmask_b32 %1, %4, %0, vcc\n\t"
-                "v_cndmask_b32 %0, %0, %2, vcc"
-                : "+v"(fq), "=&v"(m), "=&v"(t) : "v"(keep), "v"(neg_one), "v"(one) : "vcc");
-        f[q] = fq; msn[q] = m;
-    }
-    pk_scale8<SEL>(acc, msn);
-}
+// acc = f16(acc * ms), a rescale
+__device__ __forceinline__ void pk_scale(uint32_t & acc, uint32_t m) { asm("v_pk_mul_f16 %0, %0, %1" : "+v"(acc) : "v"(m)); }
 // two f32 factors -> one register of two f16 (round to nearest even, as the conversion in front of vdupq_n_f16)
 __device__ __forceinline__ uint32_t pk_factors(float f0, float f1) {
     uint32_t r;
@@ -1256,85 +1192,73 @@ __global__ void __launch_bounds__(512, 2) k_fattn_seq_tile(fa_args a) {
 }
 
 // ------------------------------------------------------------------------------------------------------
-// k_fattn_pk_tile: the tile kernel for the packed-f16 form of the step (MI355X_FA_F16_PK).
+// k_fattn_pk_tile: N > 8, the packed-f16 form of the step (MI355X_FA_F16_PK)
 //
-// Same roles, tiles and barriers as k_fattn_seq_tile.  With 8 instead of 24 vector instructions per key the chains of
-// that kernel's layout (a lane = one query x 16 d, every lane reading the key's 32 bytes of V) are bound by the LDS
-// reads, not by the vector units: a V register that arrives serves one instruction.  Here a lane owns 4 queries x 4 d
-// (lane = query quad l / 16 of the wavefront's 16 queries, d slice l % 16), so a key costs it one 8-byte read of V for
-// 8 instructions, and the factors arrive as f16, two keys to a register and the four queries of the quad side by side:
-// one 16-byte read per pair of keys.  Per key and lane 12 bytes from LDS instead of 36.
-//   factor tile  fp[key pair][query ^ swizzle]: 32 rows of 64 registers, each register the factors of keys 2 p, 2 p + 1
-//                for one query (vs, or -ms where the key raises that query's maximum); the producers' thread (query,
-//                16-key run) writes a column piece of 8, and the swizzle (bit 4 of the query index flipped in the rows
-//                of odd runs) spreads a wavefront's 64 writes over all banks twice instead of 16 banks four times
-//   raise masks  per chain wavefront and tile 64 bits: does key k raise the maximum of any of its 16 queries?  Built
-//                by the producer wavefront that has the same 16 queries; the chain tests them with scalar
-//                instructions, so a pair of keys without a raise costs its 16 multiply-adds and nothing else.
+// A workgroup owns TQ queries of one head and walks the keys in tiles of 64.  Two roles, one barrier per tile: four chain
+// wavefronts, one to a SIMD, walk tile t - 1 key by key, while PW producer wavefronts make the factors of tile t.
+//
+//   chains     a lane owns QL queries x 4 d (lane = query group l / 16, d slice l % 16): a key costs it one read of V for 2 QL
+//              v_pk_fma_f16, and the factors arrive as f16, two keys to a register and the lane's queries side by side.  A block of 16 keys in which no query of the wavefront gets a new maximum is its multiply-adds and nothing
+//              else; the others begin with a rescale of the accumulators.
+//   producers  scores come transposed out of v_mfma_f32_16x16x32_f16 (K rows as the A operand, Q as the B operand, which stays
+//              in registers): lane l holds query l % 16 and the keys 16 b + 4 (l / 16) + e, b, e = 0 .. 3 — so running maximum,
+//              denominator and factors never leave the registers of the lanes they belong to.  A block of 16 keys that
+//              raises no maximum in the wavefront is four exponentials of fma(c, scale, -M) and their sum; the others take the
+//              block's maximum over the four lanes of a query (two lane swaps) first.  The denominator is kept per lane, as the
+//              sum of exp2(s - M) of the lane's own keys, and added up at the end.
+//              K and V rows go from memory straight into LDS (global_load_lds), a tile ahead.
+//   factor tile  fp[key pair][query]: each register the f16 factors vs of keys 2 p, 2 p + 1 for one query; fm[block][query] the
+//                rescale ms in front of a block, for blocks with one.  The four lanes of a query write rows 2 apart: where a row
+//                is a multiple of the banks, those would collide, so the column (and with 32 columns the row of the pair) is
+//                flipped by the lane's group (fp_row, fp_flip).
+// The running maximum moves at the beginning of a block of 16 keys instead of at the key, at most 15 keys early: a key in front of
+// the new maximum takes its factor at the new scale, where the reference takes it at the old one and rescales the sum after it.
+// From the block's end on both are at the same scale, which matters — with flat attention the f16 sum of 1500 keys stagnates
+// in a way that depends on the scale of the factors: with a maximum on a grid of powers of two, whose rescales would be
+// exact, results were 3e-4 NMSE away from the reference's sequence and closer to the exact sum.  Key by key, with a scalar test
+// per key in the chains, a block with a raise cost three times one without.
+//
+// What bounds it: one wavefront issues a vector instruction every 5 clocks (2.3 ns; two on a SIMD one every 1.9 ns), and LDS
+// returns a 16-byte read in 1.84 ns, an 8-byte read in 1.02 ns per CU (and a pair of 8-byte reads as one instruction in
+// 3.4 ns, which is why the addresses are kept apart).  A workgroup that has its CU to itself is one wavefront per SIMD and takes
+// the chain's length times 5 clocks, so a small grid wants few queries to the workgroup, a large one few LDS reads to the
+// multiply-add:
+//   QL = 4, 64 queries   8 multiply-adds to a key: 0.24 ns of LDS each
+//   QL = 2, 32 queries   half the instructions per wavefront; 0.38 ns
+// (A lane of 4 queries x 8 d, 128 queries to the workgroup, 0.17 ns, came out level with QL = 4 at its best.)
+// Measured, us, with the exact per-key form that was here before in front (64 queries, factors as f32 pairs through LDS):
+//   N 1500 x KV 1536 x 20 heads 105 -> QL 4: 85; 12 heads 96 -> 78; 6 heads 73 -> QL 4: 49, QL 2: 58; 487 x 512 x 6: 31 -> QL 2: 17;
+//   227 x 1536 x 20: 73 -> QL 4: 48, QL 2: 40; 27 x 1536 x 12: 70 -> 39; 27 x 256 x 12 with a mask: 22 -> 12
 // ------------------------------------------------------------------------------------------------------
 
-#define P_FP_ROW   T_Q                                    // registers per key-pair row of the factor tile
-#define P_FP_TILE  ((T_KV / 2) * P_FP_ROW)
-#define P_LDS_BYTES ((T_Q * T_LDH + T_KV * T_LDH + 2 * T_KV * FA_D) * 2 + T_Q * T_LDF * 4 + 2 * P_FP_TILE * 4 + 2 * 4 * 2 * 4 + 2 * T_Q * 4)   // 69184
+#define P_KV       64
+#define P_M_START  (-3.0e38f)     // below every score and finite: no difference is (-inf) - (-inf), a masked key gives the factor 0
 
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-// The factor step of a run of 16 scores, written out: s[i] becomes its factor (negated where key i raises the row's maximum),
-// M the running maximum, (P, A) the run's part of the denominator (S_after = S_before * P + A), bit i of `bits` the raise.
-// The common key raises no maximum in the whole wavefront (85 % of the keys of the encoder's launches) and takes the
-// straight path — test, difference, exponential, sum and a branch not taken; a raise anywhere in the wavefront sends it
-// through the general form at the end of the block and back.  As C++ the same loop met after every key in a join
-// for which the compiler copied three to five registers, on the straight path too: nine vector instructions and two taken
-// branches per key.  (The s_nop behind v_exp_f32 is the wait state its result needs in front of a vector instruction.)
-// The factor is 2^-|s - M|: 2^(s - M), or 2^(M - s) where s raises the maximum.  M starts at PKT_M_START, a finite number
-// below every score, so that the difference is never (-inf) - (-inf): a masked key (s = -inf) gives -inf and the factor 0
-// whatever was seen before it, the first real key of a row raises the maximum with the factor 2^-huge = 0, as with -inf.
-#define PKT_M_START (-3.0e38f)
-#define PKT_KEY(i) \
-    "v_cmp_gt_f32 vcc, %[s" #i "], %[M]\n" \
-    "v_sub_f32 %[t], %[s" #i "], %[M]\n" \
-    "s_cbranch_vccnz 1" #i "f\n" \
-    "v_exp_f32_e64 %[s" #i "], -|%[t]|\n" \
-    "s_nop 0\n" \
-    "v_add_f32 %[A], %[A], %[s" #i "]\n" \
-    "2" #i ":\n"
-#define PKT_RAISE(i) \
-    "1" #i ":\n" \
-    "v_max_f32 %[M], %[M], %[s" #i "]\n" \
-    "v_exp_f32_e64 %[ex], -|%[t]|\n" \
-    "s_nop 0\n" \
-    "v_cndmask_b32_e64 %[ms], 1.0, %[ex], vcc\n" \
-    "v_cndmask_b32_e64 %[vs], %[ex], 1.0, vcc\n" \
-    "v_mul_f32 %[P], %[P], %[ms]\n" \
-    "v_fma_f32 %[A], %[A], %[ms], %[vs]\n" \
-    "v_cndmask_b32_e64 %[s" #i "], %[ex], -%[ex], vcc\n" \
-    "v_cndmask_b32_e64 %[ms], 0, 1, vcc\n" \
-    "v_lshl_or_b32 %[bits], %[ms], " #i ", %[bits]\n" \
-    "s_branch 2" #i "b\n"
-__device__ __forceinline__ void pkt_factor_run(float (&sv)[16], float & M, float & P, float & A, uint32_t & bits) {
-    float t, ex, ms, vs;
-    asm volatile(
-        PKT_KEY(0) PKT_KEY(1) PKT_KEY(2) PKT_KEY(3) PKT_KEY(4) PKT_KEY(5) PKT_KEY(6) PKT_KEY(7)
-        PKT_KEY(8) PKT_KEY(9) PKT_KEY(10) PKT_KEY(11) PKT_KEY(12) PKT_KEY(13) PKT_KEY(14) PKT_KEY(15)
-        "s_branch 3f\n"
-        PKT_RAISE(0) PKT_RAISE(1) PKT_RAISE(2) PKT_RAISE(3) PKT_RAISE(4) PKT_RAISE(5) PKT_RAISE(6) PKT_RAISE(7)
-        PKT_RAISE(8) PKT_RAISE(9) PKT_RAISE(10) PKT_RAISE(11) PKT_RAISE(12) PKT_RAISE(13) PKT_RAISE(14) PKT_RAISE(15)
-        "3:\n"
-        : [s0] "+v"(sv[0]), [s1] "+v"(sv[1]), [s2] "+v"(sv[2]), [s3] "+v"(sv[3]), [s4] "+v"(sv[4]), [s5] "+v"(sv[5]), [s6] "+v"(sv[6]), [s7] "+v"(sv[7]),
-          [s8] "+v"(sv[8]), [s9] "+v"(sv[9]), [s10] "+v"(sv[10]), [s11] "+v"(sv[11]), [s12] "+v"(sv[12]), [s13] "+v"(sv[13]), [s14] "+v"(sv[14]), [s15] "+v"(sv[15]),
-          [M] "+v"(M), [P] "+v"(P), [A] "+v"(A), [bits] "+v"(bits), [t] "=&v"(t), [ex] "=&v"(ex), [ms] "=&v"(ms), [vs] "=&v"(vs)
-        : : "vcc");
+__device__ __forceinline__ void wait_loads() {                // everything requested has arrived, rows on their way into LDS included
+    __builtin_amdgcn_s_waitcnt((0 << 14) | (7 << 4) | (15 << 8));
+    __builtin_amdgcn_sched_barrier(0);
 }
 
-__global__ void __launch_bounds__(512, 2) k_fattn_pk_tile(fa_args a) {
+template <int QL> constexpr int p_queries() { return 16 * QL; }                          // four wavefronts of four groups
+template <int QL> constexpr int p_lds_bytes() { return 2 * P_KV * FA_D * 2 * 2 + 2 * (P_KV / 2 + 4) * p_queries<QL>() * 4 + 2 * 4 * 4 + p_queries<QL>() * 4; }
+
+// where a factor tile keeps (key pair, query): register fp_row(pair) + (query ^ fp_flip(pair)); (pair / 2) % 4 is the group of the
+// lane that writes it
+template <int TQ> __device__ __forceinline__ constexpr int fp_row(int pair)  { return TQ >= 64 ? pair * TQ : (pair ^ (pair >> 2 & 1)) * 32; }
+template <int TQ> __device__ __forceinline__ constexpr int fp_flip(int pair) { return TQ >= 64 ? (pair >> 1 & 3) << 4 : (pair >> 1 & 1) << 4; }
+
+template <int QL, int PW>
+__global__ void __launch_bounds__(256 + 64 * PW, 2) k_fattn_pk_tile(fa_args a) {
+    constexpr int TQ = p_queries<QL>(), QB = TQ / (16 * PW);      // QB: blocks of 16 queries per producer wavefront
+    constexpr int FP_TILE = (P_KV / 2) * TQ;
+    constexpr int DL = 4, SL = FA_D / DL, WQ = TQ / 4;                // a lane's d; d slices (lanes of a query group); queries per chain wavefront
     extern __shared__ __attribute__((aligned(16))) char t_smem[];
-    half_t *   q_s  = (half_t *) t_smem;                      // [T_Q * T_LDH]
-    half_t *   k_s  = q_s + T_Q * T_LDH;                      // [T_KV * T_LDH]
-    half_t *   v_s2 = k_s + T_KV * T_LDH;                     // [2][T_KV * FA_D]
-    float *    sc_s = (float *)(v_s2 + 2 * T_KV * FA_D);      // [T_Q * T_LDF]   scores of the tile in work (producers only)
-    uint32_t * fp_s = (uint32_t *)(sc_s + T_Q * T_LDF);       // [2][P_FP_TILE]
-    uint32_t * rm_s = fp_s + 2 * P_FP_TILE;                   // [2][4][2]
-    float *    m_run = (float *)(rm_s + 16), * s_run = m_run + T_Q;
+    char *     k_s   = t_smem;                                // [2][64 rows of 128 bytes], chunks swizzled
+    char *     v_s   = k_s + 2 * P_KV * FA_D * 2;             // [2][64 rows of 128 bytes]
+    uint32_t * fp_s  = (uint32_t *)(v_s + 2 * P_KV * FA_D * 2);
+    uint32_t * fm_s  = fp_s + 2 * FP_TILE;                    // [2][4][TQ]
+    uint32_t * rm_s  = fm_s + 2 * 4 * TQ;                     // [2][PW]     bit b: block b of the tile begins with a rescale
+    float *    s_run = (float *)(rm_s + 2 * PW);              // [TQ]
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1342,218 +1266,305 @@ __global__ void __launch_bounds__(512, 2) k_fattn_pk_tile(fa_args a) {
     const uint32_t lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), total = gridDim.x * gridDim.y * gridDim.z;
     const uint32_t xcd = lin % 8, per = total / 8, extra = total % 8;
     const uint32_t item = xcd * per + (xcd < extra ? xcd : extra) + lin / 8;
-    const int64_t n0 = (int64_t)(item % gridDim.x) * T_Q, h = (item / gridDim.x) % gridDim.y, i3 = item / (gridDim.x * gridDim.y);
-    const int n_tiles = (int)((a.KV + T_KV - 1) / T_KV);
+    const int64_t n0 = (int64_t)(item % gridDim.x) * TQ, h = (item / gridDim.x) % gridDim.y, i3 = item / (gridDim.x * gridDim.y);
+    const int n_tiles = (int)((a.KV + P_KV - 1) / P_KV);
 
     if (wave >= 4) {
         // ---- producers ---------------------------------------------------------------------------------------------------------------
-        const int tid = threadIdx.x - 256, pw = wave - 4;
-        const char * qb = a.q + h * a.q_nb2 + i3 * a.q_nb3;
+        const int pw = wave - 4, r16 = lane & 15, g = lane >> 4;
         const char * kb = a.k + (h / a.hk_ratio) * a.k_nb2 + (i3 / a.k_ne3_ratio) * a.k_nb3;
         const char * vb = a.v + (h / a.hv_ratio) * a.v_nb2 + (i3 / a.v_ne3_ratio) * a.v_nb3;
-        {   // Q tile -> f16 in LDS; thread t: row t/4, 16 values
-            const int r = tid >> 2, c = (tid & 3) * 16;
-            const int64_t n = n0 + r;
+        // Rows of a tile: 8 loads of 8 rows for K and for V, dealt to the wavefronts.  K: row pairs form 256-byte lines, the 16-byte
+        // chunk c of row r sits in slot (r & 1) * 8 + (c ^ (line & 7)), so that the 16 rows of a fragment read cover all banks once.
+        constexpr int LD = 8 / PW;
+        auto load_k = [&](int it) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (n < a.N) t = *(const float4 *)(qb + n * a.q_nb1 + (c + 4 * i) * 4);
-                half4_t hq = { (half_t) t.x, (half_t) t.y, (half_t) t.z, (half_t) t.w };
-                *(half4_t *)(q_s + r * T_LDH + c + 4 * i) = hq;
+            for (int i = 0; i < LD; ++i) {
+                const int j = pw * LD + i, line = 4 * j + g;
+                const int64_t key = (int64_t) it * P_KV + 2 * line + (r16 >> 3);
+                const char * p = kb + (key < a.KV ? key : a.KV - 1) * a.k_nb1 + ((lane & 7) ^ (line & 7)) * 16;      // (past the end: masked)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *) p, (__attribute__((address_space(3))) void *)(k_s + (it & 1) * (P_KV * FA_D * 2) + j * 1024), 16, 0, 0);
             }
-        }
-        if (tid < T_Q) { m_run[tid] = PKT_M_START; s_run[tid] = 0.0f; }
-
-        const int sq = (pw >> 1) * 32, sk = (pw & 1) * 32, l32 = lane & 31, g = lane >> 5;
-        const int kr = tid >> 2, kc = (tid & 3) * 16;
-        const float scale2 = a.scale * LOG2E_F;
-        u32x4 kreg0, kreg1, vreg0, vreg1;
-        auto load_kv = [&](int64_t key0) __attribute__((always_inline)) {
-            const int64_t key = key0 + kr < a.KV ? key0 + kr : a.KV - 1;      // rows past the end repeat the last key; their scores are masked
-            const u32x4 * kp = (const u32x4 *)(kb + key * a.k_nb1 + kc * 2);
-            const u32x4 * vp = (const u32x4 *)(vb + key * a.v_nb1 + kc * 2);
-            kreg0 = kp[0]; kreg1 = kp[1]; vreg0 = vp[0]; vreg1 = vp[1];
         };
-        load_kv(0);
-        *(u32x4 *)(k_s + kr * T_LDH + kc) = kreg0; *(u32x4 *)(k_s + kr * T_LDH + kc + 8) = kreg1;
-
-        for (int it = 0; it <= n_tiles; ++it) {
-            __syncthreads();                               // tile boundary
-            if (it == n_tiles) { __syncthreads(); break; }
-            const int64_t key0 = (int64_t) it * T_KV;
-            half_t * vs_buf = v_s2 + (it & 1) * T_KV * FA_D;
-            *(u32x4 *)(vs_buf + kr * FA_D + kc) = vreg0; *(u32x4 *)(vs_buf + kr * FA_D + kc + 8) = vreg1;
-            if (it + 1 < n_tiles) load_kv(key0 + T_KV);
-
-            {   // ---- scores: S = Q K^T on the matrix cores
-                float16_t c16;
+        auto load_v = [&](int it) __attribute__((always_inline)) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) c16[r] = 0.0f;
+            for (int i = 0; i < LD; ++i) {
+                const int j = pw * LD + i;
+                const int64_t key = (int64_t) it * P_KV + 8 * j + (lane >> 3);
+                const char * p = vb + (key < a.KV ? key : a.KV - 1) * a.v_nb1 + (lane & 7) * 16;                     // (past the end: factor 0, finite values)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *) p, (__attribute__((address_space(3))) void *)(v_s + (it & 1) * (P_KV * FA_D * 2) + j * 1024), 16, 0, 0);
+            }
+        };
+        load_k(0);
+        half8_t qf[QB][2];                                     // this lane's queries, d = 32 s + 8 g .. + 7
+        const char * mrow[QB];
 #pragma unroll
-                for (int kk = 0; kk < FA_D / 16; ++kk) {
-                    const half8_t av = *(const half8_t *)(q_s + (sq + l32) * T_LDH + kk * 16 + 8 * g);
-                    const half8_t bv = *(const half8_t *)(k_s + (sk + l32) * T_LDH + kk * 16 + 8 * g);
-                    c16 = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, c16, 0, 0, 0);
-                }
-                const int64_t key = key0 + sk + l32;
-                const bool key_ok = key < a.KV;
-                // (scores are kept in units of log2 e: the factors are then one v_exp_f32 each)
-                if (!a.mask && key0 + T_KV <= a.KV) {
+        for (int i = 0; i < QB; ++i) {
+            const int64_t nq = n0 + 16 * (QB * pw + i) + r16, n = nq < a.N ? nq : a.N - 1;
+            const char * qp = a.q + n * a.q_nb1 + h * a.q_nb2 + i3 * a.q_nb3 + g * 32;
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int qi = sq + 8 * (r >> 2) + 4 * g + (r & 3);
-                        sc_s[qi * T_LDF + sk + l32] = __fmul_rn(c16[r], scale2);
+            for (int s = 0; s < 2; ++s) {
+                const float4 x = *(const float4 *)(qp + s * 128), y = *(const float4 *)(qp + s * 128 + 16);
+                qf[i][s] = (half8_t){ (half_t) x.x, (half_t) x.y, (half_t) x.z, (half_t) x.w, (half_t) y.x, (half_t) y.y, (half_t) y.z, (half_t) y.w };
+            }
+            mrow[i] = a.mask + n * a.m_nb1;
+        }
+        const bool mask_al8 = ((uintptr_t) a.mask | (uintptr_t) a.m_nb1) % 8 == 0;
+        half4_t mk[QB][4];                                     // mask of the tile in work: keys 16 b + 4 g .. + 3
+        auto load_mask = [&](int it) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < QB; ++i)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const int64_t key = (int64_t) it * P_KV + 16 * b + 4 * g;
+                    if (mask_al8 && key + 3 < a.KV) mk[i][b] = *(const half4_t *)(mrow[i] + key * 2);
+                    else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) mk[i][b][e] = *(const half_t *)(mrow[i] + (key + e < a.KV ? key + e : a.KV - 1) * 2);
                     }
-                } else {
-                    float mv[16];
+                }
+        };
+        if (a.mask) load_mask(0);
+        const bool busy = n0 + 16 * QB * pw < a.N;             // (a tile that dst covers in part)
+        const float scale2 = a.scale * LOG2E_F;                // scores in units of log2 e: a factor is one v_exp_f32
+        const int frow = (r16 >> 1) * 256 + (r16 & 1) * 128, fsw = (r16 >> 1) & 7;
+        float M[QB], S[QB];                                    // running maximum of the query; this lane's share of its denominator
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int qi = sq + 8 * (r >> 2) + 4 * g + (r & 3);
-                        mv[r] = 0.0f;
-                        if (a.mask) {
-                            const int64_t n = n0 + qi < a.N ? n0 + qi : a.N - 1;
-                            mv[r] = (float) *(const half_t *)(a.mask + n * a.m_nb1 + (key_ok ? key : a.KV - 1) * 2);
+        for (int i = 0; i < QB; ++i) { M[i] = P_M_START; S[i] = 0.0f; }
+        wait_loads();
+
+        for (int it = 0; it < n_tiles; ++it) {
+            __syncthreads();                                   // tile boundary: K of tile it is there, the other buffers are free
+            load_v(it);
+            if (it + 1 < n_tiles) load_k(it + 1);
+            if (busy) {
+                float4_t c[QB][4];
+                const char * kt = k_s + (it & 1) * (P_KV * FA_D * 2);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+#pragma unroll
+                    for (int i = 0; i < QB; ++i) c[i][b] = (float4_t){ 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) {
+                        const half8_t kf = *(const half8_t *)(kt + b * 2048 + frow + ((4 * s + g) ^ fsw) * 16);
+#pragma unroll
+                        for (int i = 0; i < QB; ++i) c[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[i][s], c[i][b], 0, 0, 0);
+                    }
+                }
+                const bool plain = !a.mask && (int64_t)(it + 1) * P_KV <= a.KV;                // uniform
+                if (!plain) {
+#pragma unroll
+                    for (int i = 0; i < QB; ++i)
+#pragma unroll
+                        for (int b = 0; b < 4; ++b)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const float s = a.mask ? __builtin_fmaf(c[i][b][e], scale2, (float) mk[i][b][e] * LOG2E_F) : c[i][b][e] * scale2;
+                                c[i][b][e] = (int64_t) it * P_KV + 16 * b + 4 * g + e < a.KV ? s : -INFINITY;
+                            }
+                    if (a.mask && it + 1 < n_tiles) load_mask(it + 1);
+                }
+                uint32_t * fpw = fp_s + (it & 1) * FP_TILE;
+                uint32_t raises = 0;                           // uniform
+                // plain tiles: c * scale2 - M in one instruction (its sign is exact: it is > 0 only if the score is above M)
+                auto block = [&](auto is_plain, int b) __attribute__((always_inline)) {
+                    constexpr bool PLAIN = decltype(is_plain)::value;
+                    float f[QB][4];
+                    bool above = false;
+#pragma unroll
+                    for (int i = 0; i < QB; ++i) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) f[i][e] = PLAIN ? __builtin_fmaf(c[i][b][e], scale2, -M[i]) : c[i][b][e] - M[i];
+                        above = above || fmaxf(fmaxf(f[i][0], f[i][1]), fmaxf(f[i][2], f[i][3])) > 0.0f;
+                    }
+                    if (__any(above)) {
+                        raises |= 1u << b;
+#pragma unroll
+                        for (int i = 0; i < QB; ++i) {
+                            float s[4];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) s[e] = PLAIN ? c[i][b][e] * scale2 : c[i][b][e];
+                            float top = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));       // ... and over lanes +-16, +-32, the query's other keys
+                            const auto w16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(top), __float_as_uint(top), false, false);
+                            top = fmaxf(__uint_as_float(w16[0]), __uint_as_float(w16[1]));
+                            const auto w32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(top), __float_as_uint(top), false, false);
+                            const float Mn = fmaxf(M[i], fmaxf(__uint_as_float(w32[0]), __uint_as_float(w32[1])));
+                            const float ms = __builtin_amdgcn_exp2f(M[i] - Mn);            // 1 where the maximum stands, 0 for the first keys
+                            if (g == 0) fm_s[((it & 1) * 4 + b) * TQ + 16 * (QB * pw + i) + r16] = pk_factors(ms, ms);
+                            S[i] *= ms;
+                            M[i] = Mn;
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) f[i][e] = s[e] - Mn;
                         }
                     }
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int qi = sq + 8 * (r >> 2) + 4 * g + (r & 3);
-                        sc_s[qi * T_LDF + sk + l32] = key_ok ? __builtin_fmaf(c16[r], scale2, mv[r] * LOG2E_F) : -INFINITY;
+                    for (int i = 0; i < QB; ++i) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) f[i][e] = __builtin_amdgcn_exp2f(f[i][e]);
+                        S[i] += (f[i][0] + f[i][1]) + (f[i][2] + f[i][3]);
+                        // (fp_row, fp_flip of the pairs 8 b + 2 g, 8 b + 2 g + 1)
+                        const int col = 16 * (QB * pw + i) + r16;
+                        const uint32_t p0 = pk_factors(f[i][0], f[i][1]), p1 = pk_factors(f[i][2], f[i][3]);
+                        if (TQ >= 64) {
+                            uint32_t * to = fpw + (8 * b + 2 * g) * TQ + (col ^ (g << 4));
+                            to[0] = p0; to[TQ] = p1;
+                        } else {
+                            uint32_t * to = fpw + (8 * b + 2 * g) * 32 + (col ^ ((g & 1) << 4));
+                            to[0] = g & 2 ? p1 : p0; to[32] = g & 2 ? p0 : p1;
+                        }
+                    }
+                };
+                if (plain) {
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) block(std::true_type{}, b);
+                } else {
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) block(std::false_type{}, b);
+                }
+                if (lane == 0) rm_s[(it & 1) * PW + pw] = raises;
+                if (it + 1 == n_tiles) {
+#pragma unroll
+                    for (int i = 0; i < QB; ++i) {
+                        S[i] += __shfl_xor(S[i], 16, WAVE); S[i] += __shfl_xor(S[i], 32, WAVE);
+                        if (g == 0) s_run[16 * (QB * pw + i) + r16] = S[i];
                     }
                 }
             }
-            __syncthreads();                               // scores visible
-
-            {   // ---- factors: thread t: query t/4, keys 16*(t%4) .. +15
-                const int qi = tid >> 2, sgm = tid & 3;
-                const float4 * sp = (const float4 *)(sc_s + qi * T_LDF + sgm * 16);
-                float sv[16], lmax = -INFINITY;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) { const float4 t = sp[i]; sv[4*i] = t.x; sv[4*i+1] = t.y; sv[4*i+2] = t.z; sv[4*i+3] = t.w; }
-#pragma unroll
-                for (int i = 0; i < 16; ++i) lmax = fmaxf(lmax, sv[i]);
-                float M = m_run[qi];
-                const float S0 = s_run[qi];
-                const float m0 = dpp_move<float, 0x00>(lmax), m1 = dpp_move<float, 0x55>(lmax), m2 = dpp_move<float, 0xAA>(lmax);
-                if (sgm > 0) M = fmaxf(M, m0);
-                if (sgm > 1) M = fmaxf(M, m1);
-                if (sgm > 2) M = fmaxf(M, m2);
-                float P = 1.0f, A = 0.0f;
-                uint32_t rbits = 0;                        // bit i: key i of this run raises this query's maximum
-                // sv[i] -> 2^(s - M), or -2^(M - s) where key i raises the maximum (-0.0 keeps the sign)
-                pkt_factor_run(sv, M, P, A, rbits);
-                // f16 factors, two keys to a register, into column (query ^ swizzle) of this run's eight key-pair rows
-                uint32_t * fpw = fp_s + (it & 1) * P_FP_TILE + (8 * sgm) * P_FP_ROW + (qi ^ ((sgm & 1) << 4));
-#pragma unroll
-                for (int j = 0; j < 8; ++j) fpw[j * P_FP_ROW] = pk_factors(sv[2*j], sv[2*j + 1]);
-                // the raise mask of the wavefront's 16 queries: OR over the lanes of a run (lane = 4 * query + run)
-                rbits |= dpp_move<uint32_t, 0x124>(rbits);     // row_ror:4
-                rbits |= dpp_move<uint32_t, 0x128>(rbits);     // row_ror:8
-                rbits |= (uint32_t) __builtin_amdgcn_ds_swizzle((int) rbits, 0x401F);       // lane ^ 16
-                rbits |= (uint32_t) __shfl_xor((int) rbits, 32, WAVE);
-                const uint32_t r1 = dpp_move<uint32_t, 0x55>(rbits), r2 = dpp_move<uint32_t, 0xAA>(rbits), r3 = dpp_move<uint32_t, 0xFF>(rbits);
-                if (lane == 0) *(u32x2 *)(rm_s + ((it & 1) * 4 + pw) * 2) = (u32x2){ rbits | (r1 << 16), r2 | (r3 << 16) };
-                // fold the four runs of this query in key order
-                const float P1 = dpp_move<float, 0x55>(P), A1 = dpp_move<float, 0x55>(A);
-                const float P2 = dpp_move<float, 0xAA>(P), A2 = dpp_move<float, 0xAA>(A);
-                const float P3 = dpp_move<float, 0xFF>(P), A3 = dpp_move<float, 0xFF>(A);
-                const float M3 = dpp_move<float, 0xFF>(M);
-                if (sgm == 0) {
-                    float S = S0 * P + A;
-                    S = S * P1 + A1; S = S * P2 + A2; S = S * P3 + A3;
-                    s_run[qi] = S; m_run[qi] = M3;
-                }
-            }
-            if (it + 1 < n_tiles) { *(u32x4 *)(k_s + kr * T_LDH + kc) = kreg0; *(u32x4 *)(k_s + kr * T_LDH + kc + 8) = kreg1; }
+            wait_loads();                                      // V of this tile and K of the next are in LDS
         }
+        __syncthreads();
         return;
     }
 
-    // ---- chains: lane = (query quad qd, d slice ds) of the wavefront's 16 queries ----------------------------------------------------
+    // ---- chains: lane = (query group qd, d slice ds) -------------------------------------------------------------------------------------
+    // (The chains are what the kernel's time consists of; the producers only have to be done a tile ahead.)
     __builtin_amdgcn_s_setprio(1);
-    const int qd = lane >> 4, ds = lane & 15;
-    half2_t acc[8];                                        // acc[2 q + j]: d pair j of the quad's query q
+    constexpr int P = DL / 2;                                  // d pairs of a lane
+    constexpr int KG = 8;                                      // keys of a group: read together, a group ahead
+    const int qd = lane / SL, ds = lane % SL;
+    uint32_t acc[QL][P];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] = (half2_t){ (half_t) 0.0f, (half_t) 0.0f };
-    const int fcol = 16 * wave + 4 * qd;
+    for (int q = 0; q < QL; ++q)
+#pragma unroll
+        for (int j = 0; j < P; ++j) acc[q][j] = 0;
+    const int fcol = WQ * wave + QL * qd;
+    const bool busy = n0 + WQ * wave < a.N;
 
     for (int it = 0; it <= n_tiles; ++it) {
-        __syncthreads();                                   // tile boundary: tile it - 1 has its factors, its masks and its V rows
-        int barriers = 0;
-        if (it > 0) {
-            const int64_t key0 = (int64_t)(it - 1) * T_KV;
-            const int nk = (int)(a.KV - key0 < T_KV ? a.KV - key0 : T_KV);       // uniform
-            const int buf = (it - 1) & 1;
-            const uint32_t * fpb = fp_s + buf * P_FP_TILE;
-            const char * vbase = (const char *)(v_s2 + buf * T_KV * FA_D) + 8 * ds;     // + key * 128
-            const u32x2 mv = *(const u32x2 *)(rm_s + (buf * 4 + wave) * 2);
-            const uint32_t mlo = __builtin_amdgcn_readfirstlane(mv.x), mhi = __builtin_amdgcn_readfirstlane(mv.y);
-            // one group = four pairs of keys: their factors (a 16-byte read per pair) and their V values (an 8-byte read per key);
-            // the next group is read while this one is walked.  (Keys past the end carry factors of exactly 0 and the last
-            // key's finite V values: walking them changes nothing, so groups are walked whole.)
-            struct pgroup { u32x4 f[4]; u32x2 v[8]; };
-            auto gload = [&](pgroup & gr, int kp0, int swz) __attribute__((always_inline)) {
+        __syncthreads();                                       // tile boundary: tile it - 1 has its factors and its V rows
+        if (it == 0 || !busy) continue;
+        const int64_t key0 = (int64_t)(it - 1) * P_KV;
+        const int nk = (int)(a.KV - key0 < P_KV ? a.KV - key0 : P_KV);               // uniform
+        const int buf = (it - 1) & 1;
+        // every address of a group in a register of its own, so that no two reads look like neighbours to the compiler
+        const char * vb[KG];
+        const char * fb[8];                                    // (fp_row and fp_flip repeat every eight pairs)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) gr.f[j] = *(const u32x4 *)(fpb + (kp0 + j) * P_FP_ROW + (fcol ^ swz));
-#pragma unroll
-                for (int j = 0; j < 8; ++j) gr.v[j] = *(const u32x2 *)(vbase + (2 * kp0 + j) * (FA_D * 2));
-            };
-            // bits: two per pair of keys, lowest first: does the first / the second key of the pair raise a maximum in this wavefront.
-            // Only the rescale sits behind the (scalar) test; the multiply-adds are the same instructions on either path.
-            auto walk = [&](pgroup & gr, uint32_t bits) __attribute__((always_inline)) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (bits & (1u << (2*j))) pk_rescale<0>(acc, gr.f[j]);
-                    pk_mad8<0>(acc, gr.v[2*j].x, gr.v[2*j].y, gr.f[j]);
-                    if (bits & (2u << (2*j))) pk_rescale<1>(acc, gr.f[j]);
-                    pk_mad8<1>(acc, gr.v[2*j + 1].x, gr.v[2*j + 1].y, gr.f[j]);
-                }
-            };
-            auto arrived = [&](const pgroup & gr) __attribute__((always_inline)) {
-                asm volatile("" :: "v"(gr.f[3].w), "v"(gr.v[7].y));
-                __builtin_amdgcn_sched_barrier(0);
-            };
-            pgroup ga, gb;
-            gload(ga, 0, 0);
-            const int n_runs = (nk + 15) >> 4;             // runs of 16 keys = 8 pairs = two groups
-            for (int u = 0; u < n_runs; ++u) {
-                const uint32_t fld = ((u & 2) ? mhi : mlo) >> (16 * (u & 1));
-                const int swz = (u & 1) << 4;
-                arrived(ga);
-                gload(gb, 8 * u + 4, swz);
-                __builtin_amdgcn_sched_barrier(0);
-                walk(ga, fld & 0xffu);
-                arrived(gb);
-                gload(ga, u < 3 ? 8 * u + 8 : 0, u < 3 ? swz ^ 16 : 0);     // (behind the last group: any readable group, nobody walks it)
-                __builtin_amdgcn_sched_barrier(0);
-                walk(gb, (fld >> 8) & 0xffu);
-                // the producers' meeting point: after 16 keys their scores are written; the other 48 keys are the time their
-                // factor step has
-                if (u == 0) { __syncthreads(); ++barriers; }
-            }
+        for (int j = 0; j < KG; ++j) {
+            uint32_t at = (uint32_t)(buf * (P_KV * FA_D * 2) + 2 * DL * ds + 128 * j);
+            asm volatile("" : "+v"(at));
+            vb[j] = v_s + at;
         }
-        for (; barriers < 1; ++barriers) __syncthreads();
-    }
-
-    // ---- results: a lane holds 4 d of 4 queries
-    const int64_t nq0 = n0 + 16 * wave + 4 * qd;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int64_t n = nq0 + q;
-        const float inv = 1.0f / s_run[16 * wave + 4 * qd + q];
-        const float o[4] = { (float) acc[2*q][0] * inv, (float) acc[2*q][1] * inv, (float) acc[2*q + 1][0] * inv, (float) acc[2*q + 1][1] * inv };
-        if (a.d && n < a.N) *(float4 *)((float *) a.d + ((i3 * a.N + n) * a.H + h) * FA_D + 4 * ds) = make_float4(o[0], o[1], o[2], o[3]);
+        for (int j = 0; j < 8; ++j) {
+            uint32_t at = (uint32_t)(buf * FP_TILE + fp_row<TQ>(j) + (fcol ^ fp_flip<TQ>(j))) * 4;
+            if (QL == 2) asm volatile("" : "+v"(at));          // (16-byte reads are not merged)
+            fb[j] = (const char *) fp_s + at;
+        }
+        const uint32_t * fmb = fm_s + buf * 4 * TQ + fcol;
+        const uint32_t raises = __builtin_amdgcn_readfirstlane(rm_s[buf * PW + PW * wave / 4]);
+        // a group's factors (a read per pair of keys) and V values (a read per key); the next group is read while this one is
+        // walked.  (Keys past the end carry factors of exactly 0 and the last key's finite V values: walking them changes nothing,
+        // so groups are walked whole.)
+        struct pgroup { uint32_t f[KG / 2][QL]; uint32_t v[KG][P]; };
+        auto gload = [&](pgroup & gr, auto u) __attribute__((always_inline)) {       // u: group of the tile
+            constexpr int k0 = KG * decltype(u)::value;
+#pragma unroll
+            for (int j = 0; j < KG / 2; ++j) {
+                const int pair = k0 / 2 + j;
+                const char * row = fb[pair % 8] + pair / 8 * (8 * TQ * 4);
+                if constexpr (QL == 4) { const u32x4 t = *(const u32x4 *) row; gr.f[j][0] = t.x; gr.f[j][1] = t.y; gr.f[j][2] = t.z; gr.f[j][3] = t.w; }
+                else                   { const u32x2 t = *(const u32x2 *) row; gr.f[j][0] = t.x; gr.f[j][1] = t.y; }
+            }
+#pragma unroll
+            for (int j = 0; j < KG; ++j) {
+                const u32x2 t = *(const u32x2 *)(vb[j] + k0 * 128);
+                gr.v[j][0] = t.x; gr.v[j][1] = t.y;
+            }
+        };
+        auto key = [&](auto sel, pgroup & gr, int k) __attribute__((always_inline)) {
+#pragma unroll
+            for (int q = 0; q < QL; q += 2) pk_key<P, decltype(sel)::value>(acc[q], acc[q + 1], gr.v[k], gr.f[k / 2][q], gr.f[k / 2][q + 1]);
+        };
+        using first = std::integral_constant<int, 0>; using second = std::integral_constant<int, 1>;
+        // acc = f16(acc * ms) in front of block b
+        auto rescale = [&](int b) __attribute__((always_inline)) {
+            uint32_t m[QL];
+#pragma unroll
+            for (int q = 0; q < QL; ++q) m[q] = fmb[b * TQ + q];
+#pragma unroll
+            for (int q = 0; q < QL; ++q)
+#pragma unroll
+                for (int j = 0; j < P; ++j) pk_scale(acc[q][j], m[q]);
+        };
+        auto walk = [&](pgroup & gr) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < KG; k += 2) { key(first{}, gr, k); key(second{}, gr, k + 1); }
+        };
+        auto arrived = [&](const pgroup & gr) __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);                 // (behind the steps in front of it: the scheduler would lift the wait above them)
+            asm volatile("" :: "v"(gr.f[KG / 2 - 1][QL - 1]), "v"(gr.v[KG - 1][P - 1]));
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        pgroup ga, gb;
+        gload(ga, first{});
+        // two groups; W = 2 KG keys from u2 W on
+        auto run = [&](auto u2) __attribute__((always_inline)) {
+            constexpr int u = decltype(u2)::value, W = 2 * KG;
+            arrived(ga);
+            gload(gb, std::integral_constant<int, 2 * u + 1>{});
+            __builtin_amdgcn_sched_barrier(0);
+            if (u * W % 16 == 0 && (raises & (1u << (u * W / 16)))) rescale(u * W / 16);
+            walk(ga);
+            arrived(gb);
+            gload(ga, std::integral_constant<int, (u + 1) * W < P_KV ? 2 * u + 2 : 0>{});      // (behind the last group: any readable group, nobody walks it)
+            __builtin_amdgcn_sched_barrier(0);
+            walk(gb);
+        };
+        auto runs = [&](auto... us) __attribute__((always_inline)) { (((int) decltype(us)::value * 2 * KG < nk ? run(us) : (void) 0), ...); };
+        runs(first{}, second{}, std::integral_constant<int, 2>{}, std::integral_constant<int, 3>{});
+    }
+    if (!busy) return;
+
+    // ---- results: a lane holds DL d of QL queries
+#pragma unroll
+    for (int q = 0; q < QL; ++q) {
+        const int64_t n = n0 + fcol + q;
+        const float inv = 1.0f / s_run[fcol + q];
+        float o[DL];
+#pragma unroll
+        for (int j = 0; j < P; ++j) { half2_t t; __builtin_memcpy(&t, &acc[q][j], 4); o[2 * j] = (float) t[0] * inv; o[2 * j + 1] = (float) t[1] * inv; }
+        const int64_t row = ((i3 * a.N + n) * a.H + h) * FA_D + DL * ds;
+        if (a.d && n < a.N) {
+#pragma unroll
+            for (int j = 0; j < DL; j += 4) *(float4 *)((float *) a.d + row + j) = make_float4(o[j], o[j + 1], o[j + 2], o[j + 3]);
+        }
         if (a.x16) {
-            // the Q8_0-rounded f16 image of the row for the projection that follows: a block is 32 d, eight lanes of a row
-            float amax = fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fmaxf(fabsf(o[2]), fabsf(o[3])));
-            amax = lanes_max<8>(amax);
+            // the Q8_0-rounded f16 image of the row for the projection that follows: a block is 32 d, 32 / DL lanes of a row
+            float amax = 0.0f;
+#pragma unroll
+            for (int j = 0; j < DL; ++j) amax = fmaxf(amax, fabsf(o[j]));
+            amax = lanes_max<32 / DL>(amax);
             if (n < a.N) {
                 const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
                 const float dq = h2f(f2h_bits(div127(amax)));
-                half4_t hx;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) hx[e] = (half_t)((rintf(o[e] * id) + 0.0f) * dq);
-                *(half4_t *)(a.x16 + ((i3 * a.N + n) * a.H + h) * FA_D + 4 * ds) = hx;
+                for (int j = 0; j < DL; j += 4) {
+                    half4_t hx;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) hx[e] = (half_t)((rintf(o[j + e] * id) + 0.0f) * dq);
+                    *(half4_t *)(a.x16 + row + j) = hx;
+                }
             }
         }
     }
@@ -1790,6 +1801,12 @@ extern "C" size_t mi355x_flash_attn_ext_workspace_size(const mi355x_tensor * q, 
     return 0;
 }
 
+template <int QL, int PW>
+static void launch_pk_tile(const fa_args & a, dim3 grid, hipStream_t st) {
+    grid.x = (unsigned)((a.N + p_queries<QL>() - 1) / p_queries<QL>());
+    k_fattn_pk_tile<QL, PW><<<grid, 256 + 64 * PW, p_lds_bytes<QL>(), st>>>(a);
+}
+
 static int flash_attn_ext(const mi355x_tensor * q, const mi355x_tensor * k, const mi355x_tensor * v,
                           const mi355x_tensor * mask, const mi355x_tensor * mask_f16, const mi355x_tensor * dst, float scale, int mode,
                           void * workspace, size_t workspace_size, void * stream) {
@@ -1875,18 +1892,21 @@ static int flash_attn_ext(const mi355x_tensor * q, const mi355x_tensor * k, cons
             const int64_t gx = (N + T_Q - 1) / T_Q;
             if (gx > 0x7fffffff) return MI355X_ERR_UNSUPPORTED;
             dim3 grid((unsigned) gx, (unsigned) H, (unsigned) q->ne[3]);
-            // per device and kernel: they ask for more LDS than a launch gets by default
-            static std::atomic<bool> configured[64][2];
+            if (mode == MI355X_FA_F16_PK) {
+                // 32 queries to the workgroup while every workgroup has a CU of its own that way, 64 from there on: two workgroups of
+                // 32 on a CU take longer than one of 64 (58 to 49 us at N 1500 x KV 1536 x 6 heads)
+                if ((N + 31) / 32 * H * q->ne[3] <= 256) launch_pk_tile<2, 2>(a, grid, st);
+                else                                     launch_pk_tile<4, 4>(a, grid, st);
+                break;
+            }
+            static std::atomic<bool> configured[64];            // per device: the kernel asks for more LDS than a launch gets by default
             int dev = 0;
             if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) { (void) hipGetLastError(); return MI355X_ERR_HIP; }
-            const int pk = mode == MI355X_FA_F16_PK;
-            if (!configured[dev][pk].load(std::memory_order_acquire)) {
-                const void * fn = pk ? (const void *) k_fattn_pk_tile : (const void *) k_fattn_seq_tile;
-                if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, pk ? (int) P_LDS_BYTES : (int) T_LDS_BYTES) != hipSuccess) { (void) hipGetLastError(); return MI355X_ERR_HIP; }
-                configured[dev][pk].store(true, std::memory_order_release);
+            if (!configured[dev].load(std::memory_order_acquire)) {
+                if (hipFuncSetAttribute((const void *) k_fattn_seq_tile, hipFuncAttributeMaxDynamicSharedMemorySize, (int) T_LDS_BYTES) != hipSuccess) { (void) hipGetLastError(); return MI355X_ERR_HIP; }
+                configured[dev].store(true, std::memory_order_release);
             }
-            if (pk) k_fattn_pk_tile<<<grid, 512, P_LDS_BYTES, st>>>(a);
-            else    k_fattn_seq_tile<<<grid, 512, T_LDS_BYTES, st>>>(a);
+            k_fattn_seq_tile<<<grid, 512, T_LDS_BYTES, st>>>(a);
         } break;
         case FA_K_MFMA: {
             const int64_t gx = (N + M_Q - 1) / M_Q;
