@@ -550,6 +550,43 @@ def test_norm_mul_mat_group(pkg, oracle, gpu, wtype, n, k, m, count):
         assert lib.mi355x_norm_mul_mat_group(tl, tl, 1e-5, None, None, (pkg.MulMatItem * 1)(), 1, None, 0, gpu.stream) in (-1, -2)
 
 
+@pytest.mark.parametrize("wtype,n,k,m,count,emit", [("Q8_0", 8, 32, 33, 1, False), ("Q5_0", 4, 544, 31, 8, False), ("Q8_0", 1, 1024, 4097, 1, False), ("Q5_0", 7, 2048, 100, 3, False),
+                                                   ("Q8_0", 3, 1312, 2080, 1, True), ("Q5_0", 8, 1056, 32, 1, True), ("Q8_0", 6, 480, 1120, 1, True), ("Q5_0", 2, 768, 4128, 1, True),
+                                                   ("Q8_0", 5, 512, 16384, 1, False), ("Q8_0", 5, 512, 16416, 1, True)])
+def test_norm_mul_mat_group_workgroup_sizes(pkg, oracle, gpu, own_numbers, wtype, n, k, m, count, emit):
+    # workgroups of 8 and 16 wavefronts, 16, 32 and 64 lanes to a row, rows that end inside a lane's pieces, the last size in one
+    # launch and the first in two: the same rows, Q8_0 forms and products as mi355x_norm_emit_q8_0 followed by mi355x_mul_mat_group
+    lib, t = pkg.kernels(), getattr(pkg, wtype)
+    x, w, b, bias = rnd((n, k), 2.0, 0.3), rnd((k,), 0.02, 1.0), rnd((k,), 0.02), rnd((m,), 0.5)
+    d_x, d_w, d_b, d_bias = gpu.up(x), gpu.up(w), gpu.up(b), gpu.up(bias)
+    mats = [oracle.quantize(t, rnd((m, k), 0.02)) for _ in range(count)]
+    d_m = [gpu.up(q) for q in mats]
+    tws, tx = [pkg.tensor(q, t, ne=[k, m]) for q in d_m], pkg.tensor(d_x, pkg.F32)
+    need = lib.mi355x_mul_mat_workspace_size(tws[0], tx)
+
+    def run(fused):
+        d_y, ws = torch.zeros_like(d_x), torch.zeros(need, dtype=torch.uint8, device=gpu.dev)
+        image = torch.zeros(n * m * 2, dtype=torch.uint8, device=gpu.dev)
+        outs = [torch.zeros((n, m), dtype=torch.float32, device=gpu.dev) for _ in range(count)]
+        tds, ty, epi = [pkg.tensor(o, pkg.F32) for o in outs], pkg.tensor(d_y, pkg.F32), pkg.Epilogue()
+        epi.flags, epi.scale, epi.bias, epi.image = pkg.EPI_BIAS | (pkg.EPI_GELU | pkg.EPI_EMIT_Q8_0 if emit else 0), 1.0, d_bias.data_ptr(), image.data_ptr()
+        items = (pkg.MulMatItem * count)()
+        for i in range(count):
+            items[i].src0, items[i].dst, items[i].epi = C.pointer(tws[i]), C.pointer(tds[i]), C.pointer(epi)
+        if fused:
+            pkg.check(lib.mi355x_norm_mul_mat_group(tx, ty, 1e-5, d_w.data_ptr(), d_b.data_ptr(), items, count, ws.data_ptr(), need, gpu.stream))
+        else:
+            pkg.check(lib.mi355x_norm_emit_q8_0(tx, ty, 1e-5, d_w.data_ptr(), d_b.data_ptr(), ws.data_ptr(), gpu.stream))
+            pkg.check(lib.mi355x_mul_mat_group(items, count, ty, pkg.MM_WS_READY, ws.data_ptr(), need, gpu.stream))
+        return gpu.down(d_y), gpu.down(ws)[: n * k + n * (k // 32) * 8], gpu.down(image), *[gpu.down(o) for o in outs]
+
+    fused = run(True)
+    for one, two in zip(fused, run(False)):
+        assert np.array_equal(one, two)
+    want = oracle.mul_mat(t, mats[-1], fused[0]) + bias
+    assert oracle.nmse(fused[-1], oracle.gelu(want) if emit else want) <= (1e-8 if emit else 1e-10)
+
+
 @pytest.mark.parametrize("wtype,ttype,n,k,m,count", [("Q8_0", "Q8_0", 5, 1280, 1280, 3), ("Q5_0", "F16", 3, 512, 512, 3), ("Q8_0", "F16", 8, 384, 384, 3),
                                                      ("Q5_0", "Q8_0", 1, 1280, 1280, 3), ("Q8_0", "Q8_0", 2, 768, 768, 1), ("Q5_0", "Q5_0", 5, 1280, 1280, 3),
                                                      ("Q5_0", "Q5_0", 7, 512, 512, 3)])

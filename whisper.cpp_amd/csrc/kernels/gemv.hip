@@ -218,54 +218,67 @@ __global__ void __launch_bounds__(256) k_quantize_x_q8(const char * __restrict__
     }
 }
 
+// rows of a launch up to which a product is a matter of latency (a layer's products; a vocabulary is a stream)
+#define GEMV_SHORT_ROWS 16384
+// lanes per row there: a block of 32 weights per lane (K <= 2048)
+static constexpr int gemv_row_lanes(int nbk) { return nbk <= 16 ? 16 : nbk <= 32 ? 32 : 64; }
+
 // The product over activations quantized ahead (a.x: the layout above, NC rows).  Lane j of a row's LPR lanes owns blocks
 // j, j + LPR, ... (NB of them) of EVERY row it visits, so its slices of the activations are read once and stay in
 // registers while the workgroup walks its row groups: the loop is weight loads and integer dot products only.  With
 // the activations in LDS, their reads (NC x 32 bytes per 34-byte block) are what bounds the kernel, and quantizing them
 // in every workgroup costs more than the product itself once K is large.
+//
+// `prologue`: what makes those activations, when they are not in the workspace yet (the fused LayerNorm leaves them in LDS).
+// Its wavefronts request their rows BEFORE their first weight blocks (request(); request_late(), if there is one, the loads
+// whose addresses those fetched, after the weight blocks) and finish() waits for the rows only: loads are waited for in the
+// order they were issued, so the LayerNorm's reductions run while the weight blocks are on their way.  Wavefronts without a row
+// go straight to their weights: the two sides of the branch request them separately, because a load behind a join is waited for
+// as if it had been issued last.
 struct gemv_no_prologue {
+    static constexpr int ROWS = 0;                  // wavefronts that have a row to normalize
     static constexpr bool LATE = false;
     __device__ __forceinline__ void request() {}
     __device__ __forceinline__ void request_late() {}
-    __device__ __forceinline__ const char * finish(const char * x) { return x; }
+    __device__ __forceinline__ void finish() {}
+    __device__ __forceinline__ const char * publish(const char * x) { return x; }
 };
 
-// `prologue` has two halves: request() issues its own loads BEFORE the first weight blocks are requested (request_late(),
-// if it has one, the loads that depend on those, after the first weight blocks), finish() runs
-// after them and returns where the quantized activations are (the plain product: the workspace as passed; the fused
-// LayerNorm first produces them in LDS).  Loads are waited for in the order they were issued, so in this order the
-// LayerNorm's reductions run while the weight blocks are still on their way from HBM (vmcnt(3) in front of them, where
-// the other order had vmcnt(0)); every load up to finish() is unconditional (clamped address, value masked where it is
-// used), because behind a branch the compiler waits for all loads, not for a count.  Measured, the launch takes the
-// same 10.3 us either way: what the LayerNorm adds to the bare product is its own dependent chain (two reductions, the
-// block maxima, a barrier, the LDS round trip of the quantized rows), not a wait it shares with the weights.
-template <int T0, int NC, int LPR, int NB, typename PRO = gemv_no_prologue>
-__device__ __forceinline__ void gemv_qr_rows(const mm_args & a, PRO prologue = PRO()) {
+//
+// walk: how the workgroups share the row groups, worked out by the host (the size of the workgroup or of the grid is a trip to
+// memory of its own on the device, and a division a hundred instructions)
+struct gemv_walk {
+    int waves_log2;      // wavefronts of a workgroup
+    int n_groups;        // groups of rows, each what a workgroup's wavefronts do at a time
+    int step;            // groups between two of a workgroup (the grid; 1 with the Q8_0 emission)
+    int run;             // Q8_0 emission: groups of a workgroup, else 0
+};
+
+template <int T0, int NC, int LPR, int NB, int W_MAX, typename PRO = gemv_no_prologue>
+__device__ __forceinline__ void gemv_qr_rows(const mm_args & a, const gemv_walk & walk, PRO prologue = PRO()) {
     const int64_t K = a.K;
     const int nbk = (int)(K / QK);
 
     constexpr int RPW = WAVE / LPR;                 // rows per wavefront
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int RPW_LOG2 = LPR == 16 ? 2 : LPR == 32 ? 1 : 0, QK_LOG2 = 5;
+    const int rpg_log2 = walk.waves_log2 + RPW_LOG2, rpg = 1 << rpg_log2;   // rows of a group
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane % LPR, r = lane / LPR;
-    const int64_t n_groups = (a.M + 4 * RPW - 1) / (4 * RPW);
     // MI355X_EPI_EMIT_Q8_0: the results are also left quantized to Q8_0 for the product that reads them next.  A Q8_0 block is
-    // 32 consecutive rows, GPB groups of this kernel, so the groups are then dealt in runs (workgroup b: groups b T .. b T + T - 1,
-    // T a multiple of GPB) instead of round-robin, the results of a block meet in LDS and the workgroup rounds them.
-    constexpr int GPB = QK / (4 * RPW);
+    // 32 consecutive rows, 2^gpb_log2 groups of this kernel (or a group is whole blocks), so the groups are then dealt in runs (workgroup
+    // b: groups b T .. b T + T - 1, T a multiple of those) instead of round-robin, the results of a block meet in LDS and the
+    // workgroup rounds them.
+    const int gpb_log2 = rpg_log2 < QK_LOG2 ? QK_LOG2 - rpg_log2 : 0, unit_log2 = rpg_log2 < QK_LOG2 ? QK_LOG2 : rpg_log2;
     const bool emit_q8 = (a.e.flags & MI355X_EPI_EMIT_Q8_0) != 0;                          // uniform
-    const int64_t run = emit_q8 ? GPB * ((n_groups + (int64_t) GPB * gridDim.x - 1) / ((int64_t) GPB * gridDim.x)) : 0;
-    const int64_t group_end = emit_q8 ? (n_groups < (blockIdx.x + 1) * run ? n_groups : (blockIdx.x + 1) * run) : n_groups;
-    const int64_t group_step = emit_q8 ? 1 : gridDim.x;
-    __shared__ float q8_rows[MI355X_GEMV_MAX_COLS][QK];
-    int64_t group = emit_q8 ? blockIdx.x * run : blockIdx.x;
+    const int group_end = emit_q8 ? min(walk.n_groups, ((int) blockIdx.x + 1) * walk.run) : walk.n_groups;
+    __shared__ float q8_rows[NC][W_MAX * RPW < QK ? QK : W_MAX * RPW];
+    int group = emit_q8 ? (int) blockIdx.x * walk.run : (int) blockIdx.x;
     const bool idle = emit_q8 && group >= group_end;    // (a grid larger than the runs need: such a workgroup walks one group without storing)
-    int64_t row = group * (4 * RPW) + wave * RPW + r;
+    int64_t row = ((int64_t) group << rpg_log2) + wave * RPW + r;
     bool row_ok = row < a.M && !idle;
     const uint8_t * wrow = (const uint8_t *) a.w + (row_ok ? row : 0) * a.w_nb1;
 
     // a lane whose block index lies beyond the row reads the row's last block again and counts it with a zero scale
-    prologue.request();
-    __builtin_amdgcn_sched_barrier(0);                  // (the scheduler would hoist the weight loads above them again)
     wraw<T0> blk[NB];
     bool blk_ok[NB];
 #pragma unroll
@@ -274,13 +287,28 @@ __device__ __forceinline__ void gemv_qr_rows(const mm_args & a, PRO prologue = P
 #pragma unroll
         for (int b = 0; b < NB; ++b) blk[b] = load_wraw<T0>(wrow, blk_ok[b] ? j + b * LPR : nbk - 1);
     };
-    load_blocks();
-    if constexpr (PRO::LATE) {                          // loads whose addresses request() fetched: behind the first weight blocks
-        __builtin_amdgcn_sched_barrier(0);
-        prologue.request_late();
+    // the epilogue operands are fetched early, under the weight stream: lane j of a row stores column j
+    float e_bias = 0.0f, e_bcol = 0.0f, e_res = 0.0f;
+    auto fetch_epilogue = [&]() __attribute__((always_inline)) {
+        if (row_ok && j < NC) {
+            if (a.e.flags & MI355X_EPI_BIAS)     e_bias = a.e.bias[row];
+            if (a.e.flags & MI355X_EPI_BIAS_COL) e_bcol = a.e.bias[j];
+            if (a.e.flags & MI355X_EPI_RESIDUAL) e_res  = *(const float *)(a.e.residual + j * a.d_nb1 + row * 4);
+        }
+    };
+    if (wave < PRO::ROWS) {                             // uniform
+        prologue.request();
+        __builtin_amdgcn_sched_barrier(0);              // (the scheduler would hoist the weight loads above them again)
+        load_blocks();
+        if constexpr (PRO::LATE) {
+            __builtin_amdgcn_sched_barrier(0);
+            prologue.request_late();
+        }
+        prologue.finish();
+    } else {
+        load_blocks();
     }
-
-    const char * xbase = prologue.finish(a.x);
+    const char * xbase = prologue.publish(a.x);
     const int32_t * xq   = (const int32_t *) xbase;
     const float *   xd   = (const float *)(xbase + (size_t) NC * K);
     const int32_t * xsum = (const int32_t *)(xbase + (size_t) NC * K + (size_t) NC * nbk * 4);
@@ -299,24 +327,6 @@ __device__ __forceinline__ void gemv_qr_rows(const mm_args & a, PRO prologue = P
             xo[n][b] = T0 == MI355X_TYPE_Q5_0 ? 16 * xsum[n * nbk + kb] : 0;
         }
     }
-
-    // the epilogue operands of the lane that will store are fetched early, under the weight stream
-    float e_bias = 0.0f, e_bcol[NC], e_res[NC];
-#pragma unroll
-    for (int n = 0; n < NC; ++n) { e_bcol[n] = 0.0f; e_res[n] = 0.0f; }
-    auto fetch_epilogue = [&]() __attribute__((always_inline)) {
-        if (row_ok && j == 0) {
-            if (a.e.flags & MI355X_EPI_BIAS) e_bias = a.e.bias[row];
-            if (a.e.flags & MI355X_EPI_BIAS_COL) {
-#pragma unroll
-                for (int n = 0; n < NC; ++n) e_bcol[n] = a.e.bias[n];
-            }
-            if (a.e.flags & MI355X_EPI_RESIDUAL) {
-#pragma unroll
-                for (int n = 0; n < NC; ++n) e_res[n] = *(const float *)(a.e.residual + n * a.d_nb1 + row * 4);
-            }
-        }
-    };
     fetch_epilogue();
 
     for (;;) {
@@ -324,17 +334,14 @@ __device__ __forceinline__ void gemv_qr_rows(const mm_args & a, PRO prologue = P
 #pragma unroll
         for (int b = 0; b < NB; ++b) cur[b] = blk[b];
         const int64_t done_row = row;
-        const bool done_writer = row_ok && j == 0;
-        const float o_bias = e_bias;
-        float o_bcol[NC], o_res[NC];
-#pragma unroll
-        for (int n = 0; n < NC; ++n) { o_bcol[n] = e_bcol[n]; o_res[n] = e_res[n]; }
+        const bool done_writer = row_ok && j < NC;
+        const float o_bias = e_bias, o_bcol = e_bcol, o_res = e_res;
         // the next row's blocks and epilogue operands travel while this row is worked on
-        const int64_t done_group = group;
-        group += group_step;
+        const int done_group = group;
+        group += walk.step;
         const bool more = group < group_end;                // uniform
         if (more) {
-            row = group * (4 * RPW) + wave * RPW + r;
+            row = ((int64_t) group << rpg_log2) + wave * RPW + r;
             row_ok = row < a.M;
             wrow = (const uint8_t *) a.w + (row_ok ? row : 0) * a.w_nb1;
             load_blocks();
@@ -369,32 +376,33 @@ __device__ __forceinline__ void gemv_qr_rows(const mm_args & a, PRO prologue = P
         }
 #pragma unroll
         for (int n = 0; n < NC; ++n) acc[n] = lanes_sum<LPR>(acc[n]);
-        if (done_writer) {
-            const bool out_f16 = a.e.flags & MI355X_EPI_OUT_F16;
+        // lane j takes column j: one epilogue and one store per lane, and the GELU table's entries of a row come in one trip
+        float v = acc[0];
 #pragma unroll
-            for (int n = 0; n < NC; ++n) {
-                float v = acc[n] + o_bias + o_bcol[n];          // at most one of the two biases is set
-                if (a.e.flags & MI355X_EPI_GELU)     v  = gelu_f32(v, a.e.gelu);
-                if (a.e.flags & MI355X_EPI_SCALE)    v *= a.e.scale;
-                if (a.e.flags & MI355X_EPI_RESIDUAL) v += o_res[n];
-                if (out_f16) *(half_t *)(a.d + n * a.d_nb1 + done_row * 2) = (half_t) v;
-                else         *(float  *)(a.d + n * a.d_nb1 + done_row * 4) = v;
-                if (emit_q8) q8_rows[n][(int)(done_group % GPB) * (4 * RPW) + wave * RPW + r] = v;
-            }
+        for (int n = 1; n < NC; ++n) v = j == n ? acc[n] : v;
+        if (done_writer) {
+            v += o_bias + o_bcol;                           // at most one of the two biases is set
+            if (a.e.flags & MI355X_EPI_GELU)     v  = gelu_f32(v, a.e.gelu);
+            if (a.e.flags & MI355X_EPI_SCALE)    v *= a.e.scale;
+            if (a.e.flags & MI355X_EPI_RESIDUAL) v += o_res;
+            if (a.e.flags & MI355X_EPI_OUT_F16) *(half_t *)(a.d + j * a.d_nb1 + done_row * 2) = (half_t) v;
+            else                                *(float  *)(a.d + j * a.d_nb1 + done_row * 4) = v;
+            if (emit_q8) q8_rows[j][(done_group & ((1 << gpb_log2) - 1)) * rpg + wave * RPW + r] = v;
         }
-        if (emit_q8 && ((done_group % GPB) == GPB - 1 || !more)) {          // uniform: a block of 32 rows is complete (M % 32 == 0)
-            // thread (column n, row rr of the block): rounding as quantize_row_q8_0 (ggml-cpu-quants.c:808-865), into the layout of
-            // k_quantize_x_q8 for NC rows of M values
+        if (emit_q8 && (((done_group + 1) & ((1 << gpb_log2) - 1)) == 0 || !more)) {          // uniform: blocks of 32 rows are complete (M % 32 == 0)
+            // thread (block of the unit, column n, row rr of the block): rounding as quantize_row_q8_0 (ggml-cpu-quants.c:808-865),
+            // into the layout of k_quantize_x_q8 for NC rows of M values
             __syncthreads();
-            const int n = threadIdx.x >> 5, rr = threadIdx.x & 31;
-            const float v = n < NC ? q8_rows[n][rr] : 0.0f;
-            const float amax = lanes_max<32>(fabsf(v));
+            const int u = threadIdx.x >> 5, n = u % NC, rr = threadIdx.x & 31;
+            const int64_t bi = ((int64_t)(done_group >> gpb_log2) << (unit_log2 - QK_LOG2)) + u / NC, nb2 = a.M / QK;
+            const bool mine = u < NC << (unit_log2 - QK_LOG2);
+            const float x = mine ? q8_rows[n][u / NC * QK + rr] : 0.0f;
+            const float amax = lanes_max<32>(fabsf(x));
             const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
-            const int q = (int) rintf(v * id);
+            const int q = (int) rintf(x * id);
             const int qsum = lanes_sum<32>(q);
-            if (n < NC && !idle) {
+            if (mine && !idle && bi < nb2) {
                 char * img = (char *) a.e.image;
-                const int64_t bi = done_group / GPB, nb2 = a.M / QK;
                 ((int8_t *) img)[n * a.M + bi * QK + rr] = (int8_t) q;
                 if (rr == 0) {
                     ((float *)(img + (size_t) NC * a.M))[n * nb2 + bi] = h2f(f2h_bits(div127(amax)));
@@ -408,7 +416,7 @@ __device__ __forceinline__ void gemv_qr_rows(const mm_args & a, PRO prologue = P
 }
 
 template <int T0, int NC, int LPR, int NB>
-__global__ void __launch_bounds__(256) k_gemv_qr(mm_args a) { gemv_qr_rows<T0, NC, LPR, NB>(a); }
+__global__ void __launch_bounds__(256) k_gemv_qr(mm_args a, gemv_walk walk) { gemv_qr_rows<T0, NC, LPR, NB, 4>(a, walk); }
 
 // ------------------------------------------------------------------------------------------------------
 // Q8_0 weights as tiles for the matrix cores: the product over a matrix long enough to be a stream (the vocabulary
@@ -465,23 +473,33 @@ struct gemv_group_entry { const char * w; char * d; const float * bias; const ch
 struct gemv_group { gemv_group_entry e[GEMV_GROUP_MAX]; };
 
 template <int T0, int NC, int LPR, int NB>
-__global__ void __launch_bounds__(256) k_gemv_qr_group(mm_args a, gemv_group grp) {
+__global__ void __launch_bounds__(256) k_gemv_qr_group(mm_args a, gemv_walk walk, gemv_group grp) {
     const gemv_group_entry & ge = grp.e[blockIdx.y];
     a.w = ge.w; a.d = ge.d; a.d_nb1 = ge.d_nb1;
     a.e.flags = ge.flags; a.e.scale = ge.scale; a.e.bias = ge.bias; a.e.residual = ge.residual;
-    gemv_qr_rows<T0, NC, LPR, NB>(a);
+    gemv_qr_rows<T0, NC, LPR, NB, 4>(a, walk);
 }
 
-// LayerNorm in front of the products, in the same launch.  A decode step's LayerNorm has five rows to work on and is
-// over in the latency of a launch (7 us); here every workgroup normalizes the rows for itself while its first weight
-// blocks travel — the rows in registers between the passes as in k_norm — and leaves them quantized in LDS, where the
-// lanes pick up their slices.  The first workgroup also writes what a separate
-// LayerNorm would have left behind: the f32 rows and the Q8_0 form in the workspace, for whatever reads them later.
+// LayerNorm in front of the products, in the same launch.  A decode step's LayerNorm has up to eight rows to work on and is
+// over in the latency of a launch; here every workgroup normalizes the rows for itself while its first weight blocks travel —
+// the rows in registers between the passes as in k_norm — and leaves them quantized in LDS, where the lanes pick up their
+// slices.  The first workgroup also writes what a separate LayerNorm would have left behind: the f32 rows and the Q8_0 form in
+// the workspace, for whatever reads them later.
+//
+// What bounds it is that chain of dependent steps — a memory round trip, two reductions, the block maxima, a barrier, the LDS
+// round trip of the quantized rows — about 1 us on top of a launch (1.7 us) when a wavefront has a SIMD to itself, and several
+// times that when the workgroups of a CU each run it with the same few wavefronts and pieces of rows that are not there.  Hence
+// one workgroup of 8 or 16 wavefronts per CU: the LayerNorm runs once per CU, a row to a wavefront and so at most two on a
+// SIMD, on exactly the pieces a row has (JN float4s per lane), and the wavefronts without a row go ahead with the weights.
+// Measured, us, with two or three workgroups of four wavefronts to a CU in front (rows x K, columns): 3 x 768 x 768, 3: 7.9 -> 4.5;
+// 3072 x 768 to Q8_0, 3: 8.3 -> 6.0; 3 x 1280 x 1280, 5: 8.9 -> 6.5; 5120 x 1280 to Q8_0, 5: 11.2 -> 8.6, 8: 26 -> 9.9;
+// 3 x 1024 x 1024, 5: 15.4 -> 5.6 — where the product alone takes 3.7, 6.3, 4.9, 10.1, 11.7 and 4.1.
 struct gemv_norm_args {
     const char * src; int64_t src_nb1;
     const float * w; const float * b; float eps;
     char * dst; int64_t dst_nb1;       // f32 rows of the normalized activations
     char * ws;                         // their Q8_0 form (layout of k_quantize_x_q8)
+    int threads;                       // of the workgroup
     // EMB instances: row n of the source is not read but made here, token row tok_ids[n] (Q8_0, Q5_0 or F16) plus position row
     // pos_ids[n] (F32) as in k_get_rows_add, and the first workgroup writes it to x0
     const char * tok; int tok_type; int64_t tok_nb1, tok_ne1; const int32_t * tok_ids;
@@ -489,15 +507,14 @@ struct gemv_norm_args {
     char * x0;
 };
 
-// NJ > 0: the rows are exactly 256 NJ values long and both affine vectors are there (whisper's LayerNorms at 512 ... 1280):
-// NJ float4s per lane instead of eight, no guard around a term, no clamped address
-template <int NC, int NJ = 0, bool EMB = false>
+// JN: float4s per lane and row, K <= 256 JN (and, for JN = 3, 4, 5, K > 256 (JN - 1): all pieces but the last are whole); W: wavefronts of the workgroup
+template <int NC, int JN, int W, bool EMB = false>
 struct gemv_norm_prologue {
     const gemv_norm_args & nm; int64_t K; char * lds;
-    // wavefront w takes rows w and w + 4; both rows and the affine vectors are requested before anything is reduced, so
-    // the prologue is one memory round trip long
-    static constexpr int RW = (NC + 3) / 4;                 // rows per wavefront
-    static constexpr int JN = NJ ? NJ : 8;                  // float4s per lane and row
+    static constexpr int ROWS = NC < W ? NC : W;
+    // wavefront w takes rows w and, where there are more rows than wavefronts, w + W; the rows and the affine vectors are all
+    // requested before anything is reduced, so the prologue is one memory round trip long
+    static constexpr int RW = (NC + W - 1) / W;             // rows per wavefront
     float4 v[RW][JN], ww[JN], bb[JN];
     // EMB: four values of the token row as they lie in the table (Q8_0: four quants and the block's scale; Q5_0: four bytes
     // of nibbles, the scale and the block's fifth bits; F16: two words) next to the position row's four in v, and whether
@@ -507,29 +524,32 @@ struct gemv_norm_prologue {
     bool ok[RW];
     static constexpr bool LATE = EMB;
 
+    // is the lane's piece jj inside the row?
+    static __device__ __forceinline__ bool inside(int jj, int lane, int n4) { return (JN >= 3 && JN <= 5 && jj < JN - 1) || lane + jj * WAVE < n4; }
+
     __device__ __forceinline__ void request() {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         const int n4 = (int)(K / 4);
         if constexpr (EMB) {                                // the rows' indices now, the rows themselves in request_late()
 #pragma unroll
             for (int rr = 0; rr < RW; ++rr) {
-                const int row = wave + 4 * rr < NC ? wave + 4 * rr : NC - 1;
+                const int row = wave + W * rr < NC ? wave + W * rr : NC - 1;
                 r0[rr] = nm.tok_ids[row]; r1[rr] = nm.pos_ids[row];
             }
         }
         // no branch around a load: addresses are clamped into the rows, and a missing affine vector reads the source instead
-        const float4 * wp = (const float4 *)(NJ || nm.w ? (const char *) nm.w : nm.src), * bp = (const float4 *)(NJ || nm.b ? (const char *) nm.b : nm.src);
+        const float4 * wp = (const float4 *)(nm.w ? (const char *) nm.w : nm.src), * bp = (const float4 *)(nm.b ? (const char *) nm.b : nm.src);
 #pragma unroll
         for (int jj = 0; jj < JN; ++jj) {
-            const int c = NJ || lane + jj * WAVE < n4 ? lane + jj * WAVE : n4 - 1;
-            ww[jj] = wp[c]; bb[jj] = bp[c];
+            const int c = inside(jj, lane, n4) ? lane + jj * WAVE : n4 - 1;
             if constexpr (!EMB) {
 #pragma unroll
                 for (int rr = 0; rr < RW; ++rr) {
-                    const int row = wave + 4 * rr < NC ? wave + 4 * rr : NC - 1;
+                    const int row = wave + W * rr < NC ? wave + W * rr : NC - 1;
                     v[rr][jj] = ((const float4 *)(nm.src + row * nm.src_nb1))[c];
                 }
             }
+            ww[jj] = wp[c]; bb[jj] = bp[c];
         }
     }
 
@@ -544,7 +564,7 @@ struct gemv_norm_prologue {
                 const float4 *  pp = (const float4 *)(nm.pos + (int64_t)(ok[rr] ? r1[rr] : 0) * nm.pos_nb1);
 #pragma unroll
                 for (int jj = 0; jj < JN; ++jj) {
-                    const int c = NJ || lane + jj * WAVE < n4 ? lane + jj * WAVE : n4 - 1;
+                    const int c = inside(jj, lane, n4) ? lane + jj * WAVE : n4 - 1;
                     v[rr][jj] = pp[c];
                     if (nm.tok_type == MI355X_TYPE_Q8_0) {          // uniform
                         const uint8_t * blk = tp + (c >> 3) * 34;
@@ -561,8 +581,8 @@ struct gemv_norm_prologue {
         }
     }
 
-    __device__ __forceinline__ const char * finish(const char *) {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __device__ __forceinline__ void finish() {
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         const int n4 = (int)(K / 4), nbk = (int)(K / QK);
         const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
         int32_t * xq   = (int32_t *) lds;
@@ -570,7 +590,7 @@ struct gemv_norm_prologue {
         int32_t * xsum = (int32_t *)(lds + (size_t) NC * nbk * 4 + (size_t) NC * K);
 #pragma unroll
         for (int rr = 0; rr < RW; ++rr) {
-            const int row = wave + 4 * rr;
+            const int row = wave + W * rr;
             if (row >= NC) break;                           // uniform
             if constexpr (EMB) {                            // the source row: dequantized token values plus position values
 #pragma unroll
@@ -583,7 +603,7 @@ struct gemv_norm_prologue {
                         e.z = (float)(int8_t)(q >> 16) * sc;  e.w = (float)(int8_t)(q >> 24) * sc;
                     } else if (nm.tok_type == MI355X_TYPE_Q5_0) {
                         const float sc = h2f((uint16_t) d);
-                        const int c = NJ || lane + jj * WAVE < n4 ? lane + jj * WAVE : n4 - 1;
+                        const int c = inside(jj, lane, n4) ? lane + jj * WAVE : n4 - 1;
                         const int j0 = 4 * (c & 7);                                     // first of the lane's four weights in the block
                         const uint32_t nib = (j0 < 16 ? q : q >> 4) & 0x0F0F0F0Fu, hb = th[rr][jj] >> j0;
                         e.x = (float)((int)((nib & 15)         | ((hb & 1) << 4))        - 16) * sc;
@@ -596,17 +616,17 @@ struct gemv_norm_prologue {
                     float4 & t = v[rr][jj];
                     const float nan = __builtin_nanf("");
                     t.x = ok[rr] ? e.x + t.x : nan; t.y = ok[rr] ? e.y + t.y : nan; t.z = ok[rr] ? e.z + t.z : nan; t.w = ok[rr] ? e.w + t.w : nan;
-                    if (writer && (NJ || lane + jj * WAVE < n4)) ((float4 *)(nm.x0 + row * nm.src_nb1))[lane + jj * WAVE] = t;
+                    if (writer && inside(jj, lane, n4)) ((float4 *)(nm.x0 + row * nm.src_nb1))[lane + jj * WAVE] = t;
                 }
             }
             float sum = 0.0f;
 #pragma unroll
-            for (int jj = 0; jj < JN; ++jj) if (NJ || lane + jj * WAVE < n4) sum += (v[rr][jj].x + v[rr][jj].y) + (v[rr][jj].z + v[rr][jj].w);
+            for (int jj = 0; jj < JN; ++jj) if (inside(jj, lane, n4)) sum += (v[rr][jj].x + v[rr][jj].y) + (v[rr][jj].z + v[rr][jj].w);
             const float mean = wave_sum(sum) / (float) K;
             float sum2 = 0.0f;
 #pragma unroll
             for (int jj = 0; jj < JN; ++jj) {
-                if (NJ || lane + jj * WAVE < n4) {
+                if (inside(jj, lane, n4)) {
                     float4 & t = v[rr][jj];
                     t.x -= mean; t.y -= mean; t.z -= mean; t.w -= mean;
                     sum2 += (t.x*t.x + t.y*t.y) + (t.z*t.z + t.w*t.w);
@@ -626,8 +646,8 @@ struct gemv_norm_prologue {
                 r[jj] = make_float4(v[rr][jj].x * scale, v[rr][jj].y * scale, v[rr][jj].z * scale, v[rr][jj].w * scale);
                 {   // (MUL then ADD, two graph nodes: two roundings — without guards around them the two would be contracted)
 #pragma clang fp contract(off)
-                    if (NJ || nm.w) { r[jj].x *= ww[jj].x; r[jj].y *= ww[jj].y; r[jj].z *= ww[jj].z; r[jj].w *= ww[jj].w; }
-                    if (NJ || nm.b) { r[jj].x += bb[jj].x; r[jj].y += bb[jj].y; r[jj].z += bb[jj].z; r[jj].w += bb[jj].w; }
+                    if (nm.w) { r[jj].x *= ww[jj].x; r[jj].y *= ww[jj].y; r[jj].z *= ww[jj].z; r[jj].w *= ww[jj].w; }
+                    if (nm.b) { r[jj].x += bb[jj].x; r[jj].y += bb[jj].y; r[jj].z += bb[jj].z; r[jj].w += bb[jj].w; }
                 }
             }
 #pragma unroll
@@ -645,7 +665,7 @@ struct gemv_norm_prologue {
 #pragma unroll
             for (int jj = 0; jj < JN; ++jj) {
                 const int c = lane + jj * WAVE;
-                if (NJ || c < n4) {
+                if (inside(jj, lane, n4)) {
                     xq[row * n4 + c] = (q[jj][0] & 0xFF) | ((q[jj][1] & 0xFF) << 8) | ((q[jj][2] & 0xFF) << 16) | ((q[jj][3] & 0xFF) << 24);
                     xd[row * nbk + c / 8] = h2f(f2h_bits(div127(amax[jj])));
                     xsum[row * nbk + c / 8] = qsum[jj];
@@ -653,45 +673,48 @@ struct gemv_norm_prologue {
             }
             if (writer) {
 #pragma unroll
-                for (int jj = 0; jj < JN; ++jj) if (NJ || lane + jj * WAVE < n4) ((float4 *)(nm.dst + row * nm.dst_nb1))[lane + jj * WAVE] = r[jj];
+                for (int jj = 0; jj < JN; ++jj) if (inside(jj, lane, n4)) ((float4 *)(nm.dst + row * nm.dst_nb1))[lane + jj * WAVE] = r[jj];
             }
         }
+    }
+
+    __device__ __forceinline__ const char * publish(const char *) {
         __syncthreads();
-        if (writer) {                                       // the workspace copy, 16 bytes per thread and step
-            const int pieces = (int)(((size_t) NC * K + (size_t) NC * nbk * 8) / 16);
-            for (int i = threadIdx.x; i < pieces; i += 256) ((u32x4 *) nm.ws)[i] = ((const u32x4 *) lds)[i];
+        if (blockIdx.x == 0 && blockIdx.y == 0) {           // the workspace copy, 8 bytes per thread and step
+            const int pieces = (int)(((size_t) NC * K + (size_t) NC * (K / QK) * 8) / 8);
+            for (int i = threadIdx.x; i < pieces; i += nm.threads) ((uint2 *) nm.ws)[i] = ((const uint2 *) lds)[i];
         }
         return lds;
     }
 };
 
-template <int T0, int NC, int LPR, int NB, int NJ = 0, bool EMB = false>
-__global__ void __launch_bounds__(256) k_gemv_qr_norm_group(mm_args a, gemv_group grp, gemv_norm_args nm) {
+template <int T0, int NC, int JN, bool EMB>
+__global__ void __launch_bounds__(1024) k_gemv_norm_group(mm_args a, gemv_walk walk, gemv_group grp, gemv_norm_args nm) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const gemv_group_entry & ge = grp.e[blockIdx.y];
     a.w = ge.w; a.d = ge.d; a.d_nb1 = ge.d_nb1;
     a.e.flags = ge.flags; a.e.scale = ge.scale; a.e.bias = ge.bias; a.e.residual = ge.residual;
-    gemv_qr_rows<T0, NC, LPR, NB>(a, gemv_norm_prologue<NC, NJ, EMB>{ nm, a.K, smem });
+    gemv_qr_rows<T0, NC, gemv_row_lanes(JN * 8), 1, 16>(a, walk, gemv_norm_prologue<NC, JN, 8, EMB>{ nm, a.K, smem });
 }
 
 // the product over the tile-ordered vocabulary matrix with the decoder's last LayerNorm in front, the same way: the
 // LayerNorm of the step's rows runs in every workgroup while its first tile row is on the way
-template <int KSTEPS, int NC, int NJ>
+template <int KSTEPS, int NC>
 __global__ void __launch_bounds__(256, 2) k_gemv_q8_0_tiles_norm(mm_args a, gemv_norm_args nm) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    gemv_q8_0_tiles_body<KSTEPS, false>(a, nullptr, gemv_norm_prologue<NC, NJ>{ nm, a.K, smem });
+    gemv_q8_0_tiles_body<KSTEPS, false>(a, nullptr, gemv_norm_prologue<NC, (KSTEPS + 3) / 4, 4>{ nm, a.K, smem });
 }
 
 template <int KSTEPS, int NC>
-static int launch_gemv_q8_0_tiles_norm_kn(const mm_args & a, const gemv_norm_args & nm, hipStream_t st) {
+static int launch_gemv_q8_0_tiles_norm_kn(const mm_args & a, gemv_norm_args nm, hipStream_t st) {
     const int64_t n_tiles = (a.M + 15) / 16;
     const int64_t resident = 256 * 2 * 4;                 // wavefronts: two workgroups of four per CU
     const int64_t rounds = (n_tiles + resident - 1) / resident;
     const int64_t waves = (n_tiles + rounds - 1) / rounds;
     const unsigned grid = (unsigned)(waves / 4 > 0 ? waves / 4 : 1);
     const size_t lds = (size_t) NC * a.K + (size_t) NC * (a.K / QK) * 8;
-    if (KSTEPS == 20 && nm.w && nm.b) k_gemv_q8_0_tiles_norm<KSTEPS, NC, KSTEPS == 20 ? 5 : 0><<<grid, 256, lds, st>>>(a, nm);
-    else                              k_gemv_q8_0_tiles_norm<KSTEPS, NC, 0><<<grid, 256, lds, st>>>(a, nm);
+    nm.threads = 256;
+    k_gemv_q8_0_tiles_norm<KSTEPS, NC><<<grid, 256, lds, st>>>(a, nm);
     return launch_status();
 }
 template <int KSTEPS>
@@ -713,11 +736,15 @@ static int launch_gemv_q8_0_tiles_norm_k(const mm_args & a, const gemv_norm_args
 // launches and entry points
 // ------------------------------------------------------------------------------------------------------
 
-// Register-resident variant: LPR = 16, 32 or 64 lanes per row with NB <= 3 blocks per lane and N * NB <= 15 block slices of
-// activations (120 registers).  The fewest lanes per row that still give 512 workgroups (few lanes per row = few idle
-// lanes when the blocks of a row do not divide evenly), else the most.  Returns LPR, 0 when the shape does not fit.
+// Lanes per row of the register kernels, LPR = 16, 32 or 64 with NB <= 3 blocks per lane and N * NB <= 15 block slices of
+// activations (120 registers); 0 when the shape does not fit.
+//   K <= 2048, up to GEMV_SHORT_ROWS rows in the launch: one block per lane (gemv_row_lanes) — such a product is over in the
+//   latency of its loads, and the LayerNorm form, which has the same order of sums, takes what its wavefronts hold at a time.
+//   else the fewest lanes per row that still give 512 workgroups: few lanes per row are few idle lanes when the blocks of a row do
+//   not divide evenly, and few steps of the sum across lanes; else the most.
 static int gemv_r_lanes(int64_t M, int64_t N, int64_t K) {
     const int64_t nbk = K / QK;
+    if (nbk <= 64 && M <= GEMV_SHORT_ROWS) return gemv_row_lanes((int) nbk);
     int best = 0;
     for (int lpr = 64; lpr >= 16; lpr /= 2) {
         const int64_t nb = (nbk + lpr - 1) / lpr;
@@ -733,56 +760,75 @@ size_t gemv_ws_bytes(const mi355x_tensor * src0, const mi355x_tensor * src1) {
     return round256((size_t)(N * K + N * (K / QK) * 8));
 }
 
+// One resident set of workgroups of `waves` wavefronts, each walking its share of the groups of waves * rpw rows: a second, partly
+// filled set would double the time.  Returns the grid, 0 for more rows than an int counts.
+static unsigned plan_walk(gemv_walk & w, int64_t M, int waves, int rpw, int64_t resident, bool emit_q8) {
+    const int rpg = waves * rpw, gpb = rpg < QK ? QK / rpg : 1;
+    const int64_t n_groups = (M + rpg - 1) / rpg;
+    if (n_groups > 0x3fffffff) return 0;
+    const int64_t rounds = (n_groups + resident - 1) / resident, grid = (n_groups + rounds - 1) / rounds;
+    w.waves_log2 = waves == 4 ? 2 : waves == 8 ? 3 : 4;
+    w.n_groups = (int) n_groups;
+    w.run = emit_q8 ? (int)(gpb * ((n_groups + gpb * grid - 1) / (gpb * grid))) : 0;
+    w.step = emit_q8 ? 1 : (int) grid;
+    return (unsigned) grid;
+}
+
 template <int T0, int NC, int LPR, int NB>
-static int launch_gemv_r_k(const mm_args & a, unsigned grid, const gemv_group * grp, int count, const gemv_norm_args * nm, hipStream_t st) {
-    if (nm) {
-        const size_t lds = (size_t) NC * a.K + (size_t) NC * (a.K / QK) * 8;
-        // (the widest model's rows, 1280 values, have an instance without guards)
-        const bool full = a.K == 1280 && nm->w && nm->b;
-        if (nm->tok) {                                      // (made for one block per lane, the shape of a layer's Q, K and V)
-            if constexpr (NB == 1) {
-                if (full) k_gemv_qr_norm_group<T0, NC, LPR, NB, 5, true><<<dim3(grid, (unsigned) count), 256, lds, st>>>(a, *grp, *nm);
-                else      k_gemv_qr_norm_group<T0, NC, LPR, NB, 0, true><<<dim3(grid, (unsigned) count), 256, lds, st>>>(a, *grp, *nm);
-            }
-            else return MI355X_ERR_UNSUPPORTED;
-        }
-        else if (full) k_gemv_qr_norm_group<T0, NC, LPR, NB, 5><<<dim3(grid, (unsigned) count), 256, lds, st>>>(a, *grp, *nm);
-        else           k_gemv_qr_norm_group<T0, NC, LPR, NB><<<dim3(grid, (unsigned) count), 256, lds, st>>>(a, *grp, *nm);
-    }
-    else if (grp) k_gemv_qr_group<T0, NC, LPR, NB><<<dim3(grid, (unsigned) count), 256, 0, st>>>(a, *grp);
-    else          k_gemv_qr<T0, NC, LPR, NB><<<grid, 256, 0, st>>>(a);
+static int launch_gemv_r_k(const mm_args & a, hipStream_t st, const gemv_group * grp, int count) {
+    const int per_cu = NB > 1 ? 2 : 4;                      // (what the registers allow)
+    gemv_walk walk;
+    const unsigned grid = plan_walk(walk, a.M, 4, WAVE / LPR, std::max(256 * per_cu / count, 1), ((grp ? grp->e[0].flags : a.e.flags) & MI355X_EPI_EMIT_Q8_0) != 0);
+    if (!grid) return MI355X_ERR_UNSUPPORTED;
+    if (grp) k_gemv_qr_group<T0, NC, LPR, NB><<<dim3(grid, (unsigned) count), 256, 0, st>>>(a, walk, *grp);
+    else     k_gemv_qr<T0, NC, LPR, NB><<<grid, 256, 0, st>>>(a, walk);
     return launch_status();
 }
 template <int T0, int NC, int LPR>
-static int launch_gemv_r_nb(const mm_args & a, int nb, unsigned grid, const gemv_group * grp, int count, const gemv_norm_args * nm, hipStream_t st) {
+static int launch_gemv_r_nb(const mm_args & a, int nb, hipStream_t st, const gemv_group * grp, int count) {
     switch (nb) {
-        case 1: return launch_gemv_r_k<T0, NC, LPR, 1>(a, grid, grp, count, nm, st);
-        case 2: if constexpr (NC * 2 <= 15) return launch_gemv_r_k<T0, NC, LPR, 2>(a, grid, grp, count, nm, st); break;
-        case 3: if constexpr (NC * 3 <= 15) return launch_gemv_r_k<T0, NC, LPR, 3>(a, grid, grp, count, nm, st); break;
+        case 1: return launch_gemv_r_k<T0, NC, LPR, 1>(a, st, grp, count);
+        case 2: if constexpr (NC * 2 <= 15) return launch_gemv_r_k<T0, NC, LPR, 2>(a, st, grp, count); break;
+        case 3: if constexpr (NC * 3 <= 15) return launch_gemv_r_k<T0, NC, LPR, 3>(a, st, grp, count); break;
     }
     return MI355X_ERR_UNSUPPORTED;
 }
+template <int T0, int NC, int JN>
+static int launch_gemv_norm(const mm_args & a, hipStream_t st, const gemv_group & grp, int count, gemv_norm_args nm) {
+    // Eight wavefronts to the workgroup while every workgroup then has a CU of its own (a launch of 16 takes 0.5 us longer to get
+    // going), 16 from there on (two workgroups on a CU make the rows twice: 7.5 us to 6.5 for 3 x 1280 rows of 1280, 5 columns),
+    // and where eight would leave a workgroup several groups to a Q8_0 block of the image.
+    const int rpw = WAVE / gemv_row_lanes(JN * 8);
+    const bool emit_q8 = (grp.e[0].flags & MI355X_EPI_EMIT_Q8_0) != 0;
+    const int waves = (a.M + 8 * rpw - 1) / (8 * rpw) * count <= 256 && (!emit_q8 || 8 * rpw >= QK) ? 8 : 16;
+    nm.threads = 64 * waves;
+    gemv_walk walk;
+    const unsigned grid = plan_walk(walk, a.M, waves, rpw, std::max(256 / count, 1), emit_q8);
+    const size_t lds = (size_t) NC * a.K + (size_t) NC * (a.K / QK) * 8;
+    if (nm.tok) k_gemv_norm_group<T0, NC, JN, true ><<<dim3(grid, (unsigned) count), 64 * waves, lds, st>>>(a, walk, grp, nm);
+    else        k_gemv_norm_group<T0, NC, JN, false><<<dim3(grid, (unsigned) count), 64 * waves, lds, st>>>(a, walk, grp, nm);
+    return launch_status();
+}
 template <int T0, int NC>
-static int launch_gemv_r(const mm_args & a, hipStream_t st, const gemv_group * grp = nullptr, int count = 1, const gemv_norm_args * nm = nullptr) {
+static int launch_gemv_r(const mm_args & a, hipStream_t st, const gemv_group * grp, int count, const gemv_norm_args * nm) {
+    if (nm) {
+        if (a.K <= 512)  return launch_gemv_norm<T0, NC, 2>(a, st, *grp, count, *nm);
+        if (a.K <= 768)  return launch_gemv_norm<T0, NC, 3>(a, st, *grp, count, *nm);
+        if (a.K <= 1024) return launch_gemv_norm<T0, NC, 4>(a, st, *grp, count, *nm);
+        if (a.K <= 1280) return launch_gemv_norm<T0, NC, 5>(a, st, *grp, count, *nm);
+        return launch_gemv_norm<T0, NC, 8>(a, st, *grp, count, *nm);
+    }
     int lpr = gemv_r_lanes(a.M * count, NC, a.K);
     if (!lpr) return MI355X_ERR_UNSUPPORTED;
     // with the Q8_0 emission a workgroup owns whole blocks of 32 rows, so there are M / 32 workgroups at most: the fewer lanes a
     // row takes, the fewer groups each of them walks one after the other
     const bool emit_q8 = ((grp ? grp->e[0].flags : a.e.flags) & MI355X_EPI_EMIT_Q8_0) != 0;
-    if (emit_q8 && (a.K / QK + 15) / 16 <= 3 && (a.K / QK + 15) / 16 * NC <= 15) lpr = 16;
+    if (emit_q8 && a.M > GEMV_SHORT_ROWS && (a.K / QK + 15) / 16 <= 3 && (a.K / QK + 15) / 16 * NC <= 15) lpr = 16;
     const int nb = (int)((a.K / QK + lpr - 1) / lpr);
-    const int rows_per_wg = 4 * (WAVE / lpr);
-    const int64_t n_groups = (a.M + rows_per_wg - 1) / rows_per_wg;
-    // one resident set of workgroups (the registers allow 4 per CU with one block per lane, else 2), each walking its
-    // share of the row groups: a second, partly filled set would double the time
-    const int per_cu = nb > 1 ? 2 : nm ? 3 : 4;           // (the LayerNorm prologue costs the one-block kernels 50 registers)
-    const int64_t resident = 256 * per_cu / count > 0 ? 256 * per_cu / count : 1;
-    const int64_t rounds   = (n_groups + resident - 1) / resident;
-    const unsigned grid    = (unsigned)((n_groups + rounds - 1) / rounds);
     switch (lpr) {
-        case 16: return launch_gemv_r_nb<T0, NC, 16>(a, nb, grid, grp, count, nm, st);
-        case 32: return launch_gemv_r_nb<T0, NC, 32>(a, nb, grid, grp, count, nm, st);
-        default: return launch_gemv_r_nb<T0, NC, 64>(a, nb, grid, grp, count, nm, st);
+        case 16: return launch_gemv_r_nb<T0, NC, 16>(a, nb, st, grp, count);
+        case 32: return launch_gemv_r_nb<T0, NC, 32>(a, nb, st, grp, count);
+        default: return launch_gemv_r_nb<T0, NC, 64>(a, nb, st, grp, count);
     }
 }
 template <int T0>
@@ -846,9 +892,16 @@ int launch_gemv_lds(int type, const mm_args & a, hipStream_t st) {
     return type == MI355X_TYPE_Q8_0 ? launch_gemv_n<MI355X_TYPE_Q8_0>(a, st) : launch_gemv_n<MI355X_TYPE_Q5_0>(a, st);
 }
 
+// a LayerNorm in front of the products: what the kernels take, and the tensors for the case that it gets a launch of its own
+struct gemv_norm_source {
+    gemv_norm_args nm;
+    const mi355x_tensor * src, * normed;
+    const mi355x_tensor * tok, * tok_ids, * pos, * pos_ids;    // of the gathering form, else NULL
+};
+
 // the few-column form of mi355x_mul_mat_group: quantized weights of one type and shape, activations quantized once
 static int group_gemv(const mi355x_mul_mat_item * items, int count, const mi355x_tensor * src1, int flags,
-                              void * workspace, size_t workspace_size, void * stream, gemv_norm_args * nm) {
+                              void * workspace, size_t workspace_size, void * stream, gemv_norm_source * ns) {
     const mi355x_tensor * w0 = items[0].src0;
     if (count > GEMV_GROUP_MAX || src1->type != MI355X_TYPE_F32 || mm_path(w0, src1) != MM_GEMV) return MI355X_ERR_UNSUPPORTED;
     if (w0->type != MI355X_TYPE_Q8_0 && w0->type != MI355X_TYPE_Q5_0) return MI355X_ERR_UNSUPPORTED;
@@ -890,9 +943,14 @@ static int group_gemv(const mi355x_mul_mat_item * items, int count, const mi355x
     a.e.image = (grp.e[0].flags & MI355X_EPI_EMIT_Q8_0) ? (half_t *) items[0].epi->image : nullptr;
     if (any_gelu && !(a.e.gelu = gelu_table_device())) return MI355X_ERR_HIP;
     hipStream_t st = (hipStream_t) stream;
-    if (nm) {                                               // the LayerNorm in front, in the same launch: it writes src1 and the workspace
-        nm->ws = (char *) workspace;
-        return w0->type == MI355X_TYPE_Q8_0 ? launch_gemv_r_n<MI355X_TYPE_Q8_0>(a, st, &grp, count, nm) : launch_gemv_r_n<MI355X_TYPE_Q5_0>(a, st, &grp, count, nm);
+    if (ns) {                                               // the LayerNorm in front: it writes src1 and the workspace
+        ns->nm.ws = (char *) workspace;
+        if (a.M * count <= GEMV_SHORT_ROWS)                 // ... in the same launch
+            return w0->type == MI355X_TYPE_Q8_0 ? launch_gemv_r_n<MI355X_TYPE_Q8_0>(a, st, &grp, count, &ns->nm) : launch_gemv_r_n<MI355X_TYPE_Q5_0>(a, st, &grp, count, &ns->nm);
+        // a long stream of weights: a launch more is nothing beside it, and the LayerNorm's registers would cost it wavefronts
+        if (ns->tok) if (const int rc = mi355x_get_rows_add(ns->tok, ns->tok_ids, ns->pos, ns->pos_ids, ns->src, stream)) return rc;
+        if (const int rc = mi355x_norm_emit_q8_0(ns->src, ns->normed, ns->nm.eps, ns->nm.w, ns->nm.b, workspace, stream)) return rc;
+        flags |= MI355X_MM_WS_READY;
     }
     if (!(flags & MI355X_MM_WS_READY)) {
         k_quantize_x_q8<<<(unsigned)((a.N * (a.K / 4) + 255) / 256), 256, 0, st>>>(a.x, a.x_nb1, a.K, a.N, (char *) workspace);
@@ -909,7 +967,7 @@ int mul_mat_group_gemv(const mi355x_mul_mat_item * items, int count, const mi355
 
 // the checks common to the LayerNorm-and-products entries; `nm` arrives with the gather fields set or zero
 static int norm_mul_mat_group(const mi355x_tensor * src, const mi355x_tensor * normed, float eps, const float * w, const float * b,
-                              const mi355x_mul_mat_item * items, int count, void * workspace, size_t workspace_size, void * stream, gemv_norm_args nm) {
+                              const mi355x_mul_mat_item * items, int count, void * workspace, size_t workspace_size, void * stream, gemv_norm_source ns) {
     if (!src || !normed || !items || count < 1 || !(eps >= 0.0f)) return MI355X_ERR_INVALID;
     if (!items[0].src0 || !items[0].dst) return MI355X_ERR_INVALID;
     if (src->type != MI355X_TYPE_F32 || normed->type != MI355X_TYPE_F32 || src->nb[0] != 4 || normed->nb[0] != 4) return MI355X_ERR_UNSUPPORTED;
@@ -918,14 +976,16 @@ static int norm_mul_mat_group(const mi355x_tensor * src, const mi355x_tensor * n
     if (src->ne[2] != 1 || src->ne[3] != 1 || N < 1 || N > MI355X_GEMV_MAX_COLS || K % QK != 0 || K > 2048) return MI355X_ERR_UNSUPPORTED;
     if (!aligned16(src) || !aligned16(normed) || (uintptr_t) w % 16 != 0 || (uintptr_t) b % 16 != 0) return MI355X_ERR_UNSUPPORTED;
     if (blck_size(items[0].src0->type) <= 1) return MI355X_ERR_UNSUPPORTED;
+    gemv_norm_args & nm = ns.nm;
     nm.src = (const char *) src->data; nm.src_nb1 = (int64_t) src->nb[1]; nm.w = w; nm.b = b; nm.eps = eps;
     nm.dst = (char *) normed->data; nm.dst_nb1 = (int64_t) normed->nb[1]; nm.ws = nullptr;
-    return group_gemv(items, count, normed, 0, workspace, workspace_size, stream, &nm);
+    ns.src = src; ns.normed = normed;
+    return group_gemv(items, count, normed, 0, workspace, workspace_size, stream, &ns);
 }
 
 extern "C" int mi355x_norm_mul_mat_group(const mi355x_tensor * src, const mi355x_tensor * normed, float eps, const float * w, const float * b,
                                          const mi355x_mul_mat_item * items, int count, void * workspace, size_t workspace_size, void * stream) {
-    return norm_mul_mat_group(src, normed, eps, w, b, items, count, workspace, workspace_size, stream, gemv_norm_args{});
+    return norm_mul_mat_group(src, normed, eps, w, b, items, count, workspace, workspace_size, stream, gemv_norm_source{});
 }
 
 extern "C" int mi355x_embed_norm_mul_mat_group(const mi355x_tensor * tok, const mi355x_tensor * tok_ids, const mi355x_tensor * pos, const mi355x_tensor * pos_ids,
@@ -943,11 +1003,13 @@ extern "C" int mi355x_embed_norm_mul_mat_group(const mi355x_tensor * tok, const 
     const uintptr_t ta = tok->type == MI355X_TYPE_F16 ? 8 : 2;
     if ((uintptr_t) tok->data % ta != 0 || tok->nb[1] % ta != 0 || (uintptr_t) pos->data % 16 != 0 || pos->nb[1] % 16 != 0 ||
         (uintptr_t) tok_ids->data % 4 != 0 || (uintptr_t) pos_ids->data % 4 != 0) return MI355X_ERR_UNSUPPORTED;
-    gemv_norm_args nm{};
+    gemv_norm_source ns{};
+    ns.tok = tok; ns.tok_ids = tok_ids; ns.pos = pos; ns.pos_ids = pos_ids;
+    gemv_norm_args & nm = ns.nm;
     nm.tok = (const char *) tok->data; nm.tok_type = tok->type; nm.tok_nb1 = (int64_t) tok->nb[1]; nm.tok_ne1 = tok->ne[1]; nm.tok_ids = (const int32_t *) tok_ids->data;
     nm.pos = (const char *) pos->data; nm.pos_nb1 = (int64_t) pos->nb[1]; nm.pos_ne1 = pos->ne[1]; nm.pos_ids = (const int32_t *) pos_ids->data;
     nm.x0 = (char *) x0->data;
-    return norm_mul_mat_group(x0, normed, eps, w, b, items, count, workspace, workspace_size, stream, nm);
+    return norm_mul_mat_group(x0, normed, eps, w, b, items, count, workspace, workspace_size, stream, ns);
 }
 extern "C" size_t mi355x_q8_0_tiles_size(int64_t K, int64_t M) {
     if (K <= 0 || M <= 0 || K % 64 != 0) return 0;

@@ -12,15 +12,16 @@
 // the activations as they come: quantized ahead, in global memory
 struct q8t_no_prologue {
     __device__ __forceinline__ void request() {}
-    __device__ __forceinline__ const char * finish(const char * x) { return x; }
+    __device__ __forceinline__ void finish() {}
+    __device__ __forceinline__ const char * publish(const char * x) { return x; }
 };
 
 // a.w: the tiles; a.x: the activations quantized ahead (layout of k_quantize_x_q8); K = 64 KSTEPS
 // STAMPS (measurement instances only, never the product's): every wavefront leaves the device's 100 MHz clock at its start and
 // after each of its tiles in `stamps` ([wavefront][1 + tiles per wavefront]; 0 = no such tile), from which the rate of the
 // stream between its ramp and its tail can be read.
-// `pro`: where the quantized activations come from.  request() issues its loads in front of the first tile's, finish() runs
-// behind them and returns the activations' address (the plain product: a.x as passed; with a LayerNorm in front, the rows
+// `pro`: where the quantized activations come from.  request() issues its loads in front of the first tile's, finish() and
+// publish() run behind them, and publish() returns the activations' address (the plain product: a.x as passed; with a LayerNorm in front, the rows
 // it has just normalized and rounded, in LDS) — the first tile takes 7 us to arrive, which is the time such a prologue has.
 template <int KSTEPS, bool STAMPS, typename PRO>
 __device__ __forceinline__ void gemv_q8_0_tiles_body(const mm_args & a, uint64_t * stamps, PRO pro) {
@@ -59,7 +60,8 @@ __device__ __forceinline__ void gemv_q8_0_tiles_body(const mm_args & a, uint64_t
     __builtin_amdgcn_sched_barrier(0);
 
     // activations: quants as the A operand (lane = A row r, 16 k of group g), scales through LDS
-    const char *  xq = pro.finish(a.x);
+    pro.finish();
+    const char *  xq = pro.publish(a.x);
     const float * xd = (const float *)(xq + (size_t) a.N * a.K);
     const int col = r & 7;
     const bool mine = ((r < 8) == (g < 2)) && col < a.N;
