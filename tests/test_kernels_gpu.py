@@ -1090,6 +1090,46 @@ def test_gelu_scale_binary(pkg, oracle, gpu):
     assert np.array_equal(gpu.down(d_a), big + bias)
 
 
+@pytest.mark.parametrize("ne", [(1, 512, 1), (64, 64, 2), (65, 63, 3), (130, 320, 1), (3, 1, 5), (1500, 64, 2)])
+@pytest.mark.parametrize("ts,td", [("F32", "F32"), ("F32", "F16"), ("F16", "F16"), ("F16", "F32")])
+def test_cpy_transposed_and_strided_rows(pkg, oracle, gpu, own_numbers, ne, ts, td):
+    # transposes at the edges of their tiles into rows with a gap behind them, and the merge of interleaved rows (ggml's permute):
+    # every value and nothing beside them
+    n0, n1, n2 = ne
+    st, dt = (np.float32 if t == "F32" else np.float16 for t in (ts, td))
+    size = {"F32": 4, "F16": 2}
+    x = rnd((n2, n0, n1)).astype(st)                       # element (i0, i1, i2) at x[i2, i0, i1]
+    d_x, d_y = gpu.up(x), gpu.up(np.full((n2, n1, n0 + 7), 3, dtype=dt))
+    src = pkg.tensor(d_x, getattr(pkg, ts), [n0, n1, n2], [size[ts] * n1, size[ts], size[ts] * n0 * n1])
+    dst = pkg.tensor(d_y, getattr(pkg, td), [n0, n1, n2], [size[td], size[td] * (n0 + 7), size[td] * (n0 + 7) * n1])
+    pkg.check(pkg.kernels().mi355x_cpy(src, dst, gpu.stream))
+    got = gpu.down(d_y)
+    assert np.array_equal(got[:, :, :n0], np.swapaxes(x, 1, 2).astype(dt)) and np.all(got[:, :, n0:] == 3)
+    d_z = gpu.up(np.full((n1, n2, 4 * n0), 3, dtype=dt))   # rows [4 n0] x n1 x n2 -> n2 and n1 exchanged
+    y = rnd((n2, n1, 4 * n0)).astype(st)
+    d_r = gpu.up(y)
+    src = pkg.tensor(d_r, getattr(pkg, ts), [4 * n0, n2, n1], [size[ts], size[ts] * 4 * n0 * n1, size[ts] * 4 * n0])
+    pkg.check(pkg.kernels().mi355x_cpy(src, pkg.tensor(d_z, getattr(pkg, td), [4 * n0, n2, n1]), gpu.stream))
+    assert np.array_equal(gpu.down(d_z), np.swapaxes(y, 0, 1).astype(dt))
+
+
+@pytest.mark.parametrize("n,rows,heads", [(1, 3, 2), (63, 5, 1), (256, 1, 12), (1028, 700, 2), (1500, 7, 3), (1500, 600, 2), (1501, 530, 2), (2048, 1025, 1), (2049, 2, 2), (8192, 3, 1), (8193, 2, 1)])
+@pytest.mark.parametrize("masked", [None, "f32", "f16"])
+def test_soft_max_row_lengths(pkg, oracle, gpu, own_numbers, n, rows, heads, masked):
+    # one and four wavefronts to a row, 16-byte and single values, rows too long for registers; in place, with a masked half
+    lib = pkg.kernels()
+    x = rnd((heads, rows, n), 4.0)
+    m = np.zeros((rows, n), dtype=np.float32)
+    if masked:
+        m[:, 1:] = np.where(np.arange(n - 1)[None, :] % 2 == np.arange(rows)[:, None] % 2, -np.inf, rnd((rows, n - 1)).astype(np.float16))
+    d_x, d_m = gpu.up(x), gpu.up(m.astype(np.float16) if masked == "f16" else m)
+    tm = pkg.tensor(d_m, pkg.F16 if masked == "f16" else pkg.F32) if masked else None
+    pkg.check(lib.mi355x_soft_max(pkg.tensor(d_x, pkg.F32), tm, pkg.tensor(d_x, pkg.F32), 0.125, gpu.stream))
+    v = x.astype(np.float64) * 0.125 + m
+    e = np.exp(v - v.max(axis=-1, keepdims=True))
+    assert oracle.nmse(gpu.down(d_x), (e / e.sum(axis=-1, keepdims=True)).astype(np.float32)) <= 1e-12
+
+
 def test_cpy_get_rows_im2col_softmax_concat(pkg, oracle, gpu):
     lib = pkg.kernels()
     # f32 -> f16 dense and transposed

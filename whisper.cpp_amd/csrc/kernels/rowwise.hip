@@ -3,6 +3,8 @@
 // a 256-thread block.  Both are HBM-bound: one read and one write of the row.
 #include "common.h"
 
+#include <type_traits>
+
 #define ROWS_PER_BLOCK 4
 #define NORM_MAX_V4    8      // rows up to 64*4*8 = 2048 floats are held in registers between the passes (NV = float4s per lane)
 
@@ -177,6 +179,71 @@ static int norm_impl(const mi355x_tensor * src, const mi355x_tensor * dst, float
 // SOFT_MAX (ggml/src/ggml-cpu/ops.cpp:4641-4737), max_bias = 0
 // ------------------------------------------------------------------------------------------------------
 
+// A row is held in registers between its two reductions: NI pieces of VEC values per lane, WPR wavefronts to the row.  What
+// bounds it is the one read and the one write of the scores (two passes more over memory before: 1500 x 1500 x 12 heads took
+// 96 us, now 35, under the 44 that reading and writing 216 MB through HBM
+// take), or, for the few rows of a decode step, the latency of the
+// launch: then a row gets four wavefronts (8 rows of 1500: 9.5 -> 3.1 us).
+template <typename TM, int VEC, int NI, int WPR>
+__global__ void __launch_bounds__(256) k_soft_max_regs(tview s, tview d, const char * __restrict__ mask, int64_t mask_nb1, float scale) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i1 = WPR == 4 ? blockIdx.x : blockIdx.x * 4 + wave;
+    if (i1 >= (int) s.ne1) return;                             // (a wavefront of its own: no barrier below)
+    const float * x = (const float *)(s.p + i1*s.nb1 + blockIdx.y*s.nb2 + blockIdx.z*s.nb3);
+    float *       y = (float *)(d.p + i1*d.nb1 + blockIdx.y*d.nb2 + blockIdx.z*d.nb3);
+    const TM *    m = mask ? (const TM *)(mask + i1 * mask_nb1) : nullptr;   // the mask is shared by all heads
+    const int n = (int) s.ne0, t = WPR == 4 ? (int) threadIdx.x : lane;
+    typedef float vec __attribute__((ext_vector_type(VEC)));
+    typedef TM mvec __attribute__((ext_vector_type(VEC)));
+
+    // (pieces beyond the row read its first one: no branch around a load)
+    vec v[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) { const int c = (i * 64 * WPR + t) * VEC; v[i] = *(const vec *)(x + (c < n ? c : 0)); }
+    if (m) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int c = (i * 64 * WPR + t) * VEC;
+            const mvec mv = *(const mvec *)(m + (c < n ? c : 0));
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) v[i][e] = __builtin_fmaf(v[i][e], scale, (float) mv[e]);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) v[i] *= scale;
+    }
+    __shared__ float part[2][4];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        if ((i * 64 * WPR + t) * VEC >= n) v[i] = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) mx = fmaxf(mx, v[i][e]);
+    }
+    mx = wave_max(mx);
+    if (WPR == 4) {
+        if (lane == 0) part[0][wave] = mx;
+        __syncthreads();
+        mx = fmaxf(fmaxf(part[0][0], part[0][1]), fmaxf(part[0][2], part[0][3]));
+    }
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) { v[i][e] = v[i][e] == -INFINITY ? 0.0f : __expf(v[i][e] - mx); sum += v[i][e]; }
+    }
+    sum = wave_sum(sum);
+    if (WPR == 4) {
+        if (lane == 0) part[1][wave] = sum;
+        __syncthreads();
+        sum = (part[1][0] + part[1][1]) + (part[1][2] + part[1][3]);
+    }
+    const float inv = 1.0f / sum;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) { const int c = (i * 64 * WPR + t) * VEC; if (c < n) *(vec *)(y + c) = v[i] * inv; }
+}
+
+// any row length: three passes over the row, one wavefront each
 template <typename TM>
 __global__ void k_soft_max(tview s, tview d, const char * __restrict__ mask, int64_t mask_nb1, int64_t nrows, float scale) {
     const int     lane = threadIdx.x % WAVE;
@@ -218,6 +285,40 @@ extern "C" int mi355x_soft_max(const mi355x_tensor * src, const mi355x_tensor * 
     const int64_t grid = (nrows + ROWS_PER_BLOCK - 1) / ROWS_PER_BLOCK;
     if (grid > 0x7fffffff) return MI355X_ERR_UNSUPPORTED;
     hipStream_t st = (hipStream_t) stream;
+    {
+        // rows in registers: up to 2048 values for a wavefront, 8192 for four.  Four while a row each would leave the GPU short of
+        // wavefronts (up to 4 rows per CU), and 16-byte pieces where every row begins at such an address.
+        auto al = [](const mi355x_tensor * t, size_t a) { return (uintptr_t) t->data % a == 0 && t->nb[1] % a == 0 && t->nb[2] % a == 0 && t->nb[3] % a == 0; };
+        const bool f16 = mask && mask->type == MI355X_TYPE_F16;
+        const int n = (int)(src->ne[0] < 8193 ? src->ne[0] : 8193);
+        const int vec = n % 4 == 0 && al(src, 16) && al(dst, 16) && (!mask || ((uintptr_t) mask->data % (f16 ? 8 : 16) == 0 && mask->nb[1] % (f16 ? 8 : 16) == 0)) ? 4 : 1;
+        const int wpr = nrows <= 1024 || n > 2048 ? 4 : 1;
+        const int ni = (n + 64 * wpr * vec - 1) / (64 * wpr * vec);
+        const int64_t gx = wpr == 4 ? src->ne[1] : (src->ne[1] + 3) / 4;
+        if (n <= 8192 && gx <= 0x7fffffff / 4 && src->ne[2] <= 65535 && src->ne[3] <= 65535) {
+            const dim3 g((unsigned) gx, (unsigned) src->ne[2], (unsigned) src->ne[3]);
+            auto launch = [&](auto tm, auto v, auto k, auto w) {
+                k_soft_max_regs<decltype(tm), decltype(v)::value, decltype(k)::value, decltype(w)::value><<<g, 256, 0, st>>>(
+                    make_view(src), make_view(dst), mask ? (const char *) mask->data : nullptr, mask ? (int64_t) mask->nb[1] : 0, scale);
+            };
+            auto pieces = [&](auto tm, auto v, auto w) {       // 32 values per lane at most
+                constexpr int V = decltype(v)::value;
+                if      (ni * V <= 4)  launch(tm, v, std::integral_constant<int, 4 / V>{}, w);
+                else if (ni * V <= 8)  launch(tm, v, std::integral_constant<int, 8 / V>{}, w);
+                else if (ni * V <= 16) launch(tm, v, std::integral_constant<int, 16 / V>{}, w);
+                else if (ni * V <= 24) launch(tm, v, std::integral_constant<int, 24 / V>{}, w);
+                else                   launch(tm, v, std::integral_constant<int, 32 / V>{}, w);
+            };
+            auto widths = [&](auto tm, auto v) {
+                if (wpr == 4) pieces(tm, v, std::integral_constant<int, 4>{}); else pieces(tm, v, std::integral_constant<int, 1>{});
+            };
+            auto types = [&](auto tm) {
+                if (vec == 4) widths(tm, std::integral_constant<int, 4>{}); else widths(tm, std::integral_constant<int, 1>{});
+            };
+            if (f16) types(half_t{}); else types(float{});
+            return launch_status();
+        }
+    }
     // when src aliases dst the first pass must not be overwritten before the second reads it: the kernel
     // recomputes v from x in pass 2 and only then stores, lane-locally, so aliasing is safe.
     if (mask && mask->type == MI355X_TYPE_F16)
