@@ -92,6 +92,10 @@ __device__ __forceinline__ uint16_t f2h_bits(float f) {
     return h;
 }
 
+// a / b for the same counts in a whole launch, both below 2^31.  b is 1 almost always (nothing broadcast, one slice), and a 64-bit
+// division is a hundred instructions in front of a kernel's first load.
+__device__ __forceinline__ uint32_t div_count(uint32_t a, int64_t b) { return (uint32_t) b == 1 ? a : a / (uint32_t) b; }
+
 // Reductions over aligned groups of W = 4 .. 64 lanes, the result in every lane of the group: DPP steps inside the rows
 // of 16 lanes (a mirror pairs the lanes as well as an exchange does, for a commutative reduction), a swizzle across two
 // rows, a permute across the halves of the wavefront.  A DPP step costs one vector instruction; the ds_bpermute behind

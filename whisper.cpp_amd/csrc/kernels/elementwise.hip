@@ -21,7 +21,7 @@ template <int OP> __device__ __forceinline__ float bin_op(float a, float b) { re
 template <int OP>
 __global__ void k_bin_contig4(const float4 * __restrict__ a, const float4 * __restrict__ b, float4 * __restrict__ d,
                               int64_t n4, int64_t n1_4) {
-    int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t i = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x;
     if (i >= n4) return;
     float4 x = a[i];
     float4 y = b[n1_4 == n4 ? i : i % n1_4];
@@ -32,7 +32,7 @@ __global__ void k_bin_contig4(const float4 * __restrict__ a, const float4 * __re
 
 template <int OP>
 __global__ void k_bin_generic(tview a, tview b, tview d, int64_t n) {
-    int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t i = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x;
     if (i >= n) return;
     int64_t i0 = i % d.ne0; int64_t t = i / d.ne0;
     int64_t i1 = t % d.ne1; t /= d.ne1;
@@ -82,7 +82,7 @@ template <int OP> __device__ __forceinline__ float un_op(float x, float s, const
 
 template <int OP>
 __global__ void k_unary_contig4(const float4 * __restrict__ a, float4 * __restrict__ d, int64_t n4, float s, const uint16_t * __restrict__ tab) {
-    int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t i = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x;
     if (i >= n4) return;
     float4 x = a[i];
     x.x = un_op<OP>(x.x, s, tab); x.y = un_op<OP>(x.y, s, tab); x.z = un_op<OP>(x.z, s, tab); x.w = un_op<OP>(x.w, s, tab);
@@ -91,7 +91,7 @@ __global__ void k_unary_contig4(const float4 * __restrict__ a, float4 * __restri
 
 template <int OP>
 __global__ void k_unary_generic(tview a, tview d, int64_t n, float s, const uint16_t * __restrict__ tab) {
-    int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t i = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x;
     if (i >= n) return;
     int64_t i0 = i % d.ne0; int64_t t = i / d.ne0;
     int64_t i1 = t % d.ne1; t /= d.ne1;
@@ -140,7 +140,7 @@ template <> __device__ __forceinline__ void st_from_f32<half_t>(char * p, float 
 // The i-th element of src in its own index order goes to the i-th element of dst in its index order.
 template <typename TS, typename TD>
 __global__ void k_cpy_generic(tview s, tview d, int64_t n) {
-    int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t i = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x;
     if (i >= n) return;
     int64_t s0 = i % s.ne0; int64_t t = i / s.ne0;
     int64_t s1 = t % s.ne1; t /= s.ne1;
@@ -154,14 +154,14 @@ __global__ void k_cpy_generic(tview s, tview d, int64_t n) {
 
 // both sides dense: 4 elements per lane
 __global__ void k_cpy_f32_f16_contig4(const float4 * __restrict__ s, half4_t * __restrict__ d, int64_t n4) {
-    int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t i = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x;
     if (i >= n4) return;
     float4 x = s[i];
     half4_t h = { (half_t) x.x, (half_t) x.y, (half_t) x.z, (half_t) x.w };
     d[i] = h;
 }
 __global__ void k_cpy_bytes16(const uint4 * __restrict__ s, uint4 * __restrict__ d, int64_t n16) {
-    int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t i = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x;
     if (i < n16) d[i] = s[i];
 }
 
@@ -285,7 +285,7 @@ __device__ __forceinline__ float dq_elem(const uint8_t * row, int64_t k) {
 
 template <int TYPE>
 __global__ void k_dequantize_row(const uint8_t * __restrict__ src, float * __restrict__ dst, int64_t k) {
-    int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t i = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x;
     if (i < k) dst[i] = dq_elem<TYPE>(src, i);
 }
 
@@ -315,7 +315,7 @@ __global__ void k_get_rows(tview s, tview ids, tview d) {
     const bool ok = row >= 0 && row < s.ne1;
     const uint8_t * sp = (const uint8_t *) s.p + (int64_t)(ok ? row : 0)*s.nb1 + i11*s.nb2 + i12*s.nb3;
     float * dp = (float *)(d.p + i10*d.nb1 + i11*d.nb2 + i12*d.nb3);
-    for (int64_t k = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; k < d.ne0; k += (int64_t) gridDim.x * blockDim.x) {
+    for (int64_t k = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x; k < d.ne0; k += (int64_t) gridDim.x * blockDim.x) {
         dp[k] = ok ? dq_elem<TYPE>(sp, k) : __builtin_nanf("");
     }
 }
@@ -351,7 +351,7 @@ __global__ void k_get_rows_add(tview s0, tview ids0, tview s1, tview ids1, tview
     const uint8_t * sp = (const uint8_t *) s0.p + (int64_t)(ok ? r0 : 0) * s0.nb1;
     const float *   pp = (const float *)(s1.p + (int64_t)(ok ? r1 : 0) * s1.nb1);
     float * dp = (float *)(d.p + i * d.nb1);
-    for (int64_t k = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; k < d.ne0; k += (int64_t) gridDim.x * blockDim.x) {
+    for (int64_t k = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x; k < d.ne0; k += (int64_t) gridDim.x * blockDim.x) {
         dp[k] = ok ? dq_elem<TYPE>(sp, k) + pp[k] : __builtin_nanf("");
     }
 }
@@ -385,7 +385,7 @@ extern "C" int mi355x_get_rows_add(const mi355x_tensor * src0, const mi355x_tens
 // ------------------------------------------------------------------------------------------------------
 
 __global__ void k_quantize_q8_0(const float * __restrict__ x, uint8_t * __restrict__ y, int64_t nblk) {
-    const int64_t t   = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t t   = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x;
     const int64_t blk = t / QK;
     const int     j   = (int)(t % QK);
     if (blk >= nblk) return;                       // whole half-waves leave together (blockDim is a multiple of 32)
@@ -464,7 +464,7 @@ extern "C" int mi355x_im2col_1d(const mi355x_tensor * src, const mi355x_tensor *
 // ------------------------------------------------------------------------------------------------------
 
 __global__ void k_concat(tview a, tview b, tview d, int64_t n, int dim) {
-    int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t i = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x;
     if (i >= n) return;
     int64_t idx[4];
     idx[0] = i % d.ne0; int64_t t = i / d.ne0;
@@ -500,11 +500,11 @@ extern "C" int mi355x_concat(const mi355x_tensor * src0, const mi355x_tensor * s
 // ------------------------------------------------------------------------------------------------------
 
 __global__ void k_fill16(uint4 * __restrict__ d, uint32_t w, int64_t n16) {
-    int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t i = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x;
     if (i < n16) d[i] = make_uint4(w, w, w, w);
 }
 __global__ void k_fill1(uint8_t * __restrict__ d, uint8_t v, int64_t n) {
-    int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t i = (int64_t) blockIdx.x * EW_BLOCK + threadIdx.x;
     if (i < n) d[i] = v;
 }
 

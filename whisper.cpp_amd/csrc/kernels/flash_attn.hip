@@ -62,8 +62,8 @@ __global__ void __launch_bounds__(256) k_fattn_vec(fa_args a) {
     const int64_t n = wid % a.N, h = (wid / a.N) % a.H, i3 = wid / (a.N * a.H);
 
     const float * qp = (const float *)(a.q + n * a.q_nb1 + h * a.q_nb2 + i3 * a.q_nb3);
-    const char *  kb = a.k + (h / a.hk_ratio) * a.k_nb2 + (i3 / a.k_ne3_ratio) * a.k_nb3;
-    const char *  vb = a.v + (h / a.hv_ratio) * a.v_nb2 + (i3 / a.v_ne3_ratio) * a.v_nb3;
+    const char *  kb = a.k + div_count((uint32_t) h, a.hk_ratio) * a.k_nb2 + div_count((uint32_t) i3, a.k_ne3_ratio) * a.k_nb3;
+    const char *  vb = a.v + div_count((uint32_t) h, a.hv_ratio) * a.v_nb2 + div_count((uint32_t) i3, a.v_ne3_ratio) * a.v_nb3;
     const half_t * mp = a.mask ? (const half_t *)(a.mask + n * a.m_nb1) : nullptr;
 
     float q[FA_D];
@@ -324,8 +324,8 @@ __global__ void __launch_bounds__(256) k_fattn_seq_row(fa_args a, int kv_pad) {
     if (wave != 0) {
         // ---- producers ----------------------------------------------------------------------------------------------
         const float * qp = (const float *)(a.q + n * a.q_nb1 + h * a.q_nb2 + i3 * a.q_nb3);
-        const char *  kb = a.k + (h / a.hk_ratio) * a.k_nb2 + (i3 / a.k_ne3_ratio) * a.k_nb3;
-        const char *  vb = a.v + (h / a.hv_ratio) * a.v_nb2 + (i3 / a.v_ne3_ratio) * a.v_nb3;
+        const char *  kb = a.k + div_count((uint32_t) h, a.hk_ratio) * a.k_nb2 + div_count((uint32_t) i3, a.k_ne3_ratio) * a.k_nb3;
+        const char *  vb = a.v + div_count((uint32_t) h, a.hv_ratio) * a.v_nb2 + div_count((uint32_t) i3, a.v_ne3_ratio) * a.v_nb3;
         const char * mp = a.mask ? a.mask + n * a.m_nb1 : nullptr;
         const int stid = tid - WAVE, pw = wave - 1;
 
@@ -625,8 +625,8 @@ __global__ void __launch_bounds__(256) k_fattn_pk_row(fa_args a, int kv_pad) {
     if (wave != 0) {
         // ---- producers ----------------------------------------------------------------------------------------------
         const float * qp = (const float *)(a.q + n * a.q_nb1 + h * a.q_nb2 + i3 * a.q_nb3);
-        const char *  kb = a.k + (h / a.hk_ratio) * a.k_nb2 + (i3 / a.k_ne3_ratio) * a.k_nb3;
-        const char *  vb = a.v + (h / a.hv_ratio) * a.v_nb2 + (i3 / a.v_ne3_ratio) * a.v_nb3;
+        const char *  kb = a.k + div_count((uint32_t) h, a.hk_ratio) * a.k_nb2 + div_count((uint32_t) i3, a.k_ne3_ratio) * a.k_nb3;
+        const char *  vb = a.v + div_count((uint32_t) h, a.hv_ratio) * a.v_nb2 + div_count((uint32_t) i3, a.v_ne3_ratio) * a.v_nb3;
         const char * mp = a.mask ? a.mask + n * a.m_nb1 : nullptr;
         const int stid = tid - WAVE, pw = wave - 1;
         const float scale2 = a.scale * LOG2E_F;
@@ -944,8 +944,8 @@ __global__ void __launch_bounds__(512, 2) k_fattn_seq_tile(fa_args a) {
         // ---- producers ---------------------------------------------------------------------------------------------------------------
         const int tid = threadIdx.x - 256, pw = wave - 4;
         const char * qb = a.q + h * a.q_nb2 + i3 * a.q_nb3;
-        const char * kb = a.k + (h / a.hk_ratio) * a.k_nb2 + (i3 / a.k_ne3_ratio) * a.k_nb3;
-        const char * vb = a.v + (h / a.hv_ratio) * a.v_nb2 + (i3 / a.v_ne3_ratio) * a.v_nb3;
+        const char * kb = a.k + div_count((uint32_t) h, a.hk_ratio) * a.k_nb2 + div_count((uint32_t) i3, a.k_ne3_ratio) * a.k_nb3;
+        const char * vb = a.v + div_count((uint32_t) h, a.hv_ratio) * a.v_nb2 + div_count((uint32_t) i3, a.v_ne3_ratio) * a.v_nb3;
 
         // Q tile -> f16 in LDS; thread t: row t/4, 16 values
         {
@@ -1263,17 +1263,19 @@ __global__ void __launch_bounds__(256 + 64 * PW, 2) k_fattn_pk_tile(fa_args a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // an XCD gets one run of consecutive (head, query tile) pairs, head-major, so that a head's K and V stay in one or two L2s
-    const uint32_t lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), total = gridDim.x * gridDim.y * gridDim.z;
+    const uint32_t gx = (uint32_t)((a.N + TQ - 1) / TQ), gy = (uint32_t) a.H;        // (the grid; gridDim is a trip to memory of its own)
+    const uint32_t lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), total = gx * gy * (uint32_t) a.ne3;
     const uint32_t xcd = lin % 8, per = total / 8, extra = total % 8;
     const uint32_t item = xcd * per + (xcd < extra ? xcd : extra) + lin / 8;
-    const int64_t n0 = (int64_t)(item % gridDim.x) * TQ, h = (item / gridDim.x) % gridDim.y, i3 = item / (gridDim.x * gridDim.y);
+    const uint32_t heads = div_count(item, gx);
+    const int64_t n0 = (int64_t)(item - heads * gx) * TQ, i3 = a.ne3 == 1 ? 0 : heads / gy, h = heads - i3 * gy;
     const int n_tiles = (int)((a.KV + P_KV - 1) / P_KV);
 
     if (wave >= 4) {
         // ---- producers ---------------------------------------------------------------------------------------------------------------
         const int pw = wave - 4, r16 = lane & 15, g = lane >> 4;
-        const char * kb = a.k + (h / a.hk_ratio) * a.k_nb2 + (i3 / a.k_ne3_ratio) * a.k_nb3;
-        const char * vb = a.v + (h / a.hv_ratio) * a.v_nb2 + (i3 / a.v_ne3_ratio) * a.v_nb3;
+        const char * kb = a.k + div_count((uint32_t) h, a.hk_ratio) * a.k_nb2 + div_count((uint32_t) i3, a.k_ne3_ratio) * a.k_nb3;
+        const char * vb = a.v + div_count((uint32_t) h, a.hv_ratio) * a.v_nb2 + div_count((uint32_t) i3, a.v_ne3_ratio) * a.v_nb3;
         // Rows of a tile: 8 loads of 8 rows for K and for V, dealt to the wavefronts.  K: row pairs form 256-byte lines, the 16-byte
         // chunk c of row r sits in slot (r & 1) * 8 + (c ^ (line & 7)), so that the 16 rows of a fragment read cover all banks once.
         constexpr int LD = 8 / PW;
@@ -1600,8 +1602,8 @@ __global__ void __launch_bounds__(256) k_fattn_mfma(fa_args a) {
     const int wq = (wave >> 1) * 32, wk = (wave & 1) * 32;
     const int64_t n0 = (int64_t) blockIdx.x * M_Q, h = blockIdx.y, i3 = blockIdx.z;
     const char * qb = a.q + h * a.q_nb2 + i3 * a.q_nb3;
-    const char * kb = a.k + (h / a.hk_ratio) * a.k_nb2 + (i3 / a.k_ne3_ratio) * a.k_nb3;
-    const char * vb = a.v + (h / a.hv_ratio) * a.v_nb2 + (i3 / a.v_ne3_ratio) * a.v_nb3;
+    const char * kb = a.k + div_count((uint32_t) h, a.hk_ratio) * a.k_nb2 + div_count((uint32_t) i3, a.k_ne3_ratio) * a.k_nb3;
+    const char * vb = a.v + div_count((uint32_t) h, a.hv_ratio) * a.v_nb2 + div_count((uint32_t) i3, a.v_ne3_ratio) * a.v_nb3;
 
     // B operand of the first product: lane (query l32, half g) holds q[16 kk + 8 g .. + 7], rounded to f16 as the CPU backend does
     const int64_t n  = n0 + wq + l32;

@@ -17,6 +17,7 @@ bool ks_pick_group(int64_t M, int64_t N, int64_t K, int count, ks_shape & s);
 bool ks_converts(const ks_shape & s);           // the shape has a KS_X_CVT form
 // rows of src0 and src1 16-byte aligned; a.x: src1 (KS_X_CVT, KS_X_F32) or its f16 rows
 int launch_gemm_ks(const mm_args & a, const ks_shape & s, int xm, half_t * x16, int64_t x16_slice, hipStream_t st);
-int launch_gemm_ks_group(const mm_args & a, const mm_group & all, int count, const ks_shape & s, hipStream_t st);
+// x16: a.x is f32 (KS_X_CVT) and its f16 rows go there; NULL: a.x is f16 rows
+int launch_gemm_ks_group(const mm_args & a, const mm_group & all, int count, const ks_shape & s, half_t * x16, hipStream_t st);
 // any alignment, any K
 int launch_gemm_kd(const mm_args & a, int xm, hipStream_t st);

@@ -292,9 +292,8 @@ __device__ __forceinline__ void gemm_kd_tile(const mm_args & a, const char * wb,
 }
 
 // grids: m tiles x n tiles x batch
-#define KS_SLICES const int64_t b2 = blockIdx.z % a.ne12, b3 = blockIdx.z / a.ne12; \
-    const char * wb = a.w + (b2 / a.r2) * a.w_nb2 + (b3 / a.r3) * a.w_nb3, * xb = a.x + b2 * a.x_nb2 + b3 * a.x_nb3; \
-    const int64_t d_off = b2 * a.d_nb2 + b3 * a.d_nb3, m0 = (int64_t) blockIdx.x * 16 * MT, n0 = (int64_t) blockIdx.y * 16 * NT;
+#define KS_SLICES const mm_slice_ptrs z = mm_slice(a, blockIdx.z); const char * wb = z.w, * xb = z.x; const int64_t d_off = z.d_off; \
+    const int64_t m0 = (int64_t) blockIdx.x * 16 * MT, n0 = (int64_t) blockIdx.y * 16 * NT;
 
 template <int MT, int NT, int KW, int D, int XR, int XM, bool EMIT>
 __global__ void __launch_bounds__(64 * KW) k_gemm_ks(mm_args a, half_t * x16, int64_t x16_slice) {
@@ -303,12 +302,13 @@ __global__ void __launch_bounds__(64 * KW) k_gemm_ks(mm_args a, half_t * x16, in
 }
 // several products over the same activations: blockIdx.z picks the weights, the destination and the epilogue
 struct ks_group { mm_group_entry e[KS_GROUP_MAX]; };
-template <int MT, int NT, int KW, int D, int XR>
-__global__ void __launch_bounds__(64 * KW) k_gemm_ks_group(mm_args a, ks_group grp) {
+template <int MT, int NT, int KW, int D, int XR, int XM>
+__global__ void __launch_bounds__(64 * KW) k_gemm_ks_group(mm_args a, ks_group grp, half_t * x16) {
     const mm_group_entry & ge = grp.e[blockIdx.z];
     epi_args e;
     e.flags = ge.flags; e.scale = ge.scale; e.bias = ge.bias; e.residual = ge.residual; e.gelu = a.e.gelu; e.image = nullptr;
-    gemm_ks_tile<MT, NT, KW, D, XR, KS_X_F16, false>(a, ge.w, a.x, ge.d, e, 0, ge.d_nb1, (int64_t) blockIdx.x * 16 * MT, (int64_t) blockIdx.y * 16 * NT, nullptr);
+    gemm_ks_tile<MT, NT, KW, D, XR, XM, false>(a, ge.w, a.x, ge.d, e, 0, ge.d_nb1, (int64_t) blockIdx.x * 16 * MT, (int64_t) blockIdx.y * 16 * NT,
+                                               blockIdx.x == 0 && blockIdx.z == 0 ? x16 : nullptr);
 }
 template <int MT, int NT, int KW, int XM>
 __global__ void __launch_bounds__(64 * KW) k_gemm_kd(mm_args a) {
@@ -416,23 +416,28 @@ int launch_gemm_ks(const mm_args & a, const ks_shape & s, int xm, half_t * x16, 
     }
 }
 
-template <int MT, int NT, int KW, int D, int XR>
-static int launch_ks_group_t(const mm_args & a, const ks_group & grp, int count, hipStream_t st) {
-    constexpr size_t ring = (size_t) KW * D * (2 * MT + XR / 8) * 1024, red = ks_red_bytes<MT, NT, KW>(), lds = ring > red ? ring : red;
+template <int MT, int NT, int KW, int D, int XR, int XM>
+static int launch_ks_group_t(const mm_args & a, const ks_group & grp, int count, half_t * x16, hipStream_t st) {
+    constexpr size_t ring = (size_t) KW * D * (2 * MT + XR * (XM == KS_X_F16 ? 2 : 4) / 16) * 1024, red = ks_red_bytes<MT, NT, KW>(), lds = ring > red ? ring : red;
     static std::atomic<bool> configured[64];
     dim3 grid;
     if (int rc = ks_grid<MT, NT>(a, grid)) return rc;
     grid.z = (unsigned) count;
-    if (int rc = ks_configure((const void *) k_gemm_ks_group<MT, NT, KW, D, XR>, lds, configured)) return rc;
-    k_gemm_ks_group<MT, NT, KW, D, XR><<<grid, 64 * KW, lds, st>>>(a, grp);
+    if (int rc = ks_configure((const void *) k_gemm_ks_group<MT, NT, KW, D, XR, XM>, lds, configured)) return rc;
+    k_gemm_ks_group<MT, NT, KW, D, XR, XM><<<grid, 64 * KW, lds, st>>>(a, grp, x16);
     return launch_status();
 }
-int launch_gemm_ks_group(const mm_args & a, const mm_group & all, int count, const ks_shape & s, hipStream_t st) {
+template <int MT, int NT, int KW, int D, int XR>
+static int launch_ks_group_x(const mm_args & a, const ks_group & grp, int count, half_t * x16, hipStream_t st) {
+    if constexpr (NT == 1) if (x16) return launch_ks_group_t<MT, NT, KW, D, XR, KS_X_CVT>(a, grp, count, x16, st);
+    return x16 ? MI355X_ERR_UNSUPPORTED : launch_ks_group_t<MT, NT, KW, D, XR, KS_X_F16>(a, grp, count, x16, st);
+}
+int launch_gemm_ks_group(const mm_args & a, const mm_group & all, int count, const ks_shape & s, half_t * x16, hipStream_t st) {
     ks_group grp;
     for (int i = 0; i < count; ++i) grp.e[i] = all.e[i];
 #define KS_CASE(MT, NT, KW, D) if (s.mt == MT && s.nt == NT && s.kw == KW && s.d == D) { \
-        if constexpr (NT == 1) if (a.N <= 8) return launch_ks_group_t<MT, NT, KW, D, 8>(a, grp, count, st); \
-        return launch_ks_group_t<MT, NT, KW, D, 16 * NT>(a, grp, count, st); }
+        if constexpr (NT == 1) if (a.N <= 8) return launch_ks_group_x<MT, NT, KW, D, 8>(a, grp, count, x16, st); \
+        return launch_ks_group_x<MT, NT, KW, D, 16 * NT>(a, grp, count, x16, st); }
     KS_CASE(1, 1, 4, 2) KS_CASE(1, 1, 8, 2) KS_CASE(2, 1, 4, 2) KS_CASE(2, 2, 4, 2) KS_CASE(4, 4, 4, 2)
 #undef KS_CASE
     return MI355X_ERR_UNSUPPORTED;

@@ -332,12 +332,11 @@ __global__ void k_w_to_f16(const char * __restrict__ w, half_t * __restrict__ ou
 template <bool Q8>
 __global__ void k_x_to_f16(const char * __restrict__ x, half_t * __restrict__ out, int64_t K, int64_t N,
                            int64_t x_nb1, int64_t x_nb2, int64_t ne12, int64_t x_nb3, int64_t slice_halves) {
-    const int64_t t  = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t k4 = K / 4;
-    const int64_t b  = blockIdx.y;
-    if (t >= k4 * N) return;                                                // whole 8-lane groups leave together (K % 32 == 0 when Q8)
-    const int64_t n = t / k4, c = t % k4;
-    const float4 v = *(const float4 *)(x + n * x_nb1 + (b % ne12) * x_nb2 + (b / ne12) * x_nb3 + c * 16);
+    const uint32_t t = blockIdx.x * 256 + threadIdx.x, k4 = (uint32_t)(K / 4);         // (k4 N < 2^32: a batch slice of 2^34 values is no case)
+    const int64_t b = blockIdx.y;
+    if (t >= k4 * (uint32_t) N) return;                                     // whole 8-lane groups leave together (K % 32 == 0 when Q8)
+    const uint32_t n = t / k4, c = t - n * k4, b3 = div_count(blockIdx.y, ne12), b2 = blockIdx.y - b3 * (uint32_t) ne12;
+    const float4 v = *(const float4 *)(x + n * x_nb1 + b2 * x_nb2 + b3 * x_nb3 + c * 16);
     half4_t h;
     if (Q8) {
         float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
@@ -830,10 +829,8 @@ static int tile_path_width(int64_t tiles_m, int64_t tiles_n, int64_t run, int bn
 
 template <int TI, int TJ, int S, bool KTAIL, bool FULL, bool EMIT>
 __global__ void __launch_bounds__(256, 2) k_gemm_f16(mm_args a, int tiles_m, int tiles_n, int sw) {
-    const int64_t b2 = blockIdx.y % a.ne12, b3 = blockIdx.y / a.ne12;
-    gemm_f16_tile<TI, TJ, S, KTAIL, FULL, EMIT>(a, tiles_m, tiles_n, sw, xcd_run_index(blockIdx.x, tiles_m * tiles_n),
-                                          a.w + (b2 / a.r2) * a.w_nb2 + (b3 / a.r3) * a.w_nb3, a.x + b2 * a.x_nb2 + b3 * a.x_nb3,
-                                          a.d + b2 * a.d_nb2 + b3 * a.d_nb3, a.e, b2 * a.d_nb2 + b3 * a.d_nb3, a.d_nb1);
+    const mm_slice_ptrs z = mm_slice(a, blockIdx.y);
+    gemm_f16_tile<TI, TJ, S, KTAIL, FULL, EMIT>(a, tiles_m, tiles_n, sw, xcd_run_index(blockIdx.x, tiles_m * tiles_n), z.w, z.x, a.d + z.d_off, a.e, z.d_off, a.d_nb1);
 }
 
 // Several products over the same src1 in one launch (the Q, K and V projections of a layer; the cross-attention K and V
@@ -853,10 +850,8 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f16_group(mm_args a, int tiles_
 // the direct-to-LDS form of the two kernels above (K a multiple of 64)
 template <int TI, int TJ, int NBUF, bool EMIT>
 __global__ void __launch_bounds__(256, 2) k_gemm_f16_dl(mm_args a, int tiles_m, int tiles_n, int sw) {
-    const int64_t b2 = blockIdx.y % a.ne12, b3 = blockIdx.y / a.ne12;
-    gemm_f16_tile_dl<TI, TJ, NBUF, EMIT>(a, tiles_m, tiles_n, sw, xcd_run_index(blockIdx.x, tiles_m * tiles_n),
-                                         a.w + (b2 / a.r2) * a.w_nb2 + (b3 / a.r3) * a.w_nb3, a.x + b2 * a.x_nb2 + b3 * a.x_nb3,
-                                         a.d + b2 * a.d_nb2 + b3 * a.d_nb3, a.e, b2 * a.d_nb2 + b3 * a.d_nb3, a.d_nb1);
+    const mm_slice_ptrs z = mm_slice(a, blockIdx.y);
+    gemm_f16_tile_dl<TI, TJ, NBUF, EMIT>(a, tiles_m, tiles_n, sw, xcd_run_index(blockIdx.x, tiles_m * tiles_n), z.w, z.x, a.d + z.d_off, a.e, z.d_off, a.d_nb1);
 }
 template <int TI, int TJ, int NBUF>
 __global__ void __launch_bounds__(256, 2) k_gemm_f16_dl_group(mm_args a, int tiles_m, int tiles_n, int sw, mm_group grp) {
@@ -896,10 +891,8 @@ static int launch_gemm_f16_dl(const mm_args & a, hipStream_t st) {
 // the two-role form (K a multiple of 64 S)
 template <int TI, int TJ, int S, bool EMIT, int NP>
 __global__ void __launch_bounds__(256 + NP) k_gemm_f16_rs(mm_args a, int tiles_m, int tiles_n, int sw) {
-    const int64_t b2 = blockIdx.y % a.ne12, b3 = blockIdx.y / a.ne12;
-    gemm_f16_tile_rs<TI, TJ, S, EMIT, NP>(a, tiles_m, tiles_n, sw, xcd_run_index(blockIdx.x, tiles_m * tiles_n),
-                                      a.w + (b2 / a.r2) * a.w_nb2 + (b3 / a.r3) * a.w_nb3, a.x + b2 * a.x_nb2 + b3 * a.x_nb3,
-                                      a.d + b2 * a.d_nb2 + b3 * a.d_nb3, a.e, b2 * a.d_nb2 + b3 * a.d_nb3, a.d_nb1);
+    const mm_slice_ptrs z = mm_slice(a, blockIdx.y);
+    gemm_f16_tile_rs<TI, TJ, S, EMIT, NP>(a, tiles_m, tiles_n, sw, xcd_run_index(blockIdx.x, tiles_m * tiles_n), z.w, z.x, a.d + z.d_off, a.e, z.d_off, a.d_nb1);
 }
 template <int TI, int TJ> constexpr int rs_ring() { return 4; }
 #define RS_NP 512       // operand threads: 512 (three 16-byte pieces each per step of a 128 x 64 tile) beat 256 by 7 %
@@ -1170,6 +1163,10 @@ extern "C" int mi355x_mul_mat_group(const mi355x_mul_mat_item * items, int count
         if (!(flags & MI355X_MM_WS_READY)) {
             dim3 qgrid((unsigned)((a.K / 4 * a.N + 255) / 256), 1);
             const bool q8 = (flags & MI355X_MM_ACT_Q8_0) && !(flags & MI355X_MM_EXACT_ACT);
+            // a handful of columns: the products round src1 to f16 themselves, the first leaves the rows in the workspace
+            ks_shape ks;
+            if (!q8 && !(flags & MI355X_MM_PREPARE_ONLY) && ks_pick_group(a.M, a.N, a.K, count, ks) && ks_converts(ks))
+                return launch_gemm_ks_group(a, grp, count, ks, (half_t *) workspace, st);
             if (q8) k_x_to_f16<true ><<<qgrid, 256, 0, st>>>(a.x, (half_t *) workspace, a.K, a.N, a.x_nb1, 0, 1, 0, 0);
             else    k_x_to_f16<false><<<qgrid, 256, 0, st>>>(a.x, (half_t *) workspace, a.K, a.N, a.x_nb1, 0, 1, 0, 0);
         }
@@ -1177,7 +1174,7 @@ extern "C" int mi355x_mul_mat_group(const mi355x_mul_mat_item * items, int count
     }
     if (flags & MI355X_MM_PREPARE_ONLY) return launch_status();
     ks_shape ks;
-    if (ks_pick_group(a.M, a.N, a.K, count, ks)) return launch_gemm_ks_group(a, grp, count, ks, st);
+    if (ks_pick_group(a.M, a.N, a.K, count, ks)) return launch_gemm_ks_group(a, grp, count, ks, nullptr, st);
     const int64_t blocks22 = ((a.N + 127) / 128) * ((a.M + 127) / 128) * count;
     return blocks22 >= 300 ? launch_gemm_f16_group<2, 2>(a, grp, count, st) : launch_gemm_f16_group<2, 1>(a, grp, count, st);
 }

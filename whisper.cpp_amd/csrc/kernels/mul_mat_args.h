@@ -33,6 +33,12 @@ struct mm_group_entry { const char * w; char * d; const float * bias; const char
 struct mm_group { mm_group_entry e[MM_GROUP_MAX]; };
 
 #ifdef __HIPCC__
+// the operands of batch slice z (z = b2 + ne12 b3)
+struct mm_slice_ptrs { const char * w; const char * x; int64_t d_off; };
+__device__ __forceinline__ mm_slice_ptrs mm_slice(const mm_args & a, uint32_t z) {
+    const uint32_t b3 = a.ne13 == 1 ? 0 : div_count(z, a.ne12), b2 = z - b3 * (uint32_t) a.ne12;
+    return { a.w + div_count(b2, a.r2) * a.w_nb2 + div_count(b3, a.r3) * a.w_nb3, a.x + b2 * a.x_nb2 + b3 * a.x_nb3, b2 * a.d_nb2 + b3 * a.d_nb3 };
+}
 // four bits -> bit 4 of four bytes
 __device__ __forceinline__ uint32_t spread4_to_bit4(uint32_t nib) {
     return ((nib * 0x00204081u) & 0x01010101u) << 4;

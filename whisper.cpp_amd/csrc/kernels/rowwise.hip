@@ -21,11 +21,15 @@
 // 512, ... 1280 values: no guard around any load, reduction term or store (34 exec-mask branches less in a kernel whose time
 // is its chain of dependent instructions)
 template <int NV, int EMIT, bool FULL = false>
-__global__ void __launch_bounds__(ROWS_PER_BLOCK * WAVE) k_norm(tview s, tview d, int64_t nrows, float eps, const float * __restrict__ w, const float * __restrict__ b, half_t * __restrict__ x16) {
+__global__ void __launch_bounds__(ROWS_PER_BLOCK * WAVE) k_norm(tview s, tview d, int nrows, float eps, const float * __restrict__ w, const float * __restrict__ b, half_t * __restrict__ x16) {
     const int     lane = threadIdx.x % WAVE;
-    const int64_t row  = (int64_t) blockIdx.x * ROWS_PER_BLOCK + threadIdx.x / WAVE;
+    const int     row  = (int) blockIdx.x * ROWS_PER_BLOCK + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     if (row >= nrows) return;
-    const int64_t i1 = row % s.ne1, i2 = (row / s.ne1) % s.ne2, i3 = row / (s.ne1 * s.ne2);
+    uint32_t i1 = row, i2 = 0, i3 = 0;
+    if (s.ne1 != nrows) {                                       // uniform: slices
+        i2 = row / (uint32_t) s.ne1; i1 = row - i2 * (uint32_t) s.ne1;
+        i3 = i2 / (uint32_t) s.ne2;  i2 -= i3 * (uint32_t) s.ne2;
+    }
     const float * x = (const float *)(s.p + i1*s.nb1 + i2*s.nb2 + i3*s.nb3);
     float *       y = (float *)(d.p + i1*d.nb1 + i2*d.nb2 + i3*d.nb3);
     const int64_t ne0 = s.ne0;
@@ -77,17 +81,17 @@ __global__ void __launch_bounds__(ROWS_PER_BLOCK * WAVE) k_norm(tview s, tview d
                     const float dq = h2f(f2h_bits(div127(amax)));
                     if (EMIT == 1) {
                         const half4_t h = { (half_t)((rintf(r.x * id) + 0.0f) * dq), (half_t)((rintf(r.y * id) + 0.0f) * dq), (half_t)((rintf(r.z * id) + 0.0f) * dq), (half_t)((rintf(r.w * id) + 0.0f) * dq) };
-                        *(half4_t *)(x16 + row * ne0 + 4 * (int64_t) c) = h;
+                        *(half4_t *)(x16 + (int64_t) row * ne0 + 4 * (int64_t) c) = h;
                     } else {
                         const int q0 = (int) rintf(r.x * id), q1 = (int) rintf(r.y * id), q2 = (int) rintf(r.z * id), q3 = (int) rintf(r.w * id);
                         int qsum = q0 + q1 + q2 + q3;
                         qsum = lanes_sum<8>(qsum);
                         char * q8 = (char *) x16;
                         const int64_t nbk = ne0 / 32;
-                        ((int32_t *) q8)[row * (ne0 / 4) + c] = (q0 & 0xFF) | ((q1 & 0xFF) << 8) | ((q2 & 0xFF) << 16) | ((q3 & 0xFF) << 24);
+                        ((int32_t *) q8)[(int64_t) row * (ne0 / 4) + c] = (q0 & 0xFF) | ((q1 & 0xFF) << 8) | ((q2 & 0xFF) << 16) | ((q3 & 0xFF) << 24);
                         if ((c & 7) == 0) {
-                            ((float *)(q8 + nrows * ne0))[row * nbk + c / 8] = dq;
-                            ((int32_t *)(q8 + nrows * ne0 + nrows * nbk * 4))[row * nbk + c / 8] = qsum;
+                            ((float *)(q8 + (int64_t) nrows * ne0))[(int64_t) row * nbk + c / 8] = dq;
+                            ((int32_t *)(q8 + (int64_t) nrows * ne0 + (int64_t) nrows * nbk * 4))[(int64_t) row * nbk + c / 8] = qsum;
                         }
                     }
                 }
@@ -134,7 +138,7 @@ static int norm_impl(const mi355x_tensor * src, const mi355x_tensor * dst, float
     // a destination without memory is an argument of the f16-image form alone (the caller wants the image and nothing else)
     if (!src->data || (!dst->data && emit != 1)) return MI355X_ERR_INVALID;
     const int64_t grid = (nrows + ROWS_PER_BLOCK - 1) / ROWS_PER_BLOCK;
-    if (grid > 0x7fffffff) return MI355X_ERR_UNSUPPORTED;
+    if (nrows > 0x7ffffff0) return MI355X_ERR_UNSUPPORTED;
     hipStream_t st = (hipStream_t) stream;
     auto al16 = [](const void * p, const size_t * nb) {
         return (uintptr_t) p % 16 == 0 && nb[1] % 16 == 0 && nb[2] % 16 == 0 && nb[3] % 16 == 0;
