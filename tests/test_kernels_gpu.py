@@ -322,7 +322,7 @@ def test_mul_mat_gelu_epilogue_from_the_lds_table_slice(pkg, oracle, gpu):
 
 # (K, M, N): one unit of K; fewer units than wavefronts; odd rows and columns on every tile size; the K split in 8; more rows
 # than one launch of 16-row tiles is chosen for; sizes on both sides of the change to 128-wide tiles
-@pytest.mark.parametrize("k,m,n", [(64, 70, 5), (64, 300, 130), (64, 1500, 700), (128, 33, 17), (192, 1, 3), (1280, 1281, 8), (2048, 515, 16), (1280, 4113, 4),
+@pytest.mark.parametrize("k,m,n", [(64, 70, 5), (64, 300, 130), (64, 1500, 700), (128, 33, 17), (192, 1, 3), (1280, 1281, 8), (2048, 515, 16), (1280, 4113, 4), (128, 9, 8), (256, 2048, 3), (1024, 2049, 7), (5120, 1281, 5),
                                    (512, 2049, 33), (384, 1000, 487), (448, 513, 900), (256, 1030, 1024), (768, 5001, 27)])
 def test_mul_mat_split_k(pkg, oracle, gpu, own_numbers, k, m, n):
     # f16 weights, f32 activations rounded to f16: against float64 over the rounded operands, with every part of the epilogue;
@@ -348,8 +348,32 @@ def test_mul_mat_split_k(pkg, oracle, gpu, own_numbers, k, m, n):
         assert oracle.nmse(got[0], want) <= (1e-12 if out == torch.float32 else 1e-6)
 
 
+@pytest.mark.parametrize("k,m,n,count", [(512, 512, 1 + 2, 3), (1280, 1280, 5, 3), (256, 385, 8, 2), (768, 2100, 4, 2), (1280, 640, 11, 2)])
+def test_mul_mat_group_f16_few_columns(pkg, oracle, gpu, own_numbers, k, m, n, count):
+    # f32 activations rounded to f16 by the products themselves, the rows left in the workspace for a second call
+    lib = pkg.kernels()
+    ws16, x, bias = [rnd((m, k), 0.05).astype(np.float16) for _ in range(count)], rnd((n, k)), rnd((m,), 0.5)
+    d_w, d_x, d_b = [gpu.up(w.view(np.int16)) for w in ws16], gpu.up(x), gpu.up(bias)
+    tws, tx = [pkg.tensor(w, pkg.F16) for w in d_w], pkg.tensor(d_x, pkg.F32)
+    need = lib.mi355x_mul_mat_workspace_size(tws[0], tx)
+    ws = torch.full((need,), 255, dtype=torch.uint8, device=gpu.dev)
+    got = []
+    for ready in (0, pkg.MM_WS_READY):
+        outs = [torch.full((n, m), 7.0, dtype=torch.float32, device=gpu.dev) for _ in range(count)]
+        tds, epi = [pkg.tensor(o, pkg.F32) for o in outs], pkg.Epilogue(pkg.EPI_BIAS, 1.0, d_b.data_ptr(), None, None)
+        items = (pkg.MulMatItem * count)()
+        for i in range(count):
+            items[i].src0, items[i].dst, items[i].epi = C.pointer(tws[i]), C.pointer(tds[i]), C.pointer(epi)
+        pkg.check(lib.mi355x_mul_mat_group(items, count, tx, ready, ws.data_ptr(), need, gpu.stream))
+        got.append([gpu.down(o) for o in outs])
+    assert np.array_equal(gpu.down(ws)[: 2 * n * k].view(np.float16).reshape(n, k), x.astype(np.float16))
+    for i in range(count):
+        assert np.array_equal(got[0][i], got[1][i])
+        assert oracle.nmse(got[0][i], x.astype(np.float16).astype(np.float64) @ ws16[i].astype(np.float64).T + bias) <= 1e-12
+
+
 # rows that are not 16-byte aligned, any K (the transposed V of a window of 1500, 37 or 1501 positions), one or two columns
-@pytest.mark.parametrize("k,m,n,batch", [(1500, 64, 300, 3), (37, 64, 37, 2), (1501, 64, 5, 2), (1500, 64, 1, 4), (64, 1500, 2, 2), (512, 1000, 1, 1), (1280, 5003, 2, 1), (2048, 48, 1, 1), (3, 5, 40, 1)])
+@pytest.mark.parametrize("k,m,n,batch", [(1500, 64, 300, 3), (37, 64, 37, 2), (1501, 64, 5, 2), (1500, 64, 1, 4), (64, 1500, 2, 2), (512, 1000, 1, 1), (1024, 1283, 2, 1), (1280, 5003, 2, 1), (2048, 48, 1, 1), (3, 5, 40, 1)])
 def test_mul_mat_f16_keeps_f32_activations(pkg, oracle, gpu, own_numbers, k, m, n, batch):
     lib = pkg.kernels()
     w16, x = rnd((batch, m, k), 0.5).astype(np.float16), np.abs(rnd((batch, n, k), 1.0 / k))

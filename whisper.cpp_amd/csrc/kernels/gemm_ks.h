@@ -8,7 +8,7 @@ enum { KS_X_F16 = 0,        // src1 is f16 rows (or their f16 image in the works
                             // the f16 rows in the workspace (what MI355X_MM_WS_READY of a later call refers to)
        KS_X_F32 = 2 };      // src1 is f32 and stays f32: v_mfma_f32_16x16x4_f32 on the widened weights (exact products)
 
-struct ks_shape { int mt, nt, kw, d; };         // tile of 16 mt x 16 nt results, kw wavefronts that share its K range, d buffers each
+struct ks_shape { int mt, nt, kw, d, h; };      // tile of 16 mt x 16 nt results (h = 2: of 8 x 8), kw wavefronts that share its K range, d buffers each
 #define KS_GROUP_MAX 8
 
 // false: the tiled kernels of mul_mat.hip are the better ones for this size (or K is no multiple of 64)

@@ -34,7 +34,7 @@ template <int MT, int NT, int KW> constexpr size_t ks_red_bytes() { return (size
 
 // The partial tiles of the KW wavefronts meet in `red` ([KW][16 NT][LD] floats, free when every wavefront is past its loop) and
 // leave through the epilogue.  EMIT: MI355X_EPI_EMIT_F16 (a block of 32 m is 8 consecutive lanes).
-template <int MT, int NT, int KW, bool EMIT>
+template <int MT, int NT, int KW, bool EMIT, int H = 1>
 __device__ __forceinline__ void ks_finish(float4_t (&acc)[MT][NT], float * red, const mm_args & a, char * db, const epi_args & epi, int64_t batch_off,
                                           int64_t d_nb1, int64_t m0, int64_t n0) {
     static_assert(!EMIT || MT % 2 == 0, "whole Q8_0 blocks per tile");
@@ -47,15 +47,18 @@ __device__ __forceinline__ void ks_finish(float4_t (&acc)[MT][NT], float * red, 
 #pragma unroll
         for (int j = 0; j < NT; ++j) *(float4_t *)(red + (wave * 16 * NT + 16 * j + r16) * LD + 16 * i + 4 * q) = acc[i][j];
     __syncthreads();
-    constexpr int PIECES = 16 * NT * 4 * MT;            // (n, four consecutive m)
+    constexpr int MR = 16 * MT / H, NR = 16 * NT / H;   // rows and columns of the tile
+    constexpr int PIECES = NR * MR / 4;                 // (n, four consecutive m)
 #pragma unroll
     for (int p0 = 0; p0 < PIECES; p0 += 64 * KW) {
         const int p = p0 + tid;
         if (PIECES % (64 * KW) != 0 && p >= PIECES) break;
-        const int nl = p / (4 * MT), ml = p % (4 * MT) * 4;
+        const int nl = p / (MR / 4), ml = p % (MR / 4) * 4;
         float4_t v = *(const float4_t *)(red + nl * LD + ml);
 #pragma unroll
-        for (int w = 1; w < KW; ++w) v += *(const float4_t *)(red + (w * 16 * NT + nl) * LD + ml);
+        for (int w = 0; w < KW; ++w)
+#pragma unroll
+            for (int h = 0; h < H; ++h) if (w + h > 0) v += *(const float4_t *)(red + (w * 16 * NT + nl + h * NR) * LD + ml + h * MR);
         const int64_t n = n0 + nl, m = m0 + ml;
         const bool row = n < a.N, whole = m + 3 < a.M;
         if (!EMIT && (!row || m >= a.M)) continue;
@@ -100,7 +103,11 @@ __device__ __forceinline__ void ks_finish(float4_t (&acc)[MT][NT], float * red, 
 // LDS layout of f16 rows: row pairs form 256-byte lines, the 16-byte chunk c of row r sits in slot (r & 1) * 8 + (c ^ (line & 7))
 // of line r / 2 (the 16 rows of a fragment read then cover all banks once); f32 rows are one line each, chunk c in slot c ^ (r & 15).
 // XR: rows of src1 that are loaded (8 with at most 8 columns: the other columns of the result are not stored).
-template <int MT, int NT, int KW, int D, int XR, int XM, bool EMIT>
+// H = 2, at most 8 columns: the tile is 8 rows, and the 16 rows and 16 columns of the matrix instruction are those 8 rows (8
+// columns) over the first half of K and over the second, so that two of the four 8 x 8 corners of its result are partial sums of the
+// tile (the others are dropped: the matrix cores have nothing else to do).  Twice the workgroups, each with half the weights to
+// fetch: a CU takes in about 45 KB/us here whatever the wavefronts and buffers, so that is what a long K waits for.
+template <int MT, int NT, int KW, int D, int XR, int XM, bool EMIT, int H = 1>
 __device__ __forceinline__ void gemm_ks_tile(const mm_args & a, const char * wb, const char * xb, char * db, const epi_args & epi, int64_t batch_off,
                                              int64_t d_nb1, int64_t m0, int64_t n0, half_t * x16) {
     constexpr int XE = XM == KS_X_F16 ? 2 : 4;
@@ -110,18 +117,26 @@ __device__ __forceinline__ void gemm_ks_tile(const mm_args & a, const char * wb,
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r16 = lane & 15, q = lane >> 4;
     char * mine = smem + wave * (D * UNIT_BYTES);
+    constexpr int MR = 16 * MT / H, NR = 16 * NT / H;
+    const int64_t part = a.K / H;
 
     // load i covers lines 4 i .. + 3; this lane: line 4 i + lane / 16, slot lane % 16
     const char * wp[WL]; const char * xp[XL];
     auto row_of = [&](int i, int & chunk) __attribute__((always_inline)) { const int line = 4 * i + q; chunk = (lane & 7) ^ (line & 7); return 2 * line + ((lane >> 3) & 1); };
 #pragma unroll
-    for (int i = 0; i < WL; ++i) { int c; const int64_t m = m0 + row_of(i, c); wp[i] = wb + (m < a.M ? m : a.M - 1) * a.w_nb1 + c * 16; }
+    for (int i = 0; i < WL; ++i) {
+        int c;
+        const int r = row_of(i, c);
+        const int64_t m = m0 + r % MR;
+        wp[i] = wb + (m < a.M ? m : a.M - 1) * a.w_nb1 + c * 16 + r / MR * (part * 2);
+    }
 #pragma unroll
     for (int i = 0; i < XL; ++i) {
-        int c; int64_t n;
-        if constexpr (XM == KS_X_F16) n = n0 + row_of(i, c);
-        else { const int r = 4 * i + q; c = r16 ^ (r & 15); n = n0 + r; }
-        xp[i] = xb + (n < a.N ? n : a.N - 1) * a.x_nb1 + c * 16;
+        int c, r;
+        if constexpr (XM == KS_X_F16) r = row_of(i, c);
+        else { r = 4 * i + q; c = r16 ^ (r & 15); }
+        const int64_t n = n0 + r % NR;
+        xp[i] = xb + (n < a.N ? n : a.N - 1) * a.x_nb1 + c * 16 + r / NR * (part * XE);
     }
     auto load = [&](int64_t u, int buf) __attribute__((always_inline)) {
         char * to = mine + buf * UNIT_BYTES;
@@ -163,8 +178,9 @@ __device__ __forceinline__ void gemm_ks_tile(const mm_args & a, const char * wb,
                     if constexpr (XM == KS_X_CVT) {
                         const half8_t xv = { (half_t) lo.x, (half_t) lo.y, (half_t) lo.z, (half_t) lo.w, (half_t) hi.x, (half_t) hi.y, (half_t) hi.z, (half_t) hi.w };
                         if (x16) {
-                            const int64_t n = n0 + 16 * j + r16;
-                            if (r16 < XR && n < a.N) *(half8_t *)(x16 + n * a.K + u * KS_UNIT + 32 * s + 8 * q) = xv;
+                            const int rr = 16 * j + r16;
+                            const int64_t n = n0 + rr % NR;
+                            if (r16 < XR && n < a.N) *(half8_t *)(x16 + n * a.K + rr / NR * part + u * KS_UNIT + 32 * s + 8 * q) = xv;
                         }
 #pragma unroll
                         for (int i = 0; i < MT; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[i], xv, acc[i][j], 0, 0, 0);
@@ -179,7 +195,7 @@ __device__ __forceinline__ void gemm_ks_tile(const mm_args & a, const char * wb,
             }
         }
     };
-    const int units = (int)(a.K / KS_UNIT), n_mine = units > wave ? (units - wave + KW - 1) / KW : 0;
+    const int units = (int)(part / KS_UNIT), n_mine = units > wave ? (units - wave + KW - 1) / KW : 0;
 #pragma unroll
     for (int t = 0; t < D - 1; ++t) if (t < n_mine) load(wave + t * KW, t);
     int t = 0, buf = 0;
@@ -192,7 +208,7 @@ __device__ __forceinline__ void gemm_ks_tile(const mm_args & a, const char * wb,
     ks_wait_vmcnt<0>();
     for (; t < n_mine; ++t) { mma(wave + (int64_t) t * KW, buf); buf = buf + 1 == D ? 0 : buf + 1; }
     __syncthreads();                                    // (the partial tiles take the buffers' place)
-    ks_finish<MT, NT, KW, EMIT>(acc, (float *) smem, a, db, epi, batch_off, d_nb1, m0, n0);
+    ks_finish<MT, NT, KW, EMIT, H>(acc, (float *) smem, a, db, epi, batch_off, d_nb1, m0, n0);
 }
 
 template <int MT, int NT, int KW, int XM>
@@ -293,32 +309,33 @@ __device__ __forceinline__ void gemm_kd_tile(const mm_args & a, const char * wb,
 
 // grids: m tiles x n tiles x batch
 #define KS_SLICES const mm_slice_ptrs z = mm_slice(a, blockIdx.z); const char * wb = z.w, * xb = z.x; const int64_t d_off = z.d_off; \
-    const int64_t m0 = (int64_t) blockIdx.x * 16 * MT, n0 = (int64_t) blockIdx.y * 16 * NT;
+    const int64_t m0 = (int64_t) blockIdx.x * (16 * MT / H), n0 = (int64_t) blockIdx.y * (16 * NT / H);
 
-template <int MT, int NT, int KW, int D, int XR, int XM, bool EMIT>
+template <int MT, int NT, int KW, int D, int XR, int XM, bool EMIT, int H>
 __global__ void __launch_bounds__(64 * KW) k_gemm_ks(mm_args a, half_t * x16, int64_t x16_slice) {
     KS_SLICES
-    gemm_ks_tile<MT, NT, KW, D, XR, XM, EMIT>(a, wb, xb, a.d + d_off, a.e, d_off, a.d_nb1, m0, n0, x16 && blockIdx.x == 0 ? x16 + blockIdx.z * x16_slice : nullptr);
+    gemm_ks_tile<MT, NT, KW, D, XR, XM, EMIT, H>(a, wb, xb, a.d + d_off, a.e, d_off, a.d_nb1, m0, n0, x16 && blockIdx.x == 0 ? x16 + blockIdx.z * x16_slice : nullptr);
 }
 // several products over the same activations: blockIdx.z picks the weights, the destination and the epilogue
 struct ks_group { mm_group_entry e[KS_GROUP_MAX]; };
-template <int MT, int NT, int KW, int D, int XR, int XM>
+template <int MT, int NT, int KW, int D, int XR, int XM, int H>
 __global__ void __launch_bounds__(64 * KW) k_gemm_ks_group(mm_args a, ks_group grp, half_t * x16) {
     const mm_group_entry & ge = grp.e[blockIdx.z];
     epi_args e;
     e.flags = ge.flags; e.scale = ge.scale; e.bias = ge.bias; e.residual = ge.residual; e.gelu = a.e.gelu; e.image = nullptr;
-    gemm_ks_tile<MT, NT, KW, D, XR, XM, false>(a, ge.w, a.x, ge.d, e, 0, ge.d_nb1, (int64_t) blockIdx.x * 16 * MT, (int64_t) blockIdx.y * 16 * NT,
+    gemm_ks_tile<MT, NT, KW, D, XR, XM, false, H>(a, ge.w, a.x, ge.d, e, 0, ge.d_nb1, (int64_t) blockIdx.x * (16 * MT / H), (int64_t) blockIdx.y * (16 * NT / H),
                                                blockIdx.x == 0 && blockIdx.z == 0 ? x16 : nullptr);
 }
 template <int MT, int NT, int KW, int XM>
 __global__ void __launch_bounds__(64 * KW) k_gemm_kd(mm_args a) {
+    constexpr int H = 1;
     KS_SLICES
     gemm_kd_tile<MT, NT, KW, XM>(a, wb, xb, a.d + d_off, a.e, d_off, a.d_nb1, m0, n0);
 }
 
-template <int MT, int NT>
+template <int MT, int NT, int H = 1>
 static int ks_grid(const mm_args & a, dim3 & grid) {
-    const int64_t tm = (a.M + 16 * MT - 1) / (16 * MT), tn = (a.N + 16 * NT - 1) / (16 * NT), nb = a.ne12 * a.ne13;
+    const int64_t tm = (a.M + 16 * MT / H - 1) / (16 * MT / H), tn = (a.N + 16 * NT / H - 1) / (16 * NT / H), nb = a.ne12 * a.ne13;
     if (tm > 0x7fffffff || tn > 65535 || nb > 65535) return MI355X_ERR_UNSUPPORTED;
     grid = dim3((unsigned) tm, (unsigned) tn, (unsigned) nb);
     return MI355X_OK;
@@ -334,15 +351,15 @@ static int ks_configure(const void * fn, size_t lds, std::atomic<bool> * configu
     return MI355X_OK;
 }
 
-template <int MT, int NT, int KW, int D, int XR, int XM, bool EMIT>
+template <int MT, int NT, int KW, int D, int XR, int XM, bool EMIT, int H = 1>
 static int launch_ks_t(const mm_args & a, half_t * x16, int64_t slice, hipStream_t st) {
     constexpr size_t ring = (size_t) KW * D * (2 * MT + XR * (XM == KS_X_F16 ? 2 : 4) / 16) * 1024, red = ks_red_bytes<MT, NT, KW>(), lds = ring > red ? ring : red;
     static std::atomic<bool> configured[64];
     static_assert(lds <= 160 * 1024, "LDS of a CU");
     dim3 grid;
-    if (int rc = ks_grid<MT, NT>(a, grid)) return rc;
-    if (int rc = ks_configure((const void *) k_gemm_ks<MT, NT, KW, D, XR, XM, EMIT>, lds, configured)) return rc;
-    k_gemm_ks<MT, NT, KW, D, XR, XM, EMIT><<<grid, 64 * KW, lds, st>>>(a, x16, slice);
+    if (int rc = ks_grid<MT, NT, H>(a, grid)) return rc;
+    if (int rc = ks_configure((const void *) k_gemm_ks<MT, NT, KW, D, XR, XM, EMIT, H>, lds, configured)) return rc;
+    k_gemm_ks<MT, NT, KW, D, XR, XM, EMIT, H><<<grid, 64 * KW, lds, st>>>(a, x16, slice);
     return launch_status();
 }
 template <int MT, int NT, int KW, int XM>
@@ -358,9 +375,12 @@ static int launch_kd_t(const mm_args & a, hipStream_t st) {
 template <int XM, bool EMIT>
 static int launch_ks_x(const mm_args & a, const ks_shape & s, half_t * x16, int64_t slice, hipStream_t st) {
     const bool few = a.N <= 8;
-#define KS_CASE(MT, NT, KW, D) if (s.mt == MT && s.nt == NT && s.kw == KW && s.d == D) { if constexpr (!EMIT || MT % 2 == 0) { \
+#define KS_CASE(MT, NT, KW, D) if (s.h == 1 && s.mt == MT && s.nt == NT && s.kw == KW && s.d == D) { if constexpr (!EMIT || MT % 2 == 0) { \
         if constexpr (NT == 1) if (few) return launch_ks_t<MT, NT, KW, D, 8, XM, EMIT>(a, x16, slice, st); \
         return launch_ks_t<MT, NT, KW, D, 16 * NT, XM, EMIT>(a, x16, slice, st); } }
+#define KS_HALVES(KW, D) if (s.h == 2 && s.kw == KW && s.d == D) { if constexpr (!EMIT) return launch_ks_t<1, 1, KW, D, 16, XM, EMIT, 2>(a, x16, slice, st); }
+    KS_HALVES(4, 2) KS_HALVES(8, 2)
+#undef KS_HALVES
     KS_CASE(1, 1, 1, 1) KS_CASE(1, 1, 4, 2) KS_CASE(1, 1, 8, 2) KS_CASE(2, 1, 4, 2)
     if constexpr (XM != KS_X_F32) { KS_CASE(2, 2, 1, 1) KS_CASE(4, 4, 1, 1) }
     if constexpr (XM == KS_X_F16) { KS_CASE(2, 2, 4, 2) KS_CASE(4, 4, 4, 2) }
@@ -369,8 +389,11 @@ static int launch_ks_x(const mm_args & a, const ks_shape & s, half_t * x16, int6
 }
 
 // Tile and split by size (MI355X, weights from HBM, us per launch; "128-wide" is what the tiled kernels of mul_mat.hip take):
-//   up to 16 columns: 16 x 16 tiles, 4 wavefronts on their K range (1280 x 1280, 5 columns: 4.6; 64 x 64 tiles 10.3), 8 from
-//     K = 2048 (1280 x 5120: 9.6, with 4 11.4, tiled 26.3), 32 rows to a tile from 4096 rows on (51866 x 1280: 26.5; 28.0; 40.4);
+//   up to 16 columns: 16 x 16 tiles, 8 wavefronts on their K range (1280 x 1280, 5 columns: 4.1, with 4 4.5, 64 x 64 tiles 10.3;
+//     1280 x 5120: 9.4; 11.1; 26.3), above 4096 rows 32 rows to a tile and 4 wavefronts (51866 x 1280: 26.3; 16 rows 28.0; 40.4);
+//   up to 8 columns and 2048 rows, where 16-row tiles leave half the CUs idle: 8-row tiles (H = 2), 8 wavefronts from K = 1024 on
+//     (1280 x 5120: 7.8; 1024 x 4096: 6.7, 16-row tiles 7.9; 1280 x 1280: 3.9; 512 x 512: 2.9, 16-row tiles 3.1; at 3072 x 768 they
+//     lose, 6.1 to 4.2);
 //   one round of 64 x 64 tiles, at least half of one (M = 512, K = 2048, N = 1500: 12.9; 128-wide 14.3; M = 1280, K = 1280,
 //     N = 700: 10.2; 11.3), else 32 x 32 (1280 x 5120, 227 columns: 17.8; 34.9; 384 x 384, 487 columns: 3.9; 7.3), and 16 x 16 where
 //     that is under half a round as well (768 x 768, 27 columns: 3.7; 4.4; 6.8);
@@ -379,7 +402,7 @@ static int launch_ks_x(const mm_args & a, const ks_shape & s, half_t * x16, int6
 // K = 64 (attention scores) is one unit: no split, one wavefront to a tile, and what counts is the store of the result.
 static bool ks_tiles(int64_t M, int64_t N, int64_t K, int64_t nb, bool emit, ks_shape & s) {
     const int64_t t44 = (M + 63) / 64 * ((N + 63) / 64) * nb, t22 = (M + 31) / 32 * ((N + 31) / 32) * nb;
-    s.kw = 4; s.d = 2;
+    s.kw = 4; s.d = 2; s.h = 1;
     if (K == KS_UNIT) {
         s.kw = 1; s.d = 1;
         s.mt = s.nt = N <= 16 || t22 < 512 ? 1 : t44 < 512 ? 2 : 4;
@@ -387,7 +410,8 @@ static bool ks_tiles(int64_t M, int64_t N, int64_t K, int64_t nb, bool emit, ks_
     }
     if (N <= 16) {
         s.nt = 1; s.mt = emit || M > 4096 ? 2 : 1;
-        if (s.mt == 1 && K >= 2048) s.kw = 8;
+        if (s.mt == 1 && N <= 8 && M <= 2048 && nb == 1 && K % (2 * KS_UNIT) == 0) { s.h = 2; s.kw = K >= 1024 ? 8 : 4; }
+        else if (s.mt == 1) s.kw = 8;
         return true;
     }
     if (t44 > 256) { s.mt = s.nt = 2; return N <= 32; }
@@ -398,12 +422,14 @@ static bool ks_tiles(int64_t M, int64_t N, int64_t K, int64_t nb, bool emit, ks_
 bool ks_pick(int64_t M, int64_t N, int64_t K, int64_t nb, bool emit, ks_shape & s) {
     return K > 0 && K % KS_UNIT == 0 && ks_tiles(M, N, K, nb, emit, s);
 }
-// A group goes the way of its single products, on tiles chosen for all of them together; the K split, and with it the order
-// of the sums, is the same for every tile size.  A group that fills the device with 128-wide tiles goes there.
+// A group of up to 8 columns is a product with the rows of all of them.  One of more columns goes the way of its single products,
+// on tiles chosen for all of them together; the K split, and with it the order of the sums, is the same for every tile size.  A
+// group that fills the device with 128-wide tiles goes there.
 bool ks_pick_group(int64_t M, int64_t N, int64_t K, int count, ks_shape & s) {
     ks_shape one;
-    if (count > KS_GROUP_MAX || !ks_pick(M, N, K, 1, false, one) || !ks_pick(M, N, K, count, false, s)) return false;
-    return s.kw == one.kw;
+    if (count > KS_GROUP_MAX || !ks_pick(M, N, K, 1, false, one)) return false;
+    if (N <= 8) return ks_pick(M * count, N, K, 1, false, s);
+    return ks_pick(M, N, K, count, false, s) && s.kw == one.kw;
 }
 bool ks_converts(const ks_shape & s) { return s.nt == 1 || s.kw == 1; }
 
@@ -416,25 +442,26 @@ int launch_gemm_ks(const mm_args & a, const ks_shape & s, int xm, half_t * x16, 
     }
 }
 
-template <int MT, int NT, int KW, int D, int XR, int XM>
+template <int MT, int NT, int KW, int D, int XR, int XM, int H>
 static int launch_ks_group_t(const mm_args & a, const ks_group & grp, int count, half_t * x16, hipStream_t st) {
     constexpr size_t ring = (size_t) KW * D * (2 * MT + XR * (XM == KS_X_F16 ? 2 : 4) / 16) * 1024, red = ks_red_bytes<MT, NT, KW>(), lds = ring > red ? ring : red;
     static std::atomic<bool> configured[64];
     dim3 grid;
-    if (int rc = ks_grid<MT, NT>(a, grid)) return rc;
+    if (int rc = ks_grid<MT, NT, H>(a, grid)) return rc;
     grid.z = (unsigned) count;
-    if (int rc = ks_configure((const void *) k_gemm_ks_group<MT, NT, KW, D, XR, XM>, lds, configured)) return rc;
-    k_gemm_ks_group<MT, NT, KW, D, XR, XM><<<grid, 64 * KW, lds, st>>>(a, grp, x16);
+    if (int rc = ks_configure((const void *) k_gemm_ks_group<MT, NT, KW, D, XR, XM, H>, lds, configured)) return rc;
+    k_gemm_ks_group<MT, NT, KW, D, XR, XM, H><<<grid, 64 * KW, lds, st>>>(a, grp, x16);
     return launch_status();
 }
-template <int MT, int NT, int KW, int D, int XR>
+template <int MT, int NT, int KW, int D, int XR, int H = 1>
 static int launch_ks_group_x(const mm_args & a, const ks_group & grp, int count, half_t * x16, hipStream_t st) {
-    if constexpr (NT == 1) if (x16) return launch_ks_group_t<MT, NT, KW, D, XR, KS_X_CVT>(a, grp, count, x16, st);
-    return x16 ? MI355X_ERR_UNSUPPORTED : launch_ks_group_t<MT, NT, KW, D, XR, KS_X_F16>(a, grp, count, x16, st);
+    if constexpr (NT == 1) if (x16) return launch_ks_group_t<MT, NT, KW, D, XR, KS_X_CVT, H>(a, grp, count, x16, st);
+    return x16 ? MI355X_ERR_UNSUPPORTED : launch_ks_group_t<MT, NT, KW, D, XR, KS_X_F16, H>(a, grp, count, x16, st);
 }
 int launch_gemm_ks_group(const mm_args & a, const mm_group & all, int count, const ks_shape & s, half_t * x16, hipStream_t st) {
     ks_group grp;
     for (int i = 0; i < count; ++i) grp.e[i] = all.e[i];
+    if (s.h == 2) return s.kw == 8 ? launch_ks_group_x<1, 1, 8, 2, 16, 2>(a, grp, count, x16, st) : launch_ks_group_x<1, 1, 4, 2, 16, 2>(a, grp, count, x16, st);
 #define KS_CASE(MT, NT, KW, D) if (s.mt == MT && s.nt == NT && s.kw == KW && s.d == D) { \
         if constexpr (NT == 1) if (a.N <= 8) return launch_ks_group_x<MT, NT, KW, D, 8>(a, grp, count, x16, st); \
         return launch_ks_group_x<MT, NT, KW, D, 16 * NT>(a, grp, count, x16, st); }
