@@ -372,6 +372,37 @@ def test_mul_mat_group_f16_few_columns(pkg, oracle, gpu, own_numbers, k, m, n, c
         assert oracle.nmse(got[0][i], x.astype(np.float16).astype(np.float64) @ ws16[i].astype(np.float64).T + bias) <= 1e-12
 
 
+@pytest.mark.parametrize("k,m,n", [(64, 5120, 1500), (192, 5088, 1409), (128, 3840, 1500), (320, 3808, 1345), (64, 2048, 1500), (448, 2016, 1430), (64, 1280, 1500), (576, 1248, 1501),
+                                   (2048, 768, 1500), (1280, 1312, 700)])
+def test_mul_mat_direct_load_tiles(pkg, oracle, gpu, own_numbers, k, m, n):
+    # each tile shape over K shorter and longer than its ring, whole and ragged; GELU with its table fetched under the last steps
+    # and behind the loop, the image beside dst and alone, residual; the two-role kernel; an image that 64 x 64 tiles would have made
+    lib = pkg.kernels()
+    w, x, bias, res = rnd((m, k), 0.5 / np.sqrt(k)), rnd((n, k)), rnd((m,), 0.5), rnd((n, m))
+    w16, x16 = w.astype(np.float16), x.astype(np.float16)
+    base = torch.from_numpy(x16.astype(np.float64)) @ torch.from_numpy(w16.astype(np.float64)).T
+    base = base.numpy() + bias
+    d_w, d_x, d_b, d_r = gpu.up(w16.view(np.int16)), gpu.up(x16.view(np.int16)), gpu.up(bias), gpu.up(res)
+    tw, tx = pkg.tensor(d_w, pkg.F16), pkg.tensor(d_x, pkg.F16)
+
+    def run(flags, image=None):
+        d_y = torch.full((n + 1, m), 7.0, dtype=torch.float32, device=gpu.dev)
+        epi = pkg.Epilogue(pkg.EPI_BIAS | flags, 1.0, d_b.data_ptr(), d_r.data_ptr(), None if image is None else image.data_ptr())
+        pkg.check(lib.mi355x_mul_mat(tw, tx, pkg.tensor(d_y[:n], pkg.F32), C.byref(epi), None, 0, gpu.stream))
+        assert torch.all(d_y[n] == 7.0)
+        return gpu.down(d_y[:n])
+
+    assert oracle.nmse(run(pkg.EPI_RESIDUAL), base + res) <= 1e-11
+    y = run(pkg.EPI_GELU)
+    assert oracle.nmse(y, oracle.gelu(base.astype(np.float32))) <= 1e-7
+    d_h, d_i = (torch.zeros((n, m), dtype=torch.float16, device=gpu.dev) for _ in range(2))
+    y2 = run(pkg.EPI_GELU | pkg.EPI_EMIT_F16, d_h)
+    assert oracle.nmse(y2, y) <= 1e-7
+    image = oracle.dequantize(oracle.Q8_0, oracle.quantize(oracle.Q8_0, y2, act=True), m).reshape(n, m)
+    assert np.array_equal(gpu.down(d_h, np.uint16), oracle.f32_to_f16_bits(image))
+    assert np.all(run(pkg.EPI_GELU | pkg.EPI_EMIT_F16 | pkg.EPI_IMAGE_ONLY, d_i) == 7.0) and np.array_equal(gpu.down(d_i, np.uint16), gpu.down(d_h, np.uint16))
+
+
 # rows that are not 16-byte aligned, any K (the transposed V of a window of 1500, 37 or 1501 positions), one or two columns
 @pytest.mark.parametrize("k,m,n,batch", [(1500, 64, 300, 3), (37, 64, 37, 2), (1501, 64, 5, 2), (1500, 64, 1, 4), (64, 1500, 2, 2), (512, 1000, 1, 1), (1024, 1283, 2, 1), (1280, 5003, 2, 1), (2048, 48, 1, 1), (3, 5, 40, 1)])
 def test_mul_mat_f16_keeps_f32_activations(pkg, oracle, gpu, own_numbers, k, m, n, batch):

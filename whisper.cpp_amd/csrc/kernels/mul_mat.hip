@@ -30,7 +30,7 @@
 #define GELU_LDS_BYTES (2 * GELU_LDS_HALF * 2)
 
 // FULL: the whole tile lies inside dst (no row or column of the patch is clamped or masked)
-template <bool EMIT, bool FULL = false>
+template <bool FULL>
 __device__ __forceinline__ void patch_epilogue(float16_t v, const epi_args & e, char * db, int64_t batch_off, int64_t d_nb1,
                                                int64_t m, int64_t M, const int64_t (&n)[16], int64_t N, const uint16_t * gelu_lds = nullptr) {
     const bool    m_ok = FULL || m < M;
@@ -99,56 +99,22 @@ __device__ __forceinline__ void patch_epilogue(float16_t v, const epi_args & e, 
     if (e.flags & MI355X_EPI_OUT_F16) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) if (m_ok && (FULL || n[i] < N)) *(half_t *)(db + n[i] * d_nb1 + m * 2) = (half_t) v[i];
-    } else if (!EMIT || !(e.flags & MI355X_EPI_IMAGE_ONLY)) {
+    } else {
 #pragma unroll
         for (int i = 0; i < 16; ++i) if (m_ok && (FULL || n[i] < N)) *(float *)(db + n[i] * d_nb1 + m * 4) = v[i];
     }
-    if (EMIT) {
-        // The product that reads dst next rounds its rows to Q8_0 first.  The 32 lanes of a half-wavefront hold 32
-        // consecutive m of one dst row — exactly one Q8_0 block (M % 32 == 0) — so the block maximum is a 5-step
-        // butterfly, and the image f16(q * d) is written here instead of by a pass of its own over dst.
-        // The two divisions of a block (127 / amax and amax / 127) would be repeated by all 32 lanes that hold it, for each
-        // of the 16 registers: 32 IEEE divisions per lane and patch, most of this epilogue's time.  Instead lane l divides
-        // for register l % 16 of its half-wavefront, and the 16 results travel back by lane permutes.
-        // Block maxima: v_permlane16_swap of registers i and i + 8 leaves, in the even rows of 16 lanes, both halves of
-        // register i's block and, in the odd rows, both halves of register i + 8's — one swap and one maximum take the
-        // first butterfly step for two registers and halve what the other four steps (inside a row) have to carry.
-        float rmax[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 8]), false, false);
-            // (the row steps on the bit patterns: non-negative floats order like unsigned integers, and an integer maximum
-            // takes its DPP operand in the same instruction)
-            rmax[i] = __uint_as_float(lanes_reduce<16>(__float_as_uint(fmaxf(fabsf(__uint_as_float(sw[0])), fabsf(__uint_as_float(sw[1])))),
-                                                        [](uint32_t a, uint32_t b) { return a > b ? a : b; }));
-        }
-        const int lane = threadIdx.x & 63;
-        float mine = rmax[0];                               // lane (row, c) of a half-wavefront: register c % 8 + 8 (row % 2)
-#pragma unroll
-        for (int i = 1; i < 8; ++i) mine = (lane & 7) == i ? rmax[i] : mine;
-        const float id_m = mine != 0.0f ? 127.0f / mine : 0.0f;
-        const float dq_m = h2f(f2h_bits(div127(mine)));
-        const int src = ((lane & 32) << 2);                 // byte address of lane 0 of this half-wavefront for ds_bpermute
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int from = src + 4 * ((i & 7) + (i >= 8 ? 16 : 0));
-            const float id = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, id_m)));
-            const float dq = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, dq_m)));
-            if (m_ok && (FULL || n[i] < N)) e.image[n[i] * M + m] = (half_t)((rintf(v[i] * id) + 0.0f) * dq);
-        }
-    }
 }
-
 
 // The same for a patch formed the other way round (the weights as the matrix instruction's A operand): the lane owns ONE dst row
 // n and 16 of the 32 consecutive m of a patch row — m = mb + 8 q + t, q = e / 4, t = e % 4, with mb = the patch's first m +
 // 4 (lane / 32) — and lane + 32 owns the other 16.  That is half a Q8_0 block per lane: the block maximum is 8 three-operand
-// maxima and one exchange with lane + 32 instead of five cross-lane steps for each of 16 registers, both divisions are the
-// lane's own (no permutes hand them round), bias, residual and stores move four consecutive values at a time.
+// maxima and one exchange with lane + 32, both divisions are the lane's own, bias, residual and stores move four consecutive
+// values at a time.  MI355X_EPI_EMIT_F16: the image f16(q * d) of the patch, as the src1 conversion pass of the product that reads
+// dst next would make it, goes to `stage` (LDS; half4 q of this lane at 16 q).
 // M a multiple of 32 (a patch lies inside dst's columns or outside); FULL: the patch is inside and n < N.
 template <bool FULL>
 __device__ __forceinline__ void patch_epilogue_t(float16_t v, const epi_args & e, char * db, int64_t batch_off, int64_t d_nb1,
-                                                 int64_t mb, int64_t M, int64_t n, int64_t N, const uint16_t * gelu_lds) {
+                                                 int64_t mb, int64_t M, int64_t n, int64_t N, const uint16_t * gelu_lds, char * stage) {
     const bool    ok = FULL || (n < N && mb < M);
     const int64_t nc = FULL || n < N ? n : N - 1;
     const int64_t mc = FULL || mb < M ? mb : M - 32 + (mb & 31);
@@ -214,7 +180,7 @@ __device__ __forceinline__ void patch_epilogue_t(float16_t v, const epi_args & e
         for (int q = 0; q < 4; ++q)
             if (ok) *(float4 *)(db + n * d_nb1 + (mb + 8 * q) * 4) = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
     }
-    // the image: rounded to Q8_0 as the product that reads dst next rounds its rows (see patch_epilogue)
+    // the image: rounded to Q8_0 as the product that reads dst next rounds its rows (quantize_row_q8_0, then widened)
     float amax = fmaxf(fabsf(v[0]), fabsf(v[1]));
 #pragma unroll
     for (int i = 2; i < 16; ++i) amax = fmaxf(amax, fabsf(v[i]));
@@ -229,7 +195,7 @@ __device__ __forceinline__ void patch_epilogue_t(float16_t v, const epi_args & e
         // (the addend +0 of the multiply-add turns a product -0 into the +0 that an integer quant of zero gives)
         const half4_t h = { (half_t) __builtin_fmaf(rintf(v[4 * q] * id), dq, 0.0f), (half_t) __builtin_fmaf(rintf(v[4 * q + 1] * id), dq, 0.0f),
                             (half_t) __builtin_fmaf(rintf(v[4 * q + 2] * id), dq, 0.0f), (half_t) __builtin_fmaf(rintf(v[4 * q + 3] * id), dq, 0.0f) };
-        if (ok) *(half4_t *)(e.image + n * M + mb + 8 * q) = h;
+        *(half4_t *)(stage + 16 * q) = h;
     }
 }
 
@@ -366,15 +332,17 @@ __global__ void k_x_to_f16(const char * __restrict__ x, half_t * __restrict__ ou
 
 // What follows the K loop of a tile: GELU reads its table from LDS when the operand buffers, free now (the loop's last barrier
 // is behind every wavefront), are large enough to hold the part that matters (TABLE_FITS); then the 32x32 patches.
-// (NT: threads of the workgroup; the patches belong to the first 256.  TR: the patches were formed with the weights as the
-// matrix instruction's A operand — lanes own dst rows, registers own columns — which the image-emitting epilogue prefers)
-template <int TI, int TJ, bool EMIT, bool TABLE_FITS, int NT = 256, bool TR = false>
+// NT: threads of the workgroup (more than a BN x BM tile has patches for: the patches belong to the first 256).  EMIT: the patches
+// were formed with the weights as the matrix instruction's A operand — lanes own dst rows, registers own columns.  table_there: the
+// GELU slice is in LDS already.
+template <int TI, int TJ, bool EMIT, bool TABLE_FITS, int NT = 256, int BN = 64 * TI, int BM = 64 * TJ>
 __device__ __forceinline__ void gemm_tile_epilogue(float16_t (&acc)[TI][TJ], const mm_args & a, const epi_args & epi, char * db, int64_t batch_off, int64_t d_nb1,
-                                                   int64_t n0, int64_t m0, int wn, int wmo, char * smem) {
+                                                   int64_t n0, int64_t m0, int wn, int wmo, char * smem, bool table_there = false) {
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const uint16_t * gelu_lds = nullptr;
     if constexpr (TABLE_FITS) {
-        if (epi.flags & MI355X_EPI_GELU) {
+        if (table_there) gelu_lds = (const uint16_t *) smem;
+        else if (epi.flags & MI355X_EPI_GELU) {
             const u32x4 * pos = (const u32x4 *) epi.gelu, * neg = (const u32x4 *)(epi.gelu + 0x8000);
             u32x4 * dst = (u32x4 *) smem;
             constexpr int pieces = GELU_LDS_HALF * 2 / 16;
@@ -383,18 +351,30 @@ __device__ __forceinline__ void gemm_tile_epilogue(float16_t (&acc)[TI][TJ], con
             gelu_lds = (const uint16_t *) smem;
         }
     }
-    if (NT > 256 && tid >= 256) return;
-    if constexpr (TR) {
-        static_assert(EMIT, "the transposed patches are the image-emitting kernel's");
+    if (NT > 256 && BN * BM == 64 * TI * 64 * TJ && tid >= 256) return;
+    if constexpr (EMIT) {
         // accumulator register e of a 32x32 patch: column (= n) lane%32, row (= m) 8*(e/4) + 4*g + e%4
+        // The image leaves through LDS: a lane's half4s go to 32 different rows, 8 bytes each, and 32 cache lines to a store made the
+        // epilogue longer than the K loop; out of LDS a store is whole 64- or 128-byte row pieces.
+        constexpr int PITCH = 64 * TJ + 16;             // bytes of a row of the wavefront's 32 TI x 32 TJ values
+        char * stage = smem + (TABLE_FITS ? GELU_LDS_BYTES : 0) + (tid >> 6) * (32 * TI * PITCH);
         auto patches_t = [&](auto full) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < TI; ++i)
 #pragma unroll
                 for (int j = 0; j < TJ; ++j)
-                    patch_epilogue_t<decltype(full)::value>(acc[i][j], epi, db, batch_off, d_nb1, m0 + wmo + 32 * j + 4 * g, a.M, n0 + wn + 32 * i + l32, a.N, gelu_lds);
+                    patch_epilogue_t<decltype(full)::value>(acc[i][j], epi, db, batch_off, d_nb1, m0 + wmo + 32 * j + 4 * g, a.M, n0 + wn + 32 * i + l32, a.N, gelu_lds,
+                                                            stage + (32 * i + l32) * PITCH + 64 * j + 8 * g);
         };
-        if (n0 + 64 * TI <= a.N && m0 + 64 * TJ <= a.M) patches_t(std::true_type{}); else patches_t(std::false_type{});
+        if (n0 + BN <= a.N && m0 + BM <= a.M) patches_t(std::true_type{}); else patches_t(std::false_type{});
+        constexpr int CPR = 4 * TJ, RPI = 64 / CPR;     // 16-byte chunks of a row; rows of a store
+#pragma unroll
+        for (int k = 0; k < 32 * TI / RPI; ++k) {
+            const int r = k * RPI + lane / CPR, c = lane % CPR;
+            const half8_t h = *(const half8_t *)(stage + r * PITCH + c * 16);
+            const int64_t n = n0 + wn + r, m = m0 + wmo + 8 * c;
+            if (n < a.N && m < a.M) *(half8_t *)(epi.image + n * a.M + m) = h;
+        }
         return;
     }
     // accumulator register e of a 32x32 patch: row (= n) 8*(e/4) + 4*g + e%4, column (= m) lane%32
@@ -406,16 +386,15 @@ __device__ __forceinline__ void gemm_tile_epilogue(float16_t (&acc)[TI][TJ], con
             for (int e = 0; e < 16; ++e) n[e] = n0 + wn + 32 * i + 8 * (e >> 2) + 4 * g + (e & 3);
 #pragma unroll
             for (int j = 0; j < TJ; ++j)
-                patch_epilogue<EMIT, decltype(full)::value>(acc[i][j], epi, db, batch_off, d_nb1, m0 + wmo + 32 * j + l32, a.M, n, a.N, gelu_lds);
+                patch_epilogue<decltype(full)::value>(acc[i][j], epi, db, batch_off, d_nb1, m0 + wmo + 32 * j + l32, a.M, n, a.N, gelu_lds);
         }
     };
     // tiles inside dst (all but the last row of tiles when N = 1500) store without per-element bounds
-    if (n0 + 64 * TI <= a.N && m0 + 64 * TJ <= a.M) patches(std::true_type{}); else patches(std::false_type{});
+    if (n0 + BN <= a.N && m0 + BM <= a.M) patches(std::true_type{}); else patches(std::false_type{});
 }
 
-// KTAIL: K is not a multiple of 64 (but of 8); FULL: K / 64 is a multiple of S; EMIT: MI355X_EPI_EMIT_F16 (a kernel of its
-// own, because its epilogue needs more registers than two workgroups per CU leave)
-template <int TI, int TJ, int S, bool KTAIL, bool FULL, bool EMIT = false>
+// The loop with the operands on their way through registers: any K that is a multiple of 8.
+template <int TI, int TJ>
 __device__ __forceinline__ void gemm_f16_tile(const mm_args & a, int tiles_m, int tiles_n, int sw, int tile, const char * wb, const char * xb, char * db,
                                               const epi_args & epi, int64_t batch_off, int64_t d_nb1) {
     constexpr int BN = 64 * TI, BM = 64 * TJ;
@@ -441,22 +420,15 @@ __device__ __forceinline__ void gemm_f16_tile(const mm_args & a, int tiles_m, in
 #pragma unroll
     for (int i = 0; i < WR; ++i) { const int64_t m = m0 + lr + 32 * i; wp[i] = wb + (m < a.M ? m : a.M - 1) * a.w_nb1 + lc * 16; }
 
-    // S steps of operands are in flight in registers (slot = step % S)
-    u32x4 xrs[S][XR], wrs[S][WR];
+    // two steps of operands are in flight in registers (slot = step % 2); pieces beyond K are read from k = 0 and zeroed
+    u32x4 xrs[2][XR], wrs[2][WR];
     auto load = [&](u32x4 (&xr)[XR], u32x4 (&wr)[WR], int64_t k0) __attribute__((always_inline)) {
-        if (KTAIL) {                                   // pieces beyond K are read from k = 0 and zeroed
-            const bool kok = k0 + 8 * lc < a.K;
-            const int64_t ko = kok ? k0 * 2 : -(int64_t) lc * 16;
+        const bool kok = k0 + 8 * lc < a.K;
+        const int64_t ko = kok ? k0 * 2 : -(int64_t) lc * 16;
 #pragma unroll
-            for (int i = 0; i < XR; ++i) { const u32x4 v = *(const u32x4 *)(xp[i] + ko); xr[i] = kok ? v : (u32x4){0, 0, 0, 0}; }
+        for (int i = 0; i < XR; ++i) { const u32x4 v = *(const u32x4 *)(xp[i] + ko); xr[i] = kok ? v : (u32x4){0, 0, 0, 0}; }
 #pragma unroll
-            for (int i = 0; i < WR; ++i) { const u32x4 v = *(const u32x4 *)(wp[i] + ko); wr[i] = kok ? v : (u32x4){0, 0, 0, 0}; }
-        } else {
-#pragma unroll
-            for (int i = 0; i < XR; ++i) xr[i] = *(const u32x4 *)(xp[i] + k0 * 2);
-#pragma unroll
-            for (int i = 0; i < WR; ++i) wr[i] = *(const u32x4 *)(wp[i] + k0 * 2);
-        }
+        for (int i = 0; i < WR; ++i) { const u32x4 v = *(const u32x4 *)(wp[i] + ko); wr[i] = kok ? v : (u32x4){0, 0, 0, 0}; }
     };
     auto store = [&](const u32x4 (&xr)[XR], const u32x4 (&wr)[WR], int buf) __attribute__((always_inline)) {
         half_t * xs = xs_base + buf * BN * GB_LD, * ws = ws_base + buf * BM * GB_LD;
@@ -512,60 +484,25 @@ __device__ __forceinline__ void gemm_f16_tile(const mm_args & a, int tiles_m, in
             }
         }
     };
-    if constexpr (FULL) {
-        // The number of steps is a multiple of S: every step stores and loads unconditionally (beyond the end it re-reads
-        // the last step's operands, which nobody consumes).  With no load behind a branch the compiler knows how many
-        // are outstanding at every point and waits for exactly the oldest slot — with conditional loads it has to assume
-        // the younger ones were never issued, waits for all of them, and the ring degenerates to one step in flight.
-        const int last = KT - 1;
-#pragma unroll
-        for (int st = 0; st < S; ++st) load(xrs[st], wrs[st], (int64_t) st * GB_K);
-        store(xrs[0], wrs[0], 0);
-        load(xrs[0], wrs[0], (int64_t) min(S, last) * GB_K);
-        __syncthreads();
-        auto step = [&](int kt, int buf, u32x4 (&xr)[XR], u32x4 (&wr)[WR]) __attribute__((always_inline)) {   // xr / wr: slot of step kt + 1
-            mma(buf);
+    load(xrs[0], wrs[0], 0);
+    if (1 < KT) load(xrs[1], wrs[1], GB_K);
+    store(xrs[0], wrs[0], 0);
+    if (2 < KT) load(xrs[0], wrs[0], 2 * GB_K);
+    __syncthreads();
+    auto step = [&](int kt, int buf, u32x4 (&xr)[XR], u32x4 (&wr)[WR]) __attribute__((always_inline)) {   // xr / wr: slot of step kt + 1
+        mma(buf);
+        if (kt + 1 < KT) {
             store(xr, wr, buf ^ 1);                     // the last readers of that buffer passed the previous barrier
-            load(xr, wr, (int64_t) min(kt + 1 + S, last) * GB_K);
-            __syncthreads();
-        };
-        for (int kt0 = 0; kt0 < KT; kt0 += S) {         // S is even: the LDS buffer of a step is the parity of its slot
-            step(kt0 + 0, 0, xrs[1 % S], wrs[1 % S]);
-            step(kt0 + 1, 1, xrs[2 % S], wrs[2 % S]);
-            if (S > 2) { step(kt0 + 2, 0, xrs[3 % S], wrs[3 % S]); step(kt0 + 3, 1, xrs[4 % S], wrs[4 % S]); }
-            if (S > 4) { step(kt0 + 4, 0, xrs[5 % S], wrs[5 % S]); step(kt0 + 5, 1, xrs[6 % S], wrs[6 % S]); }
+            if (kt + 3 < KT) load(xr, wr, (int64_t)(kt + 3) * GB_K);
         }
-    } else {
-        load(xrs[0], wrs[0], 0);
-        if (1 < KT) load(xrs[1], wrs[1], GB_K);
-        if (S > 2) { if (2 < KT) load(xrs[2 % S], wrs[2 % S], 2 * GB_K); if (3 < KT) load(xrs[3 % S], wrs[3 % S], 3 * GB_K); }
-        if (S > 4) { if (4 < KT) load(xrs[4 % S], wrs[4 % S], 4 * GB_K); if (5 < KT) load(xrs[5 % S], wrs[5 % S], 5 * GB_K); }
-        store(xrs[0], wrs[0], 0);
-        if (S < KT) load(xrs[0], wrs[0], (int64_t) S * GB_K);
         __syncthreads();
-        auto step = [&](int kt, int buf, u32x4 (&xr)[XR], u32x4 (&wr)[WR]) __attribute__((always_inline)) {
-            mma(buf);
-            if (kt + 1 < KT) {
-                store(xr, wr, buf ^ 1);
-                if (kt + 1 + S < KT) load(xr, wr, (int64_t)(kt + 1 + S) * GB_K);
-            }
-            __syncthreads();
-        };
-        for (int kt0 = 0; kt0 < KT; kt0 += S) {
-            if (kt0 + 0 < KT) step(kt0 + 0, 0, xrs[1 % S], wrs[1 % S]);
-            if (kt0 + 1 < KT) step(kt0 + 1, 1, xrs[2 % S], wrs[2 % S]);
-            if (S > 2) {
-                if (kt0 + 2 < KT) step(kt0 + 2, 0, xrs[3 % S], wrs[3 % S]);
-                if (kt0 + 3 < KT) step(kt0 + 3, 1, xrs[4 % S], wrs[4 % S]);
-            }
-            if (S > 4) {
-                if (kt0 + 4 < KT) step(kt0 + 4, 0, xrs[5 % S], wrs[5 % S]);
-                if (kt0 + 5 < KT) step(kt0 + 5, 1, xrs[6 % S], wrs[6 % S]);
-            }
-        }
+    };
+    for (int kt0 = 0; kt0 < KT; kt0 += 2) {
+        step(kt0 + 0, 0, xrs[1], wrs[1]);
+        if (kt0 + 1 < KT) step(kt0 + 1, 1, xrs[0], wrs[0]);
     }
 
-    gemm_tile_epilogue<TI, TJ, EMIT, ((size_t) 2 * (BN + BM) * GB_LD * sizeof(half_t) >= GELU_LDS_BYTES)>(acc, a, epi, db, batch_off, d_nb1, n0, m0, wn, wmo, smem);
+    gemm_tile_epilogue<TI, TJ, false, ((size_t) 2 * (BN + BM) * GB_LD * sizeof(half_t) >= GELU_LDS_BYTES)>(acc, a, epi, db, batch_off, d_nb1, n0, m0, wn, wmo, smem);
 }
 
 // The same tile by a workgroup of eight wavefronts in two roles: wavefronts 4 .. 7 move the operands (global loads into a
@@ -574,7 +511,7 @@ __device__ __forceinline__ void gemm_f16_tile(const mm_args & a, int tiles_m, in
 // stores, during which it issues no matrix instruction; here the matrix wavefronts do nothing else, and a SIMD holds
 // one of each role per workgroup.  K a multiple of 64 S.
 // NP: threads that move operands (256 or 512), behind the 256 that multiply
-template <int TI, int TJ, int S, bool EMIT, int NP>
+template <int TI, int TJ, int S, int NP>
 __device__ __forceinline__ void gemm_f16_tile_rs(const mm_args & a, int tiles_m, int tiles_n, int sw, int tile, const char * wb, const char * xb, char * db,
                                                  const epi_args & epi, int64_t batch_off, int64_t d_nb1) {
     constexpr int BN = 64 * TI, BM = 64 * TJ;
@@ -684,14 +621,16 @@ __device__ __forceinline__ void gemm_f16_tile_rs(const mm_args & a, int tiles_m,
         }
     }
     // all eight wavefronts are behind the last barrier: the operand buffers are free
-    gemm_tile_epilogue<TI, TJ, EMIT, ((size_t) 2 * (BN + BM) * GB_LD * sizeof(half_t) >= GELU_LDS_BYTES), 256 + NP>(acc, a, epi, db, batch_off, d_nb1, n0, m0, wn, wmo, smem);
+    gemm_tile_epilogue<TI, TJ, false, ((size_t) 2 * (BN + BM) * GB_LD * sizeof(half_t) >= GELU_LDS_BYTES), 256 + NP>(acc, a, epi, db, batch_off, d_nb1, n0, m0, wn, wmo, smem);
 }
 
 // The same tile with the operands going from global memory straight into LDS (global_load_lds_dwordx4: lane l's 16 bytes
-// land at the wave's LDS base + 16 l, no register and no LDS store instruction in between).  Measured on the register-staged
-// loop above, a wavefront spends two thirds of a K step outside its matrix phase — issuing the global loads, whose return
-// path into the registers is busy, and the LDS stores — and here both phases are gone: a step is a wait, a barrier,
-// the issue of the loads NBUF - 1 steps ahead and the matrix phase.
+// land at the wave's LDS base + 16 l, no register and no LDS store instruction in between): a step is a wait, a barrier, the
+// issue of the loads NBUF - 1 steps ahead and the matrix phase of WN x WM wavefronts, 32 TI x 32 TJ results each.
+// What bounds it: a CU takes about 55 KB/us in from L2 (25 B per clock: 14 TB/s over the device), however deep the ring and however many
+// workgroups share the CU, which is less than its matrix instructions could use at these tile sizes.  So the tile is as large
+// as leaves one to a CU, and the ring as deep as LDS allows.  The barrier is a bare s_barrier behind a counted wait: __syncthreads()
+// waits for every load into LDS first, and the ring degenerates to one step in flight (128 x 64 tiles, K = 5120: 67 us, now 39).
 // LDS tile of an operand: row pairs form 256-byte lines, the 16-byte chunk c of row r sits in slot (r & 1) * 8 +
 // (c ^ ((r >> 1) & 7)) of line r >> 1 — the 16 lanes of a b128 fragment read (16 consecutive rows, one chunk) then cover 256
 // consecutive bytes' worth of banks, and a wave's load (1 KB: 8 rows) writes whole lines from whole 128-byte row pieces.
@@ -704,11 +643,17 @@ __device__ __forceinline__ void wait_vmcnt() {                // s_waitcnt vmcnt
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
-template <int TI, int TJ, int NBUF, bool EMIT>
+template <int N>
+__device__ __forceinline__ void wait_vmcnt_lds() {            // s_waitcnt vmcnt(N) lgkmcnt(0)
+    static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4));
+}
+
+template <int WN, int WM, int TI, int TJ, int NBUF, bool EMIT>
 __device__ __forceinline__ void gemm_f16_tile_dl(const mm_args & a, int tiles_m, int tiles_n, int sw, int tile, const char * wb, const char * xb, char * db,
                                                  const epi_args & epi, int64_t batch_off, int64_t d_nb1) {
-    constexpr int BN = 64 * TI, BM = 64 * TJ;
-    constexpr int XL = BN / 32, WL = BM / 32;          // 1 KB loads per wavefront and step (8 rows each)
+    constexpr int NW = WN * WM, BN = 32 * TI * WN, BM = 32 * TJ * WM;
+    constexpr int XL = BN / (8 * NW), WL = BM / (8 * NW); static_assert(BN % (8 * NW) == 0 && BM % (8 * NW) == 0, "");          // 1 KB loads per wavefront and step (8 rows each)
     constexpr int STEP_BYTES = (BN + BM) * DL_STEP_ROW;
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
@@ -718,26 +663,40 @@ __device__ __forceinline__ void gemm_f16_tile_dl(const mm_args & a, int tiles_m,
     const int64_t n0 = (int64_t)(rem / cw) * BN;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // load i of this wavefront covers rows 32 i + 8 wave .. + 7 of the tile; this lane: row lrow of the 8, chunk lchunk
+    // load i of this wavefront covers rows 8 (NW i + wave) .. + 7 of the tile; this lane: row lrow of the 8, chunk lchunk
     const int lrow = 2 * (lane >> 4) + ((lane & 15) >> 3);
     const int lchunk = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
     const char * xp[XL]; const char * wp[WL];
 #pragma unroll
-    for (int i = 0; i < XL; ++i) { const int64_t n = n0 + 32 * i + 8 * wave + lrow; xp[i] = xb + (n < a.N ? n : a.N - 1) * a.x_nb1 + lchunk * 16; }
+    for (int i = 0; i < XL; ++i) { const int64_t n = n0 + 8 * (NW * i + wave) + lrow; xp[i] = xb + (n < a.N ? n : a.N - 1) * a.x_nb1 + lchunk * 16; }
 #pragma unroll
-    for (int i = 0; i < WL; ++i) { const int64_t m = m0 + 32 * i + 8 * wave + lrow; wp[i] = wb + (m < a.M ? m : a.M - 1) * a.w_nb1 + lchunk * 16; }
+    for (int i = 0; i < WL; ++i) { const int64_t m = m0 + 8 * (NW * i + wave) + lrow; wp[i] = wb + (m < a.M ? m : a.M - 1) * a.w_nb1 + lchunk * 16; }
     auto load = [&](int step, int buf) __attribute__((always_inline)) {
         const int64_t ko = (int64_t) step * DL_STEP_ROW;
         char * xs = smem + buf * STEP_BYTES + wave * 1024, * ws = xs + BN * DL_STEP_ROW;
 #pragma unroll
         for (int i = 0; i < XL; ++i)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(xp[i] + ko), (__attribute__((address_space(3))) void *)(xs + i * 4096), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(xp[i] + ko), (__attribute__((address_space(3))) void *)(xs + i * (NW * 1024)), 16, 0, 0);
 #pragma unroll
         for (int i = 0; i < WL; ++i)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(wp[i] + ko), (__attribute__((address_space(3))) void *)(ws + i * 4096), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(wp[i] + ko), (__attribute__((address_space(3))) void *)(ws + i * (NW * 1024)), 16, 0, 0);
+    };
+    // The last NBUF - 1 steps have no later step to fetch: their loads bring the part of the GELU table that the epilogue wants,
+    // or, without a GELU, one line again and again, so that the number of loads in flight stays what the waits count on.
+    // Step KT - 1 lies in the last buffer, so the table grows from the first one on.
+    const bool gelu = epi.flags & MI355X_EPI_GELU;
+    auto load_table = [&](int s) __attribute__((always_inline)) {                // s-th of these steps
+        constexpr int HALF = GELU_LDS_BYTES / 2048;      // 1 KB pieces of a half
+        char * to = smem + s * STEP_BYTES + wave * 1024;
+#pragma unroll
+        for (int i = 0; i < XL + WL; ++i) {
+            const int p = (s * (XL + WL) + i) * NW + wave;
+            const char * t = (const char *) epi.gelu + (p < HALF ? p * 1024 : 0x8000 * 2 + (min(p, 2 * HALF - 1) - HALF) * 1024) + lane * 16;
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(gelu ? t : wb), (__attribute__((address_space(3))) void *)(to + i * (NW * 1024)), 16, 0, 0);
+        }
     };
 
-    const int wn = (wave >> 1) * 32 * TI, wmo = (wave & 1) * 32 * TJ;   // wave patch origin inside the tile
+    const int wn = (wave / WM) * 32 * TI, wmo = (wave % WM) * 32 * TJ;   // wave patch origin inside the tile
     const int l32 = lane & 31, g = lane >> 5;
     // fragment reads: row wn + 32 i + l32 (its line and half of the line), chunk 2 kk + g swizzled by the row
     const int rsw = (l32 >> 1) & 7;
@@ -759,7 +718,7 @@ __device__ __forceinline__ void gemm_f16_tile_dl(const mm_args & a, int tiles_m,
     // behind each of the first matrix instructions — a load can sit in the issue stage while the CU's vector-memory path is
     // backed up, and everything behind it waits with it: spread out, a matrix instruction is already running each time
     // (1480 clocks per step instead of 1730 with the eight loads in front); then the rest of the 4 TI TJ matrix instructions.
-    auto mma = [&](int buf, int load_step, int load_buf) __attribute__((always_inline)) {
+    auto mma = [&](int buf, auto && fetch) __attribute__((always_inline)) {
         const char * xs = smem + buf * STEP_BYTES + xrow, * ws = smem + buf * STEP_BYTES + wrow;
         half8_t av[GB_K / 16][TI], bv[GB_K / 16][TJ];
 #pragma unroll
@@ -769,7 +728,7 @@ __device__ __forceinline__ void gemm_f16_tile_dl(const mm_args & a, int tiles_m,
 #pragma unroll
             for (int j = 0; j < TJ; ++j) bv[kk][j] = *(const half8_t *)(ws + j * 4096 + koff[kk]);
         }
-        load(load_step, load_buf);
+        fetch();
 #pragma unroll
         for (int kk = 0; kk < GB_K / 16; ++kk)
 #pragma unroll
@@ -791,20 +750,32 @@ __device__ __forceinline__ void gemm_f16_tile_dl(const mm_args & a, int tiles_m,
     };
 
     const int KT = (int)(a.K / GB_K), last = KT - 1;
-    // Every step issues its XL + WL loads unconditionally (beyond the end it re-reads the last step into a buffer nobody reads
-    // again), so "all but the (NBUF - 2) (XL + WL) youngest have landed" is a constant wait.
+    // Every step issues XL + WL loads, so "all but the (NBUF - 2) (XL + WL) youngest have landed" is a constant wait.
+    int buf = (int)((uint32_t)(NBUF * KT - KT) % NBUF);         // of step 0: step KT - 1 lies in buffer NBUF - 1
+    int fill = buf;
 #pragma unroll
-    for (int st = 0; st < NBUF - 1; ++st) load(min(st, last), st);
-    int buf = 0, fill = NBUF - 1;                      // buffer of step kt; buffer that step kt + NBUF - 1 goes into
-    for (int kt = 0; kt < KT; ++kt) {
-        wait_vmcnt<(NBUF - 2) * (XL + WL)>();             // this wavefront's pieces of step kt are in LDS
-        __syncthreads();                                // ... everybody's are, and everybody is done reading step kt - 1
-        mma(buf, min(kt + NBUF - 1, last), fill);       // ... whose buffer the loads of step kt + NBUF - 1 go into
+    for (int st = 0; st < NBUF - 1; ++st) { load(min(st, last), fill); fill = fill + 1 == NBUF ? 0 : fill + 1; }
+    auto step_begins = [&]() __attribute__((always_inline)) {
+        wait_vmcnt_lds<(NBUF - 2) * (XL + WL)>();         // this wavefront's pieces of the step are in LDS, its reads of the step before are done
+        __builtin_amdgcn_s_barrier();                   // ... and everybody's.  (Not __syncthreads(), which waits for every load into LDS.)
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const int kt_tail = max(KT - (NBUF - 1), 0);
+    int kt = 0;
+    for (; kt < kt_tail; ++kt) {
+        step_begins();
+        mma(buf, [&]() __attribute__((always_inline)) { load(kt + NBUF - 1, fill); });
         buf = buf + 1 == NBUF ? 0 : buf + 1; fill = fill + 1 == NBUF ? 0 : fill + 1;
     }
-    wait_vmcnt<0>();                                    // the surplus loads still write LDS, which the epilogue reuses
+    const bool table = gelu && KT >= NBUF - 1;          // (a K shorter than the ring: the epilogue fetches the table)
+    for (; kt < KT; ++kt) {
+        step_begins();
+        mma(buf, [&]() __attribute__((always_inline)) { load_table(kt - KT + NBUF - 1); });
+        buf = buf + 1 == NBUF ? 0 : buf + 1;
+    }
+    wait_vmcnt<0>();
     __syncthreads();
-    gemm_tile_epilogue<TI, TJ, EMIT, true, 256, EMIT>(acc, a, epi, db, batch_off, d_nb1, n0, m0, wn, wmo, smem);
+    gemm_tile_epilogue<TI, TJ, EMIT, true, 64 * NW, BN, BM>(acc, a, epi, db, batch_off, d_nb1, n0, m0, wn, wmo, smem, table);
 }
 
 // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2: workgroup `lin` of `total` runs on XCD lin % 8.
@@ -827,180 +798,139 @@ static int tile_path_width(int64_t tiles_m, int64_t tiles_n, int64_t run, int bn
     return best;
 }
 
-template <int TI, int TJ, int S, bool KTAIL, bool FULL, bool EMIT>
+template <int TI, int TJ>
 __global__ void __launch_bounds__(256, 2) k_gemm_f16(mm_args a, int tiles_m, int tiles_n, int sw) {
     const mm_slice_ptrs z = mm_slice(a, blockIdx.y);
-    gemm_f16_tile<TI, TJ, S, KTAIL, FULL, EMIT>(a, tiles_m, tiles_n, sw, xcd_run_index(blockIdx.x, tiles_m * tiles_n), z.w, z.x, a.d + z.d_off, a.e, z.d_off, a.d_nb1);
+    gemm_f16_tile<TI, TJ>(a, tiles_m, tiles_n, sw, xcd_run_index(blockIdx.x, tiles_m * tiles_n), z.w, z.x, a.d + z.d_off, a.e, z.d_off, a.d_nb1);
 }
 
+// LDS of the epilogue: the GELU table slice and, with an image, the rows on their way out
+template <int NW, int TI, int TJ, bool EMIT> constexpr size_t dl_epilogue_bytes() { return GELU_LDS_BYTES + (EMIT ? (size_t) NW * 32 * TI * (64 * TJ + 16) : 0); }
+
+template <int WN, int WM, int TI, int TJ, int NBUF, bool EMIT>
+__global__ void __launch_bounds__(64 * WN * WM) k_gemm_f16_dl(mm_args a, int tiles_m, int tiles_n, int sw) {
+    const mm_slice_ptrs z = mm_slice(a, blockIdx.y);
+    gemm_f16_tile_dl<WN, WM, TI, TJ, NBUF, EMIT>(a, tiles_m, tiles_n, sw, xcd_run_index(blockIdx.x, tiles_m * tiles_n), z.w, z.x, a.d + z.d_off, a.e, z.d_off, a.d_nb1);
+}
 // Several products over the same src1 in one launch (the Q, K and V projections of a layer; the cross-attention K and V
-// of all decoder layers): blockIdx.y picks the weights, the destination and the epilogue.  One launch of 3 x 120 or
-// 64 x 120 tiles fills 256 CUs where 120 tiles at a time leave half of them idle.
-template <int TI, int TJ, int S>
-__global__ void __launch_bounds__(256, 2) k_gemm_f16_group(mm_args a, int tiles_m, int tiles_n, int sw, mm_group grp) {
-    // the products' tiles form one pool, product after product, and an XCD's run may cross from one product into the next
+// of all decoder layers): one launch of 3 x 80 or 64 x 60 tiles fills 256 CUs where 80 tiles at a time leave most of them idle.
+// The products' tiles form one pool, product after product, and an XCD's run may cross from one product into the next.
+template <int WN, int WM, int TI, int TJ, int NBUF>
+__global__ void __launch_bounds__(64 * WN * WM) k_gemm_f16_dl_group(mm_args a, int tiles_m, int tiles_n, int sw, int count, mm_group grp) {
     const int nblk = tiles_m * tiles_n;
-    const int item = xcd_run_index((int)(blockIdx.x + gridDim.x * blockIdx.y), nblk * (int) gridDim.y);
+    const int item = xcd_run_index((int) blockIdx.x, nblk * count);
     const mm_group_entry & ge = grp.e[item / nblk];
     epi_args e;
     e.flags = ge.flags; e.scale = ge.scale; e.bias = ge.bias; e.residual = ge.residual; e.gelu = a.e.gelu; e.image = nullptr;
-    gemm_f16_tile<TI, TJ, S, false, true>(a, tiles_m, tiles_n, sw, item % nblk, ge.w, a.x, ge.d, e, 0, ge.d_nb1);
+    gemm_f16_tile_dl<WN, WM, TI, TJ, NBUF, false>(a, tiles_m, tiles_n, sw, item % nblk, ge.w, a.x, ge.d, e, 0, ge.d_nb1);
 }
 
-// the direct-to-LDS form of the two kernels above (K a multiple of 64)
-template <int TI, int TJ, int NBUF, bool EMIT>
-__global__ void __launch_bounds__(256, 2) k_gemm_f16_dl(mm_args a, int tiles_m, int tiles_n, int sw) {
-    const mm_slice_ptrs z = mm_slice(a, blockIdx.y);
-    gemm_f16_tile_dl<TI, TJ, NBUF, EMIT>(a, tiles_m, tiles_n, sw, xcd_run_index(blockIdx.x, tiles_m * tiles_n), z.w, z.x, a.d + z.d_off, a.e, z.d_off, a.d_nb1);
-}
-template <int TI, int TJ, int NBUF>
-__global__ void __launch_bounds__(256, 2) k_gemm_f16_dl_group(mm_args a, int tiles_m, int tiles_n, int sw, mm_group grp) {
-    const int nblk = tiles_m * tiles_n;
-    const int item = xcd_run_index((int)(blockIdx.x + gridDim.x * blockIdx.y), nblk * (int) gridDim.y);
-    const mm_group_entry & ge = grp.e[item / nblk];
-    epi_args e;
-    e.flags = ge.flags; e.scale = ge.scale; e.bias = ge.bias; e.residual = ge.residual; e.gelu = a.e.gelu; e.image = nullptr;
-    gemm_f16_tile_dl<TI, TJ, NBUF, false>(a, tiles_m, tiles_n, sw, item % nblk, ge.w, a.x, ge.d, e, 0, ge.d_nb1);
-}
-// LDS buffers of K steps in flight by tile shape: 128 x 128 tiles keep two workgroups per CU (2 x 32 KB each)
-template <int TI, int TJ> constexpr int dl_buffers() { return TI * TJ == 4 ? 2 : 3; }
-template <int TI, int TJ> constexpr size_t dl_lds_bytes() {
-    constexpr size_t ring = (size_t) dl_buffers<TI, TJ>() * 64 * (TI + TJ) * DL_STEP_ROW;
-    return ring > GELU_LDS_BYTES ? ring : GELU_LDS_BYTES;        // the epilogue keeps the GELU table slice there
-}
-
-template <int TI, int TJ, bool EMIT>
-static int launch_gemm_f16_dl(const mm_args & a, hipStream_t st) {
-    constexpr int BN = 64 * TI, BM = 64 * TJ, NBUF = dl_buffers<TI, TJ>();
-    constexpr size_t lds = dl_lds_bytes<TI, TJ>();
-    static std::atomic<bool> configured[64];
+// more than the default 64 KB of LDS have to be asked for, once per kernel and device
+static int configure_lds(const void * fn, size_t lds, std::atomic<bool> * configured) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return MI355X_ERR_HIP;
-    if (!configured[dev].load(std::memory_order_acquire)) {
-        if (hipFuncSetAttribute((const void *) k_gemm_f16_dl<TI, TJ, NBUF, EMIT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds) != hipSuccess) return MI355X_ERR_HIP;
-        configured[dev].store(true, std::memory_order_release);
-    }
-    const int64_t tm = (a.M + BM - 1) / BM, tn = (a.N + BN - 1) / BN;
-    if (tm * tn > 0x7fffffff) return MI355X_ERR_UNSUPPORTED;
-    dim3 grid((unsigned)(tm * tn), (unsigned)(a.ne12 * a.ne13));
-    const int sw = tile_path_width(tm, tn, (tm * tn + 7) / 8, BN, BM);
-    k_gemm_f16_dl<TI, TJ, NBUF, EMIT><<<grid, 256, lds, st>>>(a, (int) tm, (int) tn, sw);
-    return launch_status();
+    if (configured[dev].load(std::memory_order_acquire)) return MI355X_OK;
+    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds) != hipSuccess) return MI355X_ERR_HIP;
+    configured[dev].store(true, std::memory_order_release);
+    return MI355X_OK;
+}
+struct tile_plan { int64_t tm, tn; int sw; dim3 grid; };
+static int plan_tiles(const mm_args & a, int bn, int bm, int count, tile_plan & p) {
+    p.tm = (a.M + bm - 1) / bm; p.tn = (a.N + bn - 1) / bn;
+    if (p.tm * p.tn * count > 0x7fffffff || a.ne12 * a.ne13 > 65535) return MI355X_ERR_UNSUPPORTED;
+    p.grid = dim3((unsigned)(p.tm * p.tn * count), (unsigned)(a.ne12 * a.ne13));
+    p.sw = tile_path_width(p.tm, p.tn, (p.tm * p.tn * count + 7) / 8, bn, bm);
+    return MI355X_OK;
 }
 
-// the two-role form (K a multiple of 64 S)
-template <int TI, int TJ, int S, bool EMIT, int NP>
-__global__ void __launch_bounds__(256 + NP) k_gemm_f16_rs(mm_args a, int tiles_m, int tiles_n, int sw) {
-    const mm_slice_ptrs z = mm_slice(a, blockIdx.y);
-    gemm_f16_tile_rs<TI, TJ, S, EMIT, NP>(a, tiles_m, tiles_n, sw, xcd_run_index(blockIdx.x, tiles_m * tiles_n), z.w, z.x, a.d + z.d_off, a.e, z.d_off, a.d_nb1);
+// grp: the products of a group (count of them), NULL for one product
+template <int WN, int WM, int TI, int TJ, int NBUF, bool EMIT>
+static int launch_dl(const mm_args & a, const mm_group * grp, int count, hipStream_t st) {
+    constexpr int BN = 32 * TI * WN, BM = 32 * TJ * WM;
+    constexpr size_t lds = std::max((size_t) NBUF * (BN + BM) * DL_STEP_ROW, dl_epilogue_bytes<WN * WM, TI, TJ, EMIT>());
+    static_assert(lds <= 160 * 1024, "LDS of a CU");
+    static std::atomic<bool> configured[64], group_configured[64];
+    tile_plan p;
+    if (int rc = plan_tiles(a, BN, BM, grp ? count : 1, p)) return rc;
+    if constexpr (!EMIT) {
+        if (grp) {
+            if (int rc = configure_lds((const void *) k_gemm_f16_dl_group<WN, WM, TI, TJ, NBUF>, lds, group_configured)) return rc;
+            k_gemm_f16_dl_group<WN, WM, TI, TJ, NBUF><<<p.grid, 64 * WN * WM, lds, st>>>(a, (int) p.tm, (int) p.tn, p.sw, count, *grp);
+            return launch_status();
+        }
+    }
+    if (int rc = configure_lds((const void *) k_gemm_f16_dl<WN, WM, TI, TJ, NBUF, EMIT>, lds, configured)) return rc;
+    k_gemm_f16_dl<WN, WM, TI, TJ, NBUF, EMIT><<<p.grid, 64 * WN * WM, lds, st>>>(a, (int) p.tm, (int) p.tn, p.sw);
+    return launch_status();
 }
-template <int TI, int TJ> constexpr int rs_ring() { return 4; }
+// The tile (n x m) by size: rounds of 256 tiles, one to a CU, times the rows of X and of W that a step of one fetches — 128 x 256 where
+// they are one round (M = 5120, N = 1500: 33 us at K = 1280; 192 x 128 46, 128 x 128 39), 192 x 128 (M = 3840: 26; 28; 37 and M = 4096,
+// 3072), 128 x 128 (M = 2048, K = 512: 10.7; 12.6 with 192 x 128, 13.5 with 128 x 64), 128 x 64 (M = 1280: 12.5; 16; 20).
+enum { DL_128x256, DL_192x128, DL_128x128, DL_128x64 };
+static int dl_pick(const mm_args & a, int count) {
+    static const int bn[4] = { 128, 192, 128, 128 }, bm[4] = { 256, 128, 128, 64 };
+    int best = DL_128x256; int64_t best_cost = INT64_MAX;
+    for (int i = 0; i < 4; ++i) {
+        const int64_t tiles = (a.N + bn[i] - 1) / bn[i] * ((a.M + bm[i] - 1) / bm[i]) * a.ne12 * a.ne13 * count, cost = (tiles + 255) / 256 * (bn[i] + bm[i]);
+        if (cost < best_cost) { best_cost = cost; best = i; }
+    }
+    return best;
+}
+template <bool EMIT>
+static int launch_gemm_f16_dl(const mm_args & a, const mm_group * grp, int count, hipStream_t st) {
+    switch (dl_pick(a, count)) {
+        case DL_128x256: return launch_dl<2, 4, 2, 2, 3, EMIT>(a, grp, count, st);
+        case DL_192x128: return launch_dl<2, 4, 3, 1, 3, EMIT>(a, grp, count, st);
+        case DL_128x128: return launch_dl<4, 2, 1, 2, 4, EMIT>(a, grp, count, st);
+        default:         return launch_dl<4, 2, 1, 1, 6, EMIT>(a, grp, count, st);
+    }
+}
+
+// the two-role form (K a multiple of 256)
 #define RS_NP 512       // operand threads: 512 (three 16-byte pieces each per step of a 128 x 64 tile) beat 256 by 7 %
-
-template <int TI, int TJ, bool EMIT>
+__global__ void __launch_bounds__(256 + RS_NP) k_gemm_f16_rs(mm_args a, int tiles_m, int tiles_n, int sw) {
+    const mm_slice_ptrs z = mm_slice(a, blockIdx.y);
+    gemm_f16_tile_rs<2, 1, 4, RS_NP>(a, tiles_m, tiles_n, sw, xcd_run_index(blockIdx.x, tiles_m * tiles_n), z.w, z.x, a.d + z.d_off, a.e, z.d_off, a.d_nb1);
+}
 static int launch_gemm_f16_rs(const mm_args & a, hipStream_t st) {
-    constexpr int BN = 64 * TI, BM = 64 * TJ, S = rs_ring<TI, TJ>();
-    constexpr size_t lds = (size_t) 2 * (BN + BM) * GB_LD * sizeof(half_t);
-    static std::atomic<bool> configured[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return MI355X_ERR_HIP;
-    if (!configured[dev].load(std::memory_order_acquire)) {
-        if (hipFuncSetAttribute((const void *) k_gemm_f16_rs<TI, TJ, S, EMIT, RS_NP>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds) != hipSuccess) return MI355X_ERR_HIP;
-        configured[dev].store(true, std::memory_order_release);
-    }
-    const int64_t tm = (a.M + BM - 1) / BM, tn = (a.N + BN - 1) / BN;
-    if (tm * tn > 0x7fffffff) return MI355X_ERR_UNSUPPORTED;
-    dim3 grid((unsigned)(tm * tn), (unsigned)(a.ne12 * a.ne13));
-    const int sw = tile_path_width(tm, tn, (tm * tn + 7) / 8, BN, BM);
-    k_gemm_f16_rs<TI, TJ, S, EMIT, RS_NP><<<grid, 256 + RS_NP, lds, st>>>(a, (int) tm, (int) tn, sw);
+    constexpr size_t lds = (size_t) 2 * (128 + 64) * GB_LD * sizeof(half_t);
+    tile_plan p;
+    if (int rc = plan_tiles(a, 128, 64, 1, p)) return rc;
+    k_gemm_f16_rs<<<p.grid, 256 + RS_NP, lds, st>>>(a, (int) p.tm, (int) p.tn, p.sw);
     return launch_status();
 }
 
-template <int TI, int TJ, int S, bool KTAIL, bool FULL, bool EMIT = false>
-static int launch_gemm_f16_k(const mm_args & a, hipStream_t st) {
-    static_assert(S % 2 == 0, "the LDS buffer index is the parity of the register slot");
-    constexpr int BN = 64 * TI, BM = 64 * TJ;
-    constexpr size_t lds = (size_t) 2 * (BN + BM) * GB_LD * sizeof(half_t);
-    static std::atomic<bool> configured[64];                         // per device: kernels may use more than the default 64 KB of LDS
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return MI355X_ERR_HIP;
-    if (!configured[dev].load(std::memory_order_acquire)) {
-        if (hipFuncSetAttribute((const void *) k_gemm_f16<TI, TJ, S, KTAIL, FULL, EMIT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds) != hipSuccess) return MI355X_ERR_HIP;
-        configured[dev].store(true, std::memory_order_release);
-    }
-    const int64_t tm = (a.M + BM - 1) / BM, tn = (a.N + BN - 1) / BN;
-    if (tm * tn > 0x7fffffff) return MI355X_ERR_UNSUPPORTED;
-    dim3 grid((unsigned)(tm * tn), (unsigned)(a.ne12 * a.ne13));
-    const int sw = tile_path_width(tm, tn, (tm * tn + 7) / 8, BN, BM);
-    k_gemm_f16<TI, TJ, S, KTAIL, FULL, EMIT><<<grid, 256, lds, st>>>(a, (int) tm, (int) tn, sw);
-    return launch_status();
-}
 template <int TI, int TJ>
 static int launch_gemm_f16(const mm_args & a, hipStream_t st) {
-    static const bool staged = getenv("MI355X_GEMM_STAGED") != nullptr;        // the register-staged loop, for comparison
-    // 128 x 64 tiles (one workgroup to a CU when M = 1280): two roles, 13.0 vs 14.9 us at K = 1280, 33.5 vs 39.9 us at K = 5120
-    if constexpr (TI * TJ == 2) {
-        if (!staged && a.K % (GB_K * rs_ring<TI, TJ>()) == 0)
-            return (a.e.flags & MI355X_EPI_EMIT_F16) ? launch_gemm_f16_rs<TI, TJ, true>(a, st) : launch_gemm_f16_rs<TI, TJ, false>(a, st);
-    }
-    // 128 x 128 tiles only: the direct loads move about half the bytes per clock of the register path, which pays where two
-    // workgroups share a CU (10 - 13 % faster) and loses on the 128 x 64 tiles that run one to a CU
-    if constexpr (TI * TJ == 4) {
-        if (a.K % GB_K == 0 && !staged) return (a.e.flags & MI355X_EPI_EMIT_F16) ? launch_gemm_f16_dl<TI, TJ, true>(a, st) : launch_gemm_f16_dl<TI, TJ, false>(a, st);
-    }
-    if (a.e.flags & MI355X_EPI_EMIT_F16) {
-        if (a.K % (2 * GB_K)) return MI355X_ERR_UNSUPPORTED;
-        return a.K % (4 * GB_K) == 0 ? launch_gemm_f16_k<TI, TJ, 4, false, true, true>(a, st) : launch_gemm_f16_k<TI, TJ, 2, false, true, true>(a, st);
-    }
-    if (a.K % GB_K) return launch_gemm_f16_k<TI, TJ, 2, true, false>(a, st);
-    const int64_t kt = a.K / GB_K;
-    if (kt % 4 == 0) return launch_gemm_f16_k<TI, TJ, 4, false, true>(a, st);
-    if (kt % 2 == 0) return launch_gemm_f16_k<TI, TJ, 2, false, true>(a, st);
-    return launch_gemm_f16_k<TI, TJ, 4, false, false>(a, st);
-}
-
-template <int TI, int TJ>
-static int launch_gemm_f16_group(const mm_args & a, const mm_group & grp, int count, hipStream_t st) {
     constexpr int BN = 64 * TI, BM = 64 * TJ;
     constexpr size_t lds = (size_t) 2 * (BN + BM) * GB_LD * sizeof(half_t);
     static std::atomic<bool> configured[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return MI355X_ERR_HIP;
-    if (!configured[dev].load(std::memory_order_acquire)) {
-        if (hipFuncSetAttribute((const void *) k_gemm_f16_group<TI, TJ, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds) != hipSuccess) return MI355X_ERR_HIP;
-        configured[dev].store(true, std::memory_order_release);
-    }
-    const int64_t tm = (a.M + BM - 1) / BM, tn = (a.N + BN - 1) / BN;
-    if (tm * tn > 0x7fffffff) return MI355X_ERR_UNSUPPORTED;
-    dim3 grid((unsigned)(tm * tn), (unsigned) count);
-    const int sw = tile_path_width(tm, tn, (tm * tn * count + 7) / 8, BN, BM);
-    static const bool staged = getenv("MI355X_GEMM_STAGED") != nullptr;
-    if constexpr (TI * TJ == 4) {
-    if (!staged) {
-        static std::atomic<bool> dl_configured[64];
-        constexpr size_t dl_lds = dl_lds_bytes<TI, TJ>();
-        if (!dl_configured[dev].load(std::memory_order_acquire)) {
-            if (hipFuncSetAttribute((const void *) k_gemm_f16_dl_group<TI, TJ, dl_buffers<TI, TJ>()>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) dl_lds) != hipSuccess) return MI355X_ERR_HIP;
-            dl_configured[dev].store(true, std::memory_order_release);
-        }
-        k_gemm_f16_dl_group<TI, TJ, dl_buffers<TI, TJ>()><<<grid, 256, dl_lds, st>>>(a, (int) tm, (int) tn, sw, grp);
-        return launch_status();
-    }
-    }
-    k_gemm_f16_group<TI, TJ, 4><<<grid, 256, lds, st>>>(a, (int) tm, (int) tn, sw, grp);
+    tile_plan p;
+    if (int rc = plan_tiles(a, BN, BM, 1, p)) return rc;
+    if (int rc = configure_lds((const void *) k_gemm_f16<TI, TJ>, lds, configured)) return rc;
+    k_gemm_f16<TI, TJ><<<p.grid, 256, lds, st>>>(a, (int) p.tm, (int) p.tn, p.sw);
     return launch_status();
 }
 
-// tile shape: small problems go to k_gemm_ks; else the largest whose grid still covers the 256 CUs about twice
+// Small problems go to k_gemm_ks; else K decides: a multiple of 64 goes over the direct loads.
 static int launch_gemm_f16_auto(const mm_args & a, hipStream_t st) {
     const int64_t nb = a.ne12 * a.ne13;
+    const bool emit = a.e.flags & MI355X_EPI_EMIT_F16;
     ks_shape ks;
-    if (ks_pick(a.M, a.N, a.K, nb, (a.e.flags & MI355X_EPI_EMIT_F16) != 0, ks)) return launch_gemm_ks(a, ks, KS_X_F16, nullptr, 0, st);
+    // (an image out of 64 x 64 tiles whose K is short: the 128-wide tiles have the better epilogue.  N = 700, M = 1280, K = 1280: 12.0 to
+    // 13.2 us; N = 400, M = 3072, K = 768: 9.4; 13.5 — but K = 5120: 34; 28)
+    if (ks_pick(a.M, a.N, a.K, nb, emit, ks) && !(emit && ks.mt == 4 && a.K < 2048)) return launch_gemm_ks(a, ks, KS_X_F16, nullptr, 0, st);
+    static const bool staged = getenv("MI355X_GEMM_STAGED") != nullptr;        // the register-staged loop, for comparison
+    if (a.K % GB_K == 0 && (!staged || emit)) {
+        // a long K on 128 x 64 tiles, nothing but sums behind it: the two-role kernel (K = 3072, M = 768: 19 us, 21 over the direct loads)
+        if (!emit && !(a.e.flags & MI355X_EPI_GELU) && a.K >= 2048 && a.K % (4 * GB_K) == 0 && dl_pick(a, 1) == DL_128x64) return launch_gemm_f16_rs(a, st);
+        return emit ? launch_gemm_f16_dl<true>(a, nullptr, 1, st) : launch_gemm_f16_dl<false>(a, nullptr, 1, st);
+    }
+    if (emit) return MI355X_ERR_UNSUPPORTED;
     auto blocks = [&](int bn, int bm) { return ((a.N + bn - 1) / bn) * ((a.M + bm - 1) / bm) * nb; };
     if (blocks(128, 128) >= 384) return launch_gemm_f16<2, 2>(a, st);
-    if (blocks(128, 64)  >= 192 || a.N > 64 || a.K % GB_K == 0) return launch_gemm_f16<2, 1>(a, st);
-    if (a.e.flags & MI355X_EPI_EMIT_F16) return MI355X_ERR_UNSUPPORTED;
-    return launch_gemm_f16_k<1, 1, 2, true, false>(a, st);       // (few tiles of a K that k_gemm_ks does not take)
+    if (blocks(128, 64)  >= 192 || a.N > 64) return launch_gemm_f16<2, 1>(a, st);
+    return launch_gemm_f16<1, 1>(a, st);       // (few tiles of a K that k_gemm_ks does not take)
 }
 
 // ------------------------------------------------------------------------------------------------------
@@ -1175,8 +1105,7 @@ extern "C" int mi355x_mul_mat_group(const mi355x_mul_mat_item * items, int count
     if (flags & MI355X_MM_PREPARE_ONLY) return launch_status();
     ks_shape ks;
     if (ks_pick_group(a.M, a.N, a.K, count, ks)) return launch_gemm_ks_group(a, grp, count, ks, nullptr, st);
-    const int64_t blocks22 = ((a.N + 127) / 128) * ((a.M + 127) / 128) * count;
-    return blocks22 >= 300 ? launch_gemm_f16_group<2, 2>(a, grp, count, st) : launch_gemm_f16_group<2, 1>(a, grp, count, st);
+    return launch_gemm_f16_dl<false>(a, &grp, count, st);
 }
 
 extern "C" int mi355x_dequantize_row_f16(int type, const void * src, void * dst, int64_t k, void * stream) {
