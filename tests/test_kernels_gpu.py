@@ -404,7 +404,7 @@ def test_mul_mat_direct_load_tiles(pkg, oracle, gpu, own_numbers, k, m, n):
 
 
 # rows that are not 16-byte aligned, any K (the transposed V of a window of 1500, 37 or 1501 positions), one or two columns
-@pytest.mark.parametrize("k,m,n,batch", [(1500, 64, 300, 3), (37, 64, 37, 2), (1501, 64, 5, 2), (1500, 64, 1, 4), (64, 1500, 2, 2), (512, 1000, 1, 1), (1024, 1283, 2, 1), (1280, 5003, 2, 1), (2048, 48, 1, 1), (3, 5, 40, 1)])
+@pytest.mark.parametrize("k,m,n,batch", [(1500, 64, 300, 3), (37, 64, 37, 2), (1501, 64, 5, 2), (1500, 64, 1, 4), (64, 1500, 2, 2), (512, 1000, 1, 1), (1024, 1283, 2, 1), (1280, 5003, 2, 1), (2048, 48, 1, 1), (3, 5, 40, 1), (68, 64, 64, 12), (132, 65, 17, 1), (191, 63, 400, 20), (321, 130, 1500, 8), (1500, 64, 1500, 12)])
 def test_mul_mat_f16_keeps_f32_activations(pkg, oracle, gpu, own_numbers, k, m, n, batch):
     lib = pkg.kernels()
     w16, x = rnd((batch, m, k), 0.5).astype(np.float16), np.abs(rnd((batch, n, k), 1.0 / k))

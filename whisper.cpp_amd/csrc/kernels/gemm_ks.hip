@@ -307,6 +307,193 @@ __device__ __forceinline__ void gemm_kd_tile(const mm_args & a, const char * wb,
     ks_finish<MT, NT, KW, false>(acc, red, a, db, epi, batch_off, d_nb1, m0, n0);
 }
 
+// k_gemm_x32: f32 activations that stay f32 (the probabilities of plain attention against the transposed V of a head), many columns.
+// v_mfma_f32_16x16x4_f32 multiplies them at a sixteenth of the bf16 rate, 22 us for 1500 x 1500 x 64 x 12 at its peak — as long as
+// the 108 MB of activations take.  So a value goes to the bf16 matrix cores in three parts, its top eight significant bits, the
+// next eight and the last eight (each a subtraction that loses nothing), a weight in two (f16 has eleven bits): six products of
+// 32 steps where the f32 form takes eight of 4, 2.7 times the rate, every product exact and every sum f32 as before.
+// A wavefront owns 16 columns and all 64 rows of the tile, so an activation is read and split once, straight from memory into
+// the operand's lanes, three units of 64 ahead; the weights of a unit are split by the workgroup together and shared through LDS.
+// A half unit's 24 matrix instructions take the splitting of the next half between them.  1500 x 1500 x 64, heads: 12 63 us -> 36
+// (a K split over four wavefronts with f32 matrix instructions in front), 20 75 -> 45, 6 39 -> 25; 700 x 700 x 12 22 -> 14.
+// (The activations through LDS, whole rows at a time, came out slower: 49 us.)
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef uint32_t ks_u4 __attribute__((ext_vector_type(4)));
+struct bf16_parts3 { ks_u4 hi, mid, lo; };
+// the bf16 in the upper halves of two registers
+__device__ __forceinline__ uint32_t pack_hi(float a, float b) { return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302); }
+__device__ __forceinline__ float top_bf16(float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
+__device__ __forceinline__ bf16_parts3 split3(const ks_f4 & x0, const ks_f4 & x1) {
+    bf16_parts3 p;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = i < 2 ? x0[2 * i] : x1[2 * i - 4], b = i < 2 ? x0[2 * i + 1] : x1[2 * i - 3];
+        const float ra = a - top_bf16(a), rb = b - top_bf16(b);
+        p.hi[i] = pack_hi(a, b); p.mid[i] = pack_hi(ra, rb); p.lo[i] = pack_hi(ra - top_bf16(ra), rb - top_bf16(rb));
+    }
+    return p;
+}
+
+template <int NW>
+__global__ void __launch_bounds__(64 * NW, 2) k_gemm_x32(mm_args a) {
+    __shared__ __attribute__((aligned(16))) char w_lds[2][2][8192];       // [buffer][part][64 rows of 128 bytes, chunks swizzled as in gemm_ks_tile]
+    const mm_slice_ptrs z = mm_slice(a, blockIdx.z);
+    const int64_t m0 = (int64_t) blockIdx.x * 64, n0 = (int64_t) blockIdx.y * (16 * NW);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, q = lane >> 4;
+    const int units = (int)(a.K / KS_UNIT), tail = (int)(a.K % KS_UNIT);      // whole ones; values behind them
+    const int64_t n = n0 + 16 * wave + r16;
+    const char * xp = z.x + (n < a.N ? n : a.N - 1) * a.x_nb1 + q * 32;
+    // this thread's weights of a unit: WC chunks of 8 values, of row wr[i] chunk wc
+    constexpr int WC = (512 + 64 * NW - 1) / (64 * NW);    // (512 chunks of 8 values in a unit)
+    int wr[WC], wc[WC]; const char * wp[WC]; bool w_ok[WC];
+#pragma unroll
+    for (int i = 0; i < WC; ++i) {
+        const int c = i * 64 * NW + tid;
+        w_ok[i] = 512 % (64 * NW) == 0 || c < 512;
+        wr[i] = (c >> 3) & 63; wc[i] = c & 7;
+        wp[i] = z.w + (m0 + wr[i] < a.M ? m0 + wr[i] : a.M - 1) * a.w_nb1 + wc[i] * 16;
+    }
+
+    struct xunit { ks_f4 v[2][2]; };
+    struct wunit { ks_h8 v[WC]; };
+    // (units past the end re-read the last one: no load behind a branch, which would be waited for with every other)
+    auto load_x = [&](xunit & x, int u) __attribute__((always_inline)) {
+        const int64_t k = (int64_t)(u < units ? u : units - 1) * (KS_UNIT * 4);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) { x.v[s][0] = *(const ks_f4 *)(xp + k + 128 * s); x.v[s][1] = *(const ks_f4 *)(xp + k + 128 * s + 16); }
+    };
+    auto load_w = [&](wunit & w, int u) __attribute__((always_inline)) {
+        const int64_t k = (int64_t)(u < units ? u : units - 1) * (KS_UNIT * 2);
+#pragma unroll
+        for (int i = 0; i < WC; ++i) w.v[i] = *(const ks_h8 *)(wp[i] + k);
+    };
+    auto store_w = [&](const wunit & w, int buf, int i) __attribute__((always_inline)) {
+        ks_u4 hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float x = (float) w.v[i][2 * e], y = (float) w.v[i][2 * e + 1];
+            hi[e] = pack_hi(x, y); lo[e] = pack_hi(x - top_bf16(x), y - top_bf16(y));
+        }
+        char * to = &w_lds[buf][0][0] + (wr[i] >> 1) * 256 + (wr[i] & 1) * 128 + (wc[i] ^ ((wr[i] >> 1) & 7)) * 16;
+        if (w_ok[i]) { *(ks_u4 *) to = hi; *(ks_u4 *)(to + 8192) = lo; }
+    };
+    float4_t acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = (float4_t){ 0.f, 0.f, 0.f, 0.f };
+    const int frow = (r16 >> 1) * 256 + (r16 & 1) * 128, fsw = (r16 >> 1) & 7;
+    struct wfrag { bf16x8_t h[4], l[4]; };
+    auto read_w = [&](wfrag & w, int buf, int s) __attribute__((always_inline)) {
+        const char * at = &w_lds[buf][0][0] + frow + ((4 * s + q) ^ fsw) * 16;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { w.h[i] = *(const bf16x8_t *)(at + i * 2048); w.l[i] = *(const bf16x8_t *)(at + i * 2048 + 8192); }
+    };
+    auto mma = [&](const wfrag & w, const bf16_parts3 & p) __attribute__((always_inline)) {
+        const bf16x8_t xh = __builtin_bit_cast(bf16x8_t, p.hi), xm = __builtin_bit_cast(bf16x8_t, p.mid), xl = __builtin_bit_cast(bf16x8_t, p.lo);
+        // (the small products first)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.l[i], xl, acc[i], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.h[i], xl, acc[i], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.l[i], xm, acc[i], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.h[i], xm, acc[i], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.l[i], xh, acc[i], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.h[i], xh, acc[i], 0, 0, 0);
+    };
+    // issue order of a half unit: a matrix instruction, then what fits into its time of the splitting for the next half
+    auto interleave = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 24; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                      // 1 matrix instruction
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);                      // 4 vector instructions
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    xunit x[4]; wunit w[2];
+    bf16_parts3 p0, p1;
+    if (units > 0) {                                       // uniform
+        load_w(w[0], 0); load_x(x[0], 0);
+        load_w(w[1], 1); load_x(x[1], 1);
+#pragma unroll
+        for (int i = 0; i < WC; ++i) store_w(w[0], 0, i);
+        load_w(w[0], 2); load_x(x[2], 2);
+        p0 = split3(x[0].v[0][0], x[0].v[0][1]);
+        __syncthreads();
+        // unit u: x[u % 4], its first half split already; w[(u + 1) % 2] holds the weights of unit u + 1
+        auto step = [&](int u, xunit & cur, const xunit & nxt, xunit & far, wunit & wn) __attribute__((always_inline)) {
+            wfrag f0, f1;
+            read_w(f0, u & 1, 0);
+            load_x(far, u + 3);
+            __builtin_amdgcn_sched_barrier(0);
+            read_w(f1, u & 1, 1);
+            p1 = split3(cur.v[1][0], cur.v[1][1]);
+            mma(f0, p0);
+#pragma unroll
+            for (int i = 0; i < WC / 2; ++i) store_w(wn, (u + 1) & 1, i);
+            interleave();
+            p0 = split3(nxt.v[0][0], nxt.v[0][1]);
+            mma(f1, p1);
+#pragma unroll
+            for (int i = WC / 2; i < WC; ++i) store_w(wn, (u + 1) & 1, i);
+            interleave();
+#pragma unroll
+            for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(p0.hi[i]), "+v"(p0.mid[i]), "+v"(p0.lo[i]));       // (split here, not where it is used)
+            load_w(wn, u + 3);
+            __syncthreads();
+        };
+        for (int u = 0;;) {
+            step(u, x[0], x[1], x[3], w[1]); if (++u >= units) break;
+            step(u, x[1], x[2], x[0], w[0]); if (++u >= units) break;
+            step(u, x[2], x[3], x[1], w[1]); if (++u >= units) break;
+            step(u, x[3], x[0], x[2], w[0]); if (++u >= units) break;
+        }
+    }
+    if (tail != 0) {                                       // the unit that K ends in: value by value, zeros behind the end
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int k = 32 * s + 8 * q + e;
+                const float v = *(const float *)(xp - q * 32 + (k < tail ? (int64_t) units * KS_UNIT + k : 0) * 4);
+                x[0].v[s][e / 4][e % 4] = k < tail ? v : 0.0f;
+            }
+#pragma unroll
+        for (int i = 0; i < WC; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int k = 8 * wc[i] + e;
+                const half_t v = *(const half_t *)(wp[i] - wc[i] * 16 + (k < tail ? (int64_t) units * KS_UNIT + k : 0) * 2);
+                w[0].v[i][e] = k < tail ? v : (half_t) 0.0f;
+            }
+#pragma unroll
+        for (int i = 0; i < WC; ++i) store_w(w[0], 0, i);
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            wfrag f;
+            read_w(f, 0, s);
+            mma(f, split3(x[0].v[s][0], x[0].v[s][1]));
+        }
+    }
+
+    if (n >= a.N) return;
+    char * db = a.d + z.d_off;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int64_t m = m0 + 16 * i + 4 * q;
+        if (a.e.flags == 0 && m + 3 < a.M) { *(ks_f4 *)(db + n * a.d_nb1 + m * 4) = (ks_f4){ acc[i][0], acc[i][1], acc[i][2], acc[i][3] }; continue; }
+        for (int e = 0; e < 4 && m + e < a.M; ++e) {
+            const float v = apply_epilogue(acc[i][e], a.e, m + e, n, z.d_off + n * a.d_nb1 + (m + e) * 4);
+            if (a.e.flags & MI355X_EPI_OUT_F16) *(half_t *)(db + n * a.d_nb1 + (m + e) * 2) = (half_t) v;
+            else                                *(float  *)(db + n * a.d_nb1 + (m + e) * 4) = v;
+        }
+    }
+}
+
 // grids: m tiles x n tiles x batch
 #define KS_SLICES const mm_slice_ptrs z = mm_slice(a, blockIdx.z); const char * wb = z.w, * xb = z.x; const int64_t d_off = z.d_off; \
     const int64_t m0 = (int64_t) blockIdx.x * (16 * MT / H), n0 = (int64_t) blockIdx.y * (16 * NT / H);
@@ -471,7 +658,7 @@ int launch_gemm_ks_group(const mm_args & a, const mm_group & all, int count, con
 }
 
 // The direct kernel, by size: a few columns on 16 x 16 tiles with as many wavefronts as the K range has units, up to 8; more
-// on 64 x 32 (64 rows are all there are of the transposed V of a head: src1 is then read once).
+// on 64 x 32 (64 rows are all there are of the transposed V of a head: src1 is then read once), or k_gemm_x32 where src1 stays f32.
 int launch_gemm_kd(const mm_args & a, int xm, hipStream_t st) {
     const bool few = a.N <= 16;
     const int kw = a.K <= KS_UNIT ? 1 : a.K < 8 * KS_UNIT ? 4 : 8;
@@ -479,6 +666,23 @@ int launch_gemm_kd(const mm_args & a, int xm, hipStream_t st) {
         if (!few) return launch_kd_t<4, 2, 4, KS_X_F16>(a, st);
         return kw == 1 ? launch_kd_t<1, 1, 1, KS_X_F16>(a, st) : kw == 4 ? launch_kd_t<1, 1, 4, KS_X_F16>(a, st) : launch_kd_t<1, 1, 8, KS_X_F16>(a, st);
     }
-    if (!few) return launch_kd_t<4, 2, 4, KS_X_F32>(a, st);
+    if (!few) {
+        // as many wavefronts to the workgroup, 4, 5 or 6, as deal the 16-column pieces out to the CUs most evenly
+        const int64_t tm = (a.M + 63) / 64, nb = a.ne12 * a.ne13;
+        int nw = 4; int64_t best = INT64_MAX;
+        for (int i : { 4, 5, 6 }) {
+            const int64_t cost = (tm * ((a.N + 16 * i - 1) / (16 * i)) * nb + 255) / 256 * i;
+            if (cost < best) { best = cost; nw = i; }
+        }
+        const int64_t tn = (a.N + 16 * nw - 1) / (16 * nw);
+        if (tm > 0x7fffffff || tn > 65535 || nb > 65535) return MI355X_ERR_UNSUPPORTED;
+        const dim3 grid((unsigned) tm, (unsigned) tn, (unsigned) nb);
+        switch (nw) {
+            case 4:  k_gemm_x32<4><<<grid, 256, 0, st>>>(a); break;
+            case 5:  k_gemm_x32<5><<<grid, 320, 0, st>>>(a); break;
+            default: k_gemm_x32<6><<<grid, 384, 0, st>>>(a); break;
+        }
+        return launch_status();
+    }
     return kw == 1 ? launch_kd_t<1, 1, 1, KS_X_F32>(a, st) : kw == 4 ? launch_kd_t<1, 1, 4, KS_X_F32>(a, st) : launch_kd_t<1, 1, 8, KS_X_F32>(a, st);
 }
