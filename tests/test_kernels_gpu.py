@@ -889,10 +889,13 @@ def test_flash_attn_packed_f16_chain(pkg, oracle, gpu, case):
     assert np.array_equal(again.view(np.uint32), got.view(np.uint32))          # the same bits on every run
 
 
-@pytest.mark.parametrize("H,N,KV,masked", [(3, 9, 1, False), (2, 32, 64, True), (2, 33, 65, True), (1, 31, 129, False),            # 32 queries to the workgroup
-                                          (128, 64, 79, False), (129, 64, 80, True), (129, 65, 127, True), (257, 17, 193, False)])   # from 257 workgroups of those on: 64
+@pytest.mark.parametrize("H,N,KV,masked", [(3, 9, 1, False), (2, 16, 64, True), (2, 17, 65, True), (128, 32, 129, False),               # 16 queries to the workgroup
+                                          (129, 32, 64, True), (128, 33, 79, False), (128, 64, 193, True),                            # from 257 workgroups of those on: 32
+                                          (129, 64, 80, True), (128, 127, 100, False),                                                 # ... 64
+                                          (257, 33, 127, True), (384, 64, 63, False),                                                  # 32 again, several to a CU
+                                          (385, 64, 70, True), (257, 65, 130, False)])                                                 # 64 without loader wavefronts
 def test_flash_attn_packed_tile_sizes(pkg, oracle, gpu, own_numbers, H, N, KV, masked):
-    # both tile sizes of the many-query kernel of the packed form at their edges, ragged ends and odd mask strides; the image
+    # the tile sizes of the many-query kernel of the packed form at their edges, ragged ends and odd mask strides; the image
     # beside dst is its rows' Q8_0 rounding
     q, kb, vb = _attention_inputs(oracle, H, N, KV)
     mask = None

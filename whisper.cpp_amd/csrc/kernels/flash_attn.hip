@@ -228,31 +228,29 @@ __device__ __forceinline__ half2_t seq_scale2(half2_t acc, float ms) {
 // rounding (2^-12 of an increment that is itself a small part of the sum) and by one rounding instead of two.  On gfx950
 // that is v_pk_fma_f16, two elements per instruction.
 //
-// One key for two of a lane's queries and P pairs of d: x[j] / y[j] hold d pair j of the first / second query, v the key's d pairs,
-// fx / fy the factors of two consecutive keys for the queries as two f16; SEL picks the first or the second of them.
+// One key for two of a lane's queries (or one) and two pairs of d: x / y hold the pairs of the first / second query, v0, v1 the key's d
+// pairs, fx / fy the factors of two consecutive keys for the queries as two f16; SEL picks the first or the second of them.
 // (asm with tied operands: the accumulators stay in the registers they are in, whatever branches surround the step)
 #define PK_FMA(acc, v, f, sel) "v_pk_fma_f16 %" #acc ", %" #v ", %" #f ", %" #acc " " sel "\n\t"
 #define PK_LO "op_sel_hi:[1,0,1]"
 #define PK_HI "op_sel:[0,1,0] op_sel_hi:[1,1,1]"
-template <int P, int SEL>
-__device__ __forceinline__ void pk_key(uint32_t (&x)[P], uint32_t (&y)[P], const uint32_t (&v)[P], uint32_t fx, uint32_t fy) {
-    static_assert(P == 2 || P == 4, "4 or 8 d to a lane");
+template <int SEL>
+__device__ __forceinline__ void pk_key(uint32_t (&x)[2], uint32_t (&y)[2], uint32_t v0, uint32_t v1, uint32_t fx, uint32_t fy) {
 #define PK_KEY2(sel) asm(PK_FMA(0, 4, 6, sel) PK_FMA(2, 4, 7, sel) PK_FMA(1, 5, 6, sel) PK_FMA(3, 5, 7, sel) \
-                         : "+v"(x[0]), "+v"(x[1]), "+v"(y[0]), "+v"(y[1]) : "v"(v[0]), "v"(v[1]), "v"(fx), "v"(fy))
-#define PK_KEY4(sel) asm(PK_FMA(0, 8, 12, sel) PK_FMA(4, 8, 13, sel) PK_FMA(1, 9, 12, sel) PK_FMA(5, 9, 13, sel) \
-                         PK_FMA(2, 10, 12, sel) PK_FMA(6, 10, 13, sel) PK_FMA(3, 11, 12, sel) PK_FMA(7, 11, 13, sel) \
-                         : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]) \
-                         : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(fx), "v"(fy))
-    if constexpr (P == 2) { if constexpr (SEL == 0) PK_KEY2(PK_LO); else PK_KEY2(PK_HI); }
-    else                  { if constexpr (SEL == 0) PK_KEY4(PK_LO); else PK_KEY4(PK_HI); }
+                         : "+v"(x[0]), "+v"(x[1]), "+v"(y[0]), "+v"(y[1]) : "v"(v0), "v"(v1), "v"(fx), "v"(fy))
+    if constexpr (SEL == 0) PK_KEY2(PK_LO); else PK_KEY2(PK_HI);
+}
+template <int SEL>
+__device__ __forceinline__ void pk_key(uint32_t (&x)[2], uint32_t v0, uint32_t v1, uint32_t f) {
+#define PK_KEY1(sel) asm(PK_FMA(0, 2, 4, sel) PK_FMA(1, 3, 4, sel) : "+v"(x[0]), "+v"(x[1]) : "v"(v0), "v"(v1), "v"(f))
+    if constexpr (SEL == 0) PK_KEY1(PK_LO); else PK_KEY1(PK_HI);
 }
 // acc = f16(acc * ms), a rescale
 __device__ __forceinline__ void pk_scale(uint32_t & acc, uint32_t m) { asm("v_pk_mul_f16 %0, %0, %1" : "+v"(acc) : "v"(m)); }
 // two f32 factors -> one register of two f16 (round to nearest even, as the conversion in front of vdupq_n_f16)
 __device__ __forceinline__ uint32_t pk_factors(float f0, float f1) {
-    uint32_t r;
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(r) : "v"(f0), "v"(f1));
-    return r;
+    typedef float float2_t __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(((float2_t){ f0, f1 }), half2_t));      // (no asm: an operand fresh from v_exp_f32 needs a wait state that only the compiler sees to)
 }
 
 // softmax factors of a run of scores that continues a running maximum M:  s[i] -> vs[i], ms[i]; also the run's
@@ -1194,23 +1192,20 @@ __global__ void __launch_bounds__(512, 2) k_fattn_seq_tile(fa_args a) {
 // ------------------------------------------------------------------------------------------------------
 // k_fattn_pk_tile: N > 8, the packed-f16 form of the step (MI355X_FA_F16_PK)
 //
-// A workgroup owns TQ queries of one head and walks the keys in tiles of 64.  Two roles, one barrier per tile: four chain
-// wavefronts, one to a SIMD, walk tile t - 1 key by key, while PW producer wavefronts make the factors of tile t.
+// A workgroup owns TQ = 16 QL queries of one head and walks the keys in tiles of 64.  Three roles, one barrier per tile: four chain
+// wavefronts, one to a SIMD, walk tile t - 1 key by key, while PW producer wavefronts make the factors of tile t and LW loader
+// wavefronts move its V rows and the K rows of the tiles behind it (LW = 0: the producers do that as well).
 //
-//   chains     a lane owns QL queries x 4 d (lane = query group l / 16, d slice l % 16): a key costs it one read of V for 2 QL
-//              v_pk_fma_f16, and the factors arrive as f16, two keys to a register and the lane's queries side by side.  A block of 16 keys in which no query of the wavefront gets a new maximum is its multiply-adds and nothing
-//              else; the others begin with a rescale of the accumulators.
+//   chains     a lane owns QL queries x 4 d (lane = query group l / 16, d slice l % 16): four keys cost it a read of V for each of its
+//              two d pairs, eight keys a read of factors for each of its queries, and a key 2 QL v_pk_fma_f16.  A block of 16 keys
+//              in which no query of the wavefront gets a new maximum is its multiply-adds and nothing else; the others begin
+//              with a rescale of the accumulators.
 //   producers  scores come transposed out of v_mfma_f32_16x16x32_f16 (K rows as the A operand, Q as the B operand, which stays
 //              in registers): lane l holds query l % 16 and the keys 16 b + 4 (l / 16) + e, b, e = 0 .. 3 — so running maximum,
-//              denominator and factors never leave the registers of the lanes they belong to.  A block of 16 keys that
-//              raises no maximum in the wavefront is four exponentials of fma(c, scale, -M) and their sum; the others take the
-//              block's maximum over the four lanes of a query (two lane swaps) first.  The denominator is kept per lane, as the
-//              sum of exp2(s - M) of the lane's own keys, and added up at the end.
-//              K and V rows go from memory straight into LDS (global_load_lds), a tile ahead.
-//   factor tile  fp[key pair][query]: each register the f16 factors vs of keys 2 p, 2 p + 1 for one query; fm[block][query] the
-//                rescale ms in front of a block, for blocks with one.  The four lanes of a query write rows 2 apart: where a row
-//                is a multiple of the banks, those would collide, so the column (and with 32 columns the row of the pair) is
-//                flipped by the lane's group (fp_row, fp_flip).
+//              denominator and factors never leave the registers of the lanes they belong to.  The denominator is kept per lane, as
+//              the sum of exp2(s - M) of the lane's own keys, and added up at the end.
+//   loaders    K rows go from memory straight into LDS (global_load_lds), V rows through registers into a dword per key and d pair.
+//              What a tile requests is awaited in the one after the next.
 // The running maximum moves at the beginning of a block of 16 keys instead of at the key, at most 15 keys early: a key in front of
 // the new maximum takes its factor at the new scale, where the reference takes it at the old one and rescales the sum after it.
 // From the block's end on both are at the same scale, which matters — with flat attention the f16 sum of 1500 keys stagnates
@@ -1218,54 +1213,51 @@ __global__ void __launch_bounds__(512, 2) k_fattn_seq_tile(fa_args a) {
 // exact, results were 3e-4 NMSE away from the reference's sequence and closer to the exact sum.  Key by key, with a scalar test
 // per key in the chains, a block with a raise cost three times one without.
 //
-// What bounds it: one wavefront issues a vector instruction every 5 clocks (2.3 ns; two on a SIMD one every 1.9 ns), and LDS
-// returns a 16-byte read in 1.84 ns, an 8-byte read in 1.02 ns per CU (and a pair of 8-byte reads as one instruction in
-// 3.4 ns, which is why the addresses are kept apart).  A workgroup that has its CU to itself is one wavefront per SIMD and takes
-// the chain's length times 5 clocks, so a small grid wants few queries to the workgroup, a large one few LDS reads to the
-// multiply-add:
-//   QL = 4, 64 queries   8 multiply-adds to a key: 0.24 ns of LDS each
-//   QL = 2, 32 queries   half the instructions per wavefront; 0.38 ns
-// (A lane of 4 queries x 8 d, 128 queries to the workgroup, 0.17 ns, came out level with QL = 4 at its best.)
+// What bounds it: one wavefront issues a vector instruction every 5 clocks (2.1 ns; two on a SIMD one every 1.9 ns), an LDS read
+// costs it 6 ns of issue whatever its width, and a load from memory 70 clocks.  A workgroup that has its CU to itself is one
+// wavefront per SIMD and role, and a tile takes as long as the slowest role: 16 QL 8 multiply-adds and (4 + QL) 8 reads of the chain,
+// some 300 instructions of a producer, or the loads (with one role for both a tile of 16 queries took 3800 clocks, 1150 of them for
+// the 16 loads, now 1900).  So a small grid wants few queries to the workgroup, a large one few reads to the multiply-add.
 // Measured, us, with the exact per-key form that was here before in front (64 queries, factors as f32 pairs through LDS):
-//   N 1500 x KV 1536 x 20 heads 105 -> QL 4: 85; 12 heads 96 -> 78; 6 heads 73 -> QL 4: 49, QL 2: 58; 487 x 512 x 6: 31 -> QL 2: 17;
-//   227 x 1536 x 20: 73 -> QL 4: 48, QL 2: 40; 27 x 1536 x 12: 70 -> 39; 27 x 256 x 12 with a mask: 22 -> 12
+//   27 x 1536 x 12 heads 70 -> QL 1: 23, QL 2: 28, QL 4: 41; 27 x 256 x 12 with a mask 22 -> 8.5; 487 x 512 x 6 31 -> QL 1: 11;
+//   227 x 1536 x 20 73 -> QL 2: 28; N 1500 x KV 1536: 6 heads 73 -> QL 4: 43; 12 heads 97 -> QL 2: 69, QL 4: 75; 20 heads 98 ... 105 ->
+//   QL 4 without loaders: 76, with them 83, QL 2: 88
+// (A lane of 4 queries x 8 d, 128 queries to the workgroup, came out level with QL = 4 at its best.)
 // ------------------------------------------------------------------------------------------------------
 
 #define P_KV       64
 #define P_M_START  (-3.0e38f)     // below every score and finite: no difference is (-inf) - (-inf), a masked key gives the factor 0
 
-__device__ __forceinline__ void wait_loads() {                // everything requested has arrived, rows on their way into LDS included
-    __builtin_amdgcn_s_waitcnt((0 << 14) | (7 << 4) | (15 << 8));
+template <int N>
+__device__ __forceinline__ void wait_loads() {                // all but the N youngest loads have arrived (rows on their way into LDS included), all LDS traffic is done
+    static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4));
     __builtin_amdgcn_sched_barrier(0);
 }
 
+#define P_VPITCH   (P_KV + 4)          // dwords of a d pair's row of the V tile: 272 bytes, 16 mod 256
+#define P_FPITCH   (2 * P_KV + 16)     // bytes of a query's row of the factor tile: 144
 template <int QL> constexpr int p_queries() { return 16 * QL; }                          // four wavefronts of four groups
-template <int QL> constexpr int p_lds_bytes() { return 2 * P_KV * FA_D * 2 * 2 + 2 * (P_KV / 2 + 4) * p_queries<QL>() * 4 + 2 * 4 * 4 + p_queries<QL>() * 4; }
+template <int QL> constexpr int p_lds_bytes() { return 3 * P_KV * FA_D * 2 + 2 * 32 * P_VPITCH * 4 + 2 * p_queries<QL>() * P_FPITCH + 2 * 4 * p_queries<QL>() * 4 + 2 * 4 * 4 + p_queries<QL>() * 4; }
 
-// where a factor tile keeps (key pair, query): register fp_row(pair) + (query ^ fp_flip(pair)); (pair / 2) % 4 is the group of the
-// lane that writes it
-template <int TQ> __device__ __forceinline__ constexpr int fp_row(int pair)  { return TQ >= 64 ? pair * TQ : (pair ^ (pair >> 2 & 1)) * 32; }
-template <int TQ> __device__ __forceinline__ constexpr int fp_flip(int pair) { return TQ >= 64 ? (pair >> 1 & 3) << 4 : (pair >> 1 & 1) << 4; }
-
-template <int QL, int PW>
-__global__ void __launch_bounds__(256 + 64 * PW, 2) k_fattn_pk_tile(fa_args a) {
+template <int QL, int PW, int LW>
+__global__ void __launch_bounds__(256 + 64 * (PW + LW), 2) k_fattn_pk_tile(fa_args a) {
     constexpr int TQ = p_queries<QL>(), QB = TQ / (16 * PW);      // QB: blocks of 16 queries per producer wavefront
-    constexpr int FP_TILE = (P_KV / 2) * TQ;
+    constexpr int V_TILE = 32 * P_VPITCH * 4, F_TILE = TQ * P_FPITCH;
     constexpr int DL = 4, SL = FA_D / DL, WQ = TQ / 4;                // a lane's d; d slices (lanes of a query group); queries per chain wavefront
     extern __shared__ __attribute__((aligned(16))) char t_smem[];
-    char *     k_s   = t_smem;                                // [2][64 rows of 128 bytes], chunks swizzled
-    char *     v_s   = k_s + 2 * P_KV * FA_D * 2;             // [2][64 rows of 128 bytes]
-    uint32_t * fp_s  = (uint32_t *)(v_s + 2 * P_KV * FA_D * 2);
-    uint32_t * fm_s  = fp_s + 2 * FP_TILE;                    // [2][4][TQ]
+    char *     k_s   = t_smem;                                // [3][64 rows of 128 bytes], chunks swizzled
+    char *     v_s   = k_s + 3 * P_KV * FA_D * 2;             // [2][32 d pairs][P_VPITCH], a dword per key; piece g (four keys) of row p at g ^ (p / 16)
+    char *     f_s   = v_s + 2 * V_TILE;                      // [2][TQ][P_FPITCH], an f16 per key
+    uint32_t * fm_s  = (uint32_t *)(f_s + 2 * F_TILE);        // [2][4][TQ]
     uint32_t * rm_s  = fm_s + 2 * 4 * TQ;                     // [2][PW]     bit b: block b of the tile begins with a rescale
     float *    s_run = (float *)(rm_s + 2 * PW);              // [TQ]
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // an XCD gets one run of consecutive (head, query tile) pairs, head-major, so that a head's K and V stay in one or two L2s
-    const uint32_t gx = (uint32_t)((a.N + TQ - 1) / TQ), gy = (uint32_t) a.H;        // (the grid; gridDim is a trip to memory of its own)
-    const uint32_t lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), total = gx * gy * (uint32_t) a.ne3;
-    const uint32_t xcd = lin % 8, per = total / 8, extra = total % 8;
+    const uint32_t gx = (uint32_t)((a.N + TQ - 1) / TQ), gy = (uint32_t) a.H, total = gx * gy * (uint32_t) a.ne3;
+    const uint32_t lin = blockIdx.x, xcd = lin % 8, per = total / 8, extra = total % 8;
     const uint32_t item = xcd * per + (xcd < extra ? xcd : extra) + lin / 8;
     const uint32_t heads = div_count(item, gx);
     const int64_t n0 = (int64_t)(item - heads * gx) * TQ, i3 = a.ne3 == 1 ? 0 : heads / gy, h = heads - i3 * gy;
@@ -1276,28 +1268,85 @@ __global__ void __launch_bounds__(256 + 64 * PW, 2) k_fattn_pk_tile(fa_args a) {
         const int pw = wave - 4, r16 = lane & 15, g = lane >> 4;
         const char * kb = a.k + div_count((uint32_t) h, a.hk_ratio) * a.k_nb2 + div_count((uint32_t) i3, a.k_ne3_ratio) * a.k_nb3;
         const char * vb = a.v + div_count((uint32_t) h, a.hv_ratio) * a.v_nb2 + div_count((uint32_t) i3, a.v_ne3_ratio) * a.v_nb3;
-        // Rows of a tile: 8 loads of 8 rows for K and for V, dealt to the wavefronts.  K: row pairs form 256-byte lines, the 16-byte
+        // K rows of a tile: 8 loads of 8 rows, dealt to the wavefronts.  Row pairs form 256-byte lines, the 16-byte
         // chunk c of row r sits in slot (r & 1) * 8 + (c ^ (line & 7)), so that the 16 rows of a fragment read cover all banks once.
-        constexpr int LD = 8 / PW;
-        auto load_k = [&](int it) __attribute__((always_inline)) {
+        // LW wavefronts of their own do the loads, or (LW = 0) the producers beside their factors.
+        constexpr int NL = LW ? LW : PW, LD = 8 / NL;
+        const int lw = LW ? pw - PW : pw;
+        const char * kp[LD];                                   // this lane's rows of the next tile to be loaded
+#pragma unroll
+        for (int i = 0; i < LD; ++i) { const int line = 4 * (lw * LD + i) + g; kp[i] = kb + (2 * line + (r16 >> 3)) * a.k_nb1 + ((lane & 7) ^ (line & 7)) * 16; }
+        const int64_t k_step = P_KV * a.k_nb1, v_step = P_KV * a.v_nb1;
+        // (parts [i0, i1) of the loads of tile 0, 1, 2, ...; past the last tile: that one again, into a buffer that nobody reads, so that
+        // the number of loads in flight stays what the waits count on)
+        auto load_k = [&](int tile, int buf, int i0, int i1) __attribute__((always_inline)) {
+            const int it = min(tile, n_tiles - 1);
+            const bool whole = (int64_t)(it + 1) * P_KV <= a.KV;               // uniform; rows past the end: the last one, masked
+            const int64_t step = tile + 1 < n_tiles ? k_step : 0;
 #pragma unroll
             for (int i = 0; i < LD; ++i) {
-                const int j = pw * LD + i, line = 4 * j + g;
-                const int64_t key = (int64_t) it * P_KV + 2 * line + (r16 >> 3);
-                const char * p = kb + (key < a.KV ? key : a.KV - 1) * a.k_nb1 + ((lane & 7) ^ (line & 7)) * 16;      // (past the end: masked)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *) p, (__attribute__((address_space(3))) void *)(k_s + (it & 1) * (P_KV * FA_D * 2) + j * 1024), 16, 0, 0);
+                if (i < i0 || i >= i1) continue;
+                const int j = lw * LD + i;
+                const char * p = kp[i];
+                if (!whole) { const int over = (int)((int64_t) it * P_KV - (a.KV - 1)) + 8 * j + 2 * g + (r16 >> 3); p -= (over > 0 ? over : 0) * a.k_nb1; }      // (no branch per lane: the load into LDS takes all lanes at once)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *) p, (__attribute__((address_space(3))) void *)(k_s + buf * (P_KV * FA_D * 2) + j * 1024), 16, 0, 0);
+                kp[i] += step;
             }
+            __builtin_amdgcn_sched_barrier(0);
         };
-        auto load_v = [&](int it) __attribute__((always_inline)) {
+        // V rows: this lane RL consecutive keys, 16 bytes (four d pairs) of each, through registers into a dword per key and pair
+        constexpr int RL = 8 / NL;
+        const int vkey = (P_KV / NL) * lw + RL * (lane >> 3), vc = lane & 7;
+        const char * vp = vb + vkey * a.v_nb1 + vc * 16;
+        auto load_v = [&](u32x4 (&vr)[RL], int tile, int i0, int i1) __attribute__((always_inline)) {
+            const int it = min(tile, n_tiles - 1);
+            const bool whole = (int64_t)(it + 1) * P_KV <= a.KV;
 #pragma unroll
-            for (int i = 0; i < LD; ++i) {
-                const int j = pw * LD + i;
-                const int64_t key = (int64_t) it * P_KV + 8 * j + (lane >> 3);
-                const char * p = vb + (key < a.KV ? key : a.KV - 1) * a.v_nb1 + (lane & 7) * 16;                     // (past the end: factor 0, finite values)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *) p, (__attribute__((address_space(3))) void *)(v_s + (it & 1) * (P_KV * FA_D * 2) + j * 1024), 16, 0, 0);
+            for (int i = 0; i < RL; ++i) {
+                if (i < i0 || i >= i1) continue;
+                const char * p = vp + i * a.v_nb1;
+                if (!whole) { const int over = (int)((int64_t) it * P_KV - (a.KV - 1)) + vkey + i; p -= (over > 0 ? over : 0) * a.v_nb1; }      // (past the end: factor 0, finite values)
+                vr[i] = *(const u32x4 *) p;
+            }
+            if (i1 == RL) vp += tile + 1 < n_tiles ? v_step : 0;
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto store_v = [&](const u32x4 (&vr)[RL], int it) __attribute__((always_inline)) {
+            char * to = v_s + (it & 1) * V_TILE + 4 * vc * (P_VPITCH * 4);
+            const int sw = vc >> 2;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if constexpr (RL == 2) *(u32x2 *)(to + j * (P_VPITCH * 4) + (((vkey >> 2) ^ sw) << 4) + (vkey & 2) * 4) = (u32x2){ vr[0][j], vr[1][j] };
+                else {
+#pragma unroll
+                    for (int h = 0; h < RL / 4; ++h)
+                        *(u32x4 *)(to + j * (P_VPITCH * 4) + ((((vkey >> 2) + h) ^ sw) << 4)) = (u32x4){ vr[4 * h][j], vr[4 * h + 1][j], vr[4 * h + 2][j], vr[4 * h + 3][j] };
+                }
             }
         };
-        load_k(0);
+        u32x4 va[RL], vc2[RL];                                 // V rows of the tile in work and of the next
+        if (LW == 0 || pw >= PW) { load_k(0, 0, 0, LD); load_v(va, 0, 0, RL); load_k(1, 1, 0, LD); }
+        if (LW != 0 && pw >= PW) {
+            wait_loads<0>();
+            int kbuf = 0;
+            auto move = [&](int it, u32x4 (&vr)[RL], u32x4 (&vnext)[RL]) __attribute__((always_inline)) {
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+                load_v(vnext, it + 1, 0, RL);
+                load_k(it + 2, kbuf == 0 ? 2 : kbuf - 1, 0, LD);
+                wait_loads<RL + LD>();                         // V of this tile is in registers, K of the next in LDS
+                store_v(vr, it);
+                __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));         // lgkmcnt(0)
+                kbuf = kbuf == 2 ? 0 : kbuf + 1;
+            };
+            for (int it = 0;;) {
+                move(it, va, vc2); if (++it == n_tiles) break;
+                move(it, vc2, va); if (++it == n_tiles) break;
+            }
+            __builtin_amdgcn_s_barrier();
+            wait_loads<0>();                                   // (the surplus loads still write LDS)
+            return;
+        }
         half8_t qf[QB][2];                                     // this lane's queries, d = 32 s + 8 g .. + 7
         const char * mrow[QB];
 #pragma unroll
@@ -1333,28 +1382,45 @@ __global__ void __launch_bounds__(256 + 64 * PW, 2) k_fattn_pk_tile(fa_args a) {
         float M[QB], S[QB];                                    // running maximum of the query; this lane's share of its denominator
 #pragma unroll
         for (int i = 0; i < QB; ++i) { M[i] = P_M_START; S[i] = 0.0f; }
-        wait_loads();
+        wait_loads<0>();
 
-        for (int it = 0; it < n_tiles; ++it) {
-            __syncthreads();                                   // tile boundary: K of tile it is there, the other buffers are free
-            load_v(it);
-            if (it + 1 < n_tiles) load_k(it + 1);
+        // Tile `it` (K in buffer kbuf, V rows in vr, both requested two tiles ago); the loads of this tile are awaited in the one after
+        // the next: a tile of the smallest grids takes less time than its rows take to arrive.
+        int kbuf = 0;
+        auto tile = [&](int it, u32x4 (&vr)[RL], u32x4 (&vnext)[RL]) __attribute__((always_inline)) {
+            // tile boundary: K of tile it is there, the other buffers are free.  (A bare barrier: __syncthreads() waits for every load into LDS.)
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            // The loads are spread over the tile's work: a load occupies the path into memory for 70 clocks, and behind one that waits for
+            // it everything else of the wavefront waits too (16 in a row: 1150 clocks of a tile's 3800).
+            const int knext = kbuf == 0 ? 2 : kbuf - 1;
+            float4_t c[QB][4];                                 // scores in units of log2 e
+            {
+                half8_t kf[4][2];
+                const char * kt = k_s + kbuf * (P_KV * FA_D * 2);
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) kf[b][s] = *(const half8_t *)(kt + b * 2048 + frow + ((4 * s + g) ^ fsw) * 16);
+                __builtin_amdgcn_sched_barrier(0);
+                if (LW == 0) load_v(vnext, it + 1, 0, RL / 2);
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+#pragma unroll
+                        for (int i = 0; i < QB; ++i) c[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[b][s], qf[i][s], s == 0 ? (float4_t){ 0.f, 0.f, 0.f, 0.f } : c[i][b], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (LW == 0) load_v(vnext, it + 1, RL / 2, RL);
+            }
             if (busy) {
-                float4_t c[QB][4];
-                const char * kt = k_s + (it & 1) * (P_KV * FA_D * 2);
-#pragma unroll
-                for (int b = 0; b < 4; ++b) {
-#pragma unroll
-                    for (int i = 0; i < QB; ++i) c[i][b] = (float4_t){ 0.f, 0.f, 0.f, 0.f };
-#pragma unroll
-                    for (int s = 0; s < 2; ++s) {
-                        const half8_t kf = *(const half8_t *)(kt + b * 2048 + frow + ((4 * s + g) ^ fsw) * 16);
-#pragma unroll
-                        for (int i = 0; i < QB; ++i) c[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[i][s], c[i][b], 0, 0, 0);
-                    }
-                }
                 const bool plain = !a.mask && (int64_t)(it + 1) * P_KV <= a.KV;                // uniform
-                if (!plain) {
+                if (plain) {
+#pragma unroll
+                    for (int i = 0; i < QB; ++i)
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) c[i][b] *= scale2;
+                } else {
 #pragma unroll
                     for (int i = 0; i < QB; ++i)
 #pragma unroll
@@ -1366,63 +1432,63 @@ __global__ void __launch_bounds__(256 + 64 * PW, 2) k_fattn_pk_tile(fa_args a) {
                             }
                     if (a.mask && it + 1 < n_tiles) load_mask(it + 1);
                 }
-                uint32_t * fpw = fp_s + (it & 1) * FP_TILE;
+                __builtin_amdgcn_sched_barrier(0);
+                if (LW == 0) load_k(it + 2, knext, 0, LD / 2);
+                // The blocks' maxima over the four lanes of a query (two lane swaps), then the maximum up to each block: no branch for the
+                // blocks that raise none, which are the fewer while a row is short, and the blocks' steps fill each other's waits.
+                float top[QB][4], mb[QB][5];
+#pragma unroll
+                for (int i = 0; i < QB; ++i)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) top[i][b] = fmaxf(fmaxf(c[i][b][0], c[i][b][1]), fmaxf(c[i][b][2], c[i][b][3]));
+#pragma unroll
+                for (int i = 0; i < QB; ++i)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        const auto w16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(top[i][b]), __float_as_uint(top[i][b]), false, false);
+                        top[i][b] = fmaxf(__uint_as_float(w16[0]), __uint_as_float(w16[1]));
+                    }
+#pragma unroll
+                for (int i = 0; i < QB; ++i)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        const auto w32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(top[i][b]), __float_as_uint(top[i][b]), false, false);
+                        top[i][b] = fmaxf(__uint_as_float(w32[0]), __uint_as_float(w32[1]));
+                    }
                 uint32_t raises = 0;                           // uniform
-                // plain tiles: c * scale2 - M in one instruction (its sign is exact: it is > 0 only if the score is above M)
-                auto block = [&](auto is_plain, int b) __attribute__((always_inline)) {
-                    constexpr bool PLAIN = decltype(is_plain)::value;
-                    float f[QB][4];
-                    bool above = false;
+                float ms[QB][4];
 #pragma unroll
-                    for (int i = 0; i < QB; ++i) {
+                for (int i = 0; i < QB; ++i) {
+                    mb[i][0] = M[i];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) f[i][e] = PLAIN ? __builtin_fmaf(c[i][b][e], scale2, -M[i]) : c[i][b][e] - M[i];
-                        above = above || fmaxf(fmaxf(f[i][0], f[i][1]), fmaxf(f[i][2], f[i][3])) > 0.0f;
-                    }
-                    if (__any(above)) {
-                        raises |= 1u << b;
-#pragma unroll
-                        for (int i = 0; i < QB; ++i) {
-                            float s[4];
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) s[e] = PLAIN ? c[i][b][e] * scale2 : c[i][b][e];
-                            float top = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));       // ... and over lanes +-16, +-32, the query's other keys
-                            const auto w16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(top), __float_as_uint(top), false, false);
-                            top = fmaxf(__uint_as_float(w16[0]), __uint_as_float(w16[1]));
-                            const auto w32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(top), __float_as_uint(top), false, false);
-                            const float Mn = fmaxf(M[i], fmaxf(__uint_as_float(w32[0]), __uint_as_float(w32[1])));
-                            const float ms = __builtin_amdgcn_exp2f(M[i] - Mn);            // 1 where the maximum stands, 0 for the first keys
-                            if (g == 0) fm_s[((it & 1) * 4 + b) * TQ + 16 * (QB * pw + i) + r16] = pk_factors(ms, ms);
-                            S[i] *= ms;
-                            M[i] = Mn;
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) f[i][e] = s[e] - Mn;
-                        }
-                    }
-#pragma unroll
-                    for (int i = 0; i < QB; ++i) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) f[i][e] = __builtin_amdgcn_exp2f(f[i][e]);
-                        S[i] += (f[i][0] + f[i][1]) + (f[i][2] + f[i][3]);
-                        // (fp_row, fp_flip of the pairs 8 b + 2 g, 8 b + 2 g + 1)
-                        const int col = 16 * (QB * pw + i) + r16;
-                        const uint32_t p0 = pk_factors(f[i][0], f[i][1]), p1 = pk_factors(f[i][2], f[i][3]);
-                        if (TQ >= 64) {
-                            uint32_t * to = fpw + (8 * b + 2 * g) * TQ + (col ^ (g << 4));
-                            to[0] = p0; to[TQ] = p1;
-                        } else {
-                            uint32_t * to = fpw + (8 * b + 2 * g) * 32 + (col ^ ((g & 1) << 4));
-                            to[0] = g & 2 ? p1 : p0; to[32] = g & 2 ? p0 : p1;
-                        }
-                    }
-                };
-                if (plain) {
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) block(std::true_type{}, b);
-                } else {
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) block(std::false_type{}, b);
+                    for (int b = 0; b < 4; ++b) { mb[i][b + 1] = fmaxf(mb[i][b], top[i][b]); ms[i][b] = __builtin_amdgcn_exp2f(mb[i][b] - mb[i][b + 1]); }      // 1 where the maximum stands, 0 for the first keys
+                    M[i] = mb[i][4];
                 }
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    bool up = false;
+#pragma unroll
+                    for (int i = 0; i < QB; ++i) up = up || mb[i][b + 1] > mb[i][b];
+                    raises |= __any(up) ? 1u << b : 0u;
+                }
+                char * fw = f_s + (it & 1) * F_TILE;
+#pragma unroll
+                for (int i = 0; i < QB; ++i) {
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) c[i][b][e] = __builtin_amdgcn_exp2f(c[i][b][e] - mb[i][b + 1]);
+                    char * to = fw + (16 * (QB * pw + i) + r16) * P_FPITCH + 8 * g;
+                    uint32_t * tm = fm_s + (it & 1) * 4 * TQ + 16 * (QB * pw + i) + r16;
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        *(u32x2 *)(to + 32 * b) = (u32x2){ pk_factors(c[i][b][0], c[i][b][1]), pk_factors(c[i][b][2], c[i][b][3]) };
+                        tm[b * TQ] = pk_factors(ms[i][b], ms[i][b]);           // (the four lanes of a query store the same)
+                        S[i] = __builtin_fmaf(S[i], ms[i][b], (c[i][b][0] + c[i][b][1]) + (c[i][b][2] + c[i][b][3]));
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                if (LW == 0) load_k(it + 2, knext, LD / 2, LD);
                 if (lane == 0) rm_s[(it & 1) * PW + pw] = raises;
                 if (it + 1 == n_tiles) {
 #pragma unroll
@@ -1432,9 +1498,20 @@ __global__ void __launch_bounds__(256 + 64 * PW, 2) k_fattn_pk_tile(fa_args a) {
                     }
                 }
             }
-            wait_loads();                                      // V of this tile and K of the next are in LDS
+            if (LW == 0 && !busy) load_k(it + 2, knext, 0, LD);
+            if (LW == 0) {
+                wait_loads<RL + LD>();                         // V of this tile is in registers, K of the next in LDS
+                store_v(vr, it);
+            }
+            __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));             // lgkmcnt(0)
+            kbuf = kbuf == 2 ? 0 : kbuf + 1;
+        };
+        for (int it = 0;;) {
+            tile(it, va, vc2); if (++it == n_tiles) break;
+            tile(it, vc2, va); if (++it == n_tiles) break;
         }
-        __syncthreads();
+        __builtin_amdgcn_s_barrier();
+        wait_loads<0>();                                       // (the surplus loads still write LDS)
         return;
     }
 
@@ -1452,53 +1529,58 @@ __global__ void __launch_bounds__(256 + 64 * PW, 2) k_fattn_pk_tile(fa_args a) {
     const int fcol = WQ * wave + QL * qd;
     const bool busy = n0 + WQ * wave < a.N;
 
+    // a group's V values (a read per d pair and four keys) and factors (a read per query); the next group is read while this one
+    // is walked, the last one of a tile is walked behind the next tile's barrier.  (Keys past the end carry factors of exactly 0 and
+    // the last key's finite V values: walking them changes nothing, so groups are walked whole.)
+    struct pgroup { u32x4 v[P][2]; u32x4 f[QL]; };
+    const char * const vrow = v_s + (P * ds) * (P_VPITCH * 4), * const frow = f_s + fcol * P_FPITCH;
+    const int vsw = (P * ds) >> 4;
+    auto gload = [&](pgroup & gr, int buf, auto u) __attribute__((always_inline)) {       // u: group of the tile
+        constexpr int U = decltype(u)::value;
+        const char * v0 = vrow + buf * V_TILE + 16 * vsw, * v1 = vrow + buf * V_TILE + 16 * (1 ^ vsw), * fr = frow + buf * F_TILE;
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            gr.v[j][0] = *(const u32x4 *)(v0 + j * (P_VPITCH * 4) + 32 * U);
+            gr.v[j][1] = *(const u32x4 *)(v1 + j * (P_VPITCH * 4) + 32 * U);
+        }
+#pragma unroll
+        for (int q = 0; q < QL; ++q) gr.f[q] = *(const u32x4 *)(fr + q * P_FPITCH + 16 * U);
+    };
+    auto walk = [&](const pgroup & gr) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < KG; ++k) {
+            const uint32_t v0 = gr.v[0][k / 4][k % 4], v1 = gr.v[1][k / 4][k % 4];
+            if constexpr (QL == 1) { if (k % 2 == 0) pk_key<0>(acc[0], v0, v1, gr.f[0][k / 2]); else pk_key<1>(acc[0], v0, v1, gr.f[0][k / 2]); }
+            else {
+#pragma unroll
+                for (int q = 0; q < QL; q += 2) {
+                    if (k % 2 == 0) pk_key<0>(acc[q], acc[q + 1], v0, v1, gr.f[q][k / 2], gr.f[q + 1][k / 2]);
+                    else            pk_key<1>(acc[q], acc[q + 1], v0, v1, gr.f[q][k / 2], gr.f[q + 1][k / 2]);
+                }
+            }
+        }
+    };
+    auto arrived = [&](const pgroup & gr) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);                     // (behind the steps in front of it: the scheduler would lift the wait above them)
+        asm volatile("" :: "v"(gr.f[QL - 1]), "v"(gr.v[P - 1][1]));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    pgroup ga, gb;
+    bool pending = false;                                      // gb holds the last group of the tile before
     for (int it = 0; it <= n_tiles; ++it) {
-        __syncthreads();                                       // tile boundary: tile it - 1 has its factors and its V rows
+        // tile boundary: tile it - 1 has its factors and its V rows.  (What this wavefront read of the tile before has arrived.)
+        __syncthreads();
         if (it == 0 || !busy) continue;
         const int64_t key0 = (int64_t)(it - 1) * P_KV;
         const int nk = (int)(a.KV - key0 < P_KV ? a.KV - key0 : P_KV);               // uniform
         const int buf = (it - 1) & 1;
-        // every address of a group in a register of its own, so that no two reads look like neighbours to the compiler
-        const char * vb[KG];
-        const char * fb[8];                                    // (fp_row and fp_flip repeat every eight pairs)
-#pragma unroll
-        for (int j = 0; j < KG; ++j) {
-            uint32_t at = (uint32_t)(buf * (P_KV * FA_D * 2) + 2 * DL * ds + 128 * j);
-            asm volatile("" : "+v"(at));
-            vb[j] = v_s + at;
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            uint32_t at = (uint32_t)(buf * FP_TILE + fp_row<TQ>(j) + (fcol ^ fp_flip<TQ>(j))) * 4;
-            if (QL == 2) asm volatile("" : "+v"(at));          // (16-byte reads are not merged)
-            fb[j] = (const char *) fp_s + at;
-        }
         const uint32_t * fmb = fm_s + buf * 4 * TQ + fcol;
-        const uint32_t raises = __builtin_amdgcn_readfirstlane(rm_s[buf * PW + PW * wave / 4]);
-        // a group's factors (a read per pair of keys) and V values (a read per key); the next group is read while this one is
-        // walked.  (Keys past the end carry factors of exactly 0 and the last key's finite V values: walking them changes nothing,
-        // so groups are walked whole.)
-        struct pgroup { uint32_t f[KG / 2][QL]; uint32_t v[KG][P]; };
-        auto gload = [&](pgroup & gr, auto u) __attribute__((always_inline)) {       // u: group of the tile
-            constexpr int k0 = KG * decltype(u)::value;
-#pragma unroll
-            for (int j = 0; j < KG / 2; ++j) {
-                const int pair = k0 / 2 + j;
-                const char * row = fb[pair % 8] + pair / 8 * (8 * TQ * 4);
-                if constexpr (QL == 4) { const u32x4 t = *(const u32x4 *) row; gr.f[j][0] = t.x; gr.f[j][1] = t.y; gr.f[j][2] = t.z; gr.f[j][3] = t.w; }
-                else                   { const u32x2 t = *(const u32x2 *) row; gr.f[j][0] = t.x; gr.f[j][1] = t.y; }
-            }
-#pragma unroll
-            for (int j = 0; j < KG; ++j) {
-                const u32x2 t = *(const u32x2 *)(vb[j] + k0 * 128);
-                gr.v[j][0] = t.x; gr.v[j][1] = t.y;
-            }
-        };
-        auto key = [&](auto sel, pgroup & gr, int k) __attribute__((always_inline)) {
-#pragma unroll
-            for (int q = 0; q < QL; q += 2) pk_key<P, decltype(sel)::value>(acc[q], acc[q + 1], gr.v[k], gr.f[k / 2][q], gr.f[k / 2][q + 1]);
-        };
-        using first = std::integral_constant<int, 0>; using second = std::integral_constant<int, 1>;
+        const uint32_t raise_v = rm_s[buf * PW + PW * wave / 4];
+        gload(ga, buf, std::integral_constant<int, 0>{});
+        __builtin_amdgcn_sched_barrier(0);
+        if (pending) walk(gb);
+        pending = false;
+        const uint32_t raises = __builtin_amdgcn_readfirstlane(raise_v);
         // acc = f16(acc * ms) in front of block b
         auto rescale = [&](int b) __attribute__((always_inline)) {
             uint32_t m[QL];
@@ -1509,33 +1591,25 @@ __global__ void __launch_bounds__(256 + 64 * PW, 2) k_fattn_pk_tile(fa_args a) {
 #pragma unroll
                 for (int j = 0; j < P; ++j) pk_scale(acc[q][j], m[q]);
         };
-        auto walk = [&](pgroup & gr) __attribute__((always_inline)) {
-#pragma unroll
-            for (int k = 0; k < KG; k += 2) { key(first{}, gr, k); key(second{}, gr, k + 1); }
-        };
-        auto arrived = [&](const pgroup & gr) __attribute__((always_inline)) {
-            __builtin_amdgcn_sched_barrier(0);                 // (behind the steps in front of it: the scheduler would lift the wait above them)
-            asm volatile("" :: "v"(gr.f[KG / 2 - 1][QL - 1]), "v"(gr.v[KG - 1][P - 1]));
-            __builtin_amdgcn_sched_barrier(0);
-        };
-        pgroup ga, gb;
-        gload(ga, first{});
-        // two groups; W = 2 KG keys from u2 W on
-        auto run = [&](auto u2) __attribute__((always_inline)) {
-            constexpr int u = decltype(u2)::value, W = 2 * KG;
+        // block b of 16 keys: two groups
+        auto run = [&](auto bb) __attribute__((always_inline)) {
+            constexpr int b = decltype(bb)::value;
             arrived(ga);
-            gload(gb, std::integral_constant<int, 2 * u + 1>{});
+            gload(gb, buf, std::integral_constant<int, 2 * b + 1>{});
             __builtin_amdgcn_sched_barrier(0);
-            if (u * W % 16 == 0 && (raises & (1u << (u * W / 16)))) rescale(u * W / 16);
+            if (raises & (1u << b)) rescale(b);
             walk(ga);
             arrived(gb);
-            gload(ga, std::integral_constant<int, (u + 1) * W < P_KV ? 2 * u + 2 : 0>{});      // (behind the last group: any readable group, nobody walks it)
-            __builtin_amdgcn_sched_barrier(0);
-            walk(gb);
+            if constexpr (b < 3) {
+                gload(ga, buf, std::integral_constant<int, 2 * b + 2>{});
+                __builtin_amdgcn_sched_barrier(0);
+                walk(gb);
+            } else pending = true;
         };
-        auto runs = [&](auto... us) __attribute__((always_inline)) { (((int) decltype(us)::value * 2 * KG < nk ? run(us) : (void) 0), ...); };
-        runs(first{}, second{}, std::integral_constant<int, 2>{}, std::integral_constant<int, 3>{});
+        auto runs = [&](auto... bs) __attribute__((always_inline)) { (((int) decltype(bs)::value * 16 < nk ? run(bs) : (void) 0), ...); };
+        runs(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{}, std::integral_constant<int, 2>{}, std::integral_constant<int, 3>{});
     }
+    if (pending) walk(gb);
     if (!busy) return;
 
     // ---- results: a lane holds DL d of QL queries
@@ -1803,10 +1877,10 @@ extern "C" size_t mi355x_flash_attn_ext_workspace_size(const mi355x_tensor * q, 
     return 0;
 }
 
-template <int QL, int PW>
-static void launch_pk_tile(const fa_args & a, dim3 grid, hipStream_t st) {
-    grid.x = (unsigned)((a.N + p_queries<QL>() - 1) / p_queries<QL>());
-    k_fattn_pk_tile<QL, PW><<<grid, 256 + 64 * PW, p_lds_bytes<QL>(), st>>>(a);
+template <int QL, int PW, int LW>
+static void launch_pk_tile(const fa_args & a, hipStream_t st) {
+    const int64_t total = (a.N + p_queries<QL>() - 1) / p_queries<QL>() * a.H * a.ne3;
+    k_fattn_pk_tile<QL, PW, LW><<<(unsigned) total, 256 + 64 * (PW + LW), p_lds_bytes<QL>(), st>>>(a);
 }
 
 static int flash_attn_ext(const mi355x_tensor * q, const mi355x_tensor * k, const mi355x_tensor * v,
@@ -1895,10 +1969,17 @@ static int flash_attn_ext(const mi355x_tensor * q, const mi355x_tensor * k, cons
             if (gx > 0x7fffffff) return MI355X_ERR_UNSUPPORTED;
             dim3 grid((unsigned) gx, (unsigned) H, (unsigned) q->ne[3]);
             if (mode == MI355X_FA_F16_PK) {
-                // 32 queries to the workgroup while every workgroup has a CU of its own that way, 64 from there on: two workgroups of
-                // 32 on a CU take longer than one of 64 (58 to 49 us at N 1500 x KV 1536 x 6 heads)
-                if ((N + 31) / 32 * H * q->ne[3] <= 256) launch_pk_tile<2, 2>(a, grid, st);
-                else                                     launch_pk_tile<4, 4>(a, grid, st);
+                // The fewest queries to the workgroup with which every workgroup still has a CU of its own.  Above 256 workgroups of 64: 32 to
+                // the workgroup as long as three of those on each CU are all there are (N 1500 x KV 1536 x 12 heads 69 us, with 64
+                // 75), else 64, whose producers load for themselves: with two workgroups to a CU there is always somebody to
+                // issue (20 heads 76 us, with loaders 83).
+                const int64_t heads = H * q->ne[3], t16 = (N + 15) / 16 * heads, t32 = (N + 31) / 32 * heads, t64 = gx * heads;
+                if (t16 > 0x7fffffff) return MI355X_ERR_UNSUPPORTED;
+                if      (t16 <= 256) launch_pk_tile<1, 1, 2>(a, st);
+                else if (t32 <= 256) launch_pk_tile<2, 2, 2>(a, st);
+                else if (t64 <= 256) launch_pk_tile<4, 4, 2>(a, st);
+                else if (t32 <= 768) launch_pk_tile<2, 2, 2>(a, st);
+                else                 launch_pk_tile<4, 4, 0>(a, st);
                 break;
             }
             static std::atomic<bool> configured[64];            // per device: the kernel asks for more LDS than a launch gets by default
