@@ -403,6 +403,23 @@ def test_mul_mat_direct_load_tiles(pkg, oracle, gpu, own_numbers, k, m, n):
     assert np.all(run(pkg.EPI_GELU | pkg.EPI_EMIT_F16 | pkg.EPI_IMAGE_ONLY, d_i) == 7.0) and np.array_equal(gpu.down(d_i, np.uint16), gpu.down(d_h, np.uint16))
 
 
+@pytest.mark.parametrize("m,n,heads", [(385, 449, 12), (1500, 1500, 12), (1503, 17, 22), (64, 577, 64), (257, 640, 11)])
+def test_mul_mat_attention_scores(pkg, oracle, gpu, own_numbers, m, n, heads):
+    # K = 64 over heads that are columns of wider rows: runs of four and of six row tiles, whole and ragged; scaled, with a residual, f16 columns
+    lib, d = pkg.kernels(), 64 * heads
+    k16, x, res = rnd((m, d)).astype(np.float16), rnd((n, d)), rnd((heads, n, m))
+    base = np.einsum("nhe,mhe->hnm", x.astype(np.float16).astype(np.float32).reshape(n, heads, 64), k16.astype(np.float32).reshape(m, heads, 64), optimize=True)
+    d_k, d_x, d_x16, d_r = gpu.up(k16.view(np.int16)), gpu.up(x), gpu.up(x.astype(np.float16).view(np.int16)), gpu.up(res)
+    tk = pkg.tensor(d_k, pkg.F16, [64, m, heads], [2, 2 * d, 128])
+    tx, tx16 = pkg.tensor(d_x, pkg.F32, [64, n, heads], [4, 4 * d, 256]), pkg.tensor(d_x16, pkg.F16, [64, n, heads], [2, 2 * d, 128])
+    ws = torch.zeros(lib.mi355x_mul_mat_workspace_size(tk, tx), dtype=torch.uint8, device=gpu.dev)
+    for t, flags, want in [(tx, 0, base), (tx16, pkg.EPI_SCALE, 0.125 * base), (tx, pkg.EPI_SCALE | pkg.EPI_RESIDUAL, 0.125 * base + res)]:
+        d_y = torch.full((heads * n + 1, m), 7.0, dtype=torch.float32, device=gpu.dev)
+        epi = pkg.Epilogue(flags, 0.125, None, d_r.data_ptr(), None)
+        pkg.check(lib.mi355x_mul_mat(tk, t, pkg.tensor(d_y[:-1].view(heads, n, m), pkg.F32), C.byref(epi), ws.data_ptr(), ws.numel(), gpu.stream))
+        assert oracle.nmse(gpu.down(d_y[:-1]).reshape(heads, n, m), want) <= 1e-11 and torch.all(d_y[-1] == 7.0)
+
+
 # rows that are not 16-byte aligned, any K (the transposed V of a window of 1500, 37 or 1501 positions), one or two columns
 @pytest.mark.parametrize("k,m,n,batch", [(1500, 64, 300, 3), (37, 64, 37, 2), (1501, 64, 5, 2), (1500, 64, 1, 4), (64, 1500, 2, 2), (512, 1000, 1, 1), (1024, 1283, 2, 1), (1280, 5003, 2, 1), (2048, 48, 1, 1), (3, 5, 40, 1), (68, 64, 64, 12), (132, 65, 17, 1), (191, 63, 400, 20), (321, 130, 1500, 8), (1500, 64, 1500, 12)])
 def test_mul_mat_f16_keeps_f32_activations(pkg, oracle, gpu, own_numbers, k, m, n, batch):

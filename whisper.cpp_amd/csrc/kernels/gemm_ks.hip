@@ -32,6 +32,33 @@ typedef half_t ks_h4 __attribute__((ext_vector_type(4), aligned(2)));
 
 template <int MT, int NT, int KW> constexpr size_t ks_red_bytes() { return (size_t) KW * 16 * NT * (16 * MT + 4) * sizeof(float); }
 
+// the epilogue of four consecutive m of a column, and their way out (EMIT: a column past N or rows past M only pass through)
+template <bool EMIT>
+__device__ __forceinline__ void ks_store4(float4_t & v, int64_t m, int64_t n, const mm_args & a, char * db, const epi_args & epi, int64_t batch_off, int64_t d_nb1) {
+    const bool row = n < a.N;
+    if (m + 3 < a.M) {
+        const int64_t nc = row ? n : a.N - 1;
+        if (epi.flags & MI355X_EPI_BIAS) v += *(const ks_f4 *)(epi.bias + m);
+        if (epi.flags & MI355X_EPI_BIAS_COL) v += epi.bias[nc];
+        if (epi.flags & MI355X_EPI_GELU) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = gelu_f32(v[e], epi.gelu);
+        }
+        if (epi.flags & MI355X_EPI_SCALE) v *= epi.scale;
+        if (epi.flags & MI355X_EPI_RESIDUAL) v += *(const ks_f4 *)(epi.residual + batch_off + nc * d_nb1 + m * 4);
+        if (row) {
+            if (epi.flags & MI355X_EPI_OUT_F16) *(ks_h4 *)(db + n * d_nb1 + m * 2) = (ks_h4){ (half_t) v[0], (half_t) v[1], (half_t) v[2], (half_t) v[3] };
+            else if (!EMIT || !(epi.flags & MI355X_EPI_IMAGE_ONLY)) *(ks_f4 *)(db + n * d_nb1 + m * 4) = v;
+        }
+    } else if (row && m < a.M) {
+        for (int e = 0; e < 4 && m + e < a.M; ++e) {
+            const float y = apply_epilogue(v[e], epi, m + e, n, batch_off + n * d_nb1 + (m + e) * 4);
+            if (epi.flags & MI355X_EPI_OUT_F16) *(half_t *)(db + n * d_nb1 + (m + e) * 2) = (half_t) y;
+            else                                *(float  *)(db + n * d_nb1 + (m + e) * 4) = y;
+        }
+    }
+}
+
 // The partial tiles of the KW wavefronts meet in `red` ([KW][16 NT][LD] floats, free when every wavefront is past its loop) and
 // leave through the epilogue.  EMIT: MI355X_EPI_EMIT_F16 (a block of 32 m is 8 consecutive lanes).
 template <int MT, int NT, int KW, bool EMIT, int H = 1>
@@ -62,27 +89,7 @@ __device__ __forceinline__ void ks_finish(float4_t (&acc)[MT][NT], float * red, 
         const int64_t n = n0 + nl, m = m0 + ml;
         const bool row = n < a.N, whole = m + 3 < a.M;
         if (!EMIT && (!row || m >= a.M)) continue;
-        const int64_t nc = row ? n : a.N - 1;
-        if (whole) {
-            if (epi.flags & MI355X_EPI_BIAS) v += *(const ks_f4 *)(epi.bias + m);
-            if (epi.flags & MI355X_EPI_BIAS_COL) v += epi.bias[nc];
-            if (epi.flags & MI355X_EPI_GELU) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = gelu_f32(v[e], epi.gelu);
-            }
-            if (epi.flags & MI355X_EPI_SCALE) v *= epi.scale;
-            if (epi.flags & MI355X_EPI_RESIDUAL) v += *(const ks_f4 *)(epi.residual + batch_off + nc * d_nb1 + m * 4);
-            if (row) {
-                if (epi.flags & MI355X_EPI_OUT_F16) *(ks_h4 *)(db + n * d_nb1 + m * 2) = (ks_h4){ (half_t) v[0], (half_t) v[1], (half_t) v[2], (half_t) v[3] };
-                else if (!EMIT || !(epi.flags & MI355X_EPI_IMAGE_ONLY)) *(ks_f4 *)(db + n * d_nb1 + m * 4) = v;
-            }
-        } else if (row && m < a.M) {
-            for (int e = 0; e < 4 && m + e < a.M; ++e) {
-                const float y = apply_epilogue(v[e], epi, m + e, n, batch_off + n * d_nb1 + (m + e) * 4);
-                if (epi.flags & MI355X_EPI_OUT_F16) *(half_t *)(db + n * d_nb1 + (m + e) * 2) = (half_t) y;
-                else                                *(float  *)(db + n * d_nb1 + (m + e) * 4) = y;
-            }
-        }
+        ks_store4<EMIT>(v, m, n, a, db, epi, batch_off, d_nb1);
         if (EMIT) {                                     // M is a multiple of 32: a block of 8 lanes is inside dst or outside
             float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
             amax = lanes_max<8>(amax);
@@ -209,6 +216,100 @@ __device__ __forceinline__ void gemm_ks_tile(const mm_args & a, const char * wb,
     for (; t < n_mine; ++t) { mma(wave + (int64_t) t * KW, buf); buf = buf + 1 == D ? 0 : buf + 1; }
     __syncthreads();                                    // (the partial tiles take the buffers' place)
     ks_finish<MT, NT, KW, EMIT, H>(acc, (float *) smem, a, db, epi, batch_off, d_nb1, m0, n0);
+}
+
+// k_gemm_k64: K = 64 (attention scores), more than a few tiles: the product is nothing beside the store of its result.  A wavefront
+// keeps its 16 columns as fragments and walks `run` tiles of 64 rows, which its workgroup of four brings to LDS two tiles ahead;
+// the results of a tile turn over in 4 KB of LDS of the wavefront's own and leave as 256-byte pieces of dst rows, behind which
+// nobody waits: the wait for a tile counts the stores of the two tiles before it among what may still be on its way.
+// 1500 x 1500, f32 columns, 12 heads: 25.5 us (a fill of the 108 MB: 18), with a workgroup of one wavefront to a 64 x 64 tile 30.5 — load,
+// product, store, one behind the other, six to a CU; 20 heads 39.7; 44, 6 heads 15.5; 19.5, 227 columns of 20 heads 9.9; 13.2.
+template <int XM>
+__global__ void __launch_bounds__(256) k_gemm_k64(mm_args a, half_t * x16, int64_t x16_slice, int run) {
+    constexpr int LD = 68;
+    extern __shared__ __attribute__((aligned(16))) char smem[];     // [3][64 rows of 128 bytes], then [4][16 * LD] floats
+    const mm_slice_ptrs z = mm_slice(a, blockIdx.z);
+    char * db = a.d + z.d_off;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, q = lane >> 4;
+    const int64_t m0 = (int64_t) blockIdx.x * (64 * run), n0 = (int64_t) blockIdx.y * 64 + 16 * wave;
+    const int tiles = (int) min((int64_t) run, (a.M - m0 + 63) / 64);
+
+    // rows of a tile: the 1 KB loads 2 wave and 2 wave + 1 (layout of gemm_ks_tile)
+    auto load = [&](int t, int buf) __attribute__((always_inline)) {
+        t = min(t, tiles - 1);                              // (past the last tile: that one again, so that the count of what is on its way holds)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int line = 4 * (2 * wave + i) + q, row = 2 * line + ((lane >> 3) & 1);
+            const int64_t m = min(m0 + 64 * t + row, a.M - 1);
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(z.w + m * a.w_nb1 + ((lane & 7) ^ (line & 7)) * 16),
+                                             (__attribute__((address_space(3))) void *)(smem + buf * 8192 + (2 * wave + i) * 1024), 16, 0, 0);
+        }
+    };
+    half8_t xv[2];
+    const int64_t n = n0 + r16;
+    const char * xp = z.x + min(n, a.N - 1) * a.x_nb1;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        if constexpr (XM == KS_X_F16) xv[s] = *(const half8_t *)(xp + (32 * s + 8 * q) * 2);
+        else {
+            const float4_t lo = *(const float4_t *)(xp + (32 * s + 8 * q) * 4), hi = *(const float4_t *)(xp + (32 * s + 8 * q) * 4 + 16);
+            xv[s] = (half8_t){ (half_t) lo.x, (half_t) lo.y, (half_t) lo.z, (half_t) lo.w, (half_t) hi.x, (half_t) hi.y, (half_t) hi.z, (half_t) hi.w };
+        }
+    }
+    if (XM == KS_X_CVT && x16 && blockIdx.x == 0 && n < a.N) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) *(half8_t *)(x16 + blockIdx.z * x16_slice + n * KS_UNIT + 32 * s + 8 * q) = xv[s];
+    }
+    ks_wait_vmcnt<0>();
+    load(0, 0);
+    load(1, 1);
+
+    // four stores to a tile, no loads: what the counted waits assume (uniform)
+    const bool counted = n0 + 16 <= a.N && !(a.e.flags & ~MI355X_EPI_SCALE);
+    const float scale = a.e.flags & MI355X_EPI_SCALE ? a.e.scale : 1.0f;
+    const int frow = (r16 >> 1) * 256 + (r16 & 1) * 128, fsw = (r16 >> 1) & 7;
+    float * mine = (float *)(smem + 3 * 8192) + wave * (16 * LD);
+    int buf = 0;
+    for (int t = 0; t < tiles; ++t) {
+        if (!counted)    ks_wait_vmcnt<0>();
+        else if (t == 0) ks_wait_vmcnt<2>();
+        else if (t == 1) ks_wait_vmcnt<2 + 4>();
+        else             ks_wait_vmcnt<4 + 2 + 4>();
+        __builtin_amdgcn_s_barrier();                       // everybody's pieces of tile t are in LDS; the buffer of tile t - 1 is free
+        __builtin_amdgcn_sched_barrier(0);
+        const char * ws = smem + buf * 8192;
+        half8_t wv[2][4];
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) wv[s][i] = *(const half8_t *)(ws + i * 2048 + frow + ((4 * s + q) ^ fsw) * 16);
+        __builtin_amdgcn_sched_barrier(0);
+        load(t + 2, buf == 0 ? 2 : buf - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        float4_t acc[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = (float4_t){ 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[s][i], xv[s], acc[i], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *(float4_t *)(mine + r16 * LD + 16 * i + 4 * q) = acc[i];
+        const int64_t mt = m0 + 64 * t + 4 * r16;
+        if (counted && m0 + 64 * t + 64 <= a.M) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) *(ks_f4 *)(db + (n0 + 4 * k + q) * a.d_nb1 + mt * 4) = *(const float4_t *)(mine + (4 * k + q) * LD + 4 * r16) * scale;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float4_t v = *(const float4_t *)(mine + (4 * k + q) * LD + 4 * r16);
+                if (n0 + 4 * k + q < a.N && mt < a.M) ks_store4<false>(v, mt, n0 + 4 * k + q, a, db, a.e, z.d_off, a.d_nb1);
+            }
+        }
+        buf = buf == 2 ? 0 : buf + 1;
+    }
+    ks_wait_vmcnt<0>();                                     // (the surplus loads still write LDS)
 }
 
 template <int MT, int NT, int KW, int XM>
@@ -559,6 +660,15 @@ static int launch_kd_t(const mm_args & a, hipStream_t st) {
     k_gemm_kd<MT, NT, KW, XM><<<grid, 64 * KW, lds, st>>>(a);
     return launch_status();
 }
+template <int XM>
+static int launch_k64(const mm_args & a, half_t * x16, int64_t slice, hipStream_t st) {
+    const int64_t t = (a.M + 63) / 64, tn = (a.N + 63) / 64, nb = a.ne12 * a.ne13;
+    const int run = (t + 5) / 6 * tn * nb >= 512 ? 6 : 4;           // (700 x 700, 12 heads: 11.4 us with 6, 9.9 with 4)
+    const int64_t tm = (t + run - 1) / run;
+    if (tm > 0x7fffffff || tn > 65535 || nb > 65535) return MI355X_ERR_UNSUPPORTED;
+    k_gemm_k64<XM><<<dim3((unsigned) tm, (unsigned) tn, (unsigned) nb), 256, 3 * 8192 + 4 * 16 * 68 * 4, st>>>(a, x16, slice, run);
+    return launch_status();
+}
 template <int XM, bool EMIT>
 static int launch_ks_x(const mm_args & a, const ks_shape & s, half_t * x16, int64_t slice, hipStream_t st) {
     const bool few = a.N <= 8;
@@ -569,7 +679,10 @@ static int launch_ks_x(const mm_args & a, const ks_shape & s, half_t * x16, int6
     KS_HALVES(4, 2) KS_HALVES(8, 2)
 #undef KS_HALVES
     KS_CASE(1, 1, 1, 1) KS_CASE(1, 1, 4, 2) KS_CASE(1, 1, 8, 2) KS_CASE(2, 1, 4, 2)
-    if constexpr (XM != KS_X_F32) { KS_CASE(2, 2, 1, 1) KS_CASE(4, 4, 1, 1) }
+    if constexpr (XM != KS_X_F32) {
+        KS_CASE(2, 2, 1, 1)
+        if constexpr (!EMIT) if (s.kw == 1 && s.mt == 4) return launch_k64<XM>(a, x16, slice, st);
+    }
     if constexpr (XM == KS_X_F16) { KS_CASE(2, 2, 4, 2) KS_CASE(4, 4, 4, 2) }
 #undef KS_CASE
     return MI355X_ERR_UNSUPPORTED;
@@ -586,7 +699,7 @@ static int launch_ks_x(const mm_args & a, const ks_shape & s, half_t * x16, int6
 //     that is under half a round as well (768 x 768, 27 columns: 3.7; 4.4; 6.8);
 //   more than a round of 64 x 64 tiles: the 128-wide tiles, which move half the bytes per product (M = 768, N = 1500: 8.9;
 //     10.7 here), except with up to 32 columns, where they are mostly padding (51865 x 768, 27 columns: 21.7; 23.9).
-// K = 64 (attention scores) is one unit: no split, one wavefront to a tile, and what counts is the store of the result.
+// K = 64 (attention scores) is one unit: no split, one wavefront to a tile; from 512 64 x 64 tiles on k_gemm_k64, for the store of the result.
 static bool ks_tiles(int64_t M, int64_t N, int64_t K, int64_t nb, bool emit, ks_shape & s) {
     const int64_t t44 = (M + 63) / 64 * ((N + 63) / 64) * nb, t22 = (M + 31) / 32 * ((N + 31) / 32) * nb;
     s.kw = 4; s.d = 2; s.h = 1;
