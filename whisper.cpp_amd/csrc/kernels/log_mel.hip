@@ -17,8 +17,11 @@
 // between them (4 and 5 are coprime: Good's mapping).  The pair's spectra come apart through bin 400 - k, which lane 20 - c
 // holds: ten values per lane through LDS.  The three pairs of a wavefront need no barrier.  Then a thread per (frame, band)
 // sums the band's range of nonzero filter weights over the powers in LDS.
-// What bounds it: f64 issue.  The transform by direct sums took 0.32 M multiply-adds a frame and was 4.2 ms for an hour of
-// audio and 53 us for 3 s; this form takes 8 k operations a frame and a memory pass costs as much as they do.
+// What bounds it: f64 issue and, between the steps of a round, LDS and load latency, so three workgroups share a CU (168 registers,
+// 52 KB of LDS), a sample that both frames of a pair want is loaded once, and the filter weights that are not zero lie in LDS
+// (read from memory one by one they were a third of the time).  An hour of audio, 80 bands, both launches: 376 us (600 with the
+// weights in memory and two workgroups to a CU; by direct sums, 0.32 M multiply-adds a frame instead of 8 k operations, 4.2 ms);
+// 128 bands 520; 3 s 18 us, nearly all of it the latency of one round and of the launches.
 #include "common.h"
 
 #define MEL_NFFT   400
@@ -31,6 +34,7 @@
 #define MEL_MAX_BANDS 128
 #define MEL_GROUPS 768          // workgroups at most: three to a CU; each walks a run of consecutive rounds
 #define MEL_LOG_BITS 6
+#define MEL_WEIGHTS 224         // nonzero filter weights in LDS for a wavefront's share of the bands (a bin belongs to two of the usual triangles: about 100)
 
 typedef double double2_t __attribute__((ext_vector_type(2)));
 
@@ -91,15 +95,16 @@ __device__ __forceinline__ double mel_log10(double x, const double2_t * __restri
 // the values of one lane visible to the other lanes of its wavefront (LDS accesses of a wavefront are carried out in order)
 __device__ __forceinline__ void wave_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); }
 
-__global__ void __launch_bounds__(256) k_log_mel_frames(const float * __restrict__ samples, int64_t n_samples, const float * __restrict__ filters,
+__global__ void __launch_bounds__(256, 3) k_log_mel_frames(const float * __restrict__ samples, int64_t n_samples, const float * __restrict__ filters,
                                                        int n_mel, int64_t n_frames, int64_t n_len, int64_t rounds_per_group,
                                                        float * __restrict__ mel, float * __restrict__ maxima) {
     __shared__ __attribute__((aligned(16))) double    xch[MEL_PAIRS * MEL_PAIR_LD];
     __shared__ __attribute__((aligned(16))) double2_t cs[MEL_NFFT];                // (cos, -sin)(2 pi i / 400)
     __shared__ __attribute__((aligned(16))) double2_t lt[1 << MEL_LOG_BITS];
-    __shared__ int16_t range[MEL_MAX_BANDS][2];                                    // a band's nonzero weights: first, one past the last
+    __shared__ int16_t range[MEL_MAX_BANDS][3];                                    // a band's nonzero weights: first, one past the last, place in weights (or -1)
+    __shared__ float weights[4 * MEL_WEIGHTS];
     __shared__ float wmax[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     for (int i = tid; i < MEL_NFFT; i += 256) {
         double s, c;
@@ -111,7 +116,9 @@ __global__ void __launch_bounds__(256) k_log_mel_frames(const float * __restrict
         lt[tid] = (double2_t){ inv, -log10(inv) };
     }
     // Mel filters are triangles over a few bins, and a zero weight adds nothing: each wavefront looks through every fourth band,
-    // eight bands' rows requested at a time.
+    // eight bands' rows requested at a time, and puts the nonzero ranges side by side in LDS (one that does not fit stays in memory;
+    // all of them for a single round: 3 s of audio 18.1 us, 18.8 with the weights moved first).
+    int used = 0;                                       // of this wavefront's share of weights
     for (int j0 = wave; j0 < n_mel; j0 += 32) {
         float w[8][4];
 #pragma unroll
@@ -128,7 +135,15 @@ __global__ void __launch_bounds__(256) k_log_mel_frames(const float * __restrict
                 const uint64_t any = __ballot(w[b][i] != 0.0f && lane + 64 * i < MEL_BINS);
                 if (any) { first = min(first, 64 * i + (int) __builtin_ctzll(any)); last = 64 * i + 64 - (int) __builtin_clzll(any); }
             }
-            if (lane == 0 && j0 + 4 * b < n_mel) { range[j0 + 4 * b][0] = (int16_t) min(first, last); range[j0 + 4 * b][1] = (int16_t) last; }
+            first = min(first, last);
+            if (j0 + 4 * b >= n_mel) break;
+            const int at = rounds_per_group > 1 && used + last - first <= MEL_WEIGHTS ? wave * MEL_WEIGHTS + used : -1;
+            if (lane == 0) { range[j0 + 4 * b][0] = (int16_t) first; range[j0 + 4 * b][1] = (int16_t) last; range[j0 + 4 * b][2] = (int16_t) at; }
+            if (at >= 0) {
+                used += last - first;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) { const int k = lane + 64 * i; if (k >= first && k < last) weights[at + k - first] = w[b][i]; }
+            }
         }
     }
     __syncthreads();
@@ -146,11 +161,11 @@ __global__ void __launch_bounds__(256) k_log_mel_frames(const float * __restrict
         {
             // sample n = t + 20 j of frames A = i0 + 2 pair and A + 1; position in the signal: reflected head, the samples, zeros
             const int64_t p0 = (i0 + 2 * pair) * MEL_HOP + t - MEL_NFFT / 2;
-            float xa[20], xb[20];
+            float x[28];                                // (frame A + 1 begins at A's sample 160: j = 8)
             if (i0 * MEL_HOP >= MEL_NFFT / 2 && (i0 + MEL_FRAMES - 1) * MEL_HOP + MEL_NFFT / 2 <= n_samples) {
                 const float * sp = samples + p0;
 #pragma unroll
-                for (int j = 0; j < 20; ++j) { xa[j] = sp[20 * j]; xb[j] = sp[20 * j + MEL_HOP]; }
+                for (int j = 0; j < 28; ++j) x[j] = sp[20 * j];
             } else {
                 auto at = [&](int64_t p) __attribute__((always_inline)) {
                     int64_t i = p < 0 ? -p : p;
@@ -159,17 +174,21 @@ __global__ void __launch_bounds__(256) k_log_mel_frames(const float * __restrict
                     return p < n_samples ? x : 0.0f;
                 };
 #pragma unroll
-                for (int j = 0; j < 20; ++j) { xa[j] = at(p0 + 20 * j); xb[j] = at(p0 + 20 * j + MEL_HOP); }
+                for (int j = 0; j < 28; ++j) x[j] = at(p0 + 20 * j);
             }
 #pragma unroll
             for (int j = 0; j < 20; ++j) {
                 const double w = 0.5 * (1.0 - cs[t + 20 * j].x);
-                z[j] = { w * (double) xa[j], w * (double) xb[j] };
+                z[j] = { w * (double) x[j], w * (double) x[j + 8] };
             }
         }
+        // (no instruction moves across: twiddles read ahead of their step would cost the registers of a third workgroup on the CU)
+        __builtin_amdgcn_sched_barrier(0);
         dft20(z);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int c = 1; c < 20; ++c) z[c] = cmul(z[c], cs[t * c]);
+        __builtin_amdgcn_sched_barrier(0);
         // 20 x 20 values change lanes, real parts first
 #pragma unroll
         for (int c = 0; c < 20; ++c) my[c * MEL_LD + t] = z[c].re;
@@ -216,8 +235,17 @@ __global__ void __launch_bounds__(256) k_log_mel_frames(const float * __restrict
             const double * pw = xch + (f >> 1) * MEL_PAIR_LD + (f & 1) * MEL_BINS;
             const float * fl = filters + j * MEL_BINS;
             double sum = 0.0;
-            const int last = range[j][1];
-            for (int k = range[j][0]; k < last; ++k) sum = __builtin_fma(pw[k], (double) fl[k], sum);
+            const int first = range[j][0], last = range[j][1], at = range[j][2];
+            auto add = [&](auto * fl) __attribute__((always_inline)) {         // fl[k]: the weight of bin k; four reads of each kind on their way
+                int k = first;
+                for (; k + 3 < last; k += 4) {
+                    const double p0 = pw[k], p1 = pw[k + 1], p2 = pw[k + 2], p3 = pw[k + 3];
+                    const float f0 = fl[k], f1 = fl[k + 1], f2 = fl[k + 2], f3 = fl[k + 3];
+                    sum = __builtin_fma(p3, (double) f3, __builtin_fma(p2, (double) f2, __builtin_fma(p1, (double) f1, __builtin_fma(p0, (double) f0, sum))));
+                }
+                for (; k < last; ++k) sum = __builtin_fma(pw[k], (double) fl[k], sum);
+            };
+            if (at >= 0) add(weights + at - first); else add(filters + j * MEL_BINS);
             if (i0 + f < n_frames) {
                 const float v = (float) mel_log10(sum > 1e-10 ? sum : 1e-10, lt);
                 mel[(int64_t) j * n_len + i0 + f] = (float)(((double) v + 4.0) / 4.0);
