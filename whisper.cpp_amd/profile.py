@@ -35,9 +35,9 @@ DEC_CMD = [str(HARNESS), "bench", "--model", DEC_MODEL, "--what", "decoder", "--
 # kernel symbol (prefix) -> the name the backend's statistics and bench.py use, and the run it is taken from (the decoder
 # command encodes a window first, with the turbo model's four decoder layers in the cross-attention launch)
 BENCH_NAMES = [
-    ("k_fattn_pk_tile", "flash_attn.seq_tile_pk", "encoder"), ("k_fattn_seq_tile", "flash_attn.seq_tile", "encoder"),
+    ("void k_fattn_pk_tile<", "flash_attn.seq_tile_pk", "encoder"), ("k_fattn_seq_tile", "flash_attn.seq_tile", "encoder"),
     ("void k_gemm_f16_dl_group", "mul_mat.gemm_group", "encoder"), ("void k_gemm_f16_dl<", "mul_mat.gemm_q5_0", "encoder"),
-    ("void k_gemm_f16_rs<", "mul_mat.gemm_q5_0", "encoder"), ("void k_norm<5, 1", "norm_affine_emit", "encoder"), ("_Z6k_normILi5ELi1E", "norm_affine_emit", "encoder"),
+    ("k_gemm_f16_rs", "mul_mat.gemm_q5_0", "encoder"), ("void k_norm<5, 1", "norm_affine_emit", "encoder"), ("_Z6k_normILi5ELi1E", "norm_affine_emit", "encoder"),
     ("k_fattn_pk_row", "flash_attn.seq_row_pk", "decoder"), ("k_fattn_seq_row", "flash_attn.seq_row", "decoder"), ("void k_gemv_q8_0_tiles<20", "mul_mat.gemv_q8_0.vocab", "decoder"),
     ("void k_gemv_q8_0_tiles_norm<20", "norm_mul_mat.gemv_q8_0.vocab", "decoder"),
 ]
@@ -91,7 +91,7 @@ def main() -> int:
         shutil.rmtree(d, ignore_errors=True)
 
     # ---- a decode step launch by launch: durations by position in the step (the steps begin where the token rows are
-    # gathered: the instance of k_gemv_qr_norm_group whose last template argument is true, else k_get_rows_add)
+    # gathered: the instance of k_gemv_norm_group whose last template argument is true, else k_get_rows_add)
     d = out / "trace_positions"
     run(["rocprofv3", "--kernel-trace", "--output-format", "csv", "-d", str(d), "--", *DEC_CMD, "--reps", "1", "--warmup", "1", "--steps", "224"], out / "trace_positions.log", 170)
     rows = []
@@ -102,7 +102,7 @@ def main() -> int:
     rows.sort()
     steps, cur = [], None
     for st, en, name in rows:
-        if "k_get_rows_add" in name or ("k_gemv_qr_norm_group" in name and (", true>" in name or "ELb1EE" in name)):
+        if "k_get_rows_add" in name or ("k_gemv_norm_group" in name and (", true>" in name or "ELb1EE" in name)):
             if cur: steps.append(cur)
             cur = []
         if cur is not None: cur.append((st, en, name))
@@ -163,7 +163,7 @@ def main() -> int:
             d = out / f"sq_{i}"
             run(["rocprofv3", "--pmc", *ctrs.split(), "--output-format", "csv", "-d", str(d), "--", *ENC_CMD, "--reps", "1", "--warmup", "0"], out / f"sq_{i}.log", 120)
             for k, v in per_kernel(d).items():
-                if k.startswith(("k_fattn", "void k_gemm_f16", "void k_norm<5, 1", "_Z6k_normILi5ELi1E")):
+                if k.startswith(("k_fattn", "void k_fattn", "k_gemm_f16", "void k_gemm_f16", "void k_norm<5, 1", "_Z6k_normILi5ELi1E")):
                     for c, (n, s) in v.items():
                         sq[k[:80]][c] = round(s / n)
             shutil.rmtree(d, ignore_errors=True)
