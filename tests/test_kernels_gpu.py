@@ -1093,6 +1093,16 @@ def test_flash_attn_strided_views_like_whisper(pkg, oracle, gpu):
 
 # ------------------------------------------------------------------------------------------------------------------
 
+@pytest.mark.parametrize("ic,iw,s0,p0", [(8, 1, 1, 1), (80, 65, 1, 1), (40, 64, 2, 1), (128, 33, 2, 0), (32, 96, 1, 2), (72, 200, 2, 3)])
+def test_im2col_three_taps(pkg, oracle, gpu, own_numbers, ic, iw, s0, p0):
+    # whole and ragged tiles of 32 positions x 32 channels, padding of none to more than a tap
+    src = rnd((ic, iw))
+    want = oracle.im2col_1d(src, 3, s0, p0, 1)
+    d_o = torch.full((want.shape[0] + 1, 3 * ic), 7.0, dtype=torch.float16, device=gpu.dev)
+    pkg.check(pkg.kernels().mi355x_im2col_1d(pkg.tensor(gpu.up(src), pkg.F32), pkg.tensor(d_o[:-1], pkg.F16), 3, s0, p0, 1, gpu.stream))
+    assert np.array_equal(gpu.down(d_o[:-1], np.uint16), want.view(np.uint16).reshape(-1, 3 * ic)) and torch.all(d_o[-1] == 7.0)
+
+
 def test_norm_and_affine(pkg, oracle, gpu):
     lib = pkg.kernels()
     for shape in [(1500, 1280), (7, 100), (3, 5000), (5, 512)]:
